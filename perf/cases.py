@@ -274,21 +274,22 @@ def _prepare_inkernel(case, seed, state, lib, stream):
 
 
 def _route(case, seed):
-    """Top-k distinct experts per token, the k-th most popular expert with probability ~ k^-1.1; rows grouped on the
-    destination PE by (expert, source PE, token).  Experts are placed at random, again if some PE would get more
-    than twice its share of the copies, which is what a receive buffer holds."""
+    """Top-k distinct experts per token, the k-th most popular expert with probability ~ k^-1.1; the experts are dealt
+    to the PEs in the order of their load, as a planner does that keeps the hottest ones apart: no PE gets more
+    than its share of the copies and the hottest expert's, at most one a token.  Rows are grouped on the
+    destination PE by (expert, source PE, token)."""
     npes, tokens, topk, experts = case["npes"], case["tokens"], case["topk"], case["experts"]
     g = torch.Generator(device="cuda")
     g.manual_seed(seed)
     gumbel = torch.empty(npes * tokens, experts, device="cuda").exponential_(generator=g).log_().neg_()
     popularity = torch.arange(1, experts + 1, device="cuda", dtype=torch.float32).log_().mul_(-1.1)
     chosen = (popularity + gumbel).topk(topk, dim=1).indices.reshape(npes, tokens * topk)
-    while True:
-        expert = torch.randperm(experts, device="cuda", generator=g)[chosen]
-        pe = expert // (experts // npes)
-        rows = torch.bincount(pe.reshape(-1), minlength=npes)
-        if int(rows.max()) <= 2 * tokens * topk:
-            break
+    loads = torch.bincount(chosen.reshape(-1), minlength=experts)
+    rank = torch.empty_like(loads)
+    rank[torch.sort(loads, descending=True, stable=True).indices] = torch.arange(experts, device="cuda")
+    expert = (rank % npes * (experts // npes) + rank // npes)[chosen]
+    pe = expert // (experts // npes)
+    rows = torch.bincount(pe.reshape(-1), minlength=npes)
     source = torch.arange(npes, device="cuda").unsqueeze(1).expand_as(expert)
     order = torch.sort((expert * npes + source).reshape(-1), stable=True).indices
     place = torch.empty_like(order)
@@ -301,7 +302,7 @@ def _route(case, seed):
 def _prepare_moe(case, seed, state, lib, stream):
     npes, tokens, topk, row = case["npes"], case["tokens"], case["topk"], case["row"]
     pe, at, expected = _route(case, seed)
-    copies, cap, sig_stride = tokens * topk, 2 * tokens * topk, 16  # a 128-byte line per signal word
+    copies, cap, sig_stride = tokens * topk, tokens * (topk + npes), 16  # a 128-byte line per signal word
     send, recv, out = (_Memory(lib, n * row) for n in (tokens, cap, copies))
     d_pe, d_row, d_expected, sig = (_Memory(lib, n) for n in (4 * copies, 8 * copies, 8 * npes, 8 * npes * sig_stride))
     _fill([_tensor(send, "bfloat16", (tokens, row // 2))], seed + 1)
