@@ -28,9 +28,6 @@ namespace nvshmem_amd {
 namespace {
 
 // Tunables (compile time).  Defaults are the values measured best on MI355X.
-#ifndef NVSHMEM_AMD_COLL_THREADS
-#define NVSHMEM_AMD_COLL_THREADS 256
-#endif
 #ifndef NVSHMEM_AMD_COPY_THREADS /* threads per block of the segment copy: one wavefront */
 #define NVSHMEM_AMD_COPY_THREADS 64
 #endif
@@ -68,14 +65,14 @@ namespace {
  * the 1M-element reduce, +20..45 % on 256 MiB collectives).  Larger sources are streamed with
  * non-temporal loads (+5 % at 2 GiB).  Stores always stream. */
 
-constexpr int kThreads = NVSHMEM_AMD_COLL_THREADS;
 constexpr int kCopyThreads = NVSHMEM_AMD_COPY_THREADS;
 
+// (any byte alignment: one global_load_dwordx4 either way)
 template <bool NTL>
 __device__ __forceinline__ nvshmemi_v4u stream_load(const char *p) {
     if (NTL && (NVSHMEM_AMD_COLL_NT & 1))
-        return __builtin_nontemporal_load(reinterpret_cast<const nvshmemi_v4u *>(p));
-    return *reinterpret_cast<const nvshmemi_v4u *>(p);
+        return __builtin_nontemporal_load(reinterpret_cast<const nvshmemi_v4u_unaligned *>(p));
+    return *reinterpret_cast<const nvshmemi_v4u_unaligned *>(p);
 }
 // How a kernel's result stores treat the caches.  All three stream (nothing here reads its output back);
 // they differ in where the line waits for memory.  Write-through stores (sc1) leave the L2 at once
@@ -257,11 +254,45 @@ __device__ __forceinline__ T fold_next(int p, T acc, T x) {
     return SCATTER ? nvshmemi_amd_reduce_op<T, OP>(acc, x) : nvshmemi_amd_fold_step<T, OP>(p, acc, x);
 }
 
+// What a reduction moves, the same for every member (the slices lie a multiple of 2 MiB apart, so an offset has the
+// same alignment in all of them): whole vectors from the first 16-byte boundary of the destination on, and the
+// elements in front of and behind them, fewer than 16 bytes on either side.  Stores are aligned that way whatever
+// the buffers are; a source on another offset is read with unaligned vector loads, which cost 3-4 % here (allreduce of
+// 8 x 25 MiB bf16: 73 us with both buffers on the same offset, aligned or not, 76 with different ones; an
+// element per thread and load, which such buffers took before, 155 and 148 us.  reducescatter of 8 x 8 x 3 MB bf16 with
+// blocks of an odd number of elements: 91 -> 42 us; with aligned blocks 39).
+struct reduce_shape_t {
+    uint64_t dst, src;   // byte offsets of the destination and the source in a slice
+    uint64_t nvec;       // whole vectors
+    uint32_t head, tail; // elements in front of and behind them
+    uint32_t lead;       // the first vector's place in its aligned 1 KiB of the destination
+};
+template <typename T>
+reduce_shape_t reduce_shape(const Runtime &rt, uint64_t dst_off, uint64_t src_off, uint64_t nelems) {
+    const uint64_t at = (uint64_t)(uintptr_t)rt.base + dst_off;
+    uint64_t head = (-at & 15) / sizeof(T);
+    if (head > nelems) head = nelems;
+    const uint64_t nvec = (nelems - head) / (16 / sizeof(T));
+    return {dst_off, src_off, nvec, (uint32_t)head, (uint32_t)(nelems - head - nvec * (16 / sizeof(T))),
+            (uint32_t)((at + head * sizeof(T)) >> 4 & 63)};
+}
+// The elements around the vectors, one per thread of the calling block's first wavefront.
+template <typename T, int OP, bool SCATTER>
+__device__ __forceinline__ void reduce_edges(char *dst, const char *src, const reduce_shape_t &s, uint64_t pe_stride,
+                                             int npes, int copies) {
+    if (threadIdx.x >= s.head + s.tail) return;
+    const uint64_t k = threadIdx.x < s.head ? threadIdx.x : s.nvec * (16 / sizeof(T)) + threadIdx.x;
+    const T *from = reinterpret_cast<const T *>(src) + k;
+    const uint64_t es = pe_stride / sizeof(T);
+    T acc = from[0];
+    for (int p = 1; p < npes; ++p) acc = fold_next<T, OP, SCATTER>(p, acc, from[(uint64_t)p * es]);
+    for (int p = 0; p < copies; ++p) reinterpret_cast<T *>(dst + (uint64_t)p * pe_stride)[k] = acc;
+}
+
 template <typename T, int OP, int NPES, bool NTL, int VPT = NVSHMEM_AMD_REDUCE_VPT, int MPW = 1>
 __global__ __launch_bounds__(NPES ? NPES / MPW * 64 : 1024) void reduce_vector_kernel(char *base, uint64_t slice_bytes,
                                                              const nvshmemi_amd_team_view_t *groups,
-                                                             uint64_t dst_off,
-                                                             uint64_t src_off, uint64_t nelems) {
+                                                             reduce_shape_t s) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
     constexpr int VEC = 16 / sizeof(T);
     // this block's team; with NPES > 0 the host has checked that every team has NPES members
@@ -274,17 +305,16 @@ __global__ __launch_bounds__(NPES ? NPES / MPW * 64 : 1024) void reduce_vector_k
     // (the wavefront's index as a scalar: the members' base addresses then stay in scalar registers)
     const unsigned pe0 = (unsigned)__builtin_amdgcn_readfirstlane(threadIdx.x >> lane_shift) * MPW,
                    i = threadIdx.x & (lanes - 1);
-    const uint64_t nvec = nelems / VEC;
+    char *const dst = base + s.dst + s.head * sizeof(T);
+    const char *const src = base + s.src + s.head * sizeof(T);
     // tiles are cut on absolute (16 * lanes)-byte boundaries of the destination, so a wavefront's
     // access is one aligned 1 KiB piece whatever the buffer's own alignment: `lead` vector slots of
     // the first tile lie in front of the buffer
     const uint64_t pe_stride = (uint64_t)g.stride * slice_bytes;  // from one member to the next
     // the block is sized for the largest team of the handle: lanes of members a team does not have idle
     auto member = [&](int m) { return NPES ? true : (int)pe0 + m < npes; };
-    const uint64_t lead = ((uint64_t)(uintptr_t)(base + dst_off) >> 4) & (lanes - 1);
     // a tile is VPT pieces of `lanes` vectors per PE: thread (pe, i) loads vector i of each piece
     constexpr unsigned tile_vecs = (unsigned)VPT << lane_shift;
-    const uint64_t ntiles = (nvec + lead + tile_vecs - 1) / tile_vecs;
     nvshmemi_v4u *stage = reinterpret_cast<nvshmemi_v4u *>(lds);           // [npes][tile_vecs]
     nvshmemi_v4u *result = stage + (size_t)npes * tile_vecs;               // [tile_vecs]
     // the unit of the fold: a 4-byte word (EPW elements) for 1- and 2-byte elements, else one element
@@ -296,83 +326,71 @@ __global__ __launch_bounds__(NPES ? NPES / MPW * 64 : 1024) void reduce_vector_k
     word_t *result_w = reinterpret_cast<word_t *>(result);
     constexpr unsigned tile_words = tile_vecs * VEC / EPW;
 
-    for (uint64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        // indices in front of the buffer wrap to huge values and are skipped like those behind it
-        const uint64_t v0 = tile * tile_vecs + i - lead;
+    // indices in front of the buffer wrap to huge values and are skipped like those behind it
+    const uint64_t v0 = (uint64_t)blockIdx.x * tile_vecs + i - s.lead;
 #pragma unroll
-        for (int u = 0; u < VPT; ++u) {
-            const uint64_t v = v0 + ((uint64_t)u << lane_shift);
-            if (v < nvec) {
+    for (int u = 0; u < VPT; ++u) {
+        const uint64_t v = v0 + ((uint64_t)u << lane_shift);
+        if (v < s.nvec) {
 #pragma unroll
-                for (int m = 0; m < MPW; ++m)
-                    if (member(m)) stage[(pe0 + m) * tile_vecs + ((unsigned)u << lane_shift) + i] =
-                        stream_load<NTL>(base + (uint64_t)(pe0 + m) * pe_stride + src_off + 16 * v);
-            }
-        }
-        __syncthreads();
-        // a thread folds one 4-byte word of the tile at a time - one element of 4 or 8 bytes, or the 2 or 4
-        // narrower elements that share the word, each folded on its own in member order - so that a tile of
-        // 1- or 2-byte elements costs as many LDS instructions as one of 4-byte elements
-        for (unsigned w = threadIdx.x; w < tile_words; w += blockDim.x) {
-            typedef nvshmemi_amd_fold_form<T, OP> form;
-            const word_t first = stage_w[w];
-            typename form::acc_t acc[EPW];
-#pragma unroll
-            for (int j = 0; j < EPW; ++j) acc[j] = form::lift(first.e[j]);
-            if (NPES) {
-#pragma unroll
-                for (int p = 1; p < NPES; ++p) {
-                    const word_t x = stage_w[(size_t)p * tile_words + w];
-#pragma unroll
-                    for (int j = 0; j < EPW; ++j) acc[j] = form::step(p, acc[j], x.e[j]);
-                }
-            } else {
-                // eight members' values fetched from LDS before they are folded, in member order
-                int p = 1;
-                for (; p + 8 <= npes; p += 8) {
-                    word_t x[8];
-#pragma unroll
-                    for (int k = 0; k < 8; ++k) x[k] = stage_w[(size_t)(p + k) * tile_words + w];
-#pragma unroll
-                    for (int k = 0; k < 8; ++k)
-#pragma unroll
-                        for (int j = 0; j < EPW; ++j) acc[j] = form::step(p + k, acc[j], x[k].e[j]);
-                }
-                for (; p < npes; ++p) {
-                    const word_t x = stage_w[(size_t)p * tile_words + w];
-#pragma unroll
-                    for (int j = 0; j < EPW; ++j) acc[j] = form::step(p, acc[j], x.e[j]);
-                }
-            }
-            word_t out;
-#pragma unroll
-            for (int j = 0; j < EPW; ++j) out.e[j] = form::lower(acc[j]);
-            result_w[w] = out;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int u = 0; u < VPT; ++u) {
-            const uint64_t v = v0 + ((uint64_t)u << lane_shift);
-            const nvshmemi_v4u r = result[((unsigned)u << lane_shift) + i];
-            if (v < nvec) {
-#pragma unroll
-                for (int m = 0; m < MPW; ++m)
-                    if (member(m)) stream_store<NVSHMEM_AMD_STORE_REDUCE>(base + (uint64_t)(pe0 + m) * pe_stride + dst_off + 16 * v, r);
-            }
+            for (int m = 0; m < MPW; ++m)
+                if (member(m)) stage[(pe0 + m) * tile_vecs + ((unsigned)u << lane_shift) + i] =
+                    stream_load<NTL>(src + (uint64_t)(pe0 + m) * pe_stride + 16 * v);
         }
     }
-    // elements behind the last full vector
-    const uint64_t done = nvec * VEC;
-    const uint64_t gid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid < nelems - done) {
-        const uint64_t k = done + gid;
-        const T *s = reinterpret_cast<const T *>(base + src_off);
-        T *d = reinterpret_cast<T *>(base + dst_off);
-        const uint64_t es = pe_stride / sizeof(T);
-        T acc = s[k];
-        for (int p = 1; p < npes; ++p) acc = nvshmemi_amd_fold_step<T, OP>(p, acc, s[(uint64_t)p * es + k]);
-        for (int p = 0; p < npes; ++p) d[(uint64_t)p * es + k] = acc;
+    __syncthreads();
+    // a thread folds one 4-byte word of the tile at a time - one element of 4 or 8 bytes, or the 2 or 4
+    // narrower elements that share the word, each folded on its own in member order - so that a tile of
+    // 1- or 2-byte elements costs as many LDS instructions as one of 4-byte elements
+    for (unsigned w = threadIdx.x; w < tile_words; w += blockDim.x) {
+        typedef nvshmemi_amd_fold_form<T, OP> form;
+        const word_t first = stage_w[w];
+        typename form::acc_t acc[EPW];
+#pragma unroll
+        for (int j = 0; j < EPW; ++j) acc[j] = form::lift(first.e[j]);
+        if (NPES) {
+#pragma unroll
+            for (int p = 1; p < NPES; ++p) {
+                const word_t x = stage_w[(size_t)p * tile_words + w];
+#pragma unroll
+                for (int j = 0; j < EPW; ++j) acc[j] = form::step(p, acc[j], x.e[j]);
+            }
+        } else {
+            // eight members' values fetched from LDS before they are folded, in member order
+            int p = 1;
+            for (; p + 8 <= npes; p += 8) {
+                word_t x[8];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) x[k] = stage_w[(size_t)(p + k) * tile_words + w];
+#pragma unroll
+                for (int k = 0; k < 8; ++k)
+#pragma unroll
+                    for (int j = 0; j < EPW; ++j) acc[j] = form::step(p + k, acc[j], x[k].e[j]);
+            }
+            for (; p < npes; ++p) {
+                const word_t x = stage_w[(size_t)p * tile_words + w];
+#pragma unroll
+                for (int j = 0; j < EPW; ++j) acc[j] = form::step(p, acc[j], x.e[j]);
+            }
+        }
+        word_t out;
+#pragma unroll
+        for (int j = 0; j < EPW; ++j) out.e[j] = form::lower(acc[j]);
+        result_w[w] = out;
     }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < VPT; ++u) {
+        const uint64_t v = v0 + ((uint64_t)u << lane_shift);
+        const nvshmemi_v4u r = result[((unsigned)u << lane_shift) + i];
+        if (v < s.nvec) {
+#pragma unroll
+            for (int m = 0; m < MPW; ++m)
+                if (member(m)) stream_store<NVSHMEM_AMD_STORE_REDUCE>(dst + (uint64_t)(pe0 + m) * pe_stride + 16 * v, r);
+        }
+    }
+    if (blockIdx.x == 0)
+        reduce_edges<T, OP, false>(base + s.dst, base + s.src, s, pe_stride, npes, npes);
 }
 
 // Allreduce without LDS, for teams the LDS-staged kernel serves badly (more than 16 members: its block
@@ -384,7 +402,7 @@ __global__ __launch_bounds__(NPES ? NPES / MPW * 64 : 1024) void reduce_vector_k
 template <typename T, int OP, int NPES, bool NTL, bool ROOT_ONLY = false>
 __global__ __launch_bounds__(64) void reduce_gather_kernel(char *base, uint64_t slice_bytes,
                                                            const nvshmemi_amd_team_view_t *groups,
-                                                           uint64_t dst_off, uint64_t src_off, uint64_t nelems) {
+                                                           reduce_shape_t s) {
     constexpr int VEC = 16 / sizeof(T);
     constexpr int kBatch = 8;
     constexpr int kBatches = NPES ? (NPES + kBatch - 1) / kBatch : 1, kStores = NPES ? NPES : 1;  // unroll counts
@@ -396,11 +414,9 @@ __global__ __launch_bounds__(64) void reduce_gather_kernel(char *base, uint64_t 
     const int npes = NPES ? NPES : g.size;
     base += (uint64_t)g.start * slice_bytes;
     const uint64_t pe_stride = (uint64_t)g.stride * slice_bytes;
-    const uint64_t nvec = nelems / VEC;
-    const uint64_t lead = ((uint64_t)(uintptr_t)(base + dst_off) >> 4) & 63;
-    const uint64_t v = (uint64_t)blockIdx.x * 64 + threadIdx.x - lead;
-    if (v < nvec) {
-        const char *src = base + src_off + 16 * v;
+    const uint64_t v = (uint64_t)blockIdx.x * 64 + threadIdx.x - s.lead;
+    if (v < s.nvec) {
+        const char *src = base + s.src + s.head * sizeof(T) + 16 * v;
         pack_t acc;
 #pragma unroll kBatches
         for (int p0 = 0; p0 < npes; p0 += kBatch) {
@@ -420,7 +436,7 @@ __global__ __launch_bounds__(64) void reduce_gather_kernel(char *base, uint64_t 
                     }
                 }
         }
-        char *dst = base + dst_off + 16 * v;
+        char *dst = base + s.dst + s.head * sizeof(T) + 16 * v;
         if (ROOT_ONLY) {
             stream_store<NVSHMEM_AMD_STORE_REDUCESCATTER>(dst, acc.v);
         } else {
@@ -428,18 +444,8 @@ __global__ __launch_bounds__(64) void reduce_gather_kernel(char *base, uint64_t 
             for (int p = 0; p < npes; ++p) stream_store<NVSHMEM_AMD_STORE_REDUCE>(dst + (uint64_t)p * pe_stride, acc.v);
         }
     }
-    // elements behind the last full vector
-    const uint64_t done = nvec * VEC;
-    const uint64_t gid = (uint64_t)blockIdx.x * 64 + threadIdx.x;
-    if (gid < nelems - done) {
-        const uint64_t k = done + gid;
-        const T *s = reinterpret_cast<const T *>(base + src_off);
-        T *d = reinterpret_cast<T *>(base + dst_off);
-        const uint64_t es = pe_stride / sizeof(T);
-        T acc = s[k];
-        for (int p = 1; p < npes; ++p) acc = nvshmemi_amd_fold_step<T, OP>(p, acc, s[(uint64_t)p * es + k]);
-        for (int p = 0; p < (ROOT_ONLY ? 1 : npes); ++p) d[(uint64_t)p * es + k] = acc;
-    }
+    if (blockIdx.x == 0)
+        reduce_edges<T, OP, false>(base + s.dst, base + s.src, s, pe_stride, npes, ROOT_ONLY ? 1 : npes);
 }
 
 // reducescatter without LDS: a block is ONE wavefront, lane i loads vector i of a 1 KiB piece of block q
@@ -451,8 +457,7 @@ __global__ __launch_bounds__(64) void reduce_gather_kernel(char *base, uint64_t 
 template <typename T, int OP, int NPES, bool NTL>
 __global__ __launch_bounds__(64) void reducescatter_gather_kernel(char *base, uint64_t slice_bytes,
                                                                   const nvshmemi_amd_team_view_t *groups,
-                                                                  uint64_t dst_off, uint64_t src_off,
-                                                                  uint64_t nelems) {
+                                                                  reduce_shape_t s, uint64_t block_bytes) {
     constexpr int VEC = 16 / sizeof(T);
     constexpr int kBatch = 8;  // loads in flight per lane
     union pack_t {
@@ -464,13 +469,16 @@ __global__ __launch_bounds__(64) void reducescatter_gather_kernel(char *base, ui
     if ((int)blockIdx.y >= npes) return;
     base += (uint64_t)g.start * slice_bytes;
     const uint64_t pe_stride = (uint64_t)g.stride * slice_bytes;
-    const uint64_t nvec = nelems / VEC;
-    src_off += (uint64_t)blockIdx.y * nelems * sizeof(T);
-    // pieces are cut on absolute 1 KiB boundaries of the source: `lead` slots of piece 0 lie in front
-    const uint64_t lead = ((uint64_t)(uintptr_t)(base + src_off) >> 4) & 63;
+    const char *const block = base + s.src + (uint64_t)blockIdx.y * block_bytes;
+    char *const dst = base + (uint64_t)blockIdx.y * pe_stride + s.dst;
+    if (blockIdx.x == 0) reduce_edges<T, OP, true>(dst, block, s, pe_stride, npes, 1);
+    // pieces are cut on absolute 1 KiB boundaries of the source (up to the last 15 bytes, where it lies on another
+    // offset than the destination): `lead` slots of piece 0 lie in front
+    const char *const body = block + s.head * sizeof(T);
+    const uint64_t lead = ((uint64_t)(uintptr_t)body >> 4) & 63;
     const uint64_t v = (uint64_t)blockIdx.x * 64 + threadIdx.x - lead;
-    if (v >= nvec) return;  // also the slots in front of the block (wrapped)
-    const char *src = base + src_off + 16 * v;
+    if (v >= s.nvec) return;  // also the slots in front of the block (wrapped)
+    const char *src = body + 16 * v;
     pack_t acc;
     for (int p0 = 0; p0 < npes; p0 += kBatch) {
         pack_t x[kBatch];
@@ -488,29 +496,7 @@ __global__ __launch_bounds__(64) void reducescatter_gather_kernel(char *base, ui
                 }
             }
     }
-    stream_store<NVSHMEM_AMD_STORE_REDUCESCATTER>(base + (uint64_t)blockIdx.y * pe_stride + dst_off + 16 * v, acc.v);
-}
-
-// Element-at-a-time variant for buffers that are not 16-byte aligned.
-template <typename T, int OP, bool SCATTER = false>
-__global__ __launch_bounds__(kThreads) void reduce_scalar_kernel(char *base, uint64_t slice_bytes,
-                                                                 const nvshmemi_amd_team_view_t *groups,
-                                                                 uint64_t dst_off, uint64_t src_off,
-                                                                 uint64_t nelems) {
-    const nvshmemi_amd_team_view_t g = groups[blockIdx.z];
-    const int npes = g.size;
-    if (SCATTER && (int)blockIdx.y >= npes) return;
-    base += (uint64_t)g.start * slice_bytes;
-    const uint64_t gsz = (uint64_t)gridDim.x * kThreads;
-    const uint64_t es = ((uint64_t)g.stride * slice_bytes) / sizeof(T);
-    const T *s = reinterpret_cast<const T *>(base + src_off) + (SCATTER ? (uint64_t)blockIdx.y * nelems : 0);
-    T *d = reinterpret_cast<T *>(base + dst_off) + (SCATTER ? (uint64_t)blockIdx.y * es : 0);
-    for (uint64_t i = (uint64_t)blockIdx.x * kThreads + threadIdx.x; i < nelems; i += gsz) {
-        T acc = s[i];
-        for (int pe = 1; pe < npes; ++pe) acc = fold_next<T, OP, SCATTER>(pe, acc, s[(uint64_t)pe * es + i]);
-        if (SCATTER) d[i] = acc;
-        else for (int pe = 0; pe < npes; ++pe) d[(uint64_t)pe * es + i] = acc;
-    }
+    stream_store<NVSHMEM_AMD_STORE_REDUCESCATTER>(dst + s.head * sizeof(T) + 16 * v, acc.v);
 }
 
 #ifndef NVSHMEM_AMD_STORE_FCOLLECT_CHUNKED
@@ -594,9 +580,10 @@ static int launch_broadcast(Runtime &rt, const TeamLaunch &tl, uint64_t doff, ui
 template <typename T, int OP>
 void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t src_off,
                    uint64_t nelems, hipStream_t stream) {
-    const bool vector_ok = ((dst_off | src_off) & 15) == 0;
     const unsigned ngroups = (unsigned)tl.ngroups;
-    // Which vector kernel.  From Runtime::lds_reduce_bytes of sources in all (64 MiB; a quarter
+    const reduce_shape_t shape = reduce_shape<T>(rt, dst_off, src_off, nelems);
+    const uint64_t nvec = shape.nvec;
+    // Which kernel.  From Runtime::lds_reduce_bytes of sources in all (64 MiB; a quarter
     // of that for teams of 17 to 32 members, four times for larger ones) the LDS-staged
     // kernel wins for every team of 3 to 64 members; below that, and for 2 members, the gather kernel does.
     // fp32 sum on a stream, LDS-staged / gather in TB/s, sources of 32 MiB | 64 MiB | 128 MiB in all: 4 members
@@ -634,27 +621,25 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
     // 32: 6.09 / 6.09 and 6.09 / 6.51, 48: 5.68 / 5.78 and 5.57 / 6.25, 64: 5.55 / 5.97 and 5.59 / 6.56.  So: from
     // Runtime::two_step_reduce_members (16) members on when the sources hold two_step_reduce_bytes (512 MiB: 16 members 6.2 against 6.0 TB/s fused there, 32 members 6.3 against 5.8) or more,
     // and from three times that many members whatever the size.
-    if (vector_ok && rt.two_step_reduce_members && tl.min_size >= (int)rt.two_step_reduce_members &&
+    if (rt.two_step_reduce_members && tl.min_size >= (int)rt.two_step_reduce_members &&
         (total_bytes >= rt.two_step_reduce_bytes || tl.min_size >= 3 * (int)rt.two_step_reduce_members) &&
         total_bytes >= lds_from_bytes) {
-        const uint64_t nvec = nelems / (16 / sizeof(T));
         uint64_t blocks = (nvec + 63 + 63) / 64;
         if (blocks <= 0x7fffffffull) {
             const dim3 grid((unsigned)blocks, 1, ngroups);
             if (stream_source)
                 hipLaunchKernelGGL((reduce_gather_kernel<T, OP, 0, true, true>), grid, dim3(64), 0, stream, rt.base,
-                                   rt.heap_size, tl.groups, dst_off, src_off, nelems);
+                                   rt.heap_size, tl.groups, shape);
             else
                 hipLaunchKernelGGL((reduce_gather_kernel<T, OP, 0, false, true>), grid, dim3(64), 0, stream, rt.base,
-                                   rt.heap_size, tl.groups, dst_off, src_off, nelems);
+                                   rt.heap_size, tl.groups, shape);
             (void)launch_broadcast(rt, tl, dst_off, dst_off, nelems * sizeof(T), 0, stream, true);
             return;
         }
     }
-    if (vector_ok && mpw && total_bytes >= lds_from_bytes) {
+    if (mpw && total_bytes >= lds_from_bytes) {
         const uint32_t lane_shift = 6;
         const unsigned threads = (unsigned)((tl.max_size + mpw - 1) / mpw) << lane_shift;
-        const uint64_t nvec = nelems / (16 / sizeof(T));
         // A tile of two vectors per thread halves the barriers per byte: worth 5 % for 16-bit elements with one
         // member per wavefront (bf16 sum at 8 x 128 MiB 5.83 -> 6.14 TB/s), less than the two members per
         // wavefront they now use with one vector; it costs 4-byte and 8-byte elements 3-4 %.
@@ -662,7 +647,10 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
         const int vpt = (ct_size == 8 || ct_size == 16) ? kVptNarrow : NVSHMEM_AMD_REDUCE_VPT;
         const uint64_t tile_vecs = (uint64_t)vpt << lane_shift;
         uint64_t blocks = (nvec + (1u << lane_shift) + tile_vecs - 1) / tile_vecs;  // room for the lead-in
-        if (blocks > 0x7fffffffull) blocks = 0x7fffffffull;  // the tile loop covers the rest
+        if (blocks > 0x7fffffffull) {
+            set_error("reduce: message too large");
+            return;
+        }
         const size_t lds = ((size_t)tl.max_size + 1) * 16 * tile_vecs;
         const dim3 grid((unsigned)blocks, 1, ngroups);
 #define NVSHMEM_AMD_LAUNCH_REDUCE(N, MPW) NVSHMEM_AMD_LAUNCH_REDUCE_V(N, MPW, NVSHMEM_AMD_REDUCE_VPT)
@@ -670,12 +658,10 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
     do {                                                                                          \
         if (stream_source)                                                                        \
             hipLaunchKernelGGL((reduce_vector_kernel<T, OP, N, true, VPT, MPW>), grid, dim3(threads), lds,  \
-                               stream, rt.base, rt.heap_size, tl.groups, dst_off,    \
-                               src_off, nelems);                                                  \
+                               stream, rt.base, rt.heap_size, tl.groups, shape);                                                  \
         else                                                                                      \
             hipLaunchKernelGGL((reduce_vector_kernel<T, OP, N, false, VPT, MPW>), grid, dim3(threads), lds, \
-                               stream, rt.base, rt.heap_size, tl.groups, dst_off,    \
-                               src_off, nelems);                                                  \
+                               stream, rt.base, rt.heap_size, tl.groups, shape);                                                  \
     } while (0)
         if (ct_size == 8) NVSHMEM_AMD_LAUNCH_REDUCE_V(8, kNarrowMpw, kVptNarrow);
         else if (ct_size == 16) NVSHMEM_AMD_LAUNCH_REDUCE_V(16, kNarrowMpw, kVptNarrow);
@@ -684,9 +670,8 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
         else NVSHMEM_AMD_LAUNCH_REDUCE(0, 4);
 #undef NVSHMEM_AMD_LAUNCH_REDUCE
 #undef NVSHMEM_AMD_LAUNCH_REDUCE_V
-    } else if (vector_ok) {
-        const uint64_t nvec = nelems / (16 / sizeof(T));
-        uint64_t blocks = (nvec + 63 + 63) / 64;  // room for the lead-in; at least one block for the tail
+    } else {
+        uint64_t blocks = (nvec + 63 + 63) / 64;  // room for the lead-in; at least one block for the edges
         if (blocks > 0x7fffffffull) {
             set_error("reduce: message too large");
             return;
@@ -696,23 +681,16 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
     do {                                                                                               \
         if (stream_source)                                                                             \
             hipLaunchKernelGGL((reduce_gather_kernel<T, OP, N, true>), grid, dim3(64), 0, stream, rt.base, \
-                               rt.heap_size, tl.groups, dst_off, src_off, nelems);                    \
+                               rt.heap_size, tl.groups, shape);                    \
         else                                                                                           \
             hipLaunchKernelGGL((reduce_gather_kernel<T, OP, N, false>), grid, dim3(64), 0, stream, rt.base, \
-                               rt.heap_size, tl.groups, dst_off, src_off, nelems);                    \
+                               rt.heap_size, tl.groups, shape);                    \
     } while (0)
         // (sixteen members unrolled measured slower than the loop: 5.2 against 5.4 TB/s)
         if (fixed_size == 4) NVSHMEM_AMD_LAUNCH_GATHER_REDUCE(4);
         else if (fixed_size == 8) NVSHMEM_AMD_LAUNCH_GATHER_REDUCE(8);
         else NVSHMEM_AMD_LAUNCH_GATHER_REDUCE(0);
 #undef NVSHMEM_AMD_LAUNCH_GATHER_REDUCE
-    } else {
-        uint64_t blocks = (nelems + kThreads - 1) / kThreads;
-        const uint64_t cap = (uint64_t)rt.num_cus * 64 / ngroups + 1;
-        if (blocks > cap) blocks = cap;
-        hipLaunchKernelGGL((reduce_scalar_kernel<T, OP>), dim3((unsigned)blocks, 1, ngroups),
-                           dim3(kThreads), 0, stream, rt.base, rt.heap_size, tl.groups, dst_off,
-                           src_off, nelems);
     }
 }
 
@@ -720,37 +698,25 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
 template <typename T, int OP>
 void launch_reducescatter(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t src_off,
                           uint64_t nelems, hipStream_t stream) {
-    const bool vector_ok = ((dst_off | src_off | (nelems * sizeof(T))) & 15) == 0;
-    const unsigned ngroups = (unsigned)tl.ngroups;
-    if (vector_ok) {
-        const uint64_t nvec = nelems / (16 / sizeof(T));
-        uint64_t blocks = (nvec + 63 + 63) / 64;  // room for the lead-in
-        if (blocks > 0x7fffffffull) {
-            set_error("reducescatter: message too large");
-            return;
-        }
-        const dim3 grid((unsigned)blocks, (unsigned)tl.max_size, ngroups);
-        const bool stream_source =
-            total_members(tl) * tl.max_size * nelems * sizeof(T) > rt.cacheable_source_bytes;
+    const reduce_shape_t shape = reduce_shape<T>(rt, dst_off, src_off, nelems);
+    const uint64_t blocks = (shape.nvec + 63 + 63) / 64;  // room for the lead-in; at least one block for the edges
+    if (blocks > 0x7fffffffull) {
+        set_error("reducescatter: message too large");
+        return;
+    }
+    const dim3 grid((unsigned)blocks, (unsigned)tl.max_size, (unsigned)tl.ngroups);
+    const bool stream_source = total_members(tl) * tl.max_size * nelems * sizeof(T) > rt.cacheable_source_bytes;
 #define NVSHMEM_AMD_LAUNCH_GATHER(N, NTL)                                                         \
     hipLaunchKernelGGL((reducescatter_gather_kernel<T, OP, N, NTL>), grid, dim3(64), 0, stream,   \
-                       rt.base, rt.heap_size, tl.groups, dst_off, src_off, nelems)
-        if (tl.min_size == 8 && tl.max_size == 8) {
-            if (stream_source) NVSHMEM_AMD_LAUNCH_GATHER(8, true);
-            else NVSHMEM_AMD_LAUNCH_GATHER(8, false);
-        } else {
-            if (stream_source) NVSHMEM_AMD_LAUNCH_GATHER(0, true);
-            else NVSHMEM_AMD_LAUNCH_GATHER(0, false);
-        }
-#undef NVSHMEM_AMD_LAUNCH_GATHER
+                       rt.base, rt.heap_size, tl.groups, shape, nelems * sizeof(T))
+    if (tl.min_size == 8 && tl.max_size == 8) {
+        if (stream_source) NVSHMEM_AMD_LAUNCH_GATHER(8, true);
+        else NVSHMEM_AMD_LAUNCH_GATHER(8, false);
     } else {
-        uint64_t blocks = (nelems + kThreads - 1) / kThreads;
-        const uint64_t cap = (uint64_t)rt.num_cus * 64 / ((uint64_t)tl.max_size * ngroups) + 1;
-        if (blocks > cap) blocks = cap;
-        hipLaunchKernelGGL((reduce_scalar_kernel<T, OP, true>),
-                           dim3((unsigned)blocks, (unsigned)tl.max_size, ngroups), dim3(kThreads), 0,
-                           stream, rt.base, rt.heap_size, tl.groups, dst_off, src_off, nelems);
+        if (stream_source) NVSHMEM_AMD_LAUNCH_GATHER(0, true);
+        else NVSHMEM_AMD_LAUNCH_GATHER(0, false);
     }
+#undef NVSHMEM_AMD_LAUNCH_GATHER
 }
 
 typedef void (*reduce_launcher_t)(Runtime &, const TeamLaunch &, uint64_t, uint64_t, uint64_t,
