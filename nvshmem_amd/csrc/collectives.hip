@@ -28,15 +28,6 @@ namespace nvshmem_amd {
 namespace {
 
 // Tunables (compile time).  Defaults are the values measured best on MI355X.
-#ifndef NVSHMEM_AMD_COPY_THREADS /* threads per block of the segment copy: one wavefront */
-#define NVSHMEM_AMD_COPY_THREADS 64
-#endif
-#ifndef NVSHMEM_AMD_ALLTOALL_UNROLL /* vectors per lane in an alltoall tile */
-#define NVSHMEM_AMD_ALLTOALL_UNROLL 1
-#endif
-#ifndef NVSHMEM_AMD_FCOLLECT_UNROLL /* vectors per lane in an fcollect tile */
-#define NVSHMEM_AMD_FCOLLECT_UNROLL 1
-#endif
 #ifndef NVSHMEM_AMD_REDUCE_VPT /* vectors a thread of the fused reduce loads per tile */
 #define NVSHMEM_AMD_REDUCE_VPT 1
 #endif
@@ -65,7 +56,6 @@ namespace {
  * the 1M-element reduce, +20..45 % on 256 MiB collectives).  Larger sources are streamed with
  * non-temporal loads (+5 % at 2 GiB).  Stores always stream. */
 
-constexpr int kCopyThreads = NVSHMEM_AMD_COPY_THREADS;
 
 // (any byte alignment: one global_load_dwordx4 either way)
 template <bool NTL>
@@ -95,6 +85,17 @@ enum { kStoreStream = 0 /* nt */, kStoreThrough = 1 /* sc1 */, kStoreThroughStre
 #ifndef NVSHMEM_AMD_STORE_REDUCESCATTER
 #define NVSHMEM_AMD_STORE_REDUCESCATTER kStoreThrough
 #endif
+// The team a block serves: among the kernel's arguments when the handle names one team, else row `group` of the
+// device's team table (which costs a load that everything else waits for).
+struct team_arg_t {
+    nvshmemi_amd_team_view_t one;
+    const nvshmemi_amd_team_view_t *table;  // null: one
+};
+static team_arg_t team_arg(const TeamLaunch &tl) { return {tl.first, tl.ngroups > 1 ? tl.groups : nullptr}; }
+__device__ __forceinline__ nvshmemi_amd_team_view_t team_of(const team_arg_t &t, unsigned group) {
+    return t.table ? t.table[group] : t.one;
+}
+
 // The asm forms end in s_nop 1: the compiler does not know the statement is a store of more than 8 bytes
 // and would not keep the wait state this GPU needs before the data registers are written again.
 template <int STORE>
@@ -108,130 +109,127 @@ __device__ __forceinline__ void stream_store(char *p, nvshmemi_v4u v) {
     else
         *reinterpret_cast<nvshmemi_v4u *>(p) = v;
 }
+// The same at p + off, p the same for all lanes: the address stays a scalar base and a 32-bit offset per lane.  (The
+// s_nop in front: a vector instruction that wrote the base - the compiler may have moved it out of a vector
+// register - must be five wait states away.)
+template <int STORE>
+__device__ __forceinline__ void stream_store_at(char *p, unsigned off, nvshmemi_v4u v) {
+    if (STORE == kStoreThrough)
+        asm volatile("s_nop 4\n\tglobal_store_dwordx4 %0, %1, %2 sc1\n\ts_nop 1" : : "v"(off), "v"(v), "s"(p) : "memory");
+    else if (STORE == kStoreThroughStream)
+        asm volatile("s_nop 4\n\tglobal_store_dwordx4 %0, %1, %2 sc1 nt\n\ts_nop 1" : : "v"(off), "v"(v), "s"(p) : "memory");
+    else
+        stream_store<STORE>(p + off, v);
+}
 
 // ---------------------------------------------------------------------------------------------
-// Segment copy: fcollect and alltoall are sets of contiguous (source, destination) segments.
-// grid.y indexes the segment, grid.x the tile inside it.  A block is ONE wavefront that moves ONE
-// aligned 1 KiB piece (64 lanes x 16 bytes): on MI355X this shape measured fastest by a clear
+// Segment copy: fcollect and alltoall are sets of contiguous (source, destination) segments, a broadcast is one.
+// grid.y (alltoall: grid.y and grid.z) indexes the segment, grid.x the tile inside it.  A block is ONE wavefront that
+// moves ONE aligned 1 KiB piece (64 lanes x 16 bytes): on MI355X this shape measured fastest by a clear
 // margin (6.7-6.8 TB/s for alltoall, against 6.0 TB/s with 256-thread blocks and 8 KiB tiles and
 // 4.0 TB/s with 32 KiB tiles), because the blocks in flight then cover a narrow, moving window of
 // addresses.  The destination is written with aligned vectors only: block 0 of a segment copies
 // the byte head in front of the first aligned destination vector and the byte tail behind the
 // last one.
+//
+// fcollect and broadcast store the piece to every member, in one of two ways:
+//  - back to back, while the whole grid is in flight at once.  Small messages are latency: with the stores of a loop
+//    that waits for each before the next, every destination costs a quarter of a microsecond (16 B to 64 KiB per
+//    member, replayed from a graph: fcollect to 8 / 16 members 3.8 / 5.5 us one by one, 1.8 / 2.1 back to back,
+//    broadcast to 8 3.7 and 1.7);
+//  - PACED, one destination after the other, each store acknowledged before the next is issued, in larger grids.
+//    They are bound by how the memory system takes writes, and that favours few write fronts: blocks that start
+//    together then write to one destination at a time instead of all 8 or 16 (broadcast of 32 MiB to 8: 47.4 us back
+//    to back, 42.8 paced), and the fewer wavefronts take part, the narrower each front.  So the launch also limits
+//    how many a compute unit holds (paced_lds_bytes).
 // ---------------------------------------------------------------------------------------------
 
 enum { kModeFcollect = 0, kModeAlltoall = 1, kModeBroadcast = 2 };
 
-// Copies the vectors v0 + t + u*kCopyThreads (u < unroll) that fall inside [0, nvec); indices in front of
-// the segment wrap to huge unsigned values and are skipped the same way as those behind it.
-template <bool SRC_ALIGNED, bool REPLICATE, int kCopyUnroll, bool NTL, int STORE>
-__device__ __forceinline__ void copy_tile(char *__restrict__ dst, const char *__restrict__ src,
-                                          uint64_t v0, uint64_t nvec, uint64_t rep_stride, int r0,
-                                          int r1) {
-    nvshmemi_v4u v[kCopyUnroll];
-#pragma unroll
-    for (int u = 0; u < kCopyUnroll; ++u) {
-        const uint64_t i = v0 + threadIdx.x + (uint64_t)u * kCopyThreads;
-        if (i < nvec) v[u] = SRC_ALIGNED ? stream_load<NTL>(src + 16 * i) : nvshmemi_amd_load16<false>(src + 16 * i);
-    }
-    if (REPLICATE) {
-        for (int r = r0; r < r1; ++r) {
-            char *d = dst + (uint64_t)r * rep_stride;
-#pragma unroll
-            for (int u = 0; u < kCopyUnroll; ++u) {
-                const uint64_t i = v0 + threadIdx.x + (uint64_t)u * kCopyThreads;
-                if (i < nvec) stream_store<STORE>(d + 16 * i, v[u]);
-            }
-        }
-    } else {
-#pragma unroll
-        for (int u = 0; u < kCopyUnroll; ++u) {
-            const uint64_t i = v0 + threadIdx.x + (uint64_t)u * kCopyThreads;
-            if (i < nvec) stream_store<STORE>(dst + 16 * i, v[u]);
-        }
-    }
-}
+struct segment_args_t {
+    char *base;
+    uint64_t slice_bytes;
+    team_arg_t team;
+    uint64_t dst_off, src_off, seg_bytes;
+    uint32_t root;
+};
 
-template <int MODE, int kCopyUnroll, bool NTL, int STORE>
-__global__ __launch_bounds__(kCopyThreads) void segment_copy_kernel(char *base, uint64_t slice_bytes,
-                                                                const nvshmemi_amd_team_view_t *groups,
-                                                                int max_size, uint64_t dst_off,
-                                                                uint64_t src_off, uint64_t seg_bytes,
-                                                                int root, uint32_t part_shift, uint32_t chunk_shift) {
+template <int MODE, bool NTL, bool PACED, int STORE>
+__global__ __launch_bounds__(64) void segment_copy_kernel(segment_args_t a) {
     // this block's team: members are the PEs start + i*stride, i < size
-    const nvshmemi_amd_team_view_t g = groups[blockIdx.z];
+    unsigned p = MODE == kModeAlltoall ? blockIdx.z : blockIdx.y, group = MODE == kModeAlltoall ? 0 : blockIdx.z;
+    if (MODE == kModeAlltoall && a.team.table) {
+        group = p / gridDim.y;
+        p -= group * gridDim.y;
+    }
+    const nvshmemi_amd_team_view_t g = team_of(a.team, group);
     const unsigned npes = (unsigned)g.size;
-    base += (uint64_t)g.start * slice_bytes;
-    const uint64_t rep_stride = (uint64_t)g.stride * slice_bytes;  // from one member to the next
-    const unsigned seg = blockIdx.y;
+    char *const base = a.base + (uint64_t)(unsigned)g.start * a.slice_bytes;
+    const uint64_t rep_stride = (uint64_t)(unsigned)g.stride * a.slice_bytes;  // from one member to the next
     const char *src;
     char *dst;
-    int nrep;
+    unsigned nrep = npes;
     if (MODE == kModeFcollect) {
         // segment p: member p's source -> slot p of every member's destination
-        if (seg >= npes) return;
-        src = base + seg * rep_stride + src_off;
-        dst = base + dst_off + (uint64_t)seg * seg_bytes;
-        nrep = (int)npes;
+        if (p >= npes) return;
+        src = base + p * rep_stride + a.src_off;
+        dst = base + a.dst_off + p * a.seg_bytes;
     } else if (MODE == kModeBroadcast) {
         // one segment: the root's source -> every member's destination
-        src = base + (uint64_t)root * rep_stride + src_off;
-        dst = base + dst_off;
-        nrep = (int)npes;
+        src = base + a.root * rep_stride + a.src_off;
+        dst = base + a.dst_off;
     } else {
         // segment (p, q): block q of member p's source -> slot p of member q's destination
-        const unsigned p = seg / (unsigned)max_size, q = seg % (unsigned)max_size;
+        const unsigned q = blockIdx.y;
         if (p >= npes || q >= npes) return;
-        src = base + p * rep_stride + src_off + (uint64_t)q * seg_bytes;
-        dst = base + q * rep_stride + dst_off + (uint64_t)p * seg_bytes;
+        src = base + p * rep_stride + a.src_off + q * a.seg_bytes;
+        dst = base + q * rep_stride + a.dst_off + p * a.seg_bytes;
         nrep = 1;
     }
-
-    uint64_t head = (uint64_t)(-(uintptr_t)dst & 15);
-    if (head > seg_bytes) head = seg_bytes;
-    const uint64_t nvec_total = (seg_bytes - head) / 16;
-    const uint64_t tail_start = head + nvec_total * 16;
-
+    const unsigned lane = threadIdx.x;
+    unsigned head = (unsigned)(-(uintptr_t)dst) & 15;
+    if (head > a.seg_bytes) head = (unsigned)a.seg_bytes;
+    const uint64_t nvec = (a.seg_bytes - head) / 16;
     if (blockIdx.x == 0) {
-        // at most 15 + 15 bytes per replica
-        const uint64_t edge = head + (seg_bytes - tail_start);
-        for (uint64_t e = threadIdx.x; e < edge * (uint64_t)nrep; e += kCopyThreads) {
-            const uint64_t r = e / edge, k = e % edge;
-            const uint64_t pos = k < head ? k : tail_start + (k - head);
-            dst[r * rep_stride + pos] = src[pos];
+        // at most 15 + 15 bytes, lane k the k-th of them, every second destination on either half of the lanes
+        const unsigned edge = head + ((unsigned)(a.seg_bytes - head) & 15), k = lane & 31;
+        if (k < edge) {
+            const uint64_t pos = k < head ? k : nvec * 16 + k;
+            const char b = src[pos];
+            for (unsigned r = lane >> 5; r < nrep; r += 2) dst[r * rep_stride + pos] = b;
         }
     }
     // tiles are cut on absolute 1 KiB boundaries of the destination: `lead` vector slots of tile 0
     // lie in front of the segment
-    const uint64_t lead = ((uint64_t)(uintptr_t)(dst + head) >> 4) & 63;
-    constexpr uint64_t kTileVectors = (uint64_t)kCopyThreads * kCopyUnroll;
-    // fcollect / broadcast with part_shift > 0: 2^part_shift blocks share a tile and split its destinations.  The
-    // sharers of a tile are 2^chunk_shift blocks apart: the grid walks a chunk of 2^chunk_shift tiles once per
-    // group of destinations, so the blocks in flight write to few destinations at a time, each a run of
-    // consecutive pieces, and re-read the chunk from the L2 of the XCD that fetched it (sharers are a multiple of
-    // 8 blocks apart).  The host passes both shifts as zero or both as non-zero.
-    uint64_t tile_index = blockIdx.x;
-    unsigned part_index = 0;
-    if (chunk_shift) {
-        part_index = (blockIdx.x >> chunk_shift) & ((1u << part_shift) - 1);
-        tile_index = (blockIdx.x & ((1u << chunk_shift) - 1)) +
-                     (((uint64_t)blockIdx.x >> (chunk_shift + part_shift)) << chunk_shift);
-    }
-    const uint64_t v0 = tile_index * kTileVectors - lead;
-    if ((int64_t)v0 >= (int64_t)nvec_total) return;
-    const char *s = src + head;
-    char *d = dst + head;
-    const bool aligned = (((uintptr_t)s) & 15) == 0;
-    if (MODE != kModeAlltoall) {
-        const int per = (nrep + (1 << part_shift) - 1) >> part_shift;
-        const int r0 = (int)part_index * per;
-        const int r1 = r0 + per < nrep ? r0 + per : nrep;
-        if (r0 >= nrep) return;  // a team smaller than the grid's largest: nothing left for this sharer
-        if (aligned) copy_tile<true, true, kCopyUnroll, NTL, STORE>(d, s, v0, nvec_total, rep_stride, r0, r1);
-        else copy_tile<false, true, kCopyUnroll, NTL, STORE>(d, s, v0, nvec_total, rep_stride, r0, r1);
+    const unsigned lead = (unsigned)((uintptr_t)(dst + head) >> 4) & 63;
+    const int64_t v0 = (int64_t)blockIdx.x * 64 - lead, left = (int64_t)nvec - v0;
+    if (left <= 0) return;
+    // this lane's vector, as an unsigned index: slots in front of the segment wrap and are skipped like those behind it
+    const unsigned first = blockIdx.x == 0 ? lead : 0, end = left < 64 ? (unsigned)left : 64;
+    if (lane - first >= end - first) return;
+    const nvshmemi_v4u v = stream_load<NTL>(src + head + 16 * v0 + 16 * lane);
+    char *d = dst + head + 16 * v0;
+    auto store = [&](char *to) { stream_store_at<STORE>(to, 16 * lane, v); };
+    if (MODE == kModeAlltoall) {
+        store(d);
+    } else if (PACED) {
+        store(d);
+        while (--nrep) {
+            d += rep_stride;
+            nvshmemi_amd_wait_vm();
+            store(d);
+        }
     } else {
-        if (aligned) copy_tile<true, false, kCopyUnroll, NTL, STORE>(d, s, v0, nvec_total, rep_stride, 0, 1);
-        else copy_tile<false, false, kCopyUnroll, NTL, STORE>(d, s, v0, nvec_total, rep_stride, 0, 1);
+        for (; nrep >= 8; nrep -= 8, d += 8 * rep_stride) {
+#pragma unroll
+            for (int r = 0; r < 8; ++r) store(d + r * rep_stride);
+        }
+        if (nrep >= 4) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) store(d + r * rep_stride);
+            nrep -= 4, d += 4 * rep_stride;
+        }
+        for (; nrep; --nrep, d += rep_stride) store(d);
     }
 }
 
@@ -499,43 +497,8 @@ __global__ __launch_bounds__(64) void reducescatter_gather_kernel(char *base, ui
     stream_store<NVSHMEM_AMD_STORE_REDUCESCATTER>(dst + s.head * sizeof(T) + 16 * v, acc.v);
 }
 
-#ifndef NVSHMEM_AMD_STORE_FCOLLECT_CHUNKED
-#define NVSHMEM_AMD_STORE_FCOLLECT_CHUNKED kStoreThroughStream /* +2 % over nt */
-#endif
-#ifndef NVSHMEM_AMD_STORE_BROADCAST_CHUNKED
-#define NVSHMEM_AMD_STORE_BROADCAST_CHUNKED kStoreStream /* +2.5 % over sc1 nt */
-#endif
-
-// Chunked sharing, the form fcollect and broadcast of sources beyond the Infinity Cache take: a wavefront stores
-// its piece to two destinations, and the grid walks a chunk of tiles once per pair of destinations before it moves
-// on (segment_copy_kernel, chunk_shift).  A write-dominated kernel is bound by how the memory system takes its
-// writes, and that favours few write fronts: a write-only stream runs at 6.9 TB/s as ONE front sweeping memory,
-// 5.7-6.2 as 64 fronts, 4.6-5.3 as 256.  With every block storing to all 8 or 16 destinations the blocks in flight
-// feed 8 or 16 fronts of a few KiB each; chunked, they feed a few fronts of 2-4 MiB.  Measured (random data, 16 x
-// 32 MiB fcollect / 512 MiB broadcast to 8): fcollect 5.85 -> 6.30 TB/s, broadcast 6.07 -> 6.48; the chunk that
-// measured best makes chunk x groups = 16384 blocks, twice what the GPU holds at a time (fcollect: 2^11 tiles x
-// 8 pairs; broadcast: 2^12 x 4; half or double that chunk loses 1-12 %), one destination per wavefront 20 %.
-// Forms with at most four destinations per wavefront whose sharers are neighbouring blocks, or the wavefronts of
-// one block, measured 5.85 / 6.03 TB/s on the same two workloads.  Cache-resident sources keep one wavefront per
-// piece storing to every member: a split costs them up to 9 %.
-#ifndef NVSHMEM_AMD_CHUNKED_REPLICAS_PER_WAVE
-#define NVSHMEM_AMD_CHUNKED_REPLICAS_PER_WAVE 2
-#endif
-#ifndef NVSHMEM_AMD_CHUNK_CYCLE_SHIFT /* log2 of chunk tiles x destination groups */
-#define NVSHMEM_AMD_CHUNK_CYCLE_SHIFT 14
-#endif
-// Groups of the chunked form: the largest power of two that leaves every group at least
-// NVSHMEM_AMD_CHUNKED_REPLICAS_PER_WAVE destinations (16 members: 8 groups of 2; 24: 8 of 3; 5: 2 groups of 3 and 2),
-// so that no group is empty.
-static uint32_t chunked_part_shift(int max_size) {
-    uint32_t shift = 0;
-    while ((max_size >> (shift + 1)) >= NVSHMEM_AMD_CHUNKED_REPLICAS_PER_WAVE) ++shift;
-    return shift;
-}
-static uint32_t chunk_shift_for(uint32_t part_shift) {
-    const uint32_t cycle = NVSHMEM_AMD_CHUNK_CYCLE_SHIFT;
-    return cycle > part_shift + 8 ? cycle - part_shift : 8;   // at least 256 tiles (a multiple of the 8 XCDs) per chunk
-}
+// Tiles of a segment, wherever it starts.
+static uint64_t segment_tiles(uint64_t seg_bytes) { return (seg_bytes / 16 + 63 + 63) / 64; }
 
 // members of all teams of the handle together
 static uint64_t total_members(const TeamLaunch &tl) {
@@ -543,31 +506,43 @@ static uint64_t total_members(const TeamLaunch &tl) {
     return (uint64_t)tl.ngroups * (uint64_t)tl.max_size;
 }
 
+// How fcollect and broadcast store: paced beyond Runtime::paced_copy_blocks (9 to a compute unit: 8 pieces and what a
+// message that is no power of two adds), up to which a grid is in flight all at once.  us paced / back to back at 1024, 2048 and 4096 blocks: fcollect to 4 members 2.8 / 2.2,
+// 3.2 / 2.8 and 4.1 / 4.0; to 8 4.2 / 2.8, 4.7 / 4.4 and 6.5 / 7.1; to 16 6.1 / 4.0, 7.0 / 6.6 and 11.1 / 12.2;
+// broadcast to 8 4.2 / 2.7, 4.7 / 4.1 and 6.3 / 6.5.
+static bool paced_copy(const Runtime &rt, uint64_t blocks) { return blocks > rt.paced_copy_blocks; }
+// Dynamic LDS that nobody uses: it limits the wavefronts of a paced copy that a compute unit (160 KiB) holds.  16 of
+// the 32 possible when the cache can hold the sources from one call to the next; their loads take longer from memory
+// and more wavefronts are needed to cover that, 24, or 20 with 16 destinations and more, which keep a wavefront
+// storing for longer.  us with 32 / 24 / 20 / 16 (sources | destinations in all): fcollect 8 members 32 MiB | 256 MiB
+// 43.3 / 43.1 / 42.9 / 42.3, 16 members 64 MiB | 1 GiB 177.9 / 167.1 / 162.1 / 157.4, 8 members 128 MiB | 1 GiB
+// 202 / 186 / 190 / 192, 4 members 128 MiB | 512 MiB 106.3 / 104.8 / 108.9 / 113.8, 16 members 128 MiB | 2 GiB 395 /
+// 341-376 / 345-373 / 376; broadcast 8 members 64 MiB | 512 MiB 85.1 / 83.1 / 82.3 / 81.7, 256 MiB | 2 GiB 376 / 372 /
+// 380 / 395, 64 members 32 MiB | 2 GiB 324-362 / 325-361 / 321-360 / 347.
+static size_t paced_lds_bytes(const Runtime &rt, uint64_t source_bytes, int members) {
+    const unsigned waves = source_bytes * 2 < rt.cacheable_source_bytes ? 16 : members < 16 ? 24 : 20;
+    return ((size_t)160 << 10) / waves & ~(size_t)127;
+}
+
 // Launches the broadcast kernel: member `root`'s [soff, +bytes) to every member's [doff, +bytes).
 static int launch_broadcast(Runtime &rt, const TeamLaunch &tl, uint64_t doff, uint64_t soff, uint64_t bytes, int root,
-                            hipStream_t stream, bool force_chunked = false) {
-    // The chunked form from Runtime::chunked_copy_bytes (128 MiB) on: measured level with the plain form at
-    // 64 MiB and 3-5 % ahead from 128 MiB for 4 and 8 members (teams of fewer than four members have one group
-    // of destinations and keep the plain form).  A source that cannot stay in the Infinity Cache is streamed.
-    const bool big_source = bytes * (uint64_t)tl.ngroups > rt.cacheable_source_bytes;
-    const bool chunked = force_chunked || bytes * (uint64_t)tl.ngroups >= rt.chunked_copy_bytes;
-    const uint32_t part_shift = chunked ? chunked_part_shift(tl.max_size) : 0;
-    const uint32_t chunk_shift = part_shift ? chunk_shift_for(part_shift) : 0;
-    uint64_t tiles = (bytes / 16 + 64 + kCopyThreads - 1) / kCopyThreads + 1;
-    tiles = ((tiles + (1ull << chunk_shift) - 1) >> chunk_shift << chunk_shift) << part_shift;  // whole chunks
+                            hipStream_t stream) {
+    const uint64_t tiles = segment_tiles(bytes), sources = bytes * (uint64_t)tl.ngroups;
     if (tiles > 0x7fffffffull) {
         set_error("broadcast: message too large");
         return NVSHMEMX_ERROR_INVALID_VALUE;
     }
-    const dim3 grid((unsigned)tiles, 1, (unsigned)tl.ngroups), block(kCopyThreads);
-    // blocks that share a piece re-read it from the cache, so the loads stay cacheable then
-#define NVSHMEM_AMD_LAUNCH_BROADCAST(NTL, STORE)                                                      \
-    hipLaunchKernelGGL((segment_copy_kernel<kModeBroadcast, 1, NTL, STORE>), grid, block, 0, stream,    \
-                       rt.base, rt.heap_size, tl.groups, tl.max_size, doff, soff, (uint64_t)bytes, root, \
-                       part_shift, chunk_shift)
-    if (chunk_shift != 0) NVSHMEM_AMD_LAUNCH_BROADCAST(false, NVSHMEM_AMD_STORE_BROADCAST_CHUNKED);
-    else if (big_source) NVSHMEM_AMD_LAUNCH_BROADCAST(true, NVSHMEM_AMD_STORE_REPLICATE);
-    else NVSHMEM_AMD_LAUNCH_BROADCAST(false, NVSHMEM_AMD_STORE_REPLICATE);
+    const dim3 grid((unsigned)tiles, 1, (unsigned)tl.ngroups);
+    const segment_args_t args = {rt.base, rt.heap_size, team_arg(tl), doff, soff, bytes, (uint32_t)root};
+    const bool paced = paced_copy(rt, tiles * (uint64_t)tl.ngroups);
+    const size_t lds = paced ? paced_lds_bytes(rt, sources, tl.max_size) : 0;
+    // a source that cannot stay in the Infinity Cache is streamed
+#define NVSHMEM_AMD_LAUNCH_BROADCAST(NTL, PACED)                                                                \
+    hipLaunchKernelGGL((segment_copy_kernel<kModeBroadcast, NTL, PACED, NVSHMEM_AMD_STORE_REPLICATE>), grid,      \
+                       dim3(64), lds, stream, args)
+    if (!paced) NVSHMEM_AMD_LAUNCH_BROADCAST(false, false);
+    else if (sources > rt.cacheable_source_bytes) NVSHMEM_AMD_LAUNCH_BROADCAST(true, true);
+    else NVSHMEM_AMD_LAUNCH_BROADCAST(false, true);
 #undef NVSHMEM_AMD_LAUNCH_BROADCAST
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
@@ -614,7 +589,7 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
     else if (tl.max_size >= 3 && tl.max_size <= 32) mpw = 2;
     else if (tl.max_size > 32 && tl.max_size <= 64) mpw = 4;
     // Two-step allreduce of large teams: fold into member 0's destination (n loads and ONE store per vector, the
-    // shape of the reducescatter), then broadcast that in the chunked form.  It moves 2 n + 2 units where the fused
+    // shape of the reducescatter), then broadcast that.  It moves 2 n + 2 units where the fused
     // kernel moves 2 n, but every block of the fused kernel feeds n write fronts of 1 KiB pieces, and its fold
     // serialises n steps between two barriers.  fp32 sum, TB/s, fused / two-step at 512 MiB and 2 GiB of sources in
     // all: 12 members 6.41 / 6.18 and 6.28 / 6.29, 16: 6.26 / 6.19 and 6.02 / 6.41, 24: 5.84 / 5.71 and 5.69 / 6.23,
@@ -633,7 +608,7 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
             else
                 hipLaunchKernelGGL((reduce_gather_kernel<T, OP, 0, false, true>), grid, dim3(64), 0, stream, rt.base,
                                    rt.heap_size, tl.groups, shape);
-            (void)launch_broadcast(rt, tl, dst_off, dst_off, nelems * sizeof(T), 0, stream, true);
+            (void)launch_broadcast(rt, tl, dst_off, dst_off, nelems * sizeof(T), 0, stream);
             return;
         }
     }
@@ -892,42 +867,27 @@ static int segment_collective(int mode, const char *what, nvshmem_team_t team, v
         set_error("%s: dest and source overlap", what);
         return NVSHMEMX_ERROR_INVALID_VALUE;
     }
-    const uint64_t tile_vectors = (uint64_t)kCopyThreads * (mode == kModeFcollect ? NVSHMEM_AMD_FCOLLECT_UNROLL
-                                                                              : NVSHMEM_AMD_ALLTOALL_UNROLL);
-    const bool big_source = src_bytes * total_members(tl) > rt.cacheable_source_bytes;
-    // An fcollect takes the chunked form when its sources hold Runtime::chunked_copy_bytes (128 MiB) or more and
-    // its destinations eight times that: with the sources still in the Infinity Cache it is the n-fold larger
-    // destinations that decide.  Chunked / plain in TB/s at 64 | 128 | 256 MiB of sources: 16 members 6.3 / 6.5 |
-    // 7.2 / 6.6 | 7.7 / 6.5, 8 members 6.4 / 6.9 | 7.3 / 6.9 | 7.9 / 6.9, 4 members 6.7 / 7.7 | 7.7 / 8.0 | 8.4 / 8.1.
-    const uint64_t all_sources = src_bytes * total_members(tl);
-    const bool chunked = mode == kModeFcollect && all_sources >= rt.chunked_copy_bytes &&
-                         all_sources * n >= 8 * rt.chunked_copy_bytes;
-    const uint32_t part_shift = chunked ? chunked_part_shift(tl.max_size) : 0;
-    const uint32_t chunk_shift = part_shift ? chunk_shift_for(part_shift) : 0;
-    uint64_t tiles = (seg_bytes / 16 + 64 + tile_vectors - 1) / tile_vectors + 1;
-    tiles = ((tiles + (1ull << chunk_shift) - 1) >> chunk_shift << chunk_shift) << part_shift;  // whole chunks
-    const unsigned segs = mode == kModeFcollect ? (unsigned)n : (unsigned)(n * n);
+    const uint64_t tiles = segment_tiles(seg_bytes), sources = src_bytes * total_members(tl);
     if (tiles > 0x7fffffffull) {
         set_error("%s: message too large", what);
         return NVSHMEMX_ERROR_INVALID_VALUE;
     }
-    // blocks that share a piece re-read it from the cache, so the loads stay cacheable then
-    const bool stream_source = part_shift == 0 && big_source;
-    const dim3 grid((unsigned)tiles, segs, (unsigned)tl.ngroups), block(kCopyThreads);
-#define NVSHMEM_AMD_LAUNCH_SEGCOPY(MODE, U, NTL, STORE)                                            \
-    hipLaunchKernelGGL((segment_copy_kernel<MODE, U, NTL, STORE>), grid, block, 0, stream, rt.base, \
-                       rt.heap_size, tl.groups, tl.max_size, doff, soff, (uint64_t)seg_bytes, 0,   \
-                       part_shift, chunk_shift)
+    const bool stream_source = sources > rt.cacheable_source_bytes;
+    const segment_args_t args = {rt.base, rt.heap_size, team_arg(tl), doff, soff, seg_bytes, 0};
+#define NVSHMEM_AMD_LAUNCH_SEGCOPY(MODE, NTL, PACED, STORE) \
+    hipLaunchKernelGGL((segment_copy_kernel<MODE, NTL, PACED, STORE>), grid, dim3(64), lds, stream, args)
     if (mode == kModeFcollect) {
-        if (chunk_shift != 0)
-            NVSHMEM_AMD_LAUNCH_SEGCOPY(kModeFcollect, NVSHMEM_AMD_FCOLLECT_UNROLL, false, NVSHMEM_AMD_STORE_FCOLLECT_CHUNKED);
-        else if (stream_source)
-            NVSHMEM_AMD_LAUNCH_SEGCOPY(kModeFcollect, NVSHMEM_AMD_FCOLLECT_UNROLL, true, NVSHMEM_AMD_STORE_REPLICATE);
-        else
-            NVSHMEM_AMD_LAUNCH_SEGCOPY(kModeFcollect, NVSHMEM_AMD_FCOLLECT_UNROLL, false, NVSHMEM_AMD_STORE_REPLICATE);
+        const dim3 grid((unsigned)tiles, (unsigned)n, (unsigned)tl.ngroups);
+        const bool paced = paced_copy(rt, tiles * n * (uint64_t)tl.ngroups);
+        const size_t lds = paced ? paced_lds_bytes(rt, sources, tl.max_size) : 0;
+        if (!paced) NVSHMEM_AMD_LAUNCH_SEGCOPY(kModeFcollect, false, false, NVSHMEM_AMD_STORE_REPLICATE);
+        else if (stream_source) NVSHMEM_AMD_LAUNCH_SEGCOPY(kModeFcollect, true, true, NVSHMEM_AMD_STORE_REPLICATE);
+        else NVSHMEM_AMD_LAUNCH_SEGCOPY(kModeFcollect, false, true, NVSHMEM_AMD_STORE_REPLICATE);
     } else {
-        if (stream_source) NVSHMEM_AMD_LAUNCH_SEGCOPY(kModeAlltoall, NVSHMEM_AMD_ALLTOALL_UNROLL, true, NVSHMEM_AMD_STORE_ALLTOALL);
-        else NVSHMEM_AMD_LAUNCH_SEGCOPY(kModeAlltoall, NVSHMEM_AMD_ALLTOALL_UNROLL, false, NVSHMEM_AMD_STORE_ALLTOALL);
+        const dim3 grid((unsigned)tiles, (unsigned)n, (unsigned)(n * tl.ngroups));
+        const size_t lds = 0;  // (one store per load: every wavefront counts)
+        if (stream_source) NVSHMEM_AMD_LAUNCH_SEGCOPY(kModeAlltoall, true, false, NVSHMEM_AMD_STORE_ALLTOALL);
+        else NVSHMEM_AMD_LAUNCH_SEGCOPY(kModeAlltoall, false, false, NVSHMEM_AMD_STORE_ALLTOALL);
     }
 #undef NVSHMEM_AMD_LAUNCH_SEGCOPY
     hipError_t e = hipGetLastError();

@@ -40,6 +40,7 @@ struct TeamTable {
 // What a collective kernel needs to serve every team of a handle.
 struct TeamLaunch {
     const nvshmemi_amd_team_view_t *groups = nullptr;  // device array, ngroups entries
+    nvshmemi_amd_team_view_t first{};                  // its first entry
     int ngroups = 0;
     int max_size = 0, min_size = 0;
 };
@@ -70,14 +71,14 @@ struct Runtime {
     // Host-launched collectives treat sources of more bytes than this (all PEs together) as too
     // large to stay in the Infinity Cache: NVSHMEM_AMD_CACHEABLE_SOURCE_BYTES, read at init
     uint64_t cacheable_source_bytes = (uint64_t)256 << 20;
-    // fcollect and broadcast take the chunked form from this many bytes of sources (all PEs together) on:
-    // NVSHMEM_AMD_CHUNKED_COPY_BYTES, read at init
-    uint64_t chunked_copy_bytes = (uint64_t)128 << 20;
+    // fcollect and broadcast store to one destination after the other in grids of more blocks than this, to all of
+    // them back to back in smaller ones: NVSHMEM_AMD_PACED_COPY_BLOCKS, read at init (default: 9 to a compute unit)
+    uint64_t paced_copy_blocks = 2304;
     // Allreduce on teams of 3 to 64 members takes the LDS-staged kernel when the sources of all PEs
     // together hold at least this many bytes (a quarter of it for teams of 17
     // to 32 members, four times for larger ones): NVSHMEM_AMD_LDS_REDUCE_BYTES, read at init
     uint64_t lds_reduce_bytes = (uint64_t)64 << 20;
-    // An allreduce beyond the cache takes two steps - fold into member 0, chunked broadcast - instead of the fused
+    // An allreduce beyond the cache takes two steps - fold into member 0, broadcast - instead of the fused
     // kernel from this team size on (NVSHMEM_AMD_TWO_STEP_REDUCE_MEMBERS, read at init; 0 = never) when the
     // sources of all members together hold at least two_step_reduce_bytes (NVSHMEM_AMD_TWO_STEP_REDUCE_BYTES), and
     // from three times the team size at any size

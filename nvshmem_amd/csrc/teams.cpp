@@ -197,6 +197,7 @@ bool resolve_team(Runtime &rt, const char *what, nvshmem_team_t team, TeamLaunch
     }
     const TeamTable &tt = rt.teams;
     out->groups = tt.dev_groups() + (size_t)team * kMaxPes;
+    out->first = tt.groups[team][0];
     out->ngroups = tt.ngroups[team];
     out->max_size = 0;
     out->min_size = kMaxPes + 1;

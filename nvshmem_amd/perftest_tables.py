@@ -18,7 +18,7 @@ latency  barrier_all / sync_all, put and get of one thread group with quiet, put
 
 collectives  the host-launched (on-stream) reduce, fcollect, broadcast, alltoall and reducescatter from 256 KiB
          to 128 MiB per PE, as the library chooses its kernels and with each of the two forms forced through
-         the environment (NVSHMEM_AMD_LDS_REDUCE_BYTES, NVSHMEM_AMD_CHUNKED_COPY_BYTES): the evidence for the
+         the environment (NVSHMEM_AMD_LDS_REDUCE_BYTES, NVSHMEM_AMD_PACED_COPY_BLOCKS): the evidence for the
          sizes at which the library switches.  Times are host wall time per call over back-to-back calls,
          so the smallest sizes show the launch rate, and sources up to 256 MiB in all stay in the Infinity
          Cache from one call to the next.
@@ -121,11 +121,11 @@ def collectives(iters):
                                                "NVSHMEM_AMD_TWO_STEP_REDUCE_MEMBERS": "0"})))
             for npes in (4, 8, 16, 32, 64)]
     jobs += [("fcollect", "fcollect", npes, "32m" if npes <= 8 else "16m",
-              (("library's choice", {}), ("chunked form at every size", {"NVSHMEM_AMD_CHUNKED_COPY_BYTES": "0"}),
-               ("plain form at every size", {"NVSHMEM_AMD_CHUNKED_COPY_BYTES": never}))) for npes in (4, 8, 16)]
+              (("library's choice", {}), ("one destination at a time", {"NVSHMEM_AMD_PACED_COPY_BLOCKS": "0"}),
+               ("all back to back", {"NVSHMEM_AMD_PACED_COPY_BLOCKS": never}))) for npes in (4, 8, 16)]
     jobs += [("broadcast", "broadcast", 8, "128m",
-              (("library's choice", {}), ("chunked form at every size", {"NVSHMEM_AMD_CHUNKED_COPY_BYTES": "0"}),
-               ("plain form at every size", {"NVSHMEM_AMD_CHUNKED_COPY_BYTES": never}))),
+              (("library's choice", {}), ("one destination at a time", {"NVSHMEM_AMD_PACED_COPY_BLOCKS": "0"}),
+               ("all back to back", {"NVSHMEM_AMD_PACED_COPY_BLOCKS": never}))),
              ("alltoall (bytes per destination)", "alltoall", 8, "16m", (("library's choice", {}),)),
              ("reducescatter (bytes per block)", "reducescatter", 8, "16m", (("library's choice", {}),))]
     lines, commands = [], []
