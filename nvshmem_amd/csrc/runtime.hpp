@@ -100,6 +100,17 @@ struct Runtime {
         *off = d % heap_size;
         return true;
     }
+    // The runtime's own words (barrier rows, epoch, timeout record) end every slice and are not the caller's to address.
+    uint64_t usable_bytes() const { return heap_size - NVSHMEMI_AMD_INTERNAL_BYTES; }
+    // Whether [p, p + bytes) lies inside one PE's part of the heap, and where in it.
+    bool usable(const void *p, uint64_t bytes, uint64_t *off) const {
+        return offset_of(p, off) && bytes <= usable_bytes() && *off + bytes <= usable_bytes();
+    }
+    // Whether [p, p + bytes) lies inside the heap (of one PE or several).
+    bool holds(const void *p, uint64_t bytes) const {
+        const uint64_t d = (uint64_t)((const char *)p - base), all = (uint64_t)npes * heap_size;
+        return initialized && (const char *)p >= base && bytes <= all && d <= all - bytes;
+    }
     char *slice(int pe) const { return base + (uint64_t)pe * heap_size; }
 };
 
