@@ -809,7 +809,17 @@ int nvshmemx_amd_collective_launch(const void *func, unsigned grid_x, unsigned g
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     if (rt.collective_launch == Runtime::kLaunchBySize && hipStreamIsCapturing(s, &capture) != hipSuccess)
         (void)hipGetLastError();
-    if (capture != hipStreamCaptureStatusNone) rt.launch_captured = true;
+    if (capture != hipStreamCaptureStatusNone && !rt.launch_captured) {
+        rt.launch_captured = true;
+        // a replay is not to start beside a plain launch that is still on its way: wait for the last one (not a part of
+        // the capture, hence the relaxed mode)
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        if (rt.launch_pending && hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess) {
+            const hipError_t waited = hipEventSynchronize(rt.launch_done);
+            (void)hipThreadExchangeStreamCaptureMode(&mode);
+            if (waited != hipSuccess) (void)hipGetLastError();
+        }
+    }
     const bool by_size = rt.collective_launch == Runtime::kLaunchBySize && rt.launch_done && !rt.launch_captured;
     auto other = [&](hipStream_t last) { return s != last || s == hipStreamPerThread; };  // (one handle, a stream per thread)
     const bool plain = rt.collective_launch == Runtime::kLaunchPlain ||

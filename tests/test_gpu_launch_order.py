@@ -47,3 +47,36 @@ def test_collective_launches_on_two_streams(forced, monkeypatch):
             assert (rt.download_all(errors, (1,), np.uint64) == 0).all()
         for s in set(streams):
             s.destroy()
+
+
+def test_captured_launch_behind_plain_ones():
+    """A collective launch is captured while plain ones on another stream are still on their way; every replay and the
+    launches between the replays give what they give on a stream."""
+    with runtime(NPES, 32 << 20) as rt:
+        perf = rt.perftest()
+        s, other = hip.Stream(), hip.Stream()
+        n, blocks = 8 * CHUNK * 2, 8
+        src, dst, sig = rt.malloc(n * 4), rt.calloc(n, 4), rt.calloc(blocks, 8)
+        eager, eager_sig = rt.calloc(n, 4), rt.calloc(blocks, 8)
+        rt.upload_all(src, O.fill_all("i32", NPES, n, 7))
+        rt.sync()
+        before = rt.lib.nvshmemx_amd_timeout_count()
+        for _ in range(ROUNDS):
+            assert perf.nvshmem_perftest_ring_reduce(eager, src, n, eager_sig, CHUNK, blocks, 256, other.ptr) == 0
+        with hip.Graph(s) as g:
+            assert perf.nvshmem_perftest_ring_reduce(dst, src, n, sig, CHUNK, blocks, 256, s.ptr) == 0
+        for k in range(3):
+            data = O.fill_all("i32", NPES, n, 50 + k)
+            note("replay %d" % k)
+            rt.upload_all(src, data)
+            rt.sync()
+            g.launch()
+            assert perf.nvshmem_perftest_ring_reduce(eager, src, n, eager_sig, CHUNK, blocks, 256, s.ptr) == 0
+            s.synchronize()
+            want = O.reduce("i32", "sum", data)
+            assert (rt.download_all(dst, (n,), np.int32) == want).all()
+            assert (rt.download_all(eager, (n,), np.int32) == want).all()
+        assert rt.lib.nvshmemx_amd_timeout_count() == before
+        g.destroy()
+        for x in (s, other):
+            x.destroy()
