@@ -52,6 +52,8 @@ constexpr size_t kSparseStrideBytes = 128, kSparseElements = (size_t)1 << 17;
 // Small copies spread over the compute units: 64 threads a block; 256 beyond (2^22 contiguous 16-bit elements: 15.5 us
 // with 64, 5.4 with 256).
 constexpr size_t kNarrowBlockElements = (size_t)1 << 16;
+// A launch holds fewer than 2^32 threads; copies of so many elements stay with the rectangle copy.
+constexpr size_t kKernelElements = (size_t)1 << 31;
 
 template <typename T>
 void launch_strided(void *dst, size_t dst_stride, const void *src, size_t src_stride, size_t nelems, hipStream_t stream) {
@@ -73,7 +75,8 @@ void strided_copy(char *dst, ptrdiff_t dst_stride, const char *src, ptrdiff_t sr
                rt.holds(p, ((uint64_t)(nelems - 1) * stride + 1) * es);
     };
     const bool sparse = (ds < ss ? ds : ss) * es >= kSparseStrideBytes && nelems > kSparseElements;
-    if (!sparse && (((uintptr_t)dst | (uintptr_t)src) & (es - 1)) == 0 && in_heap(dst, ds) && in_heap(src, ss)) {
+    if (!sparse && nelems <= kKernelElements && (((uintptr_t)dst | (uintptr_t)src) & (es - 1)) == 0 && in_heap(dst, ds) &&
+        in_heap(src, ss)) {
         switch (es) {
             case 1: return launch_strided<uint8_t>(dst, ds, src, ss, nelems, stream);
             case 2: return launch_strided<uint16_t>(dst, ds, src, ss, nelems, stream);
