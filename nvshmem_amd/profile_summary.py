@@ -40,7 +40,7 @@ Durations under the counter pass are a few percent longer than in the kernel tra
 (algorithmic bytes per second) are the kernel trace's."""
 
 
-COMMANDS = """Commands (on the GPU box, from the repository root; every file they run is committed):
+COMMANDS = """Commands (on a machine with the GPU, from the repository root; every file they run is committed):
   export OUT=<a scratch directory>; cd /tmp; export TMPDIR=/tmp
   export NVSHMEM_AMD_PLAIN_COLLECTIVE_LAUNCH=1   (kernels that nvshmemx_collective_launch starts are started with a plain
       launch: after a cooperative launch the profiled process crashes in an exit handler of the profiler's stack, behind
