@@ -341,10 +341,10 @@ NVSHMEMI_REPT_FOR_ALL_REDUCE_TYPES_AND_OPS(NVSHMEMI_DECL_TYPED_REDUCE_HOST)
 #undef NVSHMEMI_DECL_TYPED_REDUCE_HOST
 
 /*
- * Collective launch of a kernel that uses the device API (reference
+ * Cooperative launch of a kernel that uses the device API (reference
  * src/device/launch/collective_launch.cpp:209-212).  One launch carries every logical PE:
  * the grid's z extent is set to npes (the caller's grid z must be 1) and a block acts as PE
- * blockIdx.z, all blocks co-resident and no other collective launch beside it.  grid (0,0,0) asks for the largest co-resident grid per PE.  The launch is refused
+ * blockIdx.z.  grid (0,0,0) asks for the largest co-resident grid per PE.  The launch is refused
  * with NVSHMEMX_ERROR_COLLECTIVE_LAUNCH_FAILED when grid*npes blocks cannot be co-resident.
  * Grid and block are passed as three unsigned each to keep the ABI free of HIP types.
  */

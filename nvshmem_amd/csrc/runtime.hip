@@ -109,12 +109,6 @@ bool require_init(Runtime &rt, const char *what) {
     return false;
 }
 
-void release_launch_event(Runtime &rt) {
-    if (rt.launch_done) (void)hipEventDestroy(rt.launch_done);
-    rt.launch_done = nullptr;
-    rt.launch_pending = false;
-}
-
 uint64_t env_size(const char *name, uint64_t dflt) {
     const char *v = getenv(name);
     if (!v || !*v) return dflt;
@@ -281,15 +275,7 @@ int nvshmemx_amd_init(int npes, size_t symmetric_size) {
                             "using full\n", order);
     }
     rt.dev.heap_magic = (1ull << 40) / (rt.heap_size >> 21) + 1;
-    const char *plain = getenv("NVSHMEM_AMD_PLAIN_COLLECTIVE_LAUNCH");
-    rt.collective_launch = !plain || !*plain ? Runtime::kLaunchBySize
-                           : env_size("NVSHMEM_AMD_PLAIN_COLLECTIVE_LAUNCH", 0) != 0 ? Runtime::kLaunchPlain
-                                                                                      : Runtime::kLaunchCooperative;
-    rt.launch_pending = rt.cooperative_pending = rt.launch_captured = false;
-    if (hipEventCreateWithFlags(&rt.launch_done, hipEventDisableTiming) != hipSuccess) {
-        (void)hipGetLastError();
-        rt.launch_done = nullptr;
-    }
+    rt.plain_collective_launch = env_size("NVSHMEM_AMD_PLAIN_COLLECTIVE_LAUNCH", 0) != 0;
     rt.cacheable_source_bytes = env_size("NVSHMEM_AMD_CACHEABLE_SOURCE_BYTES", (size_t)256 << 20);
     rt.paced_copy_blocks = env_size("NVSHMEM_AMD_PACED_COPY_BLOCKS", (uint64_t)rt.num_cus * 9);
     rt.lds_reduce_bytes = env_size("NVSHMEM_AMD_LDS_REDUCE_BYTES", (size_t)64 << 20);
@@ -297,7 +283,6 @@ int nvshmemx_amd_init(int npes, size_t symmetric_size) {
     rt.two_step_reduce_bytes = env_size("NVSHMEM_AMD_TWO_STEP_REDUCE_BYTES", (size_t)512 << 20);
     if (!teams_init(rt)) {
         teams_finalize(rt);
-        release_launch_event(rt);
         (void)hipFree(rt.base);
         if (rt.timeout_flag) (void)hipHostFree(rt.timeout_flag);
         rt.timeout_flag = nullptr;
@@ -334,7 +319,6 @@ void nvshmem_finalize(void) {
     (void)report_timeouts(rt, "nvshmem_finalize");
     rt.timeouts_seen = 0;
     teams_finalize(rt);
-    release_launch_event(rt);
     (void)hipFree(rt.base);
     if (rt.timeout_flag) (void)hipHostFree(rt.timeout_flag);
     rt.timeout_flag = nullptr;
@@ -796,51 +780,20 @@ int nvshmemx_amd_collective_launch(const void *func, unsigned grid_x, unsigned g
                   per_pe, rt.npes, cap, threads);
         return NVSHMEMX_ERROR_COLLECTIVE_LAUNCH_FAILED;
     }
-    // A cooperative launch goes through a queue of its own, in step with the stream on either side: 20 us between
-    // back-to-back launches of 8 blocks, where a plain launch that records an event takes 4.0 and a plain one 2.4.
-    // What the cooperative queue gives a grid whose blocks wait for each other is that no second such grid runs
-    // beside it, each holding compute units that the other needs.  A grid of at most half of what the GPU holds
-    // therefore starts with a plain launch, and the order among collective launches is kept here: each records its
-    // end, and one on another stream waits for it on the GPU (on the same stream the stream does).  Larger grids stay
-    // cooperative, and so does a launch on another stream behind one of those, which that queue then orders; and
-    // everything once a collective launch has been captured into a graph, whose replays cannot be ordered from here.
+    // A cooperative launch guarantees that all blocks are resident together, whatever else runs on
+    // the GPU, and costs about 20 us more than a plain launch here.  The grid has just been checked
+    // against the occupancy limit, so a plain launch gives the same co-residency as long as no
+    // other kernel holds compute units while waiting for this one: NVSHMEM_AMD_PLAIN_COLLECTIVE_
+    // LAUNCH=1 opts into that for programs that launch their PE kernels one at a time.
     const dim3 grid(grid_x, grid_y, (unsigned)rt.npes), block(block_x, block_y, block_z);
-    hipStream_t s = (hipStream_t)stream;
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (rt.collective_launch == Runtime::kLaunchBySize && hipStreamIsCapturing(s, &capture) != hipSuccess)
-        (void)hipGetLastError();
-    if (capture != hipStreamCaptureStatusNone && !rt.launch_captured) {
-        rt.launch_captured = true;
-        // a replay is not to start beside a plain launch that is still on its way: wait for the last one (not a part of
-        // the capture, hence the relaxed mode)
-        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-        if (rt.launch_pending && hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess) {
-            const hipError_t waited = hipEventSynchronize(rt.launch_done);
-            (void)hipThreadExchangeStreamCaptureMode(&mode);
-            if (waited != hipSuccess) (void)hipGetLastError();
-        }
-    }
-    const bool by_size = rt.collective_launch == Runtime::kLaunchBySize && rt.launch_done && !rt.launch_captured;
-    auto other = [&](hipStream_t last) { return s != last || s == hipStreamPerThread; };  // (one handle, a stream per thread)
-    const bool plain = rt.collective_launch == Runtime::kLaunchPlain ||
-                       (by_size && 2 * per_pe <= (unsigned long long)cap &&
-                        !(rt.cooperative_pending && other(rt.cooperative_stream)));
-    hipError_t e = hipSuccess;
-    if (capture == hipStreamCaptureStatusNone && rt.launch_pending && other(rt.launch_stream))
-        e = hipStreamWaitEvent(s, rt.launch_done, 0);
-    if (e == hipSuccess) {
-        if (!plain) e = hipLaunchCooperativeKernel(func, grid, block, args, (unsigned)shared_mem, s);
-        else if (by_size) e = hipExtLaunchKernel(func, grid, block, args, shared_mem, s, nullptr, rt.launch_done, 0);
-        else e = hipLaunchKernel(func, grid, block, args, shared_mem, s);
-    }
-    if (e == hipSuccess && by_size) {
-        (plain ? rt.launch_stream : rt.cooperative_stream) = s;
-        if (plain) rt.launch_pending = true;
-        rt.cooperative_pending = !plain;  // (a plain launch behind a cooperative one is on its stream)
-    }
+    hipError_t e = rt.plain_collective_launch
+                       ? hipLaunchKernel(func, grid, block, args, shared_mem, (hipStream_t)stream)
+                       : hipLaunchCooperativeKernel(func, grid, block, args, (unsigned)shared_mem,
+                                                    (hipStream_t)stream);
     if (e != hipSuccess) {
         (void)hipGetLastError();
-        set_error("collective launch: %s failed: %s", plain ? "plain launch" : "hipLaunchCooperativeKernel",
+        set_error("collective launch: %s failed: %s",
+                  rt.plain_collective_launch ? "hipLaunchKernel" : "hipLaunchCooperativeKernel",
                   hipGetErrorString(e));
         return NVSHMEMX_ERROR_COLLECTIVE_LAUNCH_FAILED;
     }

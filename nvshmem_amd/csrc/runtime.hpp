@@ -58,16 +58,7 @@ struct Runtime {
     TeamTable teams{};
     std::set<nvshmemi_amd_state_updater_t> updaters;  // one per translation unit with a state block
     bool symbols_stale = false;
-    // How nvshmemx_collective_launch starts a grid (NVSHMEM_AMD_PLAIN_COLLECTIVE_LAUNCH, read at init): unset = by
-    // its size, 0 = always cooperatively, anything else = always with a plain launch
-    enum { kLaunchBySize, kLaunchCooperative, kLaunchPlain } collective_launch = kLaunchBySize;
-    // Collective launches run one after the other.  launch_done marks the end of the latest one that was started with
-    // a plain launch, on launch_stream; null if it could not be created (then every launch by size is cooperative).
-    hipEvent_t launch_done = nullptr;
-    hipStream_t launch_stream = nullptr, cooperative_stream = nullptr;
-    bool launch_pending = false;       // launch_done has been recorded
-    bool cooperative_pending = false;  // a cooperative launch, on cooperative_stream, is not covered by launch_done
-    bool launch_captured = false;      // a collective launch has gone into a graph, whose replays are not seen here
+    bool plain_collective_launch = false;  // NVSHMEM_AMD_PLAIN_COLLECTIVE_LAUNCH=1, read at init
     // Host-launched collectives treat sources of more bytes than this (all PEs together) as too
     // large to stay in the Infinity Cache: NVSHMEM_AMD_CACHEABLE_SOURCE_BYTES, read at init
     uint64_t cacheable_source_bytes = (uint64_t)256 << 20;

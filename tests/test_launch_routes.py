@@ -1,0 +1,23 @@
+"""Which kernels the library launches for a call, and with which grids: seen on the CPU, where nothing runs."""
+import pytest
+
+from launch_recorder import recorded  # noqa: F401
+
+COLLECTIVE_LAUNCH = """
+ok(lib.nvshmemx_amd_init(8, 1 << 20))
+launches()
+for threads, blocks in ((64, 1), (1024, 1), (256, 32), (256, 200)):
+    for stream in (None, 1, 2, 1):
+        ok(lib.nvshmemx_amd_collective_launch(1, blocks, 1, 1, threads, 1, 1, None, 0, stream))
+for kernel, cooperative, grid, block, lds in launches():
+    assert cooperative == %s, (grid, block)
+    assert grid[2] == 8
+"""
+
+
+@pytest.mark.parametrize("plain,cooperative", [(None, True), ("0", True), ("1", False)])
+def test_collective_launches_are_cooperative_unless_asked(recorded, plain, cooperative):  # noqa: F811
+    """Only the cooperative queue keeps a PE kernel apart from cooperative kernels that the program itself has on
+    another stream: side by side, each could hold compute units that the other waits for."""
+    env = {} if plain is None else {"NVSHMEM_AMD_PLAIN_COLLECTIVE_LAUNCH": plain}
+    recorded(COLLECTIVE_LAUNCH % cooperative, **env)
