@@ -145,6 +145,11 @@ __device__ __forceinline__ void stream_store_at(char *p, unsigned off, nvshmemi_
 // ---------------------------------------------------------------------------------------------
 
 enum { kModeFcollect = 0, kModeAlltoall = 1, kModeBroadcast = 2 };
+// Below this length of a segment the edge bytes are stored in front of the vectors, which mostly lie in the same lines;
+// beyond, behind them, so that the vectors of block 0 are on their way no later than those of the other blocks.  us
+// first / last: broadcast to 8 of 64 bytes on an odd address 2.0 / 2.2, of 800 2.2 / 2.1; alltoall on 16 PEs of 200 bytes
+// 2.4 / 2.5, of 1021 2.6 / 2.3, of 16372 4.4 / 3.7.
+constexpr unsigned kEdgesFirstBytes = 512;
 
 struct segment_args_t {
     char *base;
@@ -190,47 +195,61 @@ __global__ __launch_bounds__(64) void segment_copy_kernel(segment_args_t a) {
     unsigned head = (unsigned)(-(uintptr_t)dst) & 15;
     if (head > a.seg_bytes) head = (unsigned)a.seg_bytes;
     const uint64_t nvec = (a.seg_bytes - head) / 16;
-    if (blockIdx.x == 0) {
-        // at most 15 + 15 bytes, lane k the k-th of them, every second destination on either half of the lanes
-        const unsigned edge = head + ((unsigned)(a.seg_bytes - head) & 15), k = lane & 31;
-        if (k < edge) {
-            const uint64_t pos = k < head ? k : nvec * 16 + k;
-            const char b = src[pos];
-            for (unsigned r = lane >> 5; r < nrep; r += 2) dst[r * rep_stride + pos] = b;
-        }
-    }
     // tiles are cut on absolute 1 KiB boundaries of the destination: `lead` vector slots of tile 0
     // lie in front of the segment
     const unsigned lead = (unsigned)((uintptr_t)(dst + head) >> 4) & 63;
     const int64_t v0 = (int64_t)blockIdx.x * 64 - lead, left = (int64_t)nvec - v0;
-    if (left <= 0) return;
+    const bool edges = blockIdx.x == 0;  // this block also moves the bytes around the vectors
+    if (left <= 0 && !edges) return;
     // this lane's vector, as an unsigned index: slots in front of the segment wrap and are skipped like those behind it
-    const unsigned first = blockIdx.x == 0 ? lead : 0, end = left < 64 ? (unsigned)left : 64;
-    if (lane - first >= end - first) return;
-    const nvshmemi_v4u v = stream_load<NTL>(src + head + 16 * v0 + 16 * lane);
+    const unsigned first = edges ? lead : 0, end = left < 64 ? (unsigned)left : 64;
+    const bool body = lane - first < end - first;
+    nvshmemi_v4u v = {};
+    if (body) v = stream_load<NTL>(src + head + 16 * v0 + 16 * lane);
+    // at most 15 + 15 bytes, lane k the k-th of them, every second destination on either half of the lanes; they are
+    // loaded beside the vectors
+    const unsigned k = lane & 31;
+    const bool edge = edges && k < head + ((unsigned)(a.seg_bytes - head) & 15);
+    const uint64_t pos = k < head ? k : nvec * 16 + k;
+    unsigned b = 0;
+    if (edge) b = (unsigned char)src[pos];
+    auto store_edges = [&]() {
+        if (!edge) return;
+        const unsigned half = lane >> 5;
+        char *to = dst + half * rep_stride + pos;
+#pragma nounroll
+        for (unsigned r = 0; r < nrep; r += 2, to += 2 * rep_stride)
+            if (r + half < nrep) *to = (char)b;
+    };
+    const bool edges_first = a.seg_bytes < kEdgesFirstBytes;
+    if (edges_first) store_edges();
     char *d = dst + head + 16 * v0;
     auto store = [&](char *to) { stream_store_at<STORE>(to, 16 * lane, v); };
-    if (MODE == kModeAlltoall) {
-        store(d);
-    } else if (PACED) {
-        store(d);
-        while (--nrep) {
-            d += rep_stride;
-            nvshmemi_amd_wait_vm();
+    if (body) {
+        unsigned n = nrep;
+        if (MODE == kModeAlltoall) {
             store(d);
-        }
-    } else {
-        for (; nrep >= 8; nrep -= 8, d += 8 * rep_stride) {
+        } else if (PACED) {
+            store(d);
+            while (--n) {
+                d += rep_stride;
+                nvshmemi_amd_wait_vm();
+                store(d);
+            }
+        } else {
+            for (; n >= 8; n -= 8, d += 8 * rep_stride) {
 #pragma unroll
-            for (int r = 0; r < 8; ++r) store(d + r * rep_stride);
-        }
-        if (nrep >= 4) {
+                for (int r = 0; r < 8; ++r) store(d + r * rep_stride);
+            }
+            if (n >= 4) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) store(d + r * rep_stride);
-            nrep -= 4, d += 4 * rep_stride;
+                for (int r = 0; r < 4; ++r) store(d + r * rep_stride);
+                n -= 4, d += 4 * rep_stride;
+            }
+            for (; n; --n, d += rep_stride) store(d);
         }
-        for (; nrep; --nrep, d += rep_stride) store(d);
     }
+    if (!edges_first) store_edges();
 }
 
 // ---------------------------------------------------------------------------------------------

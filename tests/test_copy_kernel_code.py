@@ -1,0 +1,62 @@
+"""What the compiler made of the small form of the segment copy: messages that take a few microseconds are bound by the
+memory round trips a wavefront makes one after the other, and those can be read from the waits in its code."""
+import os
+import re
+import struct
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+LIBRARY = os.path.join(ROOT, "nvshmem_amd", "lib", "libnvshmem_amd.so")
+LLVM = "/opt/rocm/llvm/bin/"
+MODES = {"fcollect": 0, "alltoall": 1, "broadcast": 2}
+STREAMED = 2  # the store form of all three
+
+
+@pytest.fixture(scope="module")
+def code_objects(tmp_path_factory):
+    """The GPU code of the library, one ELF file per translation unit."""
+    d = tmp_path_factory.mktemp("code")
+    fat = str(d / "fatbin")
+    subprocess.run([LLVM + "llvm-objcopy", "--dump-section", ".hip_fatbin=" + fat, LIBRARY, str(d / "rest")], check=True)
+    data = open(fat, "rb").read()
+    out = []
+    for m in re.finditer(b"__CLANG_OFFLOAD_BUNDLE__", data):
+        at = m.end()
+        count, = struct.unpack_from("<Q", data, at)
+        at += 8
+        for _ in range(count):
+            offset, size, name_len = struct.unpack_from("<QQQ", data, at)
+            name = data[at + 24:at + 24 + name_len]
+            at += 24 + name_len
+            if b"gfx950" in name and size:
+                out.append(str(d / ("unit%d.elf" % len(out))))
+                open(out[-1], "wb").write(data[m.start() + offset:m.start() + offset + size])
+    assert out
+    return out
+
+
+def _kernel(code_objects, mode, streamed_loads=False, paced=False):
+    """Instructions of one segment_copy_kernel, in the order in which they are laid out."""
+    symbol = re.compile(r"segment_copy_kernelILi%dELb%dELb%dELi%dE" % (MODES[mode], streamed_loads, paced, STREAMED))
+    for path in code_objects:
+        names = subprocess.run([LLVM + "llvm-objdump", "-t", path], check=True, stdout=subprocess.PIPE, text=True).stdout.split()
+        for name in names:
+            if symbol.search(name) and re.fullmatch(r"\w+", name):
+                text = subprocess.run([LLVM + "llvm-objdump", "-d", "--no-show-raw-insn", "--disassemble-symbols=" + name, path],
+                                      check=True, stdout=subprocess.PIPE, text=True).stdout
+                return [line.split("//")[0].strip() for line in text.splitlines() if line.startswith("\t")]
+    raise AssertionError("no kernel for " + mode)
+
+
+def _places(code, what):
+    return [i for i, line in enumerate(code) if re.match(what, line)]
+
+
+@pytest.mark.parametrize("mode", sorted(MODES))
+def test_edge_bytes_wait_beside_the_vectors(code_objects, mode):
+    """The bytes around the vectors are stored after the vectors' load has gone out, not in a round trip before it."""
+    code = _kernel(code_objects, mode)
+    load, = _places(code, r"global_load_dwordx4")
+    assert min(_places(code, r"global_store_byte")) > load

@@ -61,3 +61,29 @@ def test_alltoall_of_a_family_of_teams():
                     assert np.array_equal(rt.download(dst, pe, (len(members) * n,), np.uint8), want[k]), (members, pe)
         rt.team_destroy(xt); rt.team_destroy(yt)
         rt.free(src); rt.free(dst)
+
+
+@pytest.mark.parametrize("npes", [2, 8, 16])
+def test_segments_around_the_order_of_edges_and_vectors(npes):
+    """Short segments store their edge bytes before the vectors, longer ones behind them; segments of one PE touch those
+    of its neighbours in the middle of a vector."""
+    rng = np.random.default_rng(50 + npes)
+    with runtime(npes, 2 << 20) as rt:
+        src = rt.malloc(npes * 1100 + 64); dst = rt.malloc(npes * 1100 + 64)
+        for n in (16, 17, 33, 511, 512, 513, 1039):
+            data = rng.integers(0, 256, (npes, npes * n), dtype=np.uint8)
+            one = np.ascontiguousarray(data[:, :n])
+            for doff, soff in OFFSETS:
+                rt.upload_all(src, data, soff)
+                note("npes=%d n=%d dst+%d src+%d" % (npes, n, doff, soff))
+                for what, nbytes, want in (("fcollect", npes * n, O.fcollect(one)), ("broadcast", n, O.broadcast(one, 1)),
+                                           ("alltoall", npes * n, O.alltoall(data))):
+                    rt.fill(dst, 0xCD, nbytes + 64)
+                    if what == "broadcast":
+                        rt.broadcastmem(dst + doff, src + soff, n, 1)
+                    else:
+                        (rt.fcollectmem if what == "fcollect" else rt.alltoallmem)(dst + doff, src + soff, n)
+                    got = rt.download_all(dst, (nbytes + 64,), np.uint8)
+                    assert np.array_equal(got[:, doff:doff + nbytes], want), (what, n, doff, soff)
+                    assert (got[:, :doff] == 0xCD).all() and (got[:, doff + nbytes:] == 0xCD).all(), (what, n, doff, soff)
+        rt.free(src); rt.free(dst)
