@@ -134,9 +134,9 @@ __device__ __forceinline__ void stream_store_at(char *p, unsigned off, nvshmemi_
 //
 // fcollect and broadcast store the piece to every member, in one of two ways:
 //  - back to back, while the whole grid is in flight at once.  Small messages are latency: with the stores of a loop
-//    that waits for each before the next, every destination costs a quarter of a microsecond (16 B to 64 KiB per
-//    member, replayed from a graph: fcollect to 8 / 16 members 3.8 / 5.5 us one by one, 1.8 / 2.1 back to back,
-//    broadcast to 8 3.7 and 1.7);
+//    that waits for each before the next, every destination costs a quarter of a microsecond (64 bytes to 64 KiB per
+//    member, replayed from a graph: fcollect to 8 / 16 members 3.4-4.5 / 5.4-6.9 us one by one, 1.9-2.9 / 2.0-4.1 back to
+//    back, broadcast of up to 64 KiB to 8 3.1-3.9 and 1.8-2.1);
 //  - PACED, one destination after the other, each store acknowledged before the next is issued, in larger grids.
 //    They are bound by how the memory system takes writes, and that favours few write fronts: blocks that start
 //    together then write to one destination at a time instead of all 8 or 16 (broadcast of 32 MiB to 8: 47.4 us back
@@ -213,6 +213,11 @@ __global__ __launch_bounds__(64) void segment_copy_kernel(segment_args_t a) {
     const uint64_t pos = k < head ? k : nvec * 16 + k;
     unsigned b = 0;
     if (edge) b = (unsigned char)src[pos];
+    // The wait for both loads belongs here, once: left to the compiler it stands in front of every group of stores below,
+    // where it also waits for the stores before (fcollect to 16 / 64 members of 64 bytes 2.3 / 5.5 us, like this 2.0 / 3.6).
+    // An alltoall stores once, and its edge bytes do better behind the vectors' acknowledgement (16 PEs, 65533 bytes: 6.7
+    // us against 6.85).
+    if (MODE != kModeAlltoall) asm volatile("" : "+v"(v), "+v"(b));
     auto store_edges = [&]() {
         if (!edge) return;
         const unsigned half = lane >> 5;

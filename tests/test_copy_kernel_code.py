@@ -60,3 +60,11 @@ def test_edge_bytes_wait_beside_the_vectors(code_objects, mode):
     code = _kernel(code_objects, mode)
     load, = _places(code, r"global_load_dwordx4")
     assert min(_places(code, r"global_store_byte")) > load
+
+
+@pytest.mark.parametrize("mode", ["fcollect", "broadcast"])
+def test_stores_to_several_members_do_not_wait(code_objects, mode):
+    """Back to back: the loads are waited for once, and no wait stands between the stores (or in their loops)."""
+    code = _kernel(code_objects, mode)
+    first = min(_places(code, r"global_store_dwordx4"))
+    assert not [i for i in _places(code, r"s_waitcnt.*vmcnt") if i > first]
