@@ -530,10 +530,11 @@ static uint64_t total_members(const TeamLaunch &tl) {
     return (uint64_t)tl.ngroups * (uint64_t)tl.max_size;
 }
 
-// How fcollect and broadcast store: paced beyond Runtime::paced_copy_blocks (9 to a compute unit: 8 pieces and what a
-// message that is no power of two adds), up to which a grid is in flight all at once.  us paced / back to back at 1024,
-// 2048 and 4096 blocks: fcollect to 4 members 2.8 / 2.2, 3.2 / 2.8 and 4.1 / 4.0; to 8 4.2 / 2.8, 4.7 / 4.4 and
-// 6.5 / 7.1; to 16 6.1 / 4.0, 7.0 / 6.6 and 11.1 / 12.2; broadcast to 8 4.2 / 2.7, 4.7 / 4.1 and 6.3 / 6.5.
+// How fcollect and broadcast store: paced beyond Runtime::paced_copy_blocks (33 to a compute unit: the 32 wavefronts it
+// holds and what a message that is no power of two adds), up to which a grid is in flight all at once.  us paced / back
+// to back at 1024, 4096, 8192 and 16384 blocks: fcollect to 4 members 3.3 / 2.5, 4.5 / 4.0, 7.0 / 6.4 and 11.2 / 11.5; to 8
+// 4.5 / 2.9, 7.8 / 6.4, 12.1 / 11.6 and 20.7 / 23.5; to 16 6.9 / 4.1, 14.4 / 11.7, 23.2 / 23.3 and 41.4 / 43.9;
+// broadcast to 8 4.1 / 2.9, 7.5 / 6.4, 11.9 / 11.4 and 21.0 / 23.8.
 static bool paced_copy(const Runtime &rt, uint64_t blocks) { return blocks > rt.paced_copy_blocks; }
 // Dynamic LDS that nobody uses: it limits the wavefronts of a paced copy that a compute unit (160 KiB) holds.  16 of
 // the 32 possible when the cache can hold the sources from one call to the next; their loads take longer from memory

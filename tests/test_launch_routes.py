@@ -21,3 +21,20 @@ def test_collective_launches_are_cooperative_unless_asked(recorded, plain, coope
     another stream: side by side, each could hold compute units that the other waits for."""
     env = {} if plain is None else {"NVSHMEM_AMD_PLAIN_COLLECTIVE_LAUNCH": plain}
     recorded(COLLECTIVE_LAUNCH % cooperative, **env)
+
+
+def test_copies_that_are_in_flight_all_at_once_are_not_paced(recorded):  # noqa: F811
+    """fcollect and broadcast of up to 32 pieces per compute unit store back to back, larger ones one destination at a
+    time (third template argument of the kernel)."""
+    recorded("""
+for npes in (4, 8, 16):
+    ok(lib.nvshmemx_amd_init(npes, 256 << 20))
+    a, b = lib.nvshmem_malloc(64 << 20), lib.nvshmem_malloc(128 << 20)
+    launches()
+    for blocks, paced in ((1, 0), (3000, 0), (8192, 0), (8700, 1), (20000, 1)):
+        ok(lib.nvshmemx_fcollectmem_on_stream(0, b, a, blocks // npes * 1024 or 1, None))
+        ok(lib.nvshmemx_broadcastmem_on_stream(0, b, a, blocks * 1024 - 5, 1, None))
+        for kernel, cooperative, grid, block, lds in launches():
+            assert "ELb%dELi" % paced in kernel and (lds > 0) == bool(paced), (npes, blocks, kernel, lds)
+    lib.nvshmem_finalize()
+""")
