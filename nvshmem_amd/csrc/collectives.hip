@@ -216,8 +216,9 @@ __global__ __launch_bounds__(64) void segment_copy_kernel(segment_args_t a) {
     // The wait for both loads belongs here, once: left to the compiler it stands in front of every group of stores below,
     // where it also waits for the stores before (fcollect to 16 / 64 members of 64 bytes 2.3 / 5.5 us, like this 2.0 / 3.6).
     // An alltoall stores once, and its edge bytes do better behind the vectors' acknowledgement (16 PEs, 65533 bytes: 6.7
-    // us against 6.85).
-    if (MODE != kModeAlltoall) asm volatile("" : "+v"(v), "+v"(b));
+    // us against 6.85); a paced copy waits in any case, and with streamed loads it loses 10 % by the wait out here
+    // (broadcast of 512 MiB to 8 734 us, 807 so; fcollect of 16 x 32 MiB 1446 and 1629).
+    if (MODE != kModeAlltoall && !PACED) asm volatile("" : "+v"(v), "+v"(b));
     auto store_edges = [&]() {
         if (!edge) return;
         const unsigned half = lane >> 5;
