@@ -537,16 +537,19 @@ static uint64_t total_members(const TeamLaunch &tl) {
 // 4.5 / 2.9, 7.8 / 6.4, 12.1 / 11.6 and 20.7 / 23.5; to 16 6.9 / 4.1, 14.4 / 11.7, 23.2 / 23.3 and 41.4 / 43.9;
 // broadcast to 8 4.1 / 2.9, 7.5 / 6.4, 11.9 / 11.4 and 21.0 / 23.8.
 static bool paced_copy(const Runtime &rt, uint64_t blocks) { return blocks > rt.paced_copy_blocks; }
-// Dynamic LDS that nobody uses: it limits the wavefronts of a paced copy that a compute unit (160 KiB) holds.  16 of
-// the 32 possible when the cache can hold the sources from one call to the next; their loads take longer from memory
-// and more wavefronts are needed to cover that, 24, or 20 with 16 destinations and more, which keep a wavefront
-// storing for longer.  us with 32 / 24 / 20 / 16 (sources | destinations in all): fcollect 8 members 32 MiB | 256 MiB
-// 43.3 / 43.1 / 42.9 / 42.3, 16 members 64 MiB | 1 GiB 177.9 / 167.1 / 162.1 / 157.4, 8 members 128 MiB | 1 GiB
-// 202 / 186 / 190 / 192, 4 members 128 MiB | 512 MiB 106.3 / 104.8 / 108.9 / 113.8, 16 members 128 MiB | 2 GiB 395 /
-// 341-376 / 345-373 / 376; broadcast 8 members 64 MiB | 512 MiB 85.1 / 83.1 / 82.3 / 81.7, 256 MiB | 2 GiB 376 / 372 /
-// 380 / 395, 64 members 32 MiB | 2 GiB 324-362 / 325-361 / 321-360 / 347.
+// Dynamic LDS that nobody uses: it limits the wavefronts of a paced copy that a compute unit (160 KiB) holds, and with
+// them the width of each write front.  16 of the 32 possible while the cache holds the sources.  Streamed loads take
+// longer and more wavefronts are needed to cover that: 24, and 28 from 12 destinations on, which keep a wavefront storing
+// for longer.  us with 16 / 20 / 24 / 28 wavefronts, random data, sources | destinations in all.  Cached: fcollect 4 members
+// 256 MiB | 1 GiB 178 / 183 / 186 / -, 8 members 128 MiB | 1 GiB 161 / 165 / 167 / -, 256 MiB | 2 GiB 322 / 328 / 332 / 334, 16
+// members 128 MiB | 2 GiB 304 / 312 / 318 / 322; broadcast to 8 of 256 MiB 322 / 328 / 331 / -, to 16 of 64 MiB 156 / 155 / 160 /
+// -.  Streamed: fcollect 8 members 512 MiB | 4 GiB 780 / 760 / 724 / 787, 12 members 384 MiB | 4.5 GiB 892 / 829 / 819 / 772, 16
+// members 384 MiB | 6 GiB - / 1082 / 1044 / 1019, 512 MiB | 8 GiB - / 1446 / 1387 / 1429, 1 GiB | 16 GiB - / 2916 / 2794 / 2761,
+// 32 members 512 MiB | 16 GiB - / 2681 / 2825 / 2610; broadcast of 512 MiB to 8 792 / 762 / 719 / 743, to 16 - / 1433 / 1359 /
+// 1347.  (Medians; runs of one size spread by up to 8 % from 16 destinations on, with where the memory lies.)
 static size_t paced_lds_bytes(const Runtime &rt, uint64_t source_bytes, int members) {
-    const unsigned waves = source_bytes * 2 < rt.cacheable_source_bytes ? 16 : members < 16 ? 24 : 20;
+    const bool streamed = source_bytes > rt.cacheable_source_bytes;
+    const unsigned waves = !streamed ? 16 : members < 12 ? 24 : 28;
     return ((size_t)160 << 10) / waves & ~(size_t)127;
 }
 
@@ -617,11 +620,11 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
     // Two-step allreduce of large teams: fold into member 0's destination (n loads and ONE store per vector, the
     // shape of the reducescatter), then broadcast that.  It moves 2 n + 2 units where the fused
     // kernel moves 2 n, but every block of the fused kernel feeds n write fronts of 1 KiB pieces, and its fold
-    // serialises n steps between two barriers.  fp32 sum, TB/s, fused / two-step at 512 MiB and 2 GiB of sources in
-    // all: 12 members 6.41 / 6.18 and 6.28 / 6.29, 16: 6.26 / 6.19 and 6.02 / 6.41, 24: 5.84 / 5.71 and 5.69 / 6.23,
-    // 32: 6.09 / 6.09 and 6.09 / 6.51, 48: 5.68 / 5.78 and 5.57 / 6.25, 64: 5.55 / 5.97 and 5.59 / 6.56.  So: from
-    // Runtime::two_step_reduce_members (16) members on when the sources hold two_step_reduce_bytes (512 MiB: 16 members 6.2 against 6.0 TB/s fused there, 32 members 6.3 against 5.8) or more,
-    // and from three times that many members whatever the size.
+    // serialises n steps between two barriers.  fp32 sum of random data, TB/s, fused / two-step at about 512 MiB and 2 to
+    // 4 GiB of sources in all: 12 members 6.02 / 6.03 and 6.23 / 6.20, 16: 6.12 / 6.25 and 6.12 / 6.32, 24: 5.72 / 6.24 and 5.79 /
+    // 6.39, 32: 6.28 / 6.19 and 6.35 / 6.42, 48: 5.87 / 6.38 and 5.94 / 6.47, 64: 5.86 / 5.81 and 6.01 / 6.47; at 256 MiB 16
+    // members 6.98 / 6.10, 32 6.93 / 6.27, 64 6.37 / 6.31.  So: from Runtime::two_step_reduce_members (16) members on when the
+    // sources hold two_step_reduce_bytes (512 MiB) or more, and from three times that many members whatever the size.
     if (rt.two_step_reduce_members && tl.min_size >= (int)rt.two_step_reduce_members &&
         (total_bytes >= rt.two_step_reduce_bytes || tl.min_size >= 3 * (int)rt.two_step_reduce_members) &&
         total_bytes >= lds_from_bytes) {

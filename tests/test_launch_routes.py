@@ -38,3 +38,18 @@ for npes in (4, 8, 16):
             assert "ELb%dELi" % paced in kernel and (lds > 0) == bool(paced), (npes, blocks, kernel, lds)
     lib.nvshmem_finalize()
 """)
+
+
+def test_wavefronts_of_paced_copies(recorded):  # noqa: F811
+    """A compute unit (160 KiB of LDS) holds 16 wavefronts of a paced copy whose sources the cache holds, more with
+    streamed loads (second template argument)."""
+    recorded("""
+for npes, mib, streamed, waves in ((8, 32, 0, 16), (16, 16, 0, 16), (16, 8, 0, 16), (8, 64, 1, 24), (16, 32, 1, 28), (32, 16, 1, 28)):
+    ok(lib.nvshmemx_amd_init(npes, (npes + 2) * mib << 20))
+    a, b = lib.nvshmem_malloc(mib << 20), lib.nvshmem_malloc(npes * mib << 20)
+    launches()
+    ok(lib.nvshmemx_fcollectmem_on_stream(0, b, a, mib << 20, None))
+    (kernel, _, grid, block, lds), = launches()
+    assert "ILi0ELb%dELb1E" % streamed in kernel and (160 << 10) // lds == waves, (npes, mib, kernel, lds)
+    lib.nvshmem_finalize()
+""")
