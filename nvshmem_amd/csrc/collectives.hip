@@ -308,7 +308,15 @@ __device__ __forceinline__ void reduce_edges(char *dst, const char *src, const r
     const T *from = reinterpret_cast<const T *>(src) + k;
     const uint64_t es = pe_stride / sizeof(T);
     T acc = from[0];
-    for (int p = 1; p < npes; ++p) acc = fold_next<T, OP, SCATTER>(p, acc, from[(uint64_t)p * es]);
+    constexpr int kBatch = 8;  // loads in flight (beyond the last member: that one again)
+    for (int p0 = 1; p0 < npes; p0 += kBatch) {
+        T x[kBatch];
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) x[j] = from[(uint64_t)(p0 + j < npes ? p0 + j : npes - 1) * es];
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j)
+            if (p0 + j < npes) acc = fold_next<T, OP, SCATTER>(p0 + j, acc, x[j]);
+    }
     for (int p = 0; p < copies; ++p) reinterpret_cast<T *>(dst + (uint64_t)p * pe_stride)[k] = acc;
 }
 

@@ -1,5 +1,5 @@
-"""What the compiler made of the small form of the segment copy: messages that take a few microseconds are bound by the
-memory round trips a wavefront makes one after the other, and those can be read from the waits in its code."""
+"""What the compiler made of kernels for small messages: those that take a few microseconds are bound by the memory round
+trips a wavefront makes one after the other, and these can be read from the loads and waits in its code."""
 import os
 import re
 import struct
@@ -39,7 +39,11 @@ def code_objects(tmp_path_factory):
 
 def _kernel(code_objects, mode, streamed_loads=False, paced=False):
     """Instructions of one segment_copy_kernel, in the order in which they are laid out."""
-    symbol = re.compile(r"segment_copy_kernelILi%dELb%dELb%dELi%dE" % (MODES[mode], streamed_loads, paced, STREAMED))
+    return _code(code_objects, r"segment_copy_kernelILi%dELb%dELb%dELi%dE" % (MODES[mode], streamed_loads, paced, STREAMED))
+
+
+def _code(code_objects, kernel):
+    symbol = re.compile(kernel)
     for path in code_objects:
         names = subprocess.run([LLVM + "llvm-objdump", "-t", path], check=True, stdout=subprocess.PIPE, text=True).stdout.split()
         for name in names:
@@ -47,7 +51,7 @@ def _kernel(code_objects, mode, streamed_loads=False, paced=False):
                 text = subprocess.run([LLVM + "llvm-objdump", "-d", "--no-show-raw-insn", "--disassemble-symbols=" + name, path],
                                       check=True, stdout=subprocess.PIPE, text=True).stdout
                 return [line.split("//")[0].strip() for line in text.splitlines() if line.startswith("\t")]
-    raise AssertionError("no kernel for " + mode)
+    raise AssertionError("no kernel " + kernel)
 
 
 def _places(code, what):
@@ -68,3 +72,18 @@ def test_stores_to_several_members_do_not_wait(code_objects, mode):
     code = _kernel(code_objects, mode)
     first = min(_places(code, r"global_store_dwordx4"))
     assert not [i for i in _places(code, r"s_waitcnt.*vmcnt") if i > first]
+
+
+@pytest.mark.parametrize("kernel", ["reduce_gather_kernelIfLi5ELi0ELb0ELb0E", "reducescatter_gather_kernelIfLi5ELi0ELb0E"])
+def test_edge_elements_of_many_members_are_loaded_together(code_objects, kernel):
+    """Teams whose size is not known at compile time: the elements around the vectors, one word each, are fetched from
+    eight members at a time, without a wait between the loads."""
+    code = _code(code_objects, kernel)
+    longest = run = 0
+    for line in code:
+        if re.match(r"global_load_dword ", line):
+            run += 1
+            longest = max(longest, run)
+        elif re.match(r"s_waitcnt.*vmcnt", line):
+            run = 0
+    assert longest >= 8
