@@ -591,7 +591,7 @@ static int launch_broadcast(Runtime &rt, const TeamLaunch &tl, uint64_t doff, ui
 
 template <typename T, int OP>
 void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t src_off,
-                   uint64_t nelems, hipStream_t stream) {
+                   uint64_t nelems, uint64_t all, hipStream_t stream) {
     const unsigned ngroups = (unsigned)tl.ngroups;
     const reduce_shape_t shape = reduce_shape<T>(rt, dst_off, src_off, nelems);
     const uint64_t nvec = shape.nvec;
@@ -611,7 +611,7 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
     // per lane measured best where the block stays within 16 wavefronts, and wavefronts of fewer than
     // 64 lanes per member (512- or 256-byte accesses) lost 7-22 % against the gather kernel.  The
     // compile-time team size is worth 6 % at 32 members (6.17 against 5.82), nothing at 64.
-    const uint64_t total_bytes = total_members(tl) * nelems * sizeof(T);
+    const uint64_t total_bytes = total_members(tl) * all * sizeof(T);
     const int fixed_size = tl.min_size == tl.max_size ? tl.max_size : 0;
     const bool stream_source = total_bytes > rt.cacheable_source_bytes;
     // (in bytes whatever the element type: fp32, bf16 and int64 cross over at the same 64 MiB on 8 and 16 members)
@@ -636,18 +636,15 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
     if (rt.two_step_reduce_members && tl.min_size >= (int)rt.two_step_reduce_members &&
         (total_bytes >= rt.two_step_reduce_bytes || tl.min_size >= 3 * (int)rt.two_step_reduce_members) &&
         total_bytes >= lds_from_bytes) {
-        uint64_t blocks = (nvec + 63 + 63) / 64;
-        if (blocks <= 0x7fffffffull) {
-            const dim3 grid((unsigned)blocks, 1, ngroups);
-            if (stream_source)
-                hipLaunchKernelGGL((reduce_gather_kernel<T, OP, 0, true, true>), grid, dim3(64), 0, stream, rt.base,
-                                   rt.heap_size, tl.groups, shape);
-            else
-                hipLaunchKernelGGL((reduce_gather_kernel<T, OP, 0, false, true>), grid, dim3(64), 0, stream, rt.base,
-                                   rt.heap_size, tl.groups, shape);
-            (void)launch_broadcast(rt, tl, dst_off, dst_off, nelems * sizeof(T), 0, stream);
-            return;
-        }
+        const dim3 grid((unsigned)((nvec + 63 + 63) / 64), 1, ngroups);
+        if (stream_source)
+            hipLaunchKernelGGL((reduce_gather_kernel<T, OP, 0, true, true>), grid, dim3(64), 0, stream, rt.base,
+                               rt.heap_size, tl.groups, shape);
+        else
+            hipLaunchKernelGGL((reduce_gather_kernel<T, OP, 0, false, true>), grid, dim3(64), 0, stream, rt.base,
+                               rt.heap_size, tl.groups, shape);
+        (void)launch_broadcast(rt, tl, dst_off, dst_off, nelems * sizeof(T), 0, stream);
+        return;
     }
     if (mpw && total_bytes >= lds_from_bytes) {
         const uint32_t lane_shift = 6;
@@ -658,11 +655,7 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
         constexpr int kVptNarrow = sizeof(T) <= 2 ? NVSHMEM_AMD_REDUCE_VPT_NARROW : NVSHMEM_AMD_REDUCE_VPT;
         const int vpt = (ct_size == 8 || ct_size == 16) ? kVptNarrow : NVSHMEM_AMD_REDUCE_VPT;
         const uint64_t tile_vecs = (uint64_t)vpt << lane_shift;
-        uint64_t blocks = (nvec + (1u << lane_shift) + tile_vecs - 1) / tile_vecs;  // room for the lead-in
-        if (blocks > 0x7fffffffull) {
-            set_error("reduce: message too large");
-            return;
-        }
+        const uint64_t blocks = (nvec + (1u << lane_shift) + tile_vecs - 1) / tile_vecs;  // room for the lead-in
         const size_t lds = ((size_t)tl.max_size + 1) * 16 * tile_vecs;
         const dim3 grid((unsigned)blocks, 1, ngroups);
 #define NVSHMEM_AMD_LAUNCH_REDUCE(N, MPW) NVSHMEM_AMD_LAUNCH_REDUCE_V(N, MPW, NVSHMEM_AMD_REDUCE_VPT)
@@ -683,12 +676,8 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
 #undef NVSHMEM_AMD_LAUNCH_REDUCE
 #undef NVSHMEM_AMD_LAUNCH_REDUCE_V
     } else {
-        uint64_t blocks = (nvec + 63 + 63) / 64;  // room for the lead-in; at least one block for the edges
-        if (blocks > 0x7fffffffull) {
-            set_error("reduce: message too large");
-            return;
-        }
-        const dim3 grid((unsigned)blocks, 1, ngroups);
+        // room for the lead-in; at least one block for the edges
+        const dim3 grid((unsigned)((nvec + 63 + 63) / 64), 1, ngroups);
 #define NVSHMEM_AMD_LAUNCH_GATHER_REDUCE(N)                                                            \
     do {                                                                                               \
         if (stream_source)                                                                             \
@@ -706,21 +695,17 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
     }
 }
 
-// reducescatter: grid.y = destination member; nelems is the element count of one PE's result
+// reducescatter: grid.y = destination member; nelems of the `all` elements of one PE's result
 template <typename T, int OP>
 void launch_reducescatter(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t src_off,
-                          uint64_t nelems, hipStream_t stream) {
+                          uint64_t nelems, uint64_t all, hipStream_t stream) {
     const reduce_shape_t shape = reduce_shape<T>(rt, dst_off, src_off, nelems);
     const uint64_t blocks = (shape.nvec + 63 + 63) / 64;  // room for the lead-in; at least one block for the edges
-    if (blocks > 0x7fffffffull) {
-        set_error("reducescatter: message too large");
-        return;
-    }
     const dim3 grid((unsigned)blocks, (unsigned)tl.max_size, (unsigned)tl.ngroups);
-    const bool stream_source = total_members(tl) * tl.max_size * nelems * sizeof(T) > rt.cacheable_source_bytes;
+    const bool stream_source = total_members(tl) * tl.max_size * all * sizeof(T) > rt.cacheable_source_bytes;
 #define NVSHMEM_AMD_LAUNCH_GATHER(N, NTL)                                                         \
     hipLaunchKernelGGL((reducescatter_gather_kernel<T, OP, N, NTL>), grid, dim3(64), 0, stream,   \
-                       rt.base, rt.heap_size, tl.groups, shape, nelems * sizeof(T))
+                       rt.base, rt.heap_size, tl.groups, shape, all * sizeof(T))
     if (tl.min_size == 8 && tl.max_size == 8) {
         if (stream_source) NVSHMEM_AMD_LAUNCH_GATHER(8, true);
         else NVSHMEM_AMD_LAUNCH_GATHER(8, false);
@@ -731,8 +716,17 @@ void launch_reducescatter(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, u
 #undef NVSHMEM_AMD_LAUNCH_GATHER
 }
 
-typedef void (*reduce_launcher_t)(Runtime &, const TeamLaunch &, uint64_t, uint64_t, uint64_t,
-                                  hipStream_t);
+typedef void (*reduce_launcher_t)(Runtime &, const TeamLaunch &, uint64_t, uint64_t, uint64_t, uint64_t, hipStream_t);
+
+// A launch holds fewer than 2^32 threads, and the LDS-staged kernel has up to 1024 of them for every KiB of one PE's
+// result: a reduction goes out in pieces of 2 GiB per PE, of 2^21 blocks.
+constexpr uint64_t kReducePieceBytes = (uint64_t)2 << 30;
+void launch_pieces(reduce_launcher_t fn, Runtime &rt, const TeamLaunch &tl, uint64_t doff, uint64_t soff, uint64_t nelems,
+                   size_t es, hipStream_t stream) {
+    const uint64_t piece = kReducePieceBytes / es;
+    for (uint64_t done = 0; done < nelems; done += piece)
+        fn(rt, tl, doff + done * es, soff + done * es, nelems - done < piece ? nelems - done : piece, nelems, stream);
+}
 
 template <typename T, bool SCATTER>
 reduce_launcher_t pick_arith(int op) {
@@ -809,7 +803,7 @@ int reduce_on_stream(int dtype, int op, nvshmem_team_t team, void *dest, const v
         set_error("reduce: dest and source overlap without being identical");
         return NVSHMEMX_ERROR_INVALID_VALUE;
     }
-    fn(rt, tl, doff, soff, nreduce, stream);
+    launch_pieces(fn, rt, tl, doff, soff, nreduce, es, stream);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         set_error("reduce: kernel launch failed: %s", hipGetErrorString(e));
@@ -850,7 +844,7 @@ int reducescatter_on_stream(int dtype, int op, nvshmem_team_t team, void *dest, 
         set_error("reducescatter: dest and source overlap");
         return NVSHMEMX_ERROR_INVALID_VALUE;
     }
-    fn(rt, tl, doff, soff, nreduce, stream);
+    launch_pieces(fn, rt, tl, doff, soff, nreduce, es, stream);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         set_error("reducescatter: kernel launch failed: %s", hipGetErrorString(e));

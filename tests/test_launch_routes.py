@@ -53,3 +53,27 @@ for npes, mib, streamed, waves in ((8, 32, 0, 16), (16, 16, 0, 16), (16, 8, 0, 1
     assert "ILi0ELb%dELb1E" % streamed in kernel and (160 << 10) // lds == waves, (npes, mib, kernel, lds)
     lib.nvshmem_finalize()
 """)
+
+
+@pytest.mark.parametrize("npes,gib", [(8, 9), (3, 18), (16, 5), (2, 65), (1, 65)])
+def test_the_largest_reductions_are_launched_whole(recorded, npes, gib):  # noqa: F811
+    """No launch of 2^32 threads or more, however long and ragged the buffers are: every element in one piece or another."""
+    recorded("""
+npes, nbytes = %d, %d << 30
+ok(lib.nvshmemx_amd_init(npes, nbytes + (1 << 30)))
+a = lib.nvshmem_malloc(nbytes + 64)
+launches()
+for name, es in (("float", 4), ("bfloat16", 2), ("double", 8)):
+    n = nbytes // es - 3
+    ok(_lib.typed_coll(lib, "nvshmemx_%%s_sum_reduce_on_stream" %% name, True)(0, a + es, a + es, n, None))
+    vectors = sum((grid[0] - 2) * 64 for kernel, _, grid, block, lds in launches() if "reduce_" in kernel)
+    assert n * es // 16 - 4096 <= vectors <= n * es // 16 + 64, (name, vectors)
+if npes == 1:
+    b = lib.nvshmem_malloc(1 << 20)
+    fn = _lib.typed_coll(lib, "nvshmemx_float_sum_reducescatter_on_stream", True)
+    ok(lib.nvshmem_finalize() or lib.nvshmemx_amd_init(1, 2 * nbytes + (1 << 30)))
+    a, b = lib.nvshmem_malloc(nbytes + 64), lib.nvshmem_malloc(nbytes + 64)
+    launches()
+    ok(fn(0, b + 4, a + 8, nbytes // 4 - 3, None))
+    assert sum(grid[0] * 64 for _, _, grid, _, _ in launches()) >= nbytes // 16 - 4096
+""" % (npes, gib))
