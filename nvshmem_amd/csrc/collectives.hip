@@ -282,8 +282,8 @@ __device__ __forceinline__ T fold_next(int p, T acc, T x) {
 // elements in front of and behind them, fewer than 16 bytes on either side.  Stores are aligned that way whatever
 // the buffers are; a source on another offset is read with unaligned vector loads, which cost 3-4 % here (allreduce of
 // 8 x 25 MiB bf16: 73 us with both buffers on the same offset, aligned or not, 76 with different ones; an
-// element per thread and load, which such buffers took before, 155 and 148 us.  reducescatter of 8 x 8 x 3 MB bf16 with
-// blocks of an odd number of elements: 91 -> 42 us; with aligned blocks 39).
+// element per lane and load takes 155 and 148 us.  reducescatter of 8 x 8 x 3 MB bf16 with blocks of an odd number of
+// elements: 42 us, an element per lane 91; with aligned blocks 39).
 struct reduce_shape_t {
     uint64_t dst, src;   // byte offsets of the destination and the source in a slice
     uint64_t nvec;       // whole vectors
@@ -479,6 +479,28 @@ __global__ __launch_bounds__(64) void reduce_gather_kernel(char *base, uint64_t 
         reduce_edges<T, OP, false>(base + s.dst, base + s.src, s, pe_stride, npes, ROOT_ONLY ? 1 : npes);
 }
 
+// One element per lane and load, for small messages whose buffers are no whole vectors (element_at_a_time): what
+// counts there is how long one lane is at work, and a lane of the vector kernels folds 2 to 16 elements, one after the
+// other in 1- and 2-byte types, with the edges before or behind them.
+template <typename T, int OP, bool SCATTER = false>
+__global__ __launch_bounds__(256) void reduce_element_kernel(char *base, uint64_t slice_bytes,
+                                                             const nvshmemi_amd_team_view_t *groups, uint64_t dst_off,
+                                                             uint64_t src_off, uint64_t nelems) {
+    const nvshmemi_amd_team_view_t g = groups[blockIdx.z];
+    const int npes = g.size;
+    if (SCATTER && (int)blockIdx.y >= npes) return;
+    const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= nelems) return;
+    base += (uint64_t)g.start * slice_bytes;
+    const uint64_t es = ((uint64_t)g.stride * slice_bytes) / sizeof(T);
+    const T *s = reinterpret_cast<const T *>(base + src_off) + (SCATTER ? (uint64_t)blockIdx.y * nelems : 0);
+    T *d = reinterpret_cast<T *>(base + dst_off) + (SCATTER ? (uint64_t)blockIdx.y * es : 0);
+    T acc = s[i];
+    for (int pe = 1; pe < npes; ++pe) acc = fold_next<T, OP, SCATTER>(pe, acc, s[(uint64_t)pe * es + i]);
+    if (SCATTER) d[i] = acc;
+    else for (int pe = 0; pe < npes; ++pe) d[(uint64_t)pe * es + i] = acc;
+}
+
 // reducescatter without LDS: a block is ONE wavefront, lane i loads vector i of a 1 KiB piece of block q
 // (blockIdx.y) from every member - eight independent loads in flight per lane at a time - folds them in
 // member order in registers and stores one vector into member q's destination.  The work is nearly all
@@ -589,6 +611,25 @@ static int launch_broadcast(Runtime &rt, const TeamLaunch &tl, uint64_t doff, ui
     return 0;
 }
 
+// Whether a reduction that would take a gather kernel folds one element per lane instead.  Aligned buffers never do.
+// Ragged ones with up to Runtime::element_reduce_bytes of results (512 KiB) do, except where the vector kernel is the
+// faster one all the same: allreduces of 4- and 8-byte elements on 4 and more members, and teams whose size it knows at
+// compile time, where it only loses 1- and 2-byte elements of up to 32 KiB (allreduce: 8 KiB) of results.
+// us element / vector, allreduce of 4 KiB, 64 KiB, 512 KiB and 1 MiB: int8 on 2 members 2.0 / 3.3, 2.1 / 3.2, 3.2 / 3.4 and 4.8
+// / 4.2, on 16 3.0 / 6.6, 3.3 / 6.3, 6.7 / 6.9 and 12.8 / 8.3, on 64 7.1 / 24, 8.1 / 23, 19 / 25 and 38 / 38; bf16 on 16 3.5 / 5.2,
+// 3.6 / 5.0, 5.4 / 5.7 and 13.6 / 6.9; fp32 on 2 2.0 / 2.6, 2.1 / 2.4, 2.4 / 2.6 and 2.8 / 2.9, on 3 2.4 / 2.7, 2.4 / 2.7, 2.7 /
+// 2.8, on 16 4.6 / 3.6, 4.7 / 3.6, 6.0 / 4.3; int8 on 8 2.5 / 2.6, 2.9 / 2.7.  reducescatter with 32 KiB and 512 KiB of results
+// in all: int8 on 4 members 2.4 / 3.5 and 3.5 / 3.6, on 16 3.0 / 6.5 and 4.4 / 6.4, on 8 2.6 / 2.8 and 4.1 / 2.9; fp32 on 4
+// 2.4 / 2.6 and 2.6 / 2.8, on 16 3.4 / 3.7 and 3.5 / 3.7.
+template <typename T, bool SCATTER>
+bool element_at_a_time(const Runtime &rt, const TeamLaunch &tl, bool known_size, uint64_t dst_off, uint64_t src_off,
+                       uint64_t nelems) {
+    const uint64_t bytes = nelems * sizeof(T), results = SCATTER ? bytes * (uint64_t)tl.max_size : bytes;
+    if (((dst_off | src_off | (SCATTER ? bytes : 0)) & 15) == 0) return false;
+    if (known_size) return sizeof(T) <= 2 && results <= rt.element_reduce_bytes / (SCATTER ? 16 : 64);
+    return (SCATTER || sizeof(T) <= 2 || tl.max_size <= 3) && results <= rt.element_reduce_bytes;
+}
+
 template <typename T, int OP>
 void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t src_off,
                    uint64_t nelems, uint64_t all, hipStream_t stream) {
@@ -675,6 +716,9 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
         else NVSHMEM_AMD_LAUNCH_REDUCE(0, 4);
 #undef NVSHMEM_AMD_LAUNCH_REDUCE
 #undef NVSHMEM_AMD_LAUNCH_REDUCE_V
+    } else if (element_at_a_time<T, false>(rt, tl, fixed_size == 4 || fixed_size == 8, dst_off, src_off, nelems)) {
+        hipLaunchKernelGGL((reduce_element_kernel<T, OP>), dim3((unsigned)((nelems + 255) / 256), 1, ngroups), dim3(256), 0,
+                           stream, rt.base, rt.heap_size, tl.groups, dst_off, src_off, nelems);
     } else {
         // room for the lead-in; at least one block for the edges
         const dim3 grid((unsigned)((nvec + 63 + 63) / 64), 1, ngroups);
@@ -699,6 +743,13 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
 template <typename T, int OP>
 void launch_reducescatter(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t src_off,
                           uint64_t nelems, uint64_t all, hipStream_t stream) {
+    const bool eight = tl.min_size == 8 && tl.max_size == 8;
+    if (nelems == all && element_at_a_time<T, true>(rt, tl, eight, dst_off, src_off, nelems)) {
+        const dim3 grid((unsigned)((nelems + 255) / 256), (unsigned)tl.max_size, (unsigned)tl.ngroups);
+        hipLaunchKernelGGL((reduce_element_kernel<T, OP, true>), grid, dim3(256), 0, stream, rt.base, rt.heap_size,
+                           tl.groups, dst_off, src_off, nelems);
+        return;
+    }
     const reduce_shape_t shape = reduce_shape<T>(rt, dst_off, src_off, nelems);
     const uint64_t blocks = (shape.nvec + 63 + 63) / 64;  // room for the lead-in; at least one block for the edges
     const dim3 grid((unsigned)blocks, (unsigned)tl.max_size, (unsigned)tl.ngroups);
@@ -706,7 +757,7 @@ void launch_reducescatter(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, u
 #define NVSHMEM_AMD_LAUNCH_GATHER(N, NTL)                                                         \
     hipLaunchKernelGGL((reducescatter_gather_kernel<T, OP, N, NTL>), grid, dim3(64), 0, stream,   \
                        rt.base, rt.heap_size, tl.groups, shape, all * sizeof(T))
-    if (tl.min_size == 8 && tl.max_size == 8) {
+    if (eight) {
         if (stream_source) NVSHMEM_AMD_LAUNCH_GATHER(8, true);
         else NVSHMEM_AMD_LAUNCH_GATHER(8, false);
     } else {

@@ -279,6 +279,7 @@ int nvshmemx_amd_init(int npes, size_t symmetric_size) {
     rt.cacheable_source_bytes = env_size("NVSHMEM_AMD_CACHEABLE_SOURCE_BYTES", (size_t)256 << 20);
     rt.paced_copy_blocks = env_size("NVSHMEM_AMD_PACED_COPY_BLOCKS", (uint64_t)rt.num_cus * 33);
     rt.lds_reduce_bytes = env_size("NVSHMEM_AMD_LDS_REDUCE_BYTES", (size_t)64 << 20);
+    rt.element_reduce_bytes = env_size("NVSHMEM_AMD_ELEMENT_REDUCE_BYTES", (size_t)512 << 10);
     rt.two_step_reduce_members = (unsigned)env_size("NVSHMEM_AMD_TWO_STEP_REDUCE_MEMBERS", 16);
     rt.two_step_reduce_bytes = env_size("NVSHMEM_AMD_TWO_STEP_REDUCE_BYTES", (size_t)512 << 20);
     if (!teams_init(rt)) {

@@ -69,6 +69,9 @@ struct Runtime {
     // together hold at least this many bytes (a quarter of it for teams of 17
     // to 32 members, four times for larger ones): NVSHMEM_AMD_LDS_REDUCE_BYTES, read at init
     uint64_t lds_reduce_bytes = (uint64_t)64 << 20;
+    // Reductions of ragged buffers with up to this many bytes of results fold one element per lane where that is the
+    // faster way: NVSHMEM_AMD_ELEMENT_REDUCE_BYTES, read at init (0 = never)
+    uint64_t element_reduce_bytes = (uint64_t)512 << 10;
     // An allreduce beyond the cache takes two steps - fold into member 0, broadcast - instead of the fused
     // kernel from this team size on (NVSHMEM_AMD_TWO_STEP_REDUCE_MEMBERS, read at init; 0 = never) when the
     // sources of all members together hold at least two_step_reduce_bytes (NVSHMEM_AMD_TWO_STEP_REDUCE_BYTES), and

@@ -10,7 +10,8 @@ from gpu_util import bits_equal, note, runtime
 pytestmark = pytest.mark.gpu
 
 FORMS = {
-    "gather": {"NVSHMEM_AMD_LDS_REDUCE_BYTES": str(1 << 40)},
+    "gather": {"NVSHMEM_AMD_LDS_REDUCE_BYTES": str(1 << 40), "NVSHMEM_AMD_ELEMENT_REDUCE_BYTES": "0"},
+    "element": {"NVSHMEM_AMD_LDS_REDUCE_BYTES": str(1 << 40), "NVSHMEM_AMD_ELEMENT_REDUCE_BYTES": str(1 << 40)},
     "lds": {"NVSHMEM_AMD_LDS_REDUCE_BYTES": "0", "NVSHMEM_AMD_TWO_STEP_REDUCE_MEMBERS": "0"},
     "two-step": {"NVSHMEM_AMD_LDS_REDUCE_BYTES": "0", "NVSHMEM_AMD_CHUNKED_COPY_BYTES": "0",
                  "NVSHMEM_AMD_TWO_STEP_REDUCE_MEMBERS": "2", "NVSHMEM_AMD_TWO_STEP_REDUCE_BYTES": "0"},
@@ -38,7 +39,7 @@ def _guarded(got, storage, first, n):
     return body, (got[:, :first * es] == 0xCD).all() and (got[:, (first + n) * es:] == 0xCD).all()
 
 
-@pytest.mark.parametrize("npes,form", [(2, "gather"), (8, "gather"), (8, "lds"), (5, "lds"), (16, "lds"), (16, "two-step")])
+@pytest.mark.parametrize("npes,form", [(2, "gather"), (5, "gather"), (8, "gather"), (3, "element"), (8, "element"), (16, "element"), (8, "lds"), (5, "lds"), (16, "lds"), (16, "two-step")])
 def test_ragged_allreduce(npes, form, monkeypatch):
     for k, v in FORMS[form].items():
         monkeypatch.setenv(k, v)
@@ -64,8 +65,10 @@ def test_ragged_allreduce(npes, form, monkeypatch):
         rt.free(src); rt.free(dst)
 
 
-@pytest.mark.parametrize("npes", [2, 8, 16])
-def test_ragged_reducescatter(npes):
+@pytest.mark.parametrize("npes,form", [(2, "gather"), (8, "gather"), (16, "gather"), (3, "element"), (8, "element"), (16, "element")])
+def test_ragged_reducescatter(npes, form, monkeypatch):
+    for k, v in FORMS[form].items():
+        monkeypatch.setenv(k, v)
     rng = np.random.default_rng(100 + npes)
     with runtime(npes, 4 << 20) as rt:
         src = rt.malloc(1 << 20); dst = rt.malloc(1 << 17)

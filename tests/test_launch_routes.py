@@ -77,3 +77,28 @@ if npes == 1:
     ok(fn(0, b + 4, a + 8, nbytes // 4 - 3, None))
     assert sum(grid[0] * 64 for _, _, grid, _, _ in launches()) >= nbytes // 16 - 4096
 """ % (npes, gib))
+
+
+def test_small_ragged_reductions_fold_an_element_per_lane(recorded):  # noqa: F811
+    """Ragged buffers with up to 512 KiB of results, but for the types and team sizes that the vector kernels serve faster;
+    aligned buffers never."""
+    recorded("""
+ELEMENT, VECTOR = True, False
+for npes, kind, name, nbytes, shift, element in (
+        (16, "reduce", "int8", 65537, 1, ELEMENT), (16, "reduce", "int8", 1 << 19, 1, ELEMENT), (16, "reduce", "int8", (1 << 19) + 1, 1, VECTOR),
+        (16, "reduce", "int8", 65536, 0, VECTOR), (16, "reduce", "float", 4100, 1, VECTOR), (3, "reduce", "float", 4100, 1, ELEMENT),
+        (2, "reduce", "double", 4104, 1, ELEMENT), (8, "reduce", "bfloat16", 8192, 1, ELEMENT), (8, "reduce", "bfloat16", 8194, 1, VECTOR),
+        (8, "reduce", "float", 404, 1, VECTOR), (4, "reduce", "int8", 100, 1, ELEMENT), (4, "reduce", "int8", 10000, 1, VECTOR),
+        (16, "reducescatter", "float", 32768, 1, ELEMENT), (16, "reducescatter", "float", 32772, 0, VECTOR),
+        (16, "reducescatter", "float", 32764, 0, ELEMENT), (16, "reducescatter", "float", 32752, 0, VECTOR),
+        (8, "reducescatter", "int8", 4095, 0, ELEMENT), (8, "reducescatter", "int8", 4097, 0, VECTOR), (8, "reducescatter", "float", 404, 0, VECTOR)):
+    es = {"int8": 1, "bfloat16": 2, "float": 4, "double": 8}[name]
+    ok(lib.nvshmemx_amd_init(npes, 32 << 20))
+    a, b = lib.nvshmem_malloc(16 << 20), lib.nvshmem_malloc(1 << 20)
+    launches()
+    ok(_lib.typed_coll(lib, "nvshmemx_%s_max_%s_on_stream" % (name, kind), True)(0, b + shift * es, a + shift * es, nbytes // es, None))
+    (kernel, _, grid, block, _), = launches()
+    assert ("reduce_element_kernel" in kernel) == element, (npes, kind, name, nbytes, shift, kernel)
+    assert not element or (grid[0] - 1) * block[0] < nbytes // es <= grid[0] * block[0]
+    lib.nvshmem_finalize()
+""")
