@@ -47,8 +47,8 @@ namespace {
 #ifndef NVSHMEM_AMD_REDUCE_WIDE_MPW
 #define NVSHMEM_AMD_REDUCE_WIDE_MPW 1
 #endif
-#ifndef NVSHMEM_AMD_COLL_NT /* bit 0: non-temporal loads allowed, bit 1: non-temporal stores */
-#define NVSHMEM_AMD_COLL_NT 3
+#ifndef NVSHMEM_AMD_COLL_NT /* non-temporal loads allowed */
+#define NVSHMEM_AMD_COLL_NT 1
 #endif
 /* Sources of up to Runtime::cacheable_source_bytes (all PEs together, 256 MiB unless the environment
  * says otherwise) are loaded with the default, cacheable policy: they fit the 256 MiB Infinity
@@ -56,23 +56,20 @@ namespace {
  * the 1M-element reduce, +20..45 % on 256 MiB collectives).  Larger sources are streamed with
  * non-temporal loads (+5 % at 2 GiB).  Stores always stream. */
 
-
 // (any byte alignment: one global_load_dwordx4 either way)
 template <bool NTL>
 __device__ __forceinline__ nvshmemi_v4u stream_load(const char *p) {
-    if (NTL && (NVSHMEM_AMD_COLL_NT & 1))
+    if (NTL && NVSHMEM_AMD_COLL_NT)
         return __builtin_nontemporal_load(reinterpret_cast<const nvshmemi_v4u_unaligned *>(p));
     return *reinterpret_cast<const nvshmemi_v4u_unaligned *>(p);
 }
-// How a kernel's result stores treat the caches.  All three stream (nothing here reads its output back);
-// they differ in where the line waits for memory.  Write-through stores (sc1) leave the L2 at once
-// instead of queuing behind its eviction of streaming lines: a write-only stream reaches 7.2 TB/s with
-// them against 6.3 TB/s with nt alone.  Which form wins depends on the kernel's mix (measured on MI355X,
-// random data): sc1 nt +4.5 % for the 8-member allreduce, +5..10 % for fcollect and cache-resident
-// broadcast, +1..3 % for alltoall and the gather allreduce; plain sc1 +5 % for the reducescatter, whose
-// one store per eight loads gains nothing from nt; and the kernels whose blocks share a piece through
-// the cache (destinations split over neighbouring blocks) lose 9..15 % with either, so they keep nt.
-enum { kStoreStream = 0 /* nt */, kStoreThrough = 1 /* sc1 */, kStoreThroughStream = 2 /* sc1 nt */ };
+// How a kernel's result stores treat the caches.  Both forms write through (nothing here reads its output back): the
+// line leaves the L2 at once instead of queuing behind its eviction of streaming lines, and a write-only stream
+// reaches 7.2 TB/s against 6.3 TB/s with nt alone.  Which of the two wins depends on the kernel's mix (measured on
+// MI355X, random data, against nt): sc1 nt +4.5 % for the 8-member allreduce, +5..10 % for fcollect and broadcast,
+// +1..3 % for alltoall and the gather allreduce; plain sc1 +5 % for the reducescatter, whose one store per eight loads
+// gains nothing from nt.
+enum { kStoreThrough = 1 /* sc1 */, kStoreThroughStream = 2 /* sc1 nt */ };
 #ifndef NVSHMEM_AMD_STORE_ALLTOALL
 #define NVSHMEM_AMD_STORE_ALLTOALL kStoreThroughStream
 #endif
@@ -102,12 +99,8 @@ template <int STORE>
 __device__ __forceinline__ void stream_store(char *p, nvshmemi_v4u v) {
     if (STORE == kStoreThrough)
         asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" : : "v"(p), "v"(v) : "memory");
-    else if (STORE == kStoreThroughStream)
-        asm volatile("global_store_dwordx4 %0, %1, off sc1 nt\n\ts_nop 1" : : "v"(p), "v"(v) : "memory");
-    else if (NVSHMEM_AMD_COLL_NT & 2)
-        __builtin_nontemporal_store(v, reinterpret_cast<nvshmemi_v4u *>(p));
     else
-        *reinterpret_cast<nvshmemi_v4u *>(p) = v;
+        asm volatile("global_store_dwordx4 %0, %1, off sc1 nt\n\ts_nop 1" : : "v"(p), "v"(v) : "memory");
 }
 // The same at p + off, p the same for all lanes: the address stays a scalar base and a 32-bit offset per lane.  (The
 // s_nop in front: a vector instruction that wrote the base - the compiler may have moved it out of a vector
@@ -116,10 +109,8 @@ template <int STORE>
 __device__ __forceinline__ void stream_store_at(char *p, unsigned off, nvshmemi_v4u v) {
     if (STORE == kStoreThrough)
         asm volatile("s_nop 4\n\tglobal_store_dwordx4 %0, %1, %2 sc1\n\ts_nop 1" : : "v"(off), "v"(v), "s"(p) : "memory");
-    else if (STORE == kStoreThroughStream)
-        asm volatile("s_nop 4\n\tglobal_store_dwordx4 %0, %1, %2 sc1 nt\n\ts_nop 1" : : "v"(off), "v"(v), "s"(p) : "memory");
     else
-        stream_store<STORE>(p + off, v);
+        asm volatile("s_nop 4\n\tglobal_store_dwordx4 %0, %1, %2 sc1 nt\n\ts_nop 1" : : "v"(off), "v"(v), "s"(p) : "memory");
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -13,7 +13,7 @@ FORMS = {
     "gather": {"NVSHMEM_AMD_LDS_REDUCE_BYTES": str(1 << 40), "NVSHMEM_AMD_ELEMENT_REDUCE_BYTES": "0"},
     "element": {"NVSHMEM_AMD_LDS_REDUCE_BYTES": str(1 << 40), "NVSHMEM_AMD_ELEMENT_REDUCE_BYTES": str(1 << 40)},
     "lds": {"NVSHMEM_AMD_LDS_REDUCE_BYTES": "0", "NVSHMEM_AMD_TWO_STEP_REDUCE_MEMBERS": "0"},
-    "two-step": {"NVSHMEM_AMD_LDS_REDUCE_BYTES": "0", "NVSHMEM_AMD_CHUNKED_COPY_BYTES": "0",
+    "two-step": {"NVSHMEM_AMD_LDS_REDUCE_BYTES": "0", "NVSHMEM_AMD_PACED_COPY_BLOCKS": "0",
                  "NVSHMEM_AMD_TWO_STEP_REDUCE_MEMBERS": "2", "NVSHMEM_AMD_TWO_STEP_REDUCE_BYTES": "0"},
 }
 # API type, operator, element kind, storage, (dest, source) offsets in elements

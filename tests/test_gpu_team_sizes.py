@@ -182,13 +182,12 @@ def test_small_in_kernel_collectives_with_and_without_packets(disable, plain, mo
 
 @pytest.mark.parametrize("npes", [3, 8, 13, 16, 33, 64])
 def test_large_source_policy_of_fcollect_and_broadcast(npes, monkeypatch):
-    """Sources beyond NVSHMEM_AMD_CACHEABLE_SOURCE_BYTES (read at init) are streamed, and from
-    NVSHMEM_AMD_CHUNKED_COPY_BYTES on fcollect / broadcast split the destinations of a piece over several
-    wavefronts (two per wavefront, the grid walking a chunk of the message once per pair).  With the
-    thresholds at zero every size takes that path: ragged, misaligned messages must come out the same, bytes
-    outside the destination untouched."""
+    """Sources beyond NVSHMEM_AMD_CACHEABLE_SOURCE_BYTES (read at init) are streamed, and beyond
+    NVSHMEM_AMD_PACED_COPY_BLOCKS pieces fcollect / broadcast store to one destination after the other.  With both
+    thresholds at zero every size takes the form of the largest messages, paced stores and streamed loads: ragged,
+    misaligned messages must come out the same, bytes outside the destination untouched."""
     monkeypatch.setenv("NVSHMEM_AMD_CACHEABLE_SOURCE_BYTES", "0")
-    monkeypatch.setenv("NVSHMEM_AMD_CHUNKED_COPY_BYTES", "0")
+    monkeypatch.setenv("NVSHMEM_AMD_PACED_COPY_BLOCKS", "0")
     monkeypatch.setenv("NVSHMEM_AMD_LDS_REDUCE_BYTES", "0")      # 8 and 16 members: the LDS-staged allreduce
     rng = np.random.default_rng(100 + npes)
     with runtime(npes, 1 << 24) as rt:
@@ -229,11 +228,11 @@ def test_large_source_policy_of_fcollect_and_broadcast(npes, monkeypatch):
 
 @pytest.mark.parametrize("npes", [5, 8, 16])
 def test_large_source_fcollect_and_broadcast_across_several_chunks(npes, monkeypatch):
-    """The large-source form of fcollect / broadcast walks the message in chunks of a few MiB, once per
-    group of destinations: a message of several chunks plus a ragged rest, misaligned at both ends, must
-    arrive whole on every member, with the bytes around the destination untouched."""
+    """The large-source form of fcollect / broadcast (paced stores, streamed loads) on more pieces than the GPU holds at
+    a time plus a ragged rest, misaligned at both ends: it must arrive whole on every member, with the bytes around the
+    destination untouched."""
     monkeypatch.setenv("NVSHMEM_AMD_CACHEABLE_SOURCE_BYTES", "0")
-    monkeypatch.setenv("NVSHMEM_AMD_CHUNKED_COPY_BYTES", "0")
+    monkeypatch.setenv("NVSHMEM_AMD_PACED_COPY_BLOCKS", "0")
     rng = np.random.default_rng(4100 + npes)
     nbytes = (9 << 20) + 1234
     with runtime(npes, (npes + 1) * (10 << 20) + (8 << 20)) as rt:
@@ -242,7 +241,7 @@ def test_large_source_fcollect_and_broadcast_across_several_chunks(npes, monkeyp
         for soff, doff in ((0, 0), (3, 21)):
             rt.upload_all(src, data, soff)
             rt.fill(dst, 0xCD, npes * nbytes + 256)
-            note("chunked fcollect npes=%d bytes=%d soff=%d doff=%d" % (npes, nbytes, soff, doff))
+            note("large-source fcollect npes=%d bytes=%d soff=%d doff=%d" % (npes, nbytes, soff, doff))
             rt.fcollectmem(dst + doff, src + soff, nbytes)
             want = O.fcollect(data)
             for pe in (0, npes // 2, npes - 1):
@@ -251,7 +250,7 @@ def test_large_source_fcollect_and_broadcast_across_several_chunks(npes, monkeyp
                 assert (got[:doff] == 0xCD).all() and (got[doff + npes * nbytes:] == 0xCD).all()
             root = npes - 2
             rt.fill(dst, 0xCD, npes * nbytes + 256)
-            note("chunked broadcast npes=%d bytes=%d root=%d" % (npes, nbytes, root))
+            note("large-source broadcast npes=%d bytes=%d root=%d" % (npes, nbytes, root))
             rt.broadcastmem(dst + doff, src + soff, nbytes, root)
             got = rt.download_all(dst, (nbytes + doff + 32,), np.uint8)
             assert np.array_equal(got[:, doff:doff + nbytes], O.broadcast(data, root)), (soff, doff)
@@ -278,7 +277,7 @@ def test_two_step_allreduce(npes, monkeypatch):
     NaN-carrying max, bf16, int64, families of ragged teams - must come out bit for bit the same."""
     monkeypatch.setenv("NVSHMEM_AMD_LDS_REDUCE_BYTES", "0")
     monkeypatch.setenv("NVSHMEM_AMD_CACHEABLE_SOURCE_BYTES", "0")
-    monkeypatch.setenv("NVSHMEM_AMD_CHUNKED_COPY_BYTES", "0")
+    monkeypatch.setenv("NVSHMEM_AMD_PACED_COPY_BLOCKS", "0")
     monkeypatch.setenv("NVSHMEM_AMD_TWO_STEP_REDUCE_MEMBERS", "2")
     monkeypatch.setenv("NVSHMEM_AMD_TWO_STEP_REDUCE_BYTES", "0")
     _allreduce_battery(npes, np.random.default_rng(7100 + npes), "two-step")
