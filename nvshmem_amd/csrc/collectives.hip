@@ -553,11 +553,16 @@ static uint64_t total_members(const TeamLaunch &tl) {
 }
 
 // How fcollect and broadcast store: paced beyond Runtime::paced_copy_blocks (33 to a compute unit: the 32 wavefronts it
-// holds and what a message that is no power of two adds), up to which a grid is in flight all at once.  us paced / back
-// to back at 1024, 4096, 8192 and 16384 blocks: fcollect to 4 members 3.3 / 2.5, 4.5 / 4.0, 7.0 / 6.4 and 11.2 / 11.5; to 8
-// 4.5 / 2.9, 7.8 / 6.4, 12.1 / 11.6 and 20.7 / 23.5; to 16 6.9 / 4.1, 14.4 / 11.7, 23.2 / 23.3 and 41.4 / 43.9;
-// broadcast to 8 4.1 / 2.9, 7.5 / 6.4, 11.9 / 11.4 and 21.0 / 23.8.
-static bool paced_copy(const Runtime &rt, uint64_t blocks) { return blocks > rt.paced_copy_blocks; }
+// holds and what a message that is no power of two adds), up to which a grid is in flight all at once; from 12
+// destinations on, whose stores are that many more, beyond half of that.  us paced / back to back at 1024, 4096, 6144,
+// 8192 and 16384 blocks, buffers 5 bytes short of a power of two: fcollect to 4 members 3.4 / 2.7, 4.9 / 4.2, 6.1 / 5.4, 7.0
+// / 6.4 and 11.9 / 11.6; to 8 4.7 / 3.4, 8.1 / 6.7, 10.4 / 9.2, 12.8 / 11.9 and 21.9 / 22.7; to 16 7.1 / 4.6, 14.8 / 12.4,
+// 17.4 / 18.5, 24.0 / 24.2 and 43 / 47; broadcast to 8 4.2 / 3.0, 7.6 / 6.4, 9.6 / 9.2, 11.8 / 11.8 and 20.9 / 23.2, to 16 6.3
+// / 4.2, 14.0 / 12.4, 17.8 / 18.8 and 22.5 / 24.4.  The times of 4096 blocks depend on where the buffers lie: with all of
+// them at multiples of 16 MiB paced takes 6.6 to 8 and 11.2 to 16, back to back 6.5 and 12.0; everywhere else as above.
+static bool paced_copy(const Runtime &rt, uint64_t blocks, int members) {
+    return blocks > (members < 12 ? rt.paced_copy_blocks : rt.paced_copy_blocks / 2);
+}
 // Dynamic LDS that nobody uses: it limits the wavefronts of a paced copy that a compute unit (160 KiB) holds, and with
 // them the width of each write front.  16 of the 32 possible while the cache holds the sources.  Streamed loads take
 // longer and more wavefronts are needed to cover that: 24, and 28 from 12 destinations on, which keep a wavefront storing
@@ -584,7 +589,7 @@ static int launch_broadcast(Runtime &rt, const TeamLaunch &tl, uint64_t doff, ui
     }
     const dim3 grid((unsigned)tiles, 1, (unsigned)tl.ngroups);
     const segment_args_t args = {rt.base, rt.heap_size, team_arg(tl), doff, soff, bytes, (uint32_t)root};
-    const bool paced = paced_copy(rt, tiles * (uint64_t)tl.ngroups);
+    const bool paced = paced_copy(rt, tiles * (uint64_t)tl.ngroups, tl.max_size);
     const size_t lds = paced ? paced_lds_bytes(rt, sources, tl.max_size) : 0;
     // a source that cannot stay in the Infinity Cache is streamed
 #define NVSHMEM_AMD_LAUNCH_BROADCAST(NTL, PACED)                                                                \
@@ -951,7 +956,7 @@ static int segment_collective(int mode, const char *what, nvshmem_team_t team, v
     hipLaunchKernelGGL((segment_copy_kernel<MODE, NTL, PACED, STORE>), grid, dim3(64), lds, stream, args)
     if (mode == kModeFcollect) {
         const dim3 grid((unsigned)tiles, (unsigned)n, (unsigned)tl.ngroups);
-        const bool paced = paced_copy(rt, tiles * n * (uint64_t)tl.ngroups);
+        const bool paced = paced_copy(rt, tiles * n * (uint64_t)tl.ngroups, tl.max_size);
         const size_t lds = paced ? paced_lds_bytes(rt, sources, tl.max_size) : 0;
         if (!paced) NVSHMEM_AMD_LAUNCH_SEGCOPY(kModeFcollect, false, false, NVSHMEM_AMD_STORE_REPLICATE);
         else if (stream_source) NVSHMEM_AMD_LAUNCH_SEGCOPY(kModeFcollect, true, true, NVSHMEM_AMD_STORE_REPLICATE);

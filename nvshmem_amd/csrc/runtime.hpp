@@ -63,7 +63,8 @@ struct Runtime {
     // large to stay in the Infinity Cache: NVSHMEM_AMD_CACHEABLE_SOURCE_BYTES, read at init
     uint64_t cacheable_source_bytes = (uint64_t)256 << 20;
     // fcollect and broadcast store to one destination after the other in grids of more blocks than this, to all of
-    // them back to back in smaller ones: NVSHMEM_AMD_PACED_COPY_BLOCKS, read at init (default: 33 to a compute unit)
+    // them back to back in smaller ones: NVSHMEM_AMD_PACED_COPY_BLOCKS, read at init (default: 33 to a compute unit;
+    // half of it from 12 destinations on)
     uint64_t paced_copy_blocks = 33 * 256;
     // Allreduce on teams of 3 to 64 members takes the LDS-staged kernel when the sources of all PEs
     // together hold at least this many bytes (a quarter of it for teams of 17

@@ -24,14 +24,14 @@ def test_collective_launches_are_cooperative_unless_asked(recorded, plain, coope
 
 
 def test_copies_that_are_in_flight_all_at_once_are_not_paced(recorded):  # noqa: F811
-    """fcollect and broadcast of up to 32 pieces per compute unit store back to back, larger ones one destination at a
-    time (third template argument of the kernel)."""
+    """fcollect and broadcast of up to 32 pieces per compute unit (16 from 12 members on) store back to back, larger ones
+    one destination at a time (third template argument of the kernel)."""
     recorded("""
 for npes in (4, 8, 16):
     ok(lib.nvshmemx_amd_init(npes, 256 << 20))
     a, b = lib.nvshmem_malloc(64 << 20), lib.nvshmem_malloc(128 << 20)
     launches()
-    for blocks, paced in ((1, 0), (3000, 0), (8192, 0), (8700, 1), (20000, 1)):
+    for blocks, paced in ((1, 0), (4096, 0), (5000, npes >= 12), (8192, npes >= 12), (8700, 1), (20000, 1)):
         ok(lib.nvshmemx_fcollectmem_on_stream(0, b, a, blocks // npes * 1024 or 1, None))
         ok(lib.nvshmemx_broadcastmem_on_stream(0, b, a, blocks * 1024 - 5, 1, None))
         for kernel, cooperative, grid, block, lds in launches():
