@@ -133,6 +133,9 @@ __device__ __forceinline__ void stream_store_at(char *p, unsigned off, nvshmemi_
 //    together then write to one destination at a time instead of all 8 or 16 (broadcast of 32 MiB to 8: 47.4 us back
 //    to back, 42.8 paced), and the fewer wavefronts take part, the narrower each front.  So the launch also limits
 //    how many a compute unit holds (paced_lds_bytes).
+// A CHUNKED fcollect (streamed sources, 16 members and more) is paced with two destinations to a wavefront: the grid
+// walks a chunk of tiles once per pair of destinations, re-reading it from the cache, before it goes on to the next.
+// The pieces in flight then feed a few write fronts however many members there are (chunked_copy).
 // ---------------------------------------------------------------------------------------------
 
 enum { kModeFcollect = 0, kModeAlltoall = 1, kModeBroadcast = 2 };
@@ -148,9 +151,10 @@ struct segment_args_t {
     team_arg_t team;
     uint64_t dst_off, src_off, seg_bytes;
     uint32_t root;
+    uint16_t part_shift, chunk_shift;  // chunked walk: 2^part_shift groups of destinations, chunks of 2^chunk_shift tiles
 };
 
-template <int MODE, bool NTL, bool PACED, int STORE>
+template <int MODE, bool NTL, bool PACED, int STORE, bool CHUNKED = false>
 __global__ __launch_bounds__(64) void segment_copy_kernel(segment_args_t a) {
     // this block's team: members are the PEs start + i*stride, i < size
     unsigned p = MODE == kModeAlltoall ? blockIdx.z : blockIdx.y, group = MODE == kModeAlltoall ? 0 : blockIdx.z;
@@ -182,6 +186,15 @@ __global__ __launch_bounds__(64) void segment_copy_kernel(segment_args_t a) {
         dst = base + q * rep_stride + a.dst_off + p * a.seg_bytes;
         nrep = 1;
     }
+    unsigned tile = blockIdx.x;
+    if (CHUNKED) {
+        const unsigned part = (tile >> a.chunk_shift) & ((1u << a.part_shift) - 1);
+        tile = (tile & ((1u << a.chunk_shift) - 1)) + (tile >> (a.chunk_shift + a.part_shift) << a.chunk_shift);
+        const unsigned per = (npes + (1u << a.part_shift) - 1) >> a.part_shift, r0 = part * per;
+        if (r0 >= npes) return;  // a team smaller than the grid's largest: nothing left for this group
+        nrep = npes - r0 < per ? npes - r0 : per;
+        dst += r0 * rep_stride;
+    }
     const unsigned lane = threadIdx.x;
     unsigned head = (unsigned)(-(uintptr_t)dst) & 15;
     if (head > a.seg_bytes) head = (unsigned)a.seg_bytes;
@@ -189,8 +202,8 @@ __global__ __launch_bounds__(64) void segment_copy_kernel(segment_args_t a) {
     // tiles are cut on absolute 1 KiB boundaries of the destination: `lead` vector slots of tile 0
     // lie in front of the segment
     const unsigned lead = (unsigned)((uintptr_t)(dst + head) >> 4) & 63;
-    const int64_t v0 = (int64_t)blockIdx.x * 64 - lead, left = (int64_t)nvec - v0;
-    const bool edges = blockIdx.x == 0;  // this block also moves the bytes around the vectors
+    const int64_t v0 = (int64_t)tile * 64 - lead, left = (int64_t)nvec - v0;
+    const bool edges = tile == 0;  // this block also moves the bytes around the vectors
     if (left <= 0 && !edges) return;
     // this lane's vector, as an unsigned index: slots in front of the segment wrap and are skipped like those behind it
     const unsigned first = edges ? lead : 0, end = left < 64 ? (unsigned)left : 64;
@@ -579,6 +592,19 @@ static size_t paced_lds_bytes(const Runtime &rt, uint64_t source_bytes, int memb
     return ((size_t)160 << 10) / waves & ~(size_t)127;
 }
 
+// The blocks of an fcollect of streamed sources that walks in chunks, 0 for one that does not.  us chunked / paced: int64 of 16 x 32 MiB with all buffers at powers of two
+// 1448 / 1526; elsewhere 16 x 32 MiB 1408 / 1429, 16 x 64 MiB 2782 / 2761, 24 x 16 MiB 1516 / 1552, 32 x 16 MiB 2745 / 2610 to
+// 2930, with a third of the spread between runs; 12 x 32 MiB 816 / 772, 8 x 64 MiB 768 / 724.  Broadcasts and cached
+// sources gain nothing by it (fcollect of 16 x 16 MiB 645 / 607).  The groups are the largest power of two that leaves each
+// two destinations, the chunk 2^14 blocks over all groups, twice what the GPU holds at a time.
+static uint64_t chunked_copy(segment_args_t *args, int members, uint64_t tiles) {
+    if (members < 16) return 0;
+    while (members >> (args->part_shift + 1) >= 2) ++args->part_shift;
+    args->chunk_shift = (uint16_t)(14 - args->part_shift);
+    const uint64_t chunks = (tiles + (1ull << args->chunk_shift) - 1) >> args->chunk_shift, blocks = chunks << 14;
+    return blocks * 64 >> 32 ? 0 : blocks;  // (a launch holds fewer than 2^32 threads)
+}
+
 // Launches the broadcast kernel: member `root`'s [soff, +bytes) to every member's [doff, +bytes).
 static int launch_broadcast(Runtime &rt, const TeamLaunch &tl, uint64_t doff, uint64_t soff, uint64_t bytes, int root,
                             hipStream_t stream) {
@@ -588,7 +614,7 @@ static int launch_broadcast(Runtime &rt, const TeamLaunch &tl, uint64_t doff, ui
         return NVSHMEMX_ERROR_INVALID_VALUE;
     }
     const dim3 grid((unsigned)tiles, 1, (unsigned)tl.ngroups);
-    const segment_args_t args = {rt.base, rt.heap_size, team_arg(tl), doff, soff, bytes, (uint32_t)root};
+    const segment_args_t args = {rt.base, rt.heap_size, team_arg(tl), doff, soff, bytes, (uint32_t)root, 0, 0};
     const bool paced = paced_copy(rt, tiles * (uint64_t)tl.ngroups, tl.max_size);
     const size_t lds = paced ? paced_lds_bytes(rt, sources, tl.max_size) : 0;
     // a source that cannot stay in the Infinity Cache is streamed
@@ -951,14 +977,19 @@ static int segment_collective(int mode, const char *what, nvshmem_team_t team, v
         return NVSHMEMX_ERROR_INVALID_VALUE;
     }
     const bool stream_source = sources > rt.cacheable_source_bytes;
-    const segment_args_t args = {rt.base, rt.heap_size, team_arg(tl), doff, soff, seg_bytes, 0};
+    const segment_args_t args = {rt.base, rt.heap_size, team_arg(tl), doff, soff, seg_bytes, 0, 0, 0};
 #define NVSHMEM_AMD_LAUNCH_SEGCOPY(MODE, NTL, PACED, STORE) \
     hipLaunchKernelGGL((segment_copy_kernel<MODE, NTL, PACED, STORE>), grid, dim3(64), lds, stream, args)
     if (mode == kModeFcollect) {
         const dim3 grid((unsigned)tiles, (unsigned)n, (unsigned)tl.ngroups);
         const bool paced = paced_copy(rt, tiles * n * (uint64_t)tl.ngroups, tl.max_size);
         const size_t lds = paced ? paced_lds_bytes(rt, sources, tl.max_size) : 0;
-        if (!paced) NVSHMEM_AMD_LAUNCH_SEGCOPY(kModeFcollect, false, false, NVSHMEM_AMD_STORE_REPLICATE);
+        segment_args_t chunked = args;
+        const uint64_t chunked_blocks = paced && stream_source ? chunked_copy(&chunked, tl.max_size, tiles) : 0;
+        if (chunked_blocks) {
+            hipLaunchKernelGGL((segment_copy_kernel<kModeFcollect, false, true, NVSHMEM_AMD_STORE_REPLICATE, true>),
+                               dim3((unsigned)chunked_blocks, grid.y, grid.z), dim3(64), 0, stream, chunked);
+        } else if (!paced) NVSHMEM_AMD_LAUNCH_SEGCOPY(kModeFcollect, false, false, NVSHMEM_AMD_STORE_REPLICATE);
         else if (stream_source) NVSHMEM_AMD_LAUNCH_SEGCOPY(kModeFcollect, true, true, NVSHMEM_AMD_STORE_REPLICATE);
         else NVSHMEM_AMD_LAUNCH_SEGCOPY(kModeFcollect, false, true, NVSHMEM_AMD_STORE_REPLICATE);
     } else {

@@ -44,7 +44,7 @@ def test_wavefronts_of_paced_copies(recorded):  # noqa: F811
     """A compute unit (160 KiB of LDS) holds 16 wavefronts of a paced copy whose sources the cache holds, more with
     streamed loads (second template argument)."""
     recorded("""
-for npes, mib, streamed, waves in ((8, 32, 0, 16), (16, 16, 0, 16), (16, 8, 0, 16), (8, 64, 1, 24), (16, 32, 1, 28), (32, 16, 1, 28)):
+for npes, mib, streamed, waves in ((8, 32, 0, 16), (16, 16, 0, 16), (16, 8, 0, 16), (8, 64, 1, 24), (12, 32, 1, 28)):
     ok(lib.nvshmemx_amd_init(npes, (npes + 2) * mib << 20))
     a, b = lib.nvshmem_malloc(mib << 20), lib.nvshmem_malloc(npes * mib << 20)
     launches()
@@ -100,5 +100,20 @@ for npes, kind, name, nbytes, shift, element in (
     (kernel, _, grid, block, _), = launches()
     assert ("reduce_element_kernel" in kernel) == element, (npes, kind, name, nbytes, shift, kernel)
     assert not element or (grid[0] - 1) * block[0] < nbytes // es <= grid[0] * block[0]
+    lib.nvshmem_finalize()
+""")
+
+
+def test_streamed_fcollects_of_many_members_walk_in_chunks(recorded):  # noqa: F811
+    """From 16 members on (fifth template argument): whole chunks, every tile of a segment for each group of members."""
+    recorded("""
+for npes, mib, groups in ((15, 40, 0), (16, 16, 0), (16, 24, 8), (24, 16, 8), (64, 5, 32)):
+    ok(lib.nvshmemx_amd_init(npes, (npes + 2) * mib << 20))
+    a, b = lib.nvshmem_malloc(mib << 20), lib.nvshmem_malloc(npes * mib << 20)
+    launches()
+    ok(lib.nvshmemx_fcollectmem_on_stream(0, b, a, (mib << 20) - 5, None))
+    (kernel, _, grid, block, lds), = launches()
+    assert ("ELi2ELb1EE" in kernel) == bool(groups), (npes, mib, kernel)
+    assert not groups or (grid[0] % 16384 == 0 and grid[0] // groups >= mib * 1024 > grid[0] // groups - 16384 // groups - 2)
     lib.nvshmem_finalize()
 """)
