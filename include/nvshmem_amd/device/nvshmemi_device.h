@@ -382,30 +382,10 @@ NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_copy_vectors(char *__restrict__ dst,
                                  NVSHMEMI_AMD_COPY_UNROLL, true>(dst, src, nvec, tid, nthr);
 }
 
-template <int SCOPE, int STORE = NVSHMEMI_AMD_STORE_STREAM, int LOAD = NVSHMEMI_AMD_LOAD_BY_SIZE>
-NVSHMEMI_DEVICE_INLINE void nvshmemi_memcpy_threadgroup(void *__restrict__ dst_v,
-                                                       const void *__restrict__ src_v, size_t len) {
-    char *dst = static_cast<char *>(dst_v);
-    const char *src = static_cast<const char *>(src_v);
-    const size_t tid = (size_t)nvshmemi_thread_id_in_threadgroup<SCOPE>();
-    const size_t nthr = (size_t)nvshmemi_threadgroup_size<SCOPE>();
-#if defined(NVSHMEMI_AMD_COPY_NT)
-    const bool stream_loads = (NVSHMEMI_AMD_COPY_NT & 1) != 0;
-#else
-    /* (short copies decide without reading the launch dimensions: puts keep their loads cacheable, gets
-     * stream) */
-    bool stream_loads = LOAD == NVSHMEMI_AMD_LOAD_STREAM;
-    if (len >= (LOAD == NVSHMEMI_AMD_LOAD_STREAM ? NVSHMEMI_AMD_GET_NT_BYTES : NVSHMEMI_AMD_COPY_NT_BYTES)) {
-        const float per_block = SCOPE == NVSHMEMI_THREADGROUP_BLOCK ? 1.0f
-                                : (float)(blockDim.x * blockDim.y * blockDim.z) /
-                                      (SCOPE == NVSHMEMI_THREADGROUP_WARP ? (float)NVSHMEMI_WARP_SIZE : 1.0f);
-        const float groups = (float)gridDim.x * (float)gridDim.y * (float)gridDim.z * per_block;
-        stream_loads = (float)len * groups > (float)NVSHMEMI_AMD_COPY_CACHE_BYTES;
-    } else if (LOAD == NVSHMEMI_AMD_LOAD_BY_SIZE) {
-        stream_loads = false;
-    }
-#endif
-
+/* The copy by lane `tid` of the `nthr` of its group; BLOCK_WIDE: the group is the block. */
+template <int STORE, int LOAD, bool BLOCK_WIDE>
+NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_copy_lanes(char *__restrict__ dst, const char *__restrict__ src, size_t len,
+                                                   size_t tid, size_t nthr, bool stream_loads) {
     size_t head = (size_t)(-(uintptr_t)dst & 15);
     if (head > len) head = len;
     for (size_t i = tid; i < head; i += nthr) nvshmemi_amd_store_byte<STORE>(dst + i, src[i]);
@@ -424,14 +404,39 @@ NVSHMEMI_DEVICE_INLINE void nvshmemi_memcpy_threadgroup(void *__restrict__ dst_v
             if (((uintptr_t)src & 15) == 0) nvshmemi_amd_copy_vectors<true, STORE, LOAD>(dst, src, pre, tid, nthr, stream_loads);
             else nvshmemi_amd_copy_vectors<false, STORE, LOAD>(dst, src, pre, tid, nthr, stream_loads);
         }
-        constexpr bool block_wide = SCOPE == NVSHMEMI_THREADGROUP_BLOCK;   // every wavefront of the block is here
         if (((uintptr_t)src & 15) == 0)
-            nvshmemi_amd_copy_vectors<true, STORE, LOAD, block_wide>(dst + 16 * pre, src + 16 * pre, nvec - pre, tid, nthr, stream_loads);
+            nvshmemi_amd_copy_vectors<true, STORE, LOAD, BLOCK_WIDE>(dst + 16 * pre, src + 16 * pre, nvec - pre, tid, nthr, stream_loads);
         else
-            nvshmemi_amd_copy_vectors<false, STORE, LOAD, block_wide>(dst + 16 * pre, src + 16 * pre, nvec - pre, tid, nthr, stream_loads);
+            nvshmemi_amd_copy_vectors<false, STORE, LOAD, BLOCK_WIDE>(dst + 16 * pre, src + 16 * pre, nvec - pre, tid, nthr, stream_loads);
     }
     const size_t done = nvec * 16;
     for (size_t i = done + tid; i < len; i += nthr) nvshmemi_amd_store_byte<STORE>(dst + i, src[i]);
+}
+
+template <int SCOPE, int STORE = NVSHMEMI_AMD_STORE_STREAM, int LOAD = NVSHMEMI_AMD_LOAD_BY_SIZE>
+NVSHMEMI_DEVICE_INLINE void nvshmemi_memcpy_threadgroup(void *__restrict__ dst_v,
+                                                       const void *__restrict__ src_v, size_t len) {
+    const size_t tid = (size_t)nvshmemi_thread_id_in_threadgroup<SCOPE>();
+    const size_t nthr = (size_t)nvshmemi_threadgroup_size<SCOPE>();
+#if defined(NVSHMEMI_AMD_COPY_NT)
+    const bool stream_loads = (NVSHMEMI_AMD_COPY_NT & 1) != 0;
+#else
+    /* (short copies decide without reading the launch dimensions: puts keep their loads cacheable, gets
+     * stream) */
+    bool stream_loads = LOAD == NVSHMEMI_AMD_LOAD_STREAM;
+    if (len >= (LOAD == NVSHMEMI_AMD_LOAD_STREAM ? NVSHMEMI_AMD_GET_NT_BYTES : NVSHMEMI_AMD_COPY_NT_BYTES)) {
+        const float per_block = SCOPE == NVSHMEMI_THREADGROUP_BLOCK ? 1.0f
+                                : (float)(blockDim.x * blockDim.y * blockDim.z) /
+                                      (SCOPE == NVSHMEMI_THREADGROUP_WARP ? (float)NVSHMEMI_WARP_SIZE : 1.0f);
+        const float groups = (float)gridDim.x * (float)gridDim.y * (float)gridDim.z * per_block;
+        stream_loads = (float)len * groups > (float)NVSHMEMI_AMD_COPY_CACHE_BYTES;
+    } else if (LOAD == NVSHMEMI_AMD_LOAD_BY_SIZE) {
+        stream_loads = false;
+    }
+#endif
+    /* (block scope: every wavefront of the block is here) */
+    nvshmemi_amd_copy_lanes<STORE, LOAD, SCOPE == NVSHMEMI_THREADGROUP_BLOCK>(
+        static_cast<char *>(dst_v), static_cast<const char *>(src_v), len, tid, nthr, stream_loads);
 }
 
 /* ------------------------------------------------------------------------------------------------
@@ -623,10 +628,9 @@ NVSHMEMI_DEVICE_INLINE T nvshmemi_amd_poll(const T *addr) {
     return __hip_atomic_load(addr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_record_timeout(const void *addr, uint64_t found,
-                                                        uint64_t expected) {
-    uint64_t *rec = reinterpret_cast<uint64_t *>(
-        nvshmemi_amd_remote(nvshmemi_device_state_d.timeout_record, nvshmemi_amd_my_pe()));
+NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_record_timeout_of(int pe, const void *addr, uint64_t found,
+                                                           uint64_t expected) {
+    uint64_t *rec = reinterpret_cast<uint64_t *>(nvshmemi_amd_remote(nvshmemi_device_state_d.timeout_record, pe));
     /* the count the host checks at its synchronisation points; the record's first word is this timeout's
      * number in that count (never 0), so that a report can tell a record of its own period from an older one */
     const uint64_t seq = __hip_atomic_fetch_add(nvshmemi_device_state_d.runtime_words + NVSHMEMI_AMD_TIMEOUT_COUNT_WORD,
@@ -639,19 +643,22 @@ NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_record_timeout(const void *addr, uint64
     if (nvshmemi_device_state_d.timeout_flag)
         __hip_atomic_store(nvshmemi_device_state_d.timeout_flag, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
+NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_record_timeout(const void *addr, uint64_t found, uint64_t expected) {
+    nvshmemi_amd_record_timeout_of(nvshmemi_amd_my_pe(), addr, found, expected);
+}
 
-/* Spin until `*ivar cmp value`; `ivar` is a local operand.  Returns the value that ended the wait.
+/* Spin until `*addr cmp value`, at an address that is used as it is, on behalf of PE `pe` (whose record a wait that
+ * gives up goes to).  Returns the value that ended the wait.
  * The final acquire makes data published before the signal visible to the caller; the reference's
  * typed waits fence the same way (__threadfence via nvshmemi_transfer_syncapi_update_mem). */
 template <typename T, bool ACQUIRE = true>
-NVSHMEMI_DEVICE_INLINE T nvshmemi_wait_until(T *ivar, int cmp, T value) {
-    const T *addr = reinterpret_cast<const T *>(nvshmemi_amd_local(ivar));
+NVSHMEMI_DEVICE_INLINE T nvshmemi_amd_wait_at(const T *addr, int pe, int cmp, T value) {
     const uint64_t limit = nvshmemi_device_state_d.spin_limit;
     uint64_t polls = 0;
     T found = nvshmemi_amd_poll(addr);
     while (!nvshmemi_amd_compare(found, cmp, value)) {
         if (limit && ++polls > limit) {
-            nvshmemi_amd_record_timeout(addr, (uint64_t)found, (uint64_t)value);
+            nvshmemi_amd_record_timeout_of(pe, addr, (uint64_t)found, (uint64_t)value);
             break;
         }
         __builtin_amdgcn_s_sleep(1);
@@ -660,6 +667,12 @@ NVSHMEMI_DEVICE_INLINE T nvshmemi_wait_until(T *ivar, int cmp, T value) {
     /* (a caller that waits for several variables in a row asks for no fence and issues one itself) */
     if (ACQUIRE) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     return found;
+}
+/* The same at a local operand of the calling PE. */
+template <typename T, bool ACQUIRE = true>
+NVSHMEMI_DEVICE_INLINE T nvshmemi_wait_until(T *ivar, int cmp, T value) {
+    return nvshmemi_amd_wait_at<T, ACQUIRE>(reinterpret_cast<const T *>(nvshmemi_amd_local(ivar)), nvshmemi_amd_my_pe(),
+                                            cmp, value);
 }
 
 template <typename T>

@@ -151,6 +151,7 @@ struct segment_args_t {
     team_arg_t team;
     uint64_t dst_off, src_off, seg_bytes;
     uint32_t root;
+    uint32_t members;                  // of the handle's largest team (gridDim would cost the host 0.6 us a launch: host_rma.hip)
     uint16_t part_shift, chunk_shift;  // chunked walk: 2^part_shift groups of destinations, chunks of 2^chunk_shift tiles
 };
 
@@ -159,8 +160,8 @@ __global__ __launch_bounds__(64) void segment_copy_kernel(segment_args_t a) {
     // this block's team: members are the PEs start + i*stride, i < size
     unsigned p = MODE == kModeAlltoall ? blockIdx.z : blockIdx.y, group = MODE == kModeAlltoall ? 0 : blockIdx.z;
     if (MODE == kModeAlltoall && a.team.table) {
-        group = p / gridDim.y;
-        p -= group * gridDim.y;
+        group = p / a.members;
+        p -= group * a.members;
     }
     const nvshmemi_amd_team_view_t g = team_of(a.team, group);
     const unsigned npes = (unsigned)g.size;
@@ -614,7 +615,8 @@ static int launch_broadcast(Runtime &rt, const TeamLaunch &tl, uint64_t doff, ui
         return NVSHMEMX_ERROR_INVALID_VALUE;
     }
     const dim3 grid((unsigned)tiles, 1, (unsigned)tl.ngroups);
-    const segment_args_t args = {rt.base, rt.heap_size, team_arg(tl), doff, soff, bytes, (uint32_t)root, 0, 0};
+    const segment_args_t args = {rt.base, rt.heap_size, team_arg(tl), doff, soff, bytes, (uint32_t)root,
+                                 (uint32_t)tl.max_size, 0, 0};
     const bool paced = paced_copy(rt, tiles * (uint64_t)tl.ngroups, tl.max_size);
     const size_t lds = paced ? paced_lds_bytes(rt, sources, tl.max_size) : 0;
     // a source that cannot stay in the Infinity Cache is streamed
@@ -977,7 +979,7 @@ static int segment_collective(int mode, const char *what, nvshmem_team_t team, v
         return NVSHMEMX_ERROR_INVALID_VALUE;
     }
     const bool stream_source = sources > rt.cacheable_source_bytes;
-    const segment_args_t args = {rt.base, rt.heap_size, team_arg(tl), doff, soff, seg_bytes, 0, 0, 0};
+    const segment_args_t args = {rt.base, rt.heap_size, team_arg(tl), doff, soff, seg_bytes, 0, (uint32_t)n, 0, 0};
 #define NVSHMEM_AMD_LAUNCH_SEGCOPY(MODE, NTL, PACED, STORE) \
     hipLaunchKernelGGL((segment_copy_kernel<MODE, NTL, PACED, STORE>), grid, dim3(64), lds, stream, args)
     if (mode == kModeFcollect) {

@@ -40,9 +40,17 @@ bool strided_target(Runtime &rt, const char *what, const void *sym, ptrdiff_t st
 // for a column of 2048 floats.  This kernel takes 1.3 us for the column, and neighbouring elements share their lines:
 // us rectangle copy / here for 2^20 floats 29.7 / 4.1 contiguous, 33 / 20 on every 10th, 41 / 39 on every 25th; 2^24 on
 // every 3rd 497 / 78 (with cached stores 110).
-template <typename T>
-__global__ void strided_copy_kernel(T *dst, size_t dst_stride, const T *src, size_t src_stride, size_t nelems) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+//
+// This kernel and the others behind the small on-stream calls use neither blockDim nor gridDim (nor what is built on
+// them, like the calling PE of the device API).  A kernel that does has 256 bytes of implicit arguments behind its own,
+// which the host fills in on every launch, and the host is what bounds a row of small calls: the GPU gets through a
+// queue of them at 1.5 to 2.3 us each.  us a call without and with implicit arguments, in processes whose host reaches the
+// GPU slowly: iput of 2048 floats 3.0 / 3.6, put_signal of 8 KiB 3.0 / 3.6, a wait for four words 3.0 / 3.6 (in the faster
+// processes 2.7 either way: runs on one machine are of one kind or the other).
+template <typename T, unsigned THREADS>
+__global__ __launch_bounds__(THREADS) void strided_copy_kernel(T *dst, size_t dst_stride, const T *src, size_t src_stride,
+                                                               size_t nelems) {
+    const size_t i = (size_t)blockIdx.x * THREADS + threadIdx.x;
     if (i < nelems) __builtin_nontemporal_store(src[i * src_stride], dst + i * dst_stride);
 }
 // Elements that all lie on lines of their own, on both sides, are all the rectangle copy is better at, and only when
@@ -57,9 +65,12 @@ constexpr size_t kKernelElements = (size_t)1 << 31;
 
 template <typename T>
 void launch_strided(void *dst, size_t dst_stride, const void *src, size_t src_stride, size_t nelems, hipStream_t stream) {
-    const unsigned threads = nelems > kNarrowBlockElements ? 256 : 64;
-    hipLaunchKernelGGL(strided_copy_kernel<T>, dim3((unsigned)((nelems + threads - 1) / threads)), dim3(threads), 0, stream,
-                       (T *)dst, dst_stride, (const T *)src, src_stride, nelems);
+    if (nelems > kNarrowBlockElements)
+        hipLaunchKernelGGL((strided_copy_kernel<T, 256>), dim3((unsigned)((nelems + 255) / 256)), dim3(256), 0, stream, (T *)dst,
+                           dst_stride, (const T *)src, src_stride, nelems);
+    else
+        hipLaunchKernelGGL((strided_copy_kernel<T, 64>), dim3((unsigned)((nelems + 63) / 64)), dim3(64), 0, stream, (T *)dst,
+                           dst_stride, (const T *)src, src_stride, nelems);
     NVSHMEM_AMD_HIP_CHECK(hipGetLastError());
 }
 
@@ -144,14 +155,19 @@ void g_on_stream(void *value_out, const void *source, size_t es, int pe, hipStre
     NVSHMEM_AMD_HIP_CHECK(hipStreamSynchronize(stream));
 }
 
+// The waits take the address as it is: the host thread is PE 0, whose copy of a symmetric object is what the address
+// already names, and an address in another PE's slice means that one.
+constexpr int kHostPe = 0;
+constexpr unsigned kWaitThreads = 64;
 template <typename T>
-__global__ void wait_until_kernel(T *ivar, int cmp, T value) {
-    nvshmemi_wait_until<T>(ivar, cmp, value);
+__global__ void wait_until_kernel(const T *ivar, int cmp, T value) {
+    nvshmemi_amd_wait_at<T>(ivar, kHostPe, cmp, value);
 }
 template <typename T>
-__global__ void wait_until_all_kernel(T *ivars, size_t nelems, const int *status, int cmp, T value) {
-    for (size_t i = threadIdx.x; i < nelems; i += blockDim.x)
-        if (!status || !status[i]) nvshmemi_wait_until<T>(ivars + i, cmp, value);
+__global__ __launch_bounds__(kWaitThreads) void wait_until_all_kernel(const T *ivars, size_t nelems, const int *status, int cmp,
+                                                                      T value) {
+    for (size_t i = threadIdx.x; i < nelems; i += kWaitThreads)
+        if (!status || !status[i]) nvshmemi_amd_wait_at<T>(ivars + i, kHostPe, cmp, value);
 }
 
 template <typename T>
@@ -180,16 +196,15 @@ void wait_until_all_on_stream(T *ivars, size_t nelems, const int *status, int cm
         return;
     }
     // `status` is read by the kernel: it must be device-accessible memory (or NULL), as in the reference
-    hipLaunchKernelGGL(wait_until_all_kernel<T>, dim3(1), dim3(64), 0, stream, ivars, nelems, status, cmp,
-                       value);
+    hipLaunchKernelGGL(wait_until_all_kernel<T>, dim3(1), dim3(kWaitThreads), 0, stream, ivars, nelems, status, cmp, value);
     NVSHMEM_AMD_HIP_CHECK(hipGetLastError());
 }
 
 template <typename T>
-__global__ void wait_until_all_vector_kernel(T *ivars, size_t nelems, const int *status, int cmp,
-                                             const T *values) {
-    for (size_t i = threadIdx.x; i < nelems; i += blockDim.x)
-        if (!status || !status[i]) nvshmemi_wait_until<T>(ivars + i, cmp, values[i]);
+__global__ __launch_bounds__(kWaitThreads) void wait_until_all_vector_kernel(const T *ivars, size_t nelems, const int *status,
+                                                                             int cmp, const T *values) {
+    for (size_t i = threadIdx.x; i < nelems; i += kWaitThreads)
+        if (!status || !status[i]) nvshmemi_amd_wait_at<T>(ivars + i, kHostPe, cmp, values[i]);
 }
 
 // `status` and `cmp_values` are read by the kernel: device-accessible memory, as in the reference
@@ -210,8 +225,8 @@ void wait_until_all_vector_on_stream(T *ivars, size_t nelems, const int *status,
         set_error("wait_until_all_vector_on_stream: cmp_values is NULL");
         return;
     }
-    hipLaunchKernelGGL(wait_until_all_vector_kernel<T>, dim3(1), dim3(64), 0, stream, ivars, nelems, status,
-                       cmp, values);
+    hipLaunchKernelGGL(wait_until_all_vector_kernel<T>, dim3(1), dim3(kWaitThreads), 0, stream, ivars, nelems, status, cmp,
+                       values);
     NVSHMEM_AMD_HIP_CHECK(hipGetLastError());
 }
 

@@ -129,19 +129,21 @@ __global__ void signal_op_kernel(uint64_t *sig_addr, uint64_t signal, int sig_op
     nvshmemi_signal_op_release(sig_addr, signal, sig_op, pe);
 }
 
-__global__ void signal_wait_kernel(uint64_t *sig_addr, int cmp, uint64_t cmp_value) {
-    nvshmemi_wait_until<uint64_t>(sig_addr, cmp, cmp_value);
+// (The kernels behind the small on-stream calls use neither blockDim nor gridDim, in any guise: see host_rma.hip.)
+__global__ void signal_wait_kernel(const uint64_t *word, int pe, int cmp, uint64_t cmp_value) {
+    nvshmemi_amd_wait_at<uint64_t>(word, pe, cmp, cmp_value);
 }
 
 // put_signal on a stream as one launch of one block: the payload is written through the L2, every wavefront waits for
 // its stores, and the signal follows.  (Nothing else that it would have to publish is written here, and what ran
 // before on the stream was published when it ended.)  Bound by the launch - copy and signal in two take 5.6 us a call
-// from 8 bytes to 1 MiB, this 3.5 - up to kPutSignalBlockBytes; beyond, by what one compute unit moves (us: 64 KiB 3.9,
+// from 8 bytes to 1 MiB, this 2.7 to 3.0 - up to kPutSignalBlockBytes; beyond, by what one compute unit moves (us: 64 KiB 3.9,
 // 128 KiB 5.2, 256 KiB 7.9).
 constexpr size_t kPutSignalBlockBytes = (size_t)64 << 10;
-__global__ __launch_bounds__(1024) void put_signal_kernel(char *dst, const char *src, size_t bytes, uint64_t *sig_addr,
-                                                          uint64_t signal, int sig_op, int pe) {
-    nvshmemi_memcpy_threadgroup<NVSHMEMI_THREADGROUP_BLOCK, NVSHMEMI_AMD_STORE_WRITE_THROUGH>(dst, src, bytes);
+__global__ __launch_bounds__(1024) void put_signal_kernel(char *dst, const char *src, uint32_t bytes, uint32_t threads,
+                                                          uint64_t *sig_addr, uint64_t signal, int sig_op, int pe) {
+    nvshmemi_amd_copy_lanes<NVSHMEMI_AMD_STORE_WRITE_THROUGH, NVSHMEMI_AMD_LOAD_BY_SIZE, true>(dst, src, bytes, threadIdx.x,
+                                                                                               threads, false);
     nvshmemi_amd_wait_vm();
     __syncthreads();
     if (threadIdx.x == 0) nvshmemi_signal_op(sig_addr, signal, sig_op, pe);
@@ -682,8 +684,7 @@ void nvshmemx_signal_wait_until_on_stream(uint64_t *sig_addr, int cmp, uint64_t 
         std::lock_guard<std::recursive_mutex> lock(rt.mu);
         refresh_symbols(rt, false);
     }
-    hipLaunchKernelGGL(signal_wait_kernel, dim3(1), dim3(1), 0, (hipStream_t)stream, sig_addr, cmp,
-                       cmp_value);
+    hipLaunchKernelGGL(signal_wait_kernel, dim3(1), dim3(1), 0, (hipStream_t)stream, sig_addr, 0, cmp, cmp_value);
     NVSHMEM_AMD_HIP_CHECK(hipGetLastError());
 }
 
@@ -707,8 +708,8 @@ void nvshmemx_putmem_signal_on_stream(void *dest, const void *source, size_t byt
             }
             const size_t vecs = (bytes + 15) / 16;
             const unsigned threads = vecs >= 1024 ? 1024 : (unsigned)(vecs + 63) & ~63u;
-            hipLaunchKernelGGL(put_signal_kernel, dim3(1), dim3(threads), 0, (hipStream_t)stream, dst, src, bytes,
-                               sig_addr, signal, op, pe);
+            hipLaunchKernelGGL(put_signal_kernel, dim3(1), dim3(threads), 0, (hipStream_t)stream, dst, src,
+                               (uint32_t)bytes, threads, sig_addr, signal, op, pe);
             NVSHMEM_AMD_HIP_CHECK(hipGetLastError());
             return;
         }

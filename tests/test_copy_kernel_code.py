@@ -87,3 +87,19 @@ def test_edge_elements_of_many_members_are_loaded_together(code_objects, kernel)
         elif re.match(r"s_waitcnt.*vmcnt", line):
             run = 0
     assert longest >= 8
+
+
+@pytest.mark.parametrize("kernel", [r"segment_copy_kernel", r"reduce_gather_kernel", r"reduce_element_kernel",
+                                    r"reducescatter_gather_kernel", r"put_signal_kernel", r"strided_copy_kernel",
+                                    r"signal_op_kernel", r"signal_wait_kernel", r"wait_until_kernel",
+                                    r"wait_until_all_kernel", r"wait_until_all_vector_kernel", r"scalar_p_kernel"])
+def test_kernels_of_small_calls_have_no_implicit_arguments(code_objects, kernel):
+    """The host fills in a kernel's implicit arguments on every launch, which costs it a quarter of the launch."""
+    seen = 0
+    for path in code_objects:
+        notes = subprocess.run([LLVM + "llvm-readelf", "--notes", path], check=True, stdout=subprocess.PIPE, text=True).stdout
+        for entry in re.split(r"\n\s+- \.agpr_count:", notes)[1:]:
+            if re.search(r"\.symbol:\s+\S*\d%s[IEP]\S*\.kd" % kernel, entry):
+                seen += 1
+                assert "hidden_" not in entry
+    assert seen
