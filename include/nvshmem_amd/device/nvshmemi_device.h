@@ -155,10 +155,10 @@ NVSHMEMI_DEVICE_INLINE void *nvshmemi_ptr(const void *ptr, int pe) {
  *
  * Byte-exact copy by the lanes of one thread group.  Where the reference picks the widest element
  * both pointers are aligned to and cascades, this version always stores 16-byte vectors: a byte
- * head brings dst to a 16-byte boundary, the body issues four (long copies: sixteen) independent
- * dwordx4 loads per lane before the first store (gfx950 accepts unaligned vector loads, so a src that
- * is not co-aligned only costs extra cache-line touches, not narrower instructions), and a byte tail
- * finishes.
+ * head brings dst to a 16-byte boundary, the body issues four (long copies: eight) independent
+ * dwordx4 loads per lane before the first store, and a byte tail finishes.  A src that is not
+ * co-aligned is read with unaligned dwordx4 loads, which cost extra cache-line touches on a multiple of
+ * 4 bytes and half the rate on any other; long copies read words there and shift them into place.
  * ---------------------------------------------------------------------------------------------- */
 typedef unsigned int nvshmemi_v4u __attribute__((ext_vector_type(4)));
 typedef nvshmemi_v4u __attribute__((aligned(1))) nvshmemi_v4u_unaligned;
@@ -182,6 +182,11 @@ typedef nvshmemi_v4u __attribute__((aligned(1))) nvshmemi_v4u_unaligned;
 #endif
 #ifndef NVSHMEMI_AMD_COPY_DEEP_MIN
 #define NVSHMEMI_AMD_COPY_DEEP_MIN 32
+#endif
+/* ... and this many where the source's offset is no multiple of 4 (NVSHMEMI_AMD_SRC_SHIFTED) and ordinary rounds take
+ * twice as long: one round */
+#ifndef NVSHMEMI_AMD_COPY_SHIFTED_MIN
+#define NVSHMEMI_AMD_COPY_SHIFTED_MIN NVSHMEMI_AMD_COPY_DEEP_UNROLL
 #endif
 /* Cache policy of the vector body.  Stores stream (non-temporal): a copy never reads its destination
  * back.  Loads stay cacheable for short and medium copies, because callers often push the same source
@@ -224,6 +229,15 @@ template <bool SRC_ALIGNED, bool NT_LOAD>
 NVSHMEMI_DEVICE_INLINE nvshmemi_v4u nvshmemi_amd_stream_load16(const char *p) {
     if (NT_LOAD && SRC_ALIGNED) return __builtin_nontemporal_load(reinterpret_cast<const nvshmemi_v4u *>(p));
     return nvshmemi_amd_load16<SRC_ALIGNED>(p);
+}
+/* The next lane's x (DPP wave_shl:1); `last` in the wavefront's last lane and where the next one is not active. */
+NVSHMEMI_DEVICE_INLINE unsigned nvshmemi_amd_next_lane(unsigned x, unsigned last) {
+    return (unsigned)__builtin_amdgcn_update_dpp((int)last, (int)x, 0x130, 0xf, 0xf, false);
+}
+/* The 16 bytes that start `shift` (0 to 3) bytes into the words v.x, v.y, v.z, v.w, next. */
+NVSHMEMI_DEVICE_INLINE nvshmemi_v4u nvshmemi_amd_shift_words(nvshmemi_v4u v, unsigned next, unsigned shift) {
+    return nvshmemi_v4u{__builtin_amdgcn_alignbyte(v.y, v.x, shift), __builtin_amdgcn_alignbyte(v.z, v.y, shift),
+                        __builtin_amdgcn_alignbyte(v.w, v.z, shift), __builtin_amdgcn_alignbyte(next, v.w, shift)};
 }
 /* Where the stores of a copy go: streamed (non-temporal; the lines stay dirty in this XCD's L2 until
  * they are evicted or a release writes the L2 back) or written through the L2 to memory at agent scope,
@@ -307,11 +321,20 @@ NVSHMEMI_DEVICE_INLINE size_t nvshmemi_amd_copy_rounds(char *__restrict__ dst,
  *   of 1024 threads per PE move 4.73 TB/s interleaved, 5.56 in runs and 6.05 in runs swept in address order;
  *   one such block 61, 77 and 78 GB/s.  Blocks of 256 threads or fewer share their compute unit with other
  *   blocks, whose requests interleave anyway: neither the barriers nor the sweep changes their rate.  (The
- *   number of rounds is the same for every wavefront of the block, so all of them reach every barrier.) */
+ *   number of rounds is the same for every wavefront of the block, so all of them reach every barrier.)
+ *
+ * A source on another offset than the destination takes the same rounds; where that is no multiple of 4, the
+ * fifth word of a lane's vector is the first that the next lane loaded, and one more load per round fetches the
+ * words behind each KiB for the last lane.  us for 8 PEs, byte loads in ordinary rounds / here / co-aligned: 16 MiB from one
+ * block of 1024 threads 578 / 308 / 281, 256 MiB from 16 1166 / 761 / 711; on a multiple of 4 336 / 286 and 945 / 732.
+ * (Streamed loads of lines that two lanes share: 3 % faster here, where one wavefront reads on behind the other, and a
+ * third slower in ordinary rounds, where it is another block.) */
 #ifndef NVSHMEMI_AMD_COPY_PHASED_THREADS
 #define NVSHMEMI_AMD_COPY_PHASED_THREADS 512
 #endif
-template <bool NT_LOAD, int STORE, int U, bool BLOCK_WIDE>
+/* The source's offset from the destination's 16-byte boundaries: none, some, or one that is no multiple of 4. */
+enum nvshmemi_amd_source_t { NVSHMEMI_AMD_SRC_ALIGNED = 0, NVSHMEMI_AMD_SRC_UNALIGNED = 1, NVSHMEMI_AMD_SRC_SHIFTED = 2 };
+template <int SRC, bool NT_LOAD, int STORE, int U, bool BLOCK_WIDE>
 NVSHMEMI_DEVICE_INLINE size_t nvshmemi_amd_copy_deep_rounds(char *__restrict__ dst, const char *__restrict__ src,
                                                            size_t nvec, unsigned tid, size_t nthr) {
     const size_t per_round = (size_t)U * nthr;
@@ -321,8 +344,11 @@ NVSHMEMI_DEVICE_INLINE size_t nvshmemi_amd_copy_deep_rounds(char *__restrict__ d
     const bool phased = BLOCK_WIDE && nthr >= NVSHMEMI_AMD_COPY_PHASED_THREADS;
     const size_t step = phased ? nthr * 16 : (size_t)1024;              /* from one instruction to the next */
     const size_t wave_off = wave * (phased ? (size_t)1024 : (size_t)(U * 1024));
-    const char *s0 = src + wave_off;
+    constexpr bool SHIFTED = SRC == NVSHMEMI_AMD_SRC_SHIFTED;
+    const unsigned shift = SHIFTED ? (unsigned)((uintptr_t)src & 3) : 0;
+    const char *s0 = src - shift + wave_off;
     char *d0 = dst + wave_off;
+    const unsigned behind = (tid & (U - 1)) * (unsigned)step + 1024;  /* lane u fetches the word behind the u-th KiB */
     /* In the first layout the rounds are walked from a start that differs from block to block, wrapping at
      * the end.  Blocks that each stream a slice of one large message otherwise march in step, at equal
      * offsets in slices that lie a power of two (or the PE distance) apart, and keep meeting on the same
@@ -340,11 +366,23 @@ NVSHMEMI_DEVICE_INLINE size_t nvshmemi_amd_copy_deep_rounds(char *__restrict__ d
         char *d = d0 + r * (16 * per_round);
         if (++r == rounds) r = 0;
         nvshmemi_v4u v[U];
+        unsigned last = 0;
+        if (SHIFTED) last = *reinterpret_cast<const unsigned *>(s + behind);
 #pragma unroll
-        for (int u = 0; u < U; ++u) v[u] = nvshmemi_amd_stream_load16<true, NT_LOAD>(s + u * step + lane_off);
+        for (int u = 0; u < U; ++u) {
+            const char *from = s + u * step + lane_off;
+            if (SRC == NVSHMEMI_AMD_SRC_ALIGNED) v[u] = nvshmemi_amd_stream_load16<true, NT_LOAD>(from);
+            else if (NT_LOAD) v[u] = __builtin_nontemporal_load(reinterpret_cast<const nvshmemi_v4u_unaligned *>(from));
+            else v[u] = nvshmemi_amd_load16<false>(from);
+        }
         if (BLOCK_WIDE && phased) asm volatile("s_barrier" ::: "memory");
 #pragma unroll
-        for (int u = 0; u < U; ++u) nvshmemi_amd_stream_store16<STORE>(d + u * step + lane_off, v[u]);
+        for (int u = 0; u < U; ++u) {
+            if (SHIFTED)
+                v[u] = nvshmemi_amd_shift_words(
+                    v[u], nvshmemi_amd_next_lane(v[u].x, (unsigned)__builtin_amdgcn_readlane((int)last, u)), shift);
+            nvshmemi_amd_stream_store16<STORE>(d + u * step + lane_off, v[u]);
+        }
         if (BLOCK_WIDE && phased) asm volatile("s_barrier" ::: "memory");
     }
     return rounds * per_round;
@@ -361,19 +399,22 @@ NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_copy_vectors(char *__restrict__ dst,
                                                      const char *__restrict__ src, size_t nvec,
                                                      size_t tid, size_t nthr, bool stream_loads) {
 #if NVSHMEMI_AMD_COPY_DEEP_UNROLL > NVSHMEMI_AMD_COPY_UNROLL
+#define NVSHMEMI_AMD_DEEP(SRC, NT) \
+    nvshmemi_amd_copy_deep_rounds<SRC, NT, STORE, NVSHMEMI_AMD_COPY_DEEP_UNROLL, BLOCK_WIDE>(dst, src, nvec, (unsigned)tid, nthr)
+    constexpr int SRC = SRC_ALIGNED ? NVSHMEMI_AMD_SRC_ALIGNED : NVSHMEMI_AMD_SRC_UNALIGNED;
+    const bool shifted = !SRC_ALIGNED && ((uintptr_t)src & 3) != 0;
     /* (the second bound follows from the first for whole wavefronts; spelled out, it lets the compiler drop
      * the deep rounds and their registers where the caller's length is known to be short) */
-    if (SRC_ALIGNED && (nthr & 63) == 0 && nvec >= (size_t)NVSHMEMI_AMD_COPY_DEEP_MIN * nthr &&
-        nvec >= (size_t)NVSHMEMI_AMD_COPY_DEEP_MIN * 64) {
-        const size_t done =
-            stream_loads ? nvshmemi_amd_copy_deep_rounds<true, STORE, NVSHMEMI_AMD_COPY_DEEP_UNROLL, BLOCK_WIDE>(
-                               dst, src, nvec, (unsigned)tid, nthr)
-                         : nvshmemi_amd_copy_deep_rounds<false, STORE, NVSHMEMI_AMD_COPY_DEEP_UNROLL, BLOCK_WIDE>(
-                               dst, src, nvec, (unsigned)tid, nthr);
+    const size_t least = shifted ? NVSHMEMI_AMD_COPY_SHIFTED_MIN : NVSHMEMI_AMD_COPY_DEEP_MIN;
+    if ((nthr & 63) == 0 && nvec >= least * nthr && nvec >= least * 64) {
+        size_t done;
+        if (shifted) done = stream_loads ? NVSHMEMI_AMD_DEEP(NVSHMEMI_AMD_SRC_SHIFTED, true) : NVSHMEMI_AMD_DEEP(NVSHMEMI_AMD_SRC_SHIFTED, false);
+        else done = stream_loads ? NVSHMEMI_AMD_DEEP(SRC, true) : NVSHMEMI_AMD_DEEP(SRC, false);
         dst += 16 * done;
         src += 16 * done;
         nvec -= done;
     }
+#undef NVSHMEMI_AMD_DEEP
 #endif
     if (LOAD == NVSHMEMI_AMD_LOAD_STREAM && !NVSHMEMI_AMD_COPY_NT_ALWAYS && !stream_loads)
         nvshmemi_amd_copy_rounds<SRC_ALIGNED, false, STORE, NVSHMEMI_AMD_COPY_UNROLL, true>(dst, src, nvec, tid, nthr);
@@ -382,8 +423,8 @@ NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_copy_vectors(char *__restrict__ dst,
                                  NVSHMEMI_AMD_COPY_UNROLL, true>(dst, src, nvec, tid, nthr);
 }
 
-/* The copy by lane `tid` of the `nthr` of its group; BLOCK_WIDE: the group is the block. */
-template <int STORE, int LOAD, bool BLOCK_WIDE>
+/* The copy by lane `tid` of the `nthr` of its group. */
+template <int SCOPE, int STORE, int LOAD>
 NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_copy_lanes(char *__restrict__ dst, const char *__restrict__ src, size_t len,
                                                    size_t tid, size_t nthr, bool stream_loads) {
     size_t head = (size_t)(-(uintptr_t)dst & 15);
@@ -404,10 +445,11 @@ NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_copy_lanes(char *__restrict__ dst, cons
             if (((uintptr_t)src & 15) == 0) nvshmemi_amd_copy_vectors<true, STORE, LOAD>(dst, src, pre, tid, nthr, stream_loads);
             else nvshmemi_amd_copy_vectors<false, STORE, LOAD>(dst, src, pre, tid, nthr, stream_loads);
         }
+        constexpr bool block_wide = SCOPE == NVSHMEMI_THREADGROUP_BLOCK;   // every wavefront of the block is here
         if (((uintptr_t)src & 15) == 0)
-            nvshmemi_amd_copy_vectors<true, STORE, LOAD, BLOCK_WIDE>(dst + 16 * pre, src + 16 * pre, nvec - pre, tid, nthr, stream_loads);
+            nvshmemi_amd_copy_vectors<true, STORE, LOAD, block_wide>(dst + 16 * pre, src + 16 * pre, nvec - pre, tid, nthr, stream_loads);
         else
-            nvshmemi_amd_copy_vectors<false, STORE, LOAD, BLOCK_WIDE>(dst + 16 * pre, src + 16 * pre, nvec - pre, tid, nthr, stream_loads);
+            nvshmemi_amd_copy_vectors<false, STORE, LOAD, block_wide>(dst + 16 * pre, src + 16 * pre, nvec - pre, tid, nthr, stream_loads);
     }
     const size_t done = nvec * 16;
     for (size_t i = done + tid; i < len; i += nthr) nvshmemi_amd_store_byte<STORE>(dst + i, src[i]);
@@ -434,9 +476,8 @@ NVSHMEMI_DEVICE_INLINE void nvshmemi_memcpy_threadgroup(void *__restrict__ dst_v
         stream_loads = false;
     }
 #endif
-    /* (block scope: every wavefront of the block is here) */
-    nvshmemi_amd_copy_lanes<STORE, LOAD, SCOPE == NVSHMEMI_THREADGROUP_BLOCK>(
-        static_cast<char *>(dst_v), static_cast<const char *>(src_v), len, tid, nthr, stream_loads);
+    nvshmemi_amd_copy_lanes<SCOPE, STORE, LOAD>(static_cast<char *>(dst_v), static_cast<const char *>(src_v), len, tid, nthr,
+                                                stream_loads);
 }
 
 /* ------------------------------------------------------------------------------------------------

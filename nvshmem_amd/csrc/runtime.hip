@@ -142,8 +142,8 @@ __global__ void signal_wait_kernel(const uint64_t *word, int pe, int cmp, uint64
 constexpr size_t kPutSignalBlockBytes = (size_t)64 << 10;
 __global__ __launch_bounds__(1024) void put_signal_kernel(char *dst, const char *src, uint32_t bytes, uint32_t threads,
                                                           uint64_t *sig_addr, uint64_t signal, int sig_op, int pe) {
-    nvshmemi_amd_copy_lanes<NVSHMEMI_AMD_STORE_WRITE_THROUGH, NVSHMEMI_AMD_LOAD_BY_SIZE, true>(dst, src, bytes, threadIdx.x,
-                                                                                               threads, false);
+    nvshmemi_amd_copy_lanes<NVSHMEMI_THREADGROUP_BLOCK, NVSHMEMI_AMD_STORE_WRITE_THROUGH, NVSHMEMI_AMD_LOAD_BY_SIZE>(
+        dst, src, bytes, threadIdx.x, threads, false);
     nvshmemi_amd_wait_vm();
     __syncthreads();
     if (threadIdx.x == 0) nvshmemi_signal_op(sig_addr, signal, sig_op, pe);
