@@ -401,6 +401,8 @@ NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_copy_vectors(char *__restrict__ dst,
 #if NVSHMEMI_AMD_COPY_DEEP_UNROLL > NVSHMEMI_AMD_COPY_UNROLL
 #define NVSHMEMI_AMD_DEEP(SRC, NT) \
     nvshmemi_amd_copy_deep_rounds<SRC, NT, STORE, NVSHMEMI_AMD_COPY_DEEP_UNROLL, BLOCK_WIDE>(dst, src, nvec, (unsigned)tid, nthr)
+#define NVSHMEMI_AMD_SHORT_DEEP(NT) \
+    nvshmemi_amd_copy_deep_rounds<NVSHMEMI_AMD_SRC_SHIFTED, NT, STORE, 2, false>(dst, src, nvec, (unsigned)tid, nthr)
     constexpr int SRC = SRC_ALIGNED ? NVSHMEMI_AMD_SRC_ALIGNED : NVSHMEMI_AMD_SRC_UNALIGNED;
     const bool shifted = !SRC_ALIGNED && ((uintptr_t)src & 3) != 0;
     /* (the second bound follows from the first for whole wavefronts; spelled out, it lets the compiler drop
@@ -414,7 +416,15 @@ NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_copy_vectors(char *__restrict__ dst,
         src += 16 * done;
         nvec -= done;
     }
+    /* (what is left over too: 8 PEs, one block of 1024 threads, 128 KiB 7.0 -> 5.6 us, 200 000 bytes 9.1 -> 6.4) */
+    if (shifted && (nthr & 63) == 0 && nvec >= 2 * nthr) {
+        const size_t done = NVSHMEMI_AMD_SHORT_DEEP(false);
+        dst += 16 * done;
+        src += 16 * done;
+        nvec -= done;
+    }
 #undef NVSHMEMI_AMD_DEEP
+#undef NVSHMEMI_AMD_SHORT_DEEP
 #endif
     if (LOAD == NVSHMEMI_AMD_LOAD_STREAM && !NVSHMEMI_AMD_COPY_NT_ALWAYS && !stream_loads)
         nvshmemi_amd_copy_rounds<SRC_ALIGNED, false, STORE, NVSHMEMI_AMD_COPY_UNROLL, true>(dst, src, nvec, tid, nthr);

@@ -170,15 +170,15 @@ def test_copy_engine_all_mutual_alignments(rt):
             assert np.array_equal(got, want), (soff, doff, is_get)
 
 
-# A source on another offset than the destination is read in words, eight vectors per lane and round: around one
-# round (the least that takes them) and 32 vectors per lane (the least for offsets that are a multiple of 4), in blocks
-# below and from 512 threads on, which lay a round out differently, and in wavefronts.
+# A source on another offset than the destination is read in words, eight vectors per lane and round, then two: around
+# one round of each (the least that takes them) and 32 vectors per lane (the least for offsets that are a multiple of
+# 4), in blocks below and from 512 threads on, which lay a round out differently, and in wavefronts.
 @pytest.mark.parametrize("scope,threads,lanes", [(N.SCOPE_BLOCK, 64, 64), (N.SCOPE_BLOCK, 192, 192), (N.SCOPE_BLOCK, 512, 512),
                                                  (N.SCOPE_BLOCK, 1024, 1024), (N.SCOPE_WARP, 64, 64)])
 def test_long_copies_from_another_offset(rt, scope, threads, lanes):
     for soff in range(16):
-        for doff, vectors, extra in ((0, 8, 0), (5, 8, 15), (14, 9, 4), (3, 25, 1), (9, 32, 17), (0, 39, 0)):
-            size = 16 * lanes * vectors + (1024 if vectors != 8 else 0) + extra
+        for doff, vectors, extra in ((0, 2, 0), (7, 3, 15), (0, 8, 0), (5, 8, 15), (14, 9, 4), (3, 25, 1), (9, 32, 17), (0, 39, 0)):
+            size = 16 * lanes * vectors + (1024 if vectors not in (2, 8) else 0) + extra
             for is_get in (0, 1):
                 got, want = _ring(rt, size, 1, threads, scope, is_get, soff, doff, seed=soff + 16 * vectors)
                 assert np.array_equal(got, want), (soff, doff, size, is_get)
