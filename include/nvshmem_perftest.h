@@ -240,7 +240,8 @@ int nvshmem_perftest_device_barrier(uint64_t *counter, uint64_t *errors, int rou
  *   combine:  out[t*topk+k] = recv@dest_pe[dest_row]  via nvshmemx_getmem_nbi_block.
  * sig holds npes words per PE and must be zero before dispatch.  recv holds recv_cap_rows rows on
  * every PE; a routing entry outside [0, npes) x [0, recv_cap_rows) is skipped.  blocks_per_pe
- * blocks of `threads` threads per PE; dispatch is a cooperative launch (it waits on other PEs).
+ * blocks of `threads` threads per PE.  Dispatch is two plain launches, one that sends and one block per PE
+ * that waits for what the others announced; as many blocks as can be resident together are accepted.
  * The plain entry points move one row per wavefront and publish one signal update per block and
  * destination; the _ex forms choose the scope (NVSHMEM_PERFTEST_SCOPE_WARP or _BLOCK) and, with
  * bit 8 set in `scope` (dispatch only), signal after every row with nvshmemx_putmem_signal_nbi_warp /

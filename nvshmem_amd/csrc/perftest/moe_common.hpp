@@ -27,7 +27,8 @@ __device__ __forceinline__ unsigned wave_in_block_per_lane() { return threadIdx.
 }  // namespace
 
 namespace perftest {
-// moe_rowsignal.hip: collective launch of the dispatch kernel that signals every row; `args` are the
-// kernel's twelve arguments in order.
+// moe_rowsignal.hip: the dispatch kernel that signals every row; `args` are its eleven arguments in order.
 int launch_moe_rowsignal(bool warp, int blocks_per_pe, int threads, void **args, hipStream_t stream);
+// moe_shuffle.hip: launch of a kernel whose blocks send and never wait, one grid for all PEs.
+int launch_senders(const void *fn, int blocks_per_pe, int threads, void **args, hipStream_t stream);
 }  // namespace perftest

@@ -18,10 +18,9 @@ namespace {
 // Per-row signalling: the API-literal form, one nvshmemx_putmem_signal_nbi per row.
 template <bool WARP_SCOPED>
 __global__ void moe_dispatch_rowsignal_kernel(char *recv, const char *send, const int32_t *dest_pe,
-                                              const int64_t *dest_row, const uint64_t *expected,
-                                              uint64_t *sig, int tokens, int topk,
-                                              size_t row_bytes, size_t recv_cap_rows, int sig_op,
-                                              int sig_stride) {
+                                              const int64_t *dest_row, uint64_t *sig, int tokens,
+                                              int topk, size_t row_bytes, size_t recv_cap_rows,
+                                              int sig_op, int sig_stride) {
     const int me = nvshmem_my_pe(), np = nvshmem_n_pes();
     const int32_t *my_dest_pe = (const int32_t *)nvshmem_ptr(dest_pe, me);
     const int64_t *my_dest_row = (const int64_t *)nvshmem_ptr(dest_row, me);
@@ -57,11 +56,6 @@ __global__ void moe_dispatch_rowsignal_kernel(char *recv, const char *send, cons
                                              send + (r / (size_t)topk) * row_bytes, row_bytes,
                                              sig + (size_t)me * sig_stride, 1, sig_op, my_dest_pe[r]);
     }
-    if (blockIdx.x == 0) {
-        const uint64_t *my_expected = (const uint64_t *)nvshmem_ptr(expected, me);
-        for (int src = threadIdx.x; src < np; src += blockDim.x)
-            nvshmem_signal_wait_until(sig + (size_t)src * sig_stride, NVSHMEM_CMP_GE, my_expected[src]);
-    }
 }
 
 }  // namespace
@@ -71,7 +65,7 @@ namespace perftest {
 int launch_moe_rowsignal(bool warp, int blocks_per_pe, int threads, void **args, hipStream_t stream) {
     const void *fn = warp ? (const void *)moe_dispatch_rowsignal_kernel<true>
                           : (const void *)moe_dispatch_rowsignal_kernel<false>;
-    return nvshmemx_collective_launch(fn, dim3(blocks_per_pe), dim3(threads), args, 0, stream);
+    return launch_senders(fn, blocks_per_pe, threads, args, stream);
 }
 
 }  // namespace perftest

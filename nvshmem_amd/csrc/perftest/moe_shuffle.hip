@@ -38,9 +38,8 @@ constexpr int kMaxPes = NVSHMEMI_AMD_MAX_PES;
 // destinations' signal words (one release + npes atomic adds per block instead of one per row).
 template <bool WARP_SCOPED>
 __global__ void moe_dispatch_kernel(char *recv, const char *send, const int32_t *dest_pe,
-                                    const int64_t *dest_row, const uint64_t *expected,
-                                    uint64_t *sig, int tokens, int topk, size_t row_bytes,
-                                    size_t recv_cap_rows) {
+                                    const int64_t *dest_row, uint64_t *sig, int tokens, int topk,
+                                    size_t row_bytes, size_t recv_cap_rows) {
     __shared__ unsigned tally[kMaxPes];
     const int me = nvshmem_my_pe(), np = nvshmem_n_pes();
     const int32_t *my_dest_pe = (const int32_t *)nvshmem_ptr(dest_pe, me);
@@ -81,13 +80,15 @@ __global__ void moe_dispatch_kernel(char *recv, const char *send, const int32_t 
     nvshmemx_quiet_block();
     for (int pe = threadIdx.x; pe < np; pe += blockDim.x)
         if (tally[pe]) nvshmemx_signal_op(sig + me, (uint64_t)tally[pe], NVSHMEM_SIGNAL_ADD, pe);
+}
 
-    // receiver side: block 0 of every PE waits until each source has delivered what it announced
-    if (blockIdx.x == 0) {
-        const uint64_t *my_expected = (const uint64_t *)nvshmem_ptr(expected, me);
-        for (int src = threadIdx.x; src < np; src += blockDim.x)
-            nvshmem_signal_wait_until(sig + src, NVSHMEM_CMP_GE, my_expected[src]);
-    }
+// Receiver side of the dispatches above, a launch behind them: every PE waits until each source has delivered
+// what it announced.
+__global__ __launch_bounds__(NVSHMEMI_WARP_SIZE) void moe_receive_kernel(const uint64_t *expected, uint64_t *sig,
+                                                                         int sig_stride) {
+    const uint64_t *my_expected = (const uint64_t *)nvshmem_ptr(expected, nvshmem_my_pe());
+    for (int src = threadIdx.x; src < nvshmem_n_pes(); src += NVSHMEMI_WARP_SIZE)
+        nvshmem_signal_wait_until(sig + (size_t)src * sig_stride, NVSHMEM_CMP_GE, my_expected[src]);
 }
 
 // Dispatch cut into short work items: an item is one piece of one token's row, pushed to all of the
@@ -351,6 +352,30 @@ bool moe_args_ok(const void *table_pe, const void *table_row, int tokens, int to
 
 }  // namespace
 
+namespace perftest {
+
+// Sending and waiting are two plain launches.  As one kernel whose first block of every PE also waited, the grid had to
+// be resident as a whole, and a cooperative launch runs in step with the stream on either side of it: 18 us a call more
+// (8 PEs, dispatch and combine of 64 tokens to 8 experts each in rows of 14 KiB 58.9 us, now 40.4; of 152 tokens to 4 in
+// rows of 2 KiB 38.4, now 19.7).  Blocks that only send end whatever else holds the GPU, and the wait behind them on the
+// stream has its signals when it starts.  A grid that could not have been resident is refused as before.
+int launch_senders(const void *fn, int blocks_per_pe, int threads, void **args, hipStream_t stream) {
+    int cap = 0;
+    const int rc = nvshmemx_collective_launch_query_gridsize(fn, dim3(threads), args, 0, &cap);
+    if (rc != NVSHMEMX_SUCCESS) return rc;
+    if (blocks_per_pe > cap) {
+        fprintf(stderr, "nvshmem_perftest: %d blocks per PE, at most %d of %d threads\n", blocks_per_pe, cap, threads);
+        return NVSHMEMX_ERROR_COLLECTIVE_LAUNCH_FAILED;
+    }
+    const hipError_t e = hipLaunchKernel(fn, dim3(blocks_per_pe, 1, (unsigned)nvshmem_n_pes()), dim3(threads), args, 0, stream);
+    if (e == hipSuccess) return 0;
+    (void)hipGetLastError();
+    fprintf(stderr, "nvshmem_perftest: moe_dispatch launch failed: %s\n", hipGetErrorString(e));
+    return NVSHMEMX_ERROR_COLLECTIVE_LAUNCH_FAILED;
+}
+
+}  // namespace perftest
+
 extern "C" {
 
 // scope: NVSHMEM_PERFTEST_SCOPE_WARP (row per wavefront) or _BLOCK (row per block);
@@ -376,12 +401,16 @@ int nvshmem_perftest_moe_dispatch_put_signal(void *recv, size_t recv_cap_rows, c
         return NVSHMEMX_ERROR_INVALID_VALUE;
     char *r = (char *)recv;
     const char *s = (const char *)send;
-    void *args[] = {&r, &s, &dest_pe, &dest_row, &expected, &sig, &tokens, &topk, &row_bytes,
-                    &recv_cap_rows, &sig_op, &sig_stride};
-    if (per_row) return perftest::launch_moe_rowsignal(warp, blocks_per_pe, threads, args, (hipStream_t)stream);
+    void *row_args[] = {&r, &s, &dest_pe, &dest_row, &sig, &tokens, &topk, &row_bytes, &recv_cap_rows, &sig_op,
+                        &sig_stride};
+    void *args[] = {&r, &s, &dest_pe, &dest_row, &sig, &tokens, &topk, &row_bytes, &recv_cap_rows};
     const void *fn = warp ? (const void *)moe_dispatch_kernel<true> : (const void *)moe_dispatch_kernel<false>;
-    return nvshmemx_collective_launch(fn, dim3(blocks_per_pe), dim3(threads), args, 0,
-                                      (hipStream_t)stream);
+    const int rc = per_row ? perftest::launch_moe_rowsignal(warp, blocks_per_pe, threads, row_args, (hipStream_t)stream)
+                           : perftest::launch_senders(fn, blocks_per_pe, threads, args, (hipStream_t)stream);
+    if (rc != 0) return rc;
+    hipLaunchKernelGGL(moe_receive_kernel, dim3(1, 1, (unsigned)nvshmem_n_pes()), dim3(NVSHMEMI_WARP_SIZE), 0,
+                       (hipStream_t)stream, expected, sig, sig_stride);
+    return perftest::launch_status("moe_receive");
 }
 
 int nvshmem_perftest_moe_dispatch_ex(void *recv, size_t recv_cap_rows, const void *send, const int32_t *dest_pe,

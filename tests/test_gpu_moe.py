@@ -139,6 +139,37 @@ def test_moe_routing_table_outside_the_buffer_is_skipped_not_written():
         assert (rt.download_all(recv, (8 * row,), np.uint8) == 0).all()
 
 
+@pytest.mark.parametrize("scope", [N.SCOPE_WARP, N.SCOPE_BLOCK | 256, N.SCOPE_WARP | 256 | 512])
+def test_moe_dispatch_waits_for_every_announced_row(scope):
+    """Rows that nobody sends are waited for, on the PE that expects them, until the spin limit."""
+    npes, T, K, row = 33, 8, 1, 48
+    with runtime(npes, 1 << 22) as rt:
+        perf = rt.perftest()
+        send = rt.calloc(T * row, 1); recv = rt.calloc(npes * T * row, 1)
+        d_pe = rt.malloc(T * K * 4); d_row = rt.malloc(T * K * 8)
+        expected = rt.malloc(npes * 8); sig = rt.calloc(npes, 8)
+        rt.upload_all(d_pe, np.full((npes, T * K), 2, np.int32))          # everything goes to PE 2
+        rt.upload_all(d_row, (np.arange(npes)[:, None] * T + np.arange(T)).astype(np.int64))
+        table = np.zeros((npes, npes), np.uint64)
+        table[2] = T
+        for late in (None, 0, npes - 1):
+            if late is not None:
+                table[late, npes - 1] += 1
+            rt.upload_all(expected, table)
+            rt.fill(sig, 0, npes * 8)
+            rt.lib.nvshmemx_amd_set_spin_limit(2000)
+            note("moe_dispatch scope=%#x, a row too many expected on PE %s" % (scope, late))
+            assert perf.nvshmem_perftest_moe_dispatch_ex(recv, npes * T, send, d_pe, d_row, expected, sig, T, K, row, 2, 128,
+                                                         scope, None) == 0
+            rt.sync()
+            rt.lib.nvshmemx_amd_set_spin_limit(1 << 22)
+            gave_up = [pe for pe in range(npes) if rt.read_timeout(pe)[0] != 0]
+            assert gave_up == ([] if late is None else [late]), gave_up
+            if late is not None:
+                table[late, npes - 1] -= 1
+        assert np.array_equal(rt.download_all(sig, (npes,), np.uint64), table)
+
+
 def test_config5_full_size_moe_shuffle():
     # 8 PEs x 8192 tokens x 7168 bf16, top-8 of 256 experts, Zipf(1.1): the receive buffer of the
     # busiest PE decides the symmetric allocation

@@ -23,6 +23,25 @@ def test_collective_launches_are_cooperative_unless_asked(recorded, plain, coope
     recorded(COLLECTIVE_LAUNCH % cooperative, **env)
 
 
+@pytest.mark.parametrize("scope", [1, 2, 1 | 256, 2 | 256 | 512])
+def test_token_dispatch_sends_and_waits_in_plain_launches(recorded, scope):  # noqa: F811
+    """Blocks that send never wait, so neither launch needs its grid to be resident as a whole; grids that could not be
+    are refused all the same."""
+    recorded("""
+perf = _lib.load_perftest()
+ok(lib.nvshmemx_amd_init(8, 8 << 20))
+a = lib.nvshmem_malloc(1 << 20)
+launches()
+def dispatch(blocks):
+    return perf.nvshmem_perftest_moe_dispatch_put_signal(a, 8, a, a, a, a, a, 1, 8, 2, 1024, blocks, 256, %d, None)
+assert dispatch(64) == 0
+(sender, c0, grid, block, lds), (receiver, c1, wait_grid, wait_block, lds1) = launches()
+assert "moe_dispatch" in sender and not c0 and grid == (64, 1, 8) and block == (256, 1, 1)
+assert "moe_receive" in receiver and not c1 and wait_grid == (1, 1, 8) and wait_block == (64, 1, 1)
+assert dispatch(1 << 20) != 0 and not launches()
+""" % scope)
+
+
 def test_copies_that_are_in_flight_all_at_once_are_not_paced(recorded):  # noqa: F811
     """fcollect and broadcast of up to 32 pieces per compute unit (16 from 12 members on) store back to back, larger ones
     one destination at a time (third template argument of the kernel)."""
