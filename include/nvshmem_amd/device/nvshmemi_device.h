@@ -170,6 +170,11 @@ typedef nvshmemi_v4u __attribute__((aligned(1))) nvshmemi_v4u_unaligned;
 #ifndef NVSHMEMI_AMD_COPY_UNROLL
 #define NVSHMEMI_AMD_COPY_UNROLL 4
 #endif
+/* Copies of this many vectors and more are cut on the destination's 1 KiB boundaries (64 instead: combines of 2 KiB
+ * pieces that lie 256 bytes off take three instructions for two and lose 1 %). */
+#ifndef NVSHMEMI_AMD_COPY_SKIP_MIN
+#define NVSHMEMI_AMD_COPY_SKIP_MIN 256
+#endif
 /* Long copies - a lane owns at least NVSHMEMI_AMD_COPY_DEEP_MIN vectors - run rounds of
  * NVSHMEMI_AMD_COPY_DEEP_UNROLL vectors per lane first (0 switches them off).  Eight is what fits the
  * registers the rest of the engine needs anyway.  Sixteen takes 30 more vector registers (82 in all: five
@@ -250,7 +255,10 @@ template <int STORE = NVSHMEMI_AMD_STORE_STREAM>
 NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_stream_store16(char *p, nvshmemi_v4u v) {
     if (STORE == NVSHMEMI_AMD_STORE_WRITE_THROUGH) {
         // sc1 nt: written through at agent scope and marked streaming (+3 % over plain sc1 on the per-row
-        // put_signal token dispatch); the s_nop for the same reason as in nvshmemi_amd_store16_agent
+        // put_signal token dispatch); the s_nop for the same reason as in nvshmemi_amd_store16_agent.  The compiler
+        // does not count these stores: before each of a run it would wait until no more loads are outstanding than
+        // were issued behind the one that fills this store's registers, and so for the stores in front of it.  A run
+        // of them therefore waits for all its loads first.
         asm volatile("global_store_dwordx4 %0, %1, off sc1 nt\n\ts_nop 1" : : "v"(p), "v"(v) : "memory");
         return;
     }
@@ -284,6 +292,7 @@ NVSHMEMI_DEVICE_INLINE size_t nvshmemi_amd_copy_rounds(char *__restrict__ dst,
 #pragma unroll
         for (int u = 0; u < U; ++u)
             v[u] = nvshmemi_amd_stream_load16<SRC_ALIGNED, NT_LOAD>(src + 16 * (i + u * nthr));
+        if (STORE == NVSHMEMI_AMD_STORE_WRITE_THROUGH) nvshmemi_amd_wait_vm(); /* (see nvshmemi_amd_stream_store16) */
 #pragma unroll
         for (int u = 0; u < U; ++u) nvshmemi_amd_stream_store16<STORE>(dst + 16 * (i + u * nthr), v[u]);
     }
@@ -292,6 +301,54 @@ NVSHMEMI_DEVICE_INLINE size_t nvshmemi_amd_copy_rounds(char *__restrict__ dst,
     if constexpr (CASCADE && U > 1)
         return nvshmemi_amd_copy_rounds<SRC_ALIGNED, NT_LOAD, STORE, NEXT, true>(dst, src, nvec, i, nthr);
     return i;
+}
+
+/* A short copy by one wavefront - at most U vectors per lane, both sides on 16-byte boundaries: ONE round, whatever the
+ * number of vectors.  The cascade above makes a round trip to memory for every power of two in that number, one behind
+ * the other, and another for the vectors in front of the destination's next KiB.  Here lane and vector number are offsets
+ * into buffer descriptors of just the bytes that are copied: what lies outside of them the hardware neither loads nor
+ * stores, so no instruction needs a predicate, and instruction u covers the u-th KiB of memory that the copy touches
+ * (from `skip` vectors in front of dst on), aligned.  A token dispatch with a signal per row, us, cascade / here: 8 x 1505
+ * tokens to 4 experts each in rows of 7424 bytes 100 / 71, 8 x 64 to 8 of 14 336 bytes 13.5 / 12.4; with the combine, of
+ * whose pieces a row's last one is short, 8 x 1000 to 6 in rows of 4352 bytes 159 / 126, 8 x 218 to 8 of 11 776 104 / 98.
+ * (Only for the wavefront scope.  A block's rounds are wide: few of its copies fit one, and the choice alone costs those
+ * that do not 0.1 us in 4 to 9.) */
+NVSHMEMI_DEVICE_INLINE __amdgpu_buffer_rsrc_t nvshmemi_amd_buffer(const char *p, unsigned bytes) {
+    const uint64_t a = (uint64_t)(uintptr_t)p;
+    const uint64_t base = (uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)a) |
+                          (uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(a >> 32)) << 32;
+    return __builtin_amdgcn_make_buffer_rsrc((void *)(uintptr_t)base, 0, __builtin_amdgcn_readfirstlane((int)bytes), 0x00020000);
+}
+template <bool NT_LOAD, int STORE, int U>
+NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_copy_one_round(char *dst, const char *src, unsigned nvec, unsigned skip, unsigned lane) {
+    /* as many instructions as it takes, to the next of 1, 2, 4, ... U */
+    constexpr int LESS = (U & (U - 1)) ? (U >= 16 ? 16 : U >= 8 ? 8 : U >= 4 ? 4 : 2) : U / 2;
+    if constexpr (U > 1) {
+        if (__builtin_amdgcn_readfirstlane((int)(skip + nvec)) <= LESS * 64) {
+            nvshmemi_amd_copy_one_round<NT_LOAD, STORE, LESS>(dst, src, nvec, skip, lane);
+            return;
+        }
+    }
+    /* cache policy bits of the buffer instructions: 2 nt, 16 sc1 */
+    constexpr int LOAD_BITS = NT_LOAD ? 2 : 0;
+#if defined(NVSHMEMI_AMD_COPY_NT) && !(NVSHMEMI_AMD_COPY_NT & 2)
+    constexpr int STORE_BITS = STORE == NVSHMEMI_AMD_STORE_WRITE_THROUGH ? 18 : 0;
+#else
+    constexpr int STORE_BITS = STORE == NVSHMEMI_AMD_STORE_WRITE_THROUGH ? 18 : 2;
+#endif
+    const auto from = nvshmemi_amd_buffer(src, nvec * 16), to = nvshmemi_amd_buffer(dst, nvec * 16);
+    /* The lanes in front of dst have offsets just below 2^32, outside of any copy.  Only the first instruction has
+     * such lanes; the others' offsets start from a base that is never negative, kept apart from the first's, so that
+     * no carry decides what lies inside. */
+    unsigned first = (lane - skip) * 16, next = (lane + 64 - skip) * 16;
+    asm("" : "+v"(next));
+    nvshmemi_v4u v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        v[u] = __builtin_amdgcn_raw_buffer_load_b128(from, (int)(u ? next + (unsigned)(u - 1) * 1024 : first), 0, LOAD_BITS);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        __builtin_amdgcn_raw_buffer_store_b128(v[u], to, (int)(u ? next + (unsigned)(u - 1) * 1024 : first), 0, STORE_BITS);
 }
 
 /* The translation unit's fixed choice for the loads of the ordinary rounds; the deep rounds of a long
@@ -376,6 +433,7 @@ NVSHMEMI_DEVICE_INLINE size_t nvshmemi_amd_copy_deep_rounds(char *__restrict__ d
             else v[u] = nvshmemi_amd_load16<false>(from);
         }
         if (BLOCK_WIDE && phased) asm volatile("s_barrier" ::: "memory");
+        if (STORE == NVSHMEMI_AMD_STORE_WRITE_THROUGH) nvshmemi_amd_wait_vm();
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             if (SHIFTED)
@@ -439,6 +497,26 @@ NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_copy_lanes(char *__restrict__ dst, cons
                                                    size_t tid, size_t nthr, bool stream_loads) {
     size_t head = (size_t)(-(uintptr_t)dst & 15);
     if (head > len) head = len;
+    if (SCOPE == NVSHMEMI_THREADGROUP_WARP && nthr == 64 && (((uintptr_t)dst ^ (uintptr_t)src) & 15) == 0 &&
+        len <= NVSHMEMI_AMD_COPY_UNROLL * 1024) {
+        const unsigned nvec = (unsigned)(len - head) / 16, edge = (unsigned)head, tail = (unsigned)(len - head) % 16;
+        const unsigned skip = nvec >= NVSHMEMI_AMD_COPY_SKIP_MIN ? (unsigned)(((uintptr_t)dst + edge) >> 4) & 63 : 0;
+        if (skip + nvec <= NVSHMEMI_AMD_COPY_UNROLL * 64) {
+            /* the bytes on either side of the vectors: a lane each, loaded in front of the vectors, stored behind them */
+            const unsigned lane = (unsigned)tid;
+            const bool mine = (lane < edge) | (lane - 16 < tail);
+            const unsigned at = lane < edge ? lane : edge + nvec * 16 + (lane - 16);
+            char byte = 0;
+            if (mine) byte = src[at];
+            constexpr bool nt = NVSHMEMI_AMD_COPY_NT_ALWAYS || LOAD == NVSHMEMI_AMD_LOAD_STREAM;
+            if (nt && !NVSHMEMI_AMD_COPY_NT_ALWAYS && !stream_loads)
+                nvshmemi_amd_copy_one_round<false, STORE, NVSHMEMI_AMD_COPY_UNROLL>(dst + edge, src + edge, nvec, skip, lane);
+            else
+                nvshmemi_amd_copy_one_round<nt, STORE, NVSHMEMI_AMD_COPY_UNROLL>(dst + edge, src + edge, nvec, skip, lane);
+            if (mine) nvshmemi_amd_store_byte<STORE>(dst + at, byte);
+            return;
+        }
+    }
     for (size_t i = tid; i < head; i += nthr) nvshmemi_amd_store_byte<STORE>(dst + i, src[i]);
     dst += head;
     src += head;
@@ -450,7 +528,7 @@ NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_copy_lanes(char *__restrict__ dst, cons
          * that every wavefront access of the body is one aligned 1 KiB piece (HBM serves those
          * measurably faster than pieces that straddle the boundary). */
         size_t pre = 0;
-        if (nvec >= 256) {
+        if (nvec >= NVSHMEMI_AMD_COPY_SKIP_MIN) {
             pre = (size_t)((-(uintptr_t)dst >> 4) & 63);
             if (((uintptr_t)src & 15) == 0) nvshmemi_amd_copy_vectors<true, STORE, LOAD>(dst, src, pre, tid, nthr, stream_loads);
             else nvshmemi_amd_copy_vectors<false, STORE, LOAD>(dst, src, pre, tid, nthr, stream_loads);

@@ -185,6 +185,30 @@ def test_long_copies_from_another_offset(rt, scope, threads, lanes):
 
 
 @pytest.mark.parametrize("is_get", [0, 1])
+@pytest.mark.parametrize("shift", [0, 1, 9, 16 * 5, 16 * 63 + 15])
+def test_short_copies_by_a_wavefront(rt, is_get, shift):
+    """One round by buffer descriptors, both sides on the same offset: sizes around its 1, 2 and 4 instructions (and the
+    ordinary rounds behind them), with bytes on either side of the vectors; nothing beside the copy changes."""
+    perf, room = rt.perftest(), 3 << 12
+    src, dst = rt.malloc(room), rt.malloc(room)
+    data = O.fill_all("bytes", NPES, room, 5)
+    rt.upload_all(src, data)
+    for n in [1, 2, 14, 15, 16, 17, 30, 31, 32, 33, 47, 1007, 1008, 1023, 1024, 1025, 1040, 2031, 2048, 2049, 3000, 4064, 4080,
+              4095, 4096, 4097, 4111, 4112, 5000]:
+        rt.fill(dst, 0x5A, room)
+        note("short copies by a wavefront: %d bytes, shift %d, get %d" % (n, shift, is_get))
+        assert perf.nvshmem_perftest_ring_rma(dst + shift, src + shift, n, 1, 64, N.SCOPE_WARP, is_get, 1, None) == 0
+        rt.sync()
+        got = rt.download_all(dst, (room,), np.uint8)
+        for pe in range(NPES):
+            other = (pe + 1) % NPES if is_get else (pe - 1) % NPES
+            want = np.full(room, 0x5A, np.uint8)
+            want[shift:shift + n] = data[other][shift:shift + n]
+            assert np.array_equal(got[pe], want), (n, pe)
+    rt.free(src); rt.free(dst)
+
+
+@pytest.mark.parametrize("is_get", [0, 1])
 def test_ring_put_get_256MiB_16_blocks(rt, is_get):
     # the largest message of the sweep: 256 MiB per PE, 16 blocks per PE
     size = 1 << 28

@@ -108,6 +108,15 @@ def test_moe_shuffle_small(scope):
         _shuffle(rt, 8, 33, 3, 64, 200 + 6, 2, 128, scope, check_exchange=False)   # ragged rows
 
 
+@pytest.mark.parametrize("row", [16, 31, 1008, 1040, 2064, 4080, 4112, 4352, 7424, 7440, 11776, 14320, 14336, 14352])
+@pytest.mark.parametrize("scope", [N.SCOPE_WARP, N.SCOPE_WARP | 256 | 512])
+def test_moe_shuffle_row_sizes(scope, row):
+    """Rows at the edges of what a wavefront copies in one round of 1, 2, 4, 8 or 14 instructions, on and off the KiB
+    boundaries of the receive buffer, where neighbouring rows show every byte written beside a row."""
+    with runtime(4, 1 << 24) as rt:
+        _shuffle(rt, 4, 24, 3, 8, row, 2, 256, scope, check_exchange=False)
+
+
 def test_moe_dispatch_pieces_through_the_put_api(monkeypatch):
     """NVSHMEM_PERFTEST_MOE_PUTS selects the nvshmemx_putmem_nbi_warp form of the short work items also
     for aligned rows (without it only rows that are not 16-byte aligned take it)."""
