@@ -1918,11 +1918,99 @@ NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_staged_reduce(nvshmem_team_t team, cons
     }
 }
 
+/* Rounds of the in-kernel allreduce's fold: lane `tid` of `nthr` folds vectors base + tid, base + tid + nthr, ... of the
+ * `nvec` at src (member 0's; the others' lie pe_stride elements apart) in the allreduce's order and stores each result to
+ * every member.  A round fetches V vectors from each of M members, all before the first fold: one after the other they
+ * would each pay the way to another PE's memory.  FULL rounds run while every lane has V vectors left, and with PHASED
+ * the block's wavefronts meet between the loads of a round and its stores and behind these (see nvshmemi_amd_reduce_vectors).
+ * Returns where the rounds ended. */
+enum nvshmemi_amd_rounds_t { NVSHMEMI_AMD_ROUNDS_ALL = 0, NVSHMEMI_AMD_ROUNDS_FULL = 1, NVSHMEMI_AMD_ROUNDS_PHASED = 2 };
+template <typename T, int OP, int M, int V, int KIND = NVSHMEMI_AMD_ROUNDS_ALL>
+NVSHMEMI_DEVICE_INLINE size_t nvshmemi_amd_reduce_rounds(T *dst, const T *src, size_t pe_stride, int npes, size_t nvec,
+                                                         size_t tid, size_t nthr, size_t base) {
+    constexpr size_t VEC = 16 / sizeof(T);
+    constexpr bool FULL = KIND != NVSHMEMI_AMD_ROUNDS_ALL, PHASED = KIND == NVSHMEMI_AMD_ROUNDS_PHASED;
+    static_assert(FULL || V == 1, "rounds of several vectors per lane are full ones");
+    union pack_t { nvshmemi_v4u bits; T e[VEC]; __device__ pack_t() {} };
+    for (; FULL ? base + V * nthr <= nvec : base + tid < nvec; base += V * nthr) {
+        pack_t acc[V];
+        for (int p0 = 0; p0 < npes; p0 += M) {
+            pack_t x[V][M];
+#pragma unroll
+            for (int j = 0; j < V; ++j)
+#pragma unroll
+                for (int k = 0; k < M; ++k) {
+                    const int pe = p0 + k < npes ? p0 + k : npes - 1; /* past the end: fetched again, not folded */
+                    x[j][k].bits = *reinterpret_cast<const nvshmemi_v4u *>(src + (size_t)pe * pe_stride +
+                                                                          (base + j * nthr + tid) * VEC);
+                }
+            if (PHASED) asm volatile("s_barrier" ::: "memory");
+#pragma unroll
+            for (int k = 0; k < M; ++k) {
+                const int pe = p0 + k;
+#pragma unroll
+                for (int j = 0; j < V; ++j)
+                    if (pe == 0) acc[j].bits = x[j][0].bits;
+                    else if (pe < npes) {
+#pragma unroll
+                        for (size_t e = 0; e < VEC; ++e) acc[j].e[e] = nvshmemi_amd_fold_step<T, OP>(pe, acc[j].e[e], x[j][k].e[e]);
+                    }
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < V; ++j)
+            for (int pe = 0; pe < npes; ++pe)
+                *reinterpret_cast<nvshmemi_v4u *>(dst + (size_t)pe * pe_stride + (base + j * nthr + tid) * VEC) = acc[j].bits;
+        if (PHASED) asm volatile("s_barrier" ::: "memory");
+    }
+    return base;
+}
+
+/* The fold of `nvec` whole vectors by a thread group.  Bound by what one compute unit keeps in flight, so by the loads of a
+ * lane that wait together: as many members at a time as there are, up to 16, and of fewer several vectors.
+ *  - Lanes with many vectors (WIDE_MIN) fetch 16 at a time; with fewer, half of that keeps more wavefronts at work in
+ *    the last rounds (us, kernel on an idle GPU: 8 members x 224 KiB bf16, 512 threads, 9.8, in wide rounds 10.5).
+ *  - Loads and stores of a large block's wavefronts hold each other up, as in a copy (nvshmemi_amd_copy_deep_rounds), so
+ *    the wavefronts of 512 threads and more go through them together, if the fold between is an instruction or two per
+ *    word: narrower elements lose by it (8 x 2 MiB bf16, 1024 threads: 53 us, 59 together), and so do messages that the
+ *    L2 holds much of (8 x 400 000 bytes fp32 12.5 / 12.7, 781 168 19.1 / 18.7).
+ * us with eight loads at a time, a member's twice where there are fewer than eight / here: 4 members x 2 MiB fp32 from 256
+ * threads 82 / 50, from 1024 63 / 44, 781 168 bytes from 1024 23.4 / 18.7; 8 x 2 MiB fp32 from 1024 56 / 46, bf16 from 256
+ * 83 / 75; 16 x 2 MiB fp32 from 1024 55 / 45, bf16 from 256 92 / 76; 8 x 224 KiB bf16 from 1024 9.7 / 9.5.
+ * (Stores written through the L2, which the barrier's release would find nothing of, cost up to twice the time - 8 x
+ * 781 168 bytes 19 us, 33 so - and streamed loads a third to a half more.) */
+template <typename T, int OP, int SCOPE>
+NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_reduce_vectors(T *dst, const T *src, size_t pe_stride, int npes, size_t nvec,
+                                                        size_t tid, size_t nthr) {
+    constexpr size_t WIDE_MIN = 16, PHASED_BYTES = (size_t)512 << 10;
+    size_t base = 0;
+#define NVSHMEMI_AMD_ROUNDS(...) base = nvshmemi_amd_reduce_rounds<T, OP, __VA_ARGS__>(dst, src, pe_stride, npes, nvec, tid, nthr, base)
+    if constexpr (SCOPE == NVSHMEMI_THREADGROUP_BLOCK) {
+        const bool phased = sizeof(T) >= 4 && nthr >= NVSHMEMI_AMD_COPY_PHASED_THREADS && nvec * 16 * npes >= PHASED_BYTES;
+        const bool wide = nvec >= WIDE_MIN * nthr;
+        if (npes > 8) {
+            if (phased) NVSHMEMI_AMD_ROUNDS(16, 1, NVSHMEMI_AMD_ROUNDS_PHASED);
+            NVSHMEMI_AMD_ROUNDS(16, 1);
+        } else if (npes > 4) {
+            if (phased) NVSHMEMI_AMD_ROUNDS(8, 1, NVSHMEMI_AMD_ROUNDS_PHASED);
+            else if (wide) NVSHMEMI_AMD_ROUNDS(8, 2, NVSHMEMI_AMD_ROUNDS_FULL);
+            NVSHMEMI_AMD_ROUNDS(8, 1);
+        } else {
+            if (phased) NVSHMEMI_AMD_ROUNDS(4, 2, NVSHMEMI_AMD_ROUNDS_PHASED);
+            else if (wide) NVSHMEMI_AMD_ROUNDS(4, 4, NVSHMEMI_AMD_ROUNDS_FULL);
+            NVSHMEMI_AMD_ROUNDS(4, 2, NVSHMEMI_AMD_ROUNDS_FULL);
+            NVSHMEMI_AMD_ROUNDS(4, 1);
+        }
+    } else {
+        NVSHMEMI_AMD_ROUNDS(8, 1);
+    }
+#undef NVSHMEMI_AMD_ROUNDS
+}
+
 template <typename T, int OP, int SCOPE>
 NVSHMEMI_DEVICE_INLINE int nvshmemi_reduce_threadgroup(nvshmem_team_t team, T *dest, const T *source,
                                                        size_t nreduce) {
     constexpr size_t VEC = 16 / sizeof(T);
-    struct alignas(16) pack_t { T e[VEC]; };
     const nvshmemi_amd_team_view_t tv = nvshmemi_amd_team_view(team);
     if (tv.size <= 0) return 1; /* the calling PE is not a member */
     const int me = tv.my_pe;
@@ -1960,31 +2048,7 @@ NVSHMEMI_DEVICE_INLINE int nvshmemi_reduce_threadgroup(nvshmem_team_t team, T *d
     size_t i = lo + tid;
     if (vectors) {
         const size_t nvec = (hi - lo) / VEC;
-        for (size_t v = tid; v < nvec; v += nthr) {
-            const size_t at = lo + v * VEC;
-            /* the members' vectors are fetched eight at a time, all loads before the first fold: one
-             * after the other they would each pay the way to another PE's memory */
-            pack_t acc;
-            for (int p0 = 0; p0 < npes; p0 += 8) {
-                pack_t x[8];
-#pragma unroll
-                for (int k = 0; k < 8; ++k) {
-                    const int pe = p0 + k < npes ? p0 + k : npes - 1; /* past the end: fetched again, not folded */
-                    x[k] = *reinterpret_cast<const pack_t *>(src0 + (size_t)pe * pe_stride + at);
-                }
-#pragma unroll
-                for (int k = 0; k < 8; ++k) {
-                    const int pe = p0 + k;
-                    if (pe == 0) acc = x[0];
-                    else if (pe < npes) {
-#pragma unroll
-                        for (size_t e = 0; e < VEC; ++e) acc.e[e] = nvshmemi_amd_fold_step<T, OP>(pe, acc.e[e], x[k].e[e]);
-                    }
-                }
-            }
-            for (int pe = 0; pe < npes; ++pe)
-                *reinterpret_cast<pack_t *>(dst0 + (size_t)pe * pe_stride + at) = acc;
-        }
+        nvshmemi_amd_reduce_vectors<T, OP, SCOPE>(dst0 + lo, src0 + lo, pe_stride, npes, nvec, tid, nthr);
         i = lo + nvec * VEC + tid; /* the last PE's range may end inside a vector */
     }
     for (; i < hi; i += nthr) {
