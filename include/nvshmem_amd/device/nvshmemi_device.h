@@ -315,6 +315,11 @@ NVSHMEMI_DEVICE_INLINE size_t nvshmemi_amd_copy_rounds(char *__restrict__ dst,
  * whose pieces a row's last one is short, 8 x 1000 to 6 in rows of 4352 bytes 159 / 126, 8 x 218 to 8 of 11 776 104 / 98.
  * (Only for the wavefront scope.  A block's rounds are wide: few of its copies fit one, and the choice alone costs those
  * that do not 0.1 us in 4 to 9.) */
+/* A buffer descriptor takes 48 bits of an address and reaches global memory only; the local side of a copy may be LDS. */
+NVSHMEMI_DEVICE_INLINE bool nvshmemi_amd_is_global(const void *p) {
+    const auto generic = (const __attribute__((address_space(0))) void *)p; /* (what the builtins take, also in the host's pass) */
+    return !__builtin_amdgcn_is_shared(generic) && !__builtin_amdgcn_is_private(generic);
+}
 NVSHMEMI_DEVICE_INLINE __amdgpu_buffer_rsrc_t nvshmemi_amd_buffer(const char *p, unsigned bytes) {
     const uint64_t a = (uint64_t)(uintptr_t)p;
     const uint64_t base = (uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)a) |
@@ -500,7 +505,7 @@ NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_copy_lanes(char *__restrict__ dst, cons
     size_t head = (size_t)(-(uintptr_t)dst & 15);
     if (head > len) head = len;
     if (SCOPE == NVSHMEMI_THREADGROUP_WARP && nthr == 64 && (((uintptr_t)dst ^ (uintptr_t)src) & 15) == 0 &&
-        len <= NVSHMEMI_AMD_COPY_UNROLL * 1024) {
+        len <= NVSHMEMI_AMD_COPY_UNROLL * 1024 && nvshmemi_amd_is_global(dst) && nvshmemi_amd_is_global(src)) {
         const unsigned nvec = (unsigned)(len - head) / 16, edge = (unsigned)head, tail = (unsigned)(len - head) % 16;
         const unsigned skip = nvec >= NVSHMEMI_AMD_COPY_SKIP_MIN ? (unsigned)(((uintptr_t)dst + edge) >> 4) & 63 : 0;
         if (skip + nvec <= NVSHMEMI_AMD_COPY_UNROLL * 64) {

@@ -37,6 +37,13 @@ enum { NVSHMEM_PERFTEST_SCOPE_THREAD = 0, NVSHMEM_PERFTEST_SCOPE_WARP = 1,
 int nvshmem_perftest_ring_rma(void *dest, const void *src, size_t bytes, int blocks_per_pe,
                               int threads, int scope, int is_get, int iters, void *stream);
 
+/* Copies whose local operand is LDS, by one block of one wavefront per PE: a put or put with signal of `bytes` of `src`, staged
+ * in LDS at `shift`, to dest + shift on PE (p+1)%npes (the signal adds 1 to the word at dest + NVSHMEM_PERFTEST_LDS_TILE), or a
+ * get of the peer's src into LDS at `shift`, whose whole tile (0x5A where the get does not write) then goes to the local dest. */
+enum { NVSHMEM_PERFTEST_LDS_PUT = 0, NVSHMEM_PERFTEST_LDS_GET = 1, NVSHMEM_PERFTEST_LDS_PUT_SIGNAL = 2,
+       NVSHMEM_PERFTEST_LDS_TILE = 8192 };
+int nvshmem_perftest_lds_rma(void *dest, const void *src, size_t bytes, size_t shift, int scope, int form, void *stream);
+
 /* Counter calibration: PE 0's `src` -> PE 0's `dst`, `bytes` (multiple of 16) with a plain
  * one-vector-per-thread kernel that uses nothing of the NVSHMEM API.  Reads and writes exactly
  * `bytes` each. */

@@ -62,6 +62,36 @@ __global__ void ring_rma_kernel(char *dest, const char *src, size_t bytes, size_
     }
 }
 
+// Copies whose local operand is LDS, which is neither in the heap nor in global memory.  A get leaves the whole tile at
+// dest, so that bytes beside the copy show; a put with a signal counts in the word behind dest's kLdsTile bytes.
+constexpr unsigned kLdsTile = NVSHMEM_PERFTEST_LDS_TILE;
+template <int SCOPE>
+__global__ __launch_bounds__(NVSHMEMI_WARP_SIZE) void lds_rma_kernel(char *dest, const char *src, unsigned bytes, unsigned shift,
+                                                                     int form) {
+    __shared__ __align__(16) char tile[kLdsTile];
+    const int me = nvshmem_my_pe();
+    const int peer = (me + 1 == nvshmem_n_pes()) ? 0 : me + 1;
+    const char *mine = (const char *)nvshmem_ptr(src, me);
+    char *out = (char *)nvshmem_ptr(dest, me);
+    for (unsigned i = threadIdx.x; i < kLdsTile; i += NVSHMEMI_WARP_SIZE)
+        tile[i] = form != NVSHMEM_PERFTEST_LDS_GET && i - shift < bytes ? mine[i - shift] : 0x5A;
+    __syncthreads();
+    uint64_t *sig = (uint64_t *)(dest + kLdsTile);
+    const int op = NVSHMEM_SIGNAL_ADD | NVSHMEMX_AMD_SIGNAL_PAYLOAD_ONLY;
+    if (SCOPE == NVSHMEM_PERFTEST_SCOPE_WARP) {
+        if (form == NVSHMEM_PERFTEST_LDS_GET) nvshmemx_getmem_warp(tile + shift, src, bytes, peer);
+        else if (form == NVSHMEM_PERFTEST_LDS_PUT) nvshmemx_putmem_warp(dest + shift, tile + shift, bytes, peer);
+        else nvshmemx_putmem_signal_warp(dest + shift, tile + shift, bytes, sig, 1, op, peer);
+    } else {
+        if (form == NVSHMEM_PERFTEST_LDS_GET) nvshmemx_getmem_block(tile + shift, src, bytes, peer);
+        else if (form == NVSHMEM_PERFTEST_LDS_PUT) nvshmemx_putmem_block(dest + shift, tile + shift, bytes, peer);
+        else nvshmemx_putmem_signal_block(dest + shift, tile + shift, bytes, sig, 1, op, peer);
+    }
+    __syncthreads();
+    if (form == NVSHMEM_PERFTEST_LDS_GET)
+        for (unsigned i = threadIdx.x; i < kLdsTile; i += NVSHMEMI_WARP_SIZE) out[i] = tile[i];
+}
+
 __global__ void p_g_kernel(uint64_t *words, uint64_t *out, uint64_t value_base) {
     const int me = nvshmem_my_pe(), np = nvshmem_n_pes();
     nvshmem_uint64_p(words + me, value_base + (uint64_t)me, (me + 1) % np);
@@ -398,6 +428,18 @@ int nvshmem_perftest_ring_rma(void *dest, const void *src, size_t bytes, int blo
         }
     }
     return rc;
+}
+
+int nvshmem_perftest_lds_rma(void *dest, const void *src, size_t bytes, size_t shift, int scope, int form, void *stream) {
+    if (!perftest::ready() || bytes > kLdsTile || shift > kLdsTile - bytes || form < 0 || form > NVSHMEM_PERFTEST_LDS_PUT_SIGNAL ||
+        (scope != NVSHMEM_PERFTEST_SCOPE_WARP && scope != NVSHMEM_PERFTEST_SCOPE_BLOCK) || ((uintptr_t)dest % 16) ||
+        ((uintptr_t)src % 16) || !perftest::check_range(dest, kLdsTile + sizeof(uint64_t)) || !perftest::check_range(src, bytes))
+        return NVSHMEMX_ERROR_INVALID_VALUE;
+    const auto kernel = scope == NVSHMEM_PERFTEST_SCOPE_WARP ? lds_rma_kernel<NVSHMEM_PERFTEST_SCOPE_WARP>
+                                                             : lds_rma_kernel<NVSHMEM_PERFTEST_SCOPE_BLOCK>;
+    hipLaunchKernelGGL(kernel, dim3(1, 1, (unsigned)nvshmem_n_pes()), dim3(NVSHMEMI_WARP_SIZE), 0, (hipStream_t)stream,
+                       (char *)dest, (const char *)src, (unsigned)bytes, (unsigned)shift, form);
+    return perftest::launch_status("lds_rma");
 }
 
 int nvshmem_perftest_element_bw(int what, int elem_bytes, void *dest, const void *src, size_t nelems,

@@ -208,6 +208,37 @@ def test_short_copies_by_a_wavefront(rt, is_get, shift):
     rt.free(src); rt.free(dst)
 
 
+LDS_PUT, LDS_GET, LDS_PUT_SIGNAL, LDS_TILE = 0, 1, 2, 8192
+
+
+@pytest.mark.parametrize("scope", [N.SCOPE_WARP, N.SCOPE_BLOCK])
+@pytest.mark.parametrize("form", [LDS_PUT, LDS_GET, LDS_PUT_SIGNAL])
+def test_copies_from_and_into_lds(rt, form, scope):
+    """The local operand of a copy may be any memory; the short copies of a wavefront have a form for global memory only."""
+    perf = rt.perftest()
+    src, dst = rt.malloc(LDS_TILE), rt.malloc(LDS_TILE + 8)
+    data = O.fill_all("bytes", NPES, LDS_TILE, 9)
+    rt.upload_all(src, data)
+    for n in (1, 15, 16, 64, 1000, 1024, 2048, 4095, 4096, 4097, 8000):
+        for shift in (0, 3, 16, 192):
+            if n + shift > LDS_TILE:
+                continue
+            rt.fill(dst, 0x5A, LDS_TILE)
+            rt.fill(dst + LDS_TILE, 0, 8)
+            note("copy of LDS, form %d, scope %d: %d bytes at %d" % (form, scope, n, shift))
+            assert perf.nvshmem_perftest_lds_rma(dst, src, n, shift, scope, form, None) == 0
+            rt.sync()
+            got = rt.download_all(dst, (LDS_TILE + 8,), np.uint8)
+            for pe in range(NPES):
+                other = (pe + 1) % NPES if form == LDS_GET else (pe - 1) % NPES
+                want = np.full(LDS_TILE, 0x5A, np.uint8)
+                want[shift:shift + n] = data[other][:n]
+                assert np.array_equal(got[pe][:LDS_TILE], want), (n, shift, pe)
+                assert got[pe][LDS_TILE:].view(np.uint64)[0] == (form == LDS_PUT_SIGNAL)
+    assert perf.nvshmem_perftest_lds_rma(dst, src, LDS_TILE, 1, scope, form, None) != 0
+    rt.free(src); rt.free(dst)
+
+
 @pytest.mark.parametrize("is_get", [0, 1])
 def test_ring_put_get_256MiB_16_blocks(rt, is_get):
     # the largest message of the sweep: 256 MiB per PE, 16 blocks per PE
