@@ -99,6 +99,17 @@ NVSHMEMI_DEVICE_INLINE void nvshmemi_threadgroup_sync() {
     }
 }
 
+/* The same thread number, which the compiler takes for a new one: what a block's copy computes from it - the lane's addresses
+ * in every kind of round - is computed where it is used.  Otherwise all of it is computed in front of the caller's loops and
+ * kept in vector registers through them, also for the kinds of round that no call takes: registers of kernels with copies
+ * by a block, without / with, in-kernel fcollect 98 / 61, alltoall 93 / 63, broadcast 94 / 57, a ring of puts with signals
+ * 73 / 69, a stream of them 75 / 71.  (Copies by a wavefront are short and made in great number: they lose 1 % by it, 64
+ * tokens to 8 experts in rows of 14 KiB 39.6 -> 40.0 us, and few of their kernels any register.) */
+NVSHMEMI_DEVICE_INLINE unsigned nvshmemi_amd_fresh(unsigned tid) {
+    asm volatile("" : "+v"(tid));
+    return tid;
+}
+
 /* Wait until this wavefront's outstanding vector memory operations have completed
  * (s_waitcnt vmcnt(0), gfx9 encoding: lgkmcnt and expcnt left at their maxima). */
 NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_wait_vm() { __builtin_amdgcn_s_waitcnt(0x0F70); }
@@ -387,7 +398,8 @@ NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_copy_one_round(char *dst, const char *s
  *   blocks, whose requests interleave anyway: neither the barriers nor the sweep changes their rate.  (The
  *   number of rounds is the same for every wavefront of the block, so all of them reach every barrier.)
  *
- * A source on another offset than the destination takes the same rounds; where that is no multiple of 4, the
+ * A source on another offset than the destination takes the same rounds in the block scope (in the wavefront scope they
+ * cost the callers 14 to 36 registers and up to three of seven wavefronts per SIMD); where that is no multiple of 4, the
  * fifth word of a lane's vector is the first that the next lane loaded, and one more load per round fetches the
  * words behind each KiB for the last lane.  us for 8 PEs, byte loads in ordinary rounds / here / co-aligned: 16 MiB from one
  * block of 1024 threads 578 / 308 / 281, 256 MiB from 16 1166 / 761 / 711; on a multiple of 4 336 / 286 and 945 / 732.
@@ -401,6 +413,7 @@ enum nvshmemi_amd_source_t { NVSHMEMI_AMD_SRC_ALIGNED = 0, NVSHMEMI_AMD_SRC_UNAL
 template <int SRC, bool NT_LOAD, int STORE, int U, bool BLOCK_WIDE>
 NVSHMEMI_DEVICE_INLINE size_t nvshmemi_amd_copy_deep_rounds(char *__restrict__ dst, const char *__restrict__ src,
                                                            size_t nvec, unsigned tid, size_t nthr) {
+    if (BLOCK_WIDE) tid = nvshmemi_amd_fresh(tid);
     const size_t per_round = (size_t)U * nthr;
     const size_t rounds = nvec / per_round;
     const size_t wave = (size_t)__builtin_amdgcn_readfirstlane(tid >> 6);
@@ -469,11 +482,11 @@ NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_copy_vectors(char *__restrict__ dst,
 #define NVSHMEMI_AMD_SHORT_DEEP(NT) \
     nvshmemi_amd_copy_deep_rounds<NVSHMEMI_AMD_SRC_SHIFTED, NT, STORE, 2, false>(dst, src, nvec, (unsigned)tid, nthr)
     constexpr int SRC = SRC_ALIGNED ? NVSHMEMI_AMD_SRC_ALIGNED : NVSHMEMI_AMD_SRC_UNALIGNED;
-    const bool shifted = !SRC_ALIGNED && ((uintptr_t)src & 3) != 0;
+    const bool shifted = BLOCK_WIDE && !SRC_ALIGNED && ((uintptr_t)src & 3) != 0;
     /* (the second bound follows from the first for whole wavefronts; spelled out, it lets the compiler drop
      * the deep rounds and their registers where the caller's length is known to be short) */
     const size_t least = shifted ? NVSHMEMI_AMD_COPY_SHIFTED_MIN : NVSHMEMI_AMD_COPY_DEEP_MIN;
-    if ((nthr & 63) == 0 && nvec >= least * nthr && nvec >= least * 64) {
+    if ((SRC_ALIGNED || BLOCK_WIDE) && (nthr & 63) == 0 && nvec >= least * nthr && nvec >= least * 64) {
         size_t done;
         if (shifted) done = stream_loads ? NVSHMEMI_AMD_DEEP(NVSHMEMI_AMD_SRC_SHIFTED, true) : NVSHMEMI_AMD_DEEP(NVSHMEMI_AMD_SRC_SHIFTED, false);
         else done = stream_loads ? NVSHMEMI_AMD_DEEP(SRC, true) : NVSHMEMI_AMD_DEEP(SRC, false);
@@ -491,6 +504,7 @@ NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_copy_vectors(char *__restrict__ dst,
 #undef NVSHMEMI_AMD_DEEP
 #undef NVSHMEMI_AMD_SHORT_DEEP
 #endif
+    if (BLOCK_WIDE) tid = nvshmemi_amd_fresh((unsigned)tid);
     if (LOAD == NVSHMEMI_AMD_LOAD_STREAM && !NVSHMEMI_AMD_COPY_NT_ALWAYS && !stream_loads)
         nvshmemi_amd_copy_rounds<SRC_ALIGNED, false, STORE, NVSHMEMI_AMD_COPY_UNROLL, true>(dst, src, nvec, tid, nthr);
     else
@@ -524,6 +538,7 @@ NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_copy_lanes(char *__restrict__ dst, cons
             return;
         }
     }
+    if (SCOPE == NVSHMEMI_THREADGROUP_BLOCK) tid = nvshmemi_amd_fresh((unsigned)tid);
     for (size_t i = tid; i < head; i += nthr) nvshmemi_amd_store_byte<STORE>(dst + i, src[i]);
     dst += head;
     src += head;

@@ -229,9 +229,10 @@ __global__ void moe_dispatch_signal_kernel(const int32_t *dest_pe, const int64_t
 }
 
 // PIECE > 0 (wavefront scope): a work item is PIECE bytes of a row instead of a whole row, so that
-// with one wavefront per block every block moves one short aligned piece and exits.
+// with one wavefront per block every block moves one short aligned piece and exits.  (Whole rows: the compiler takes 68
+// registers, four more than let eight wavefronts run on a SIMD, unless it is held to that; then 59 and no spills.)
 template <bool WARP_SCOPED, int PIECE = 0>
-__global__ void moe_combine_kernel(char *out, const char *recv, const int32_t *dest_pe,
+__global__ __launch_bounds__(1024, WARP_SCOPED && PIECE == 0 ? 8 : 4) void moe_combine_kernel(char *out, const char *recv, const int32_t *dest_pe,
                                    const int64_t *dest_row, int tokens, int topk,
                                    size_t row_bytes, size_t recv_cap_rows) {
     const int me = nvshmem_my_pe();
