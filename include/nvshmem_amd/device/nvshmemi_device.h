@@ -1987,37 +1987,34 @@ NVSHMEMI_DEVICE_INLINE size_t nvshmemi_amd_reduce_rounds(T *dst, const T *src, s
 }
 
 /* The fold of `nvec` whole vectors by a thread group.  Bound by what one compute unit keeps in flight, so by the loads of a
- * lane that wait together: as many members at a time as there are, up to 16, and of fewer several vectors.
- *  - Lanes with many vectors (WIDE_MIN) fetch 16 at a time; with fewer, half of that keeps more wavefronts at work in
- *    the last rounds (us, kernel on an idle GPU: 8 members x 224 KiB bf16, 512 threads, 9.8, in wide rounds 10.5).
+ * lane that wait together: eight, of as many members as there are, and with four or fewer of two vectors each.
+ *  - Eight are what leaves every caller its wavefronts.  Sixteen take 79 to 101 vector registers where these take 51 (bf16
+ *    sum 59, bf16 max 71), so five wavefronts per SIMD instead of eight, for a caller's whole kernel and for the blocks
+ *    that a collective launch accepts; from 256 threads they are faster (4 members x 2 MiB fp32 40 us, 48 here; 8 x 2 MiB
+ *    bf16 57 / 59; 16 x 2 MiB bf16 66 / 81), from 1024 they take as long.
  *  - Loads and stores of a large block's wavefronts hold each other up, as in a copy (nvshmemi_amd_copy_deep_rounds), so
  *    the wavefronts of 512 threads and more go through them together, if the fold between is an instruction or two per
  *    word: narrower elements lose by it (8 x 2 MiB bf16, 1024 threads: 53 us, 59 together), and so do messages that the
  *    L2 holds much of (8 x 400 000 bytes fp32 12.5 / 12.7, 781 168 19.1 / 18.7).
- * us with eight loads at a time, a member's twice where there are fewer than eight / here: 4 members x 2 MiB fp32 from 256
- * threads 82 / 50, from 1024 63 / 44, 781 168 bytes from 1024 23.4 / 18.7; 8 x 2 MiB fp32 from 1024 56 / 46, bf16 from 256
- * 83 / 75; 16 x 2 MiB fp32 from 1024 55 / 45, bf16 from 256 92 / 76; 8 x 224 KiB bf16 from 1024 9.7 / 9.5.
+ * us, kernel on an idle GPU, eight loads without this barrier and a member's twice where there are fewer than eight / here:
+ * 4 members x 2 MiB fp32 from 256 threads 62 / 48, from 1024 51 / 37, bf16 54 / 41, 781 168 bytes fp32 23.0 / 17.5; 8 x 2 MiB fp32
+ * from 256 46 / 40, from 1024 39.5 / 37.5, bf16 from 256 70 / 59; 16 x 2 MiB fp32 from 1024 50 / 43, bf16 from 256 87 / 81;
+ * 8 x 224 KiB bf16 from 1024 9.8 / 9.1.
  * (Stores written through the L2, which the barrier's release would find nothing of, cost up to twice the time - 8 x
  * 781 168 bytes 19 us, 33 so - and streamed loads a third to a half more.) */
 template <typename T, int OP, int SCOPE>
 NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_reduce_vectors(T *dst, const T *src, size_t pe_stride, int npes, size_t nvec,
                                                         size_t tid, size_t nthr) {
-    constexpr size_t WIDE_MIN = 16, PHASED_BYTES = (size_t)512 << 10;
+    constexpr size_t PHASED_BYTES = (size_t)512 << 10;
     size_t base = 0;
 #define NVSHMEMI_AMD_ROUNDS(...) base = nvshmemi_amd_reduce_rounds<T, OP, __VA_ARGS__>(dst, src, pe_stride, npes, nvec, tid, nthr, base)
     if constexpr (SCOPE == NVSHMEMI_THREADGROUP_BLOCK) {
         const bool phased = sizeof(T) >= 4 && nthr >= NVSHMEMI_AMD_COPY_PHASED_THREADS && nvec * 16 * npes >= PHASED_BYTES;
-        const bool wide = nvec >= WIDE_MIN * nthr;
-        if (npes > 8) {
-            if (phased) NVSHMEMI_AMD_ROUNDS(16, 1, NVSHMEMI_AMD_ROUNDS_PHASED);
-            NVSHMEMI_AMD_ROUNDS(16, 1);
-        } else if (npes > 4) {
+        if (npes > 4) {
             if (phased) NVSHMEMI_AMD_ROUNDS(8, 1, NVSHMEMI_AMD_ROUNDS_PHASED);
-            else if (wide) NVSHMEMI_AMD_ROUNDS(8, 2, NVSHMEMI_AMD_ROUNDS_FULL);
             NVSHMEMI_AMD_ROUNDS(8, 1);
         } else {
             if (phased) NVSHMEMI_AMD_ROUNDS(4, 2, NVSHMEMI_AMD_ROUNDS_PHASED);
-            else if (wide) NVSHMEMI_AMD_ROUNDS(4, 4, NVSHMEMI_AMD_ROUNDS_FULL);
             NVSHMEMI_AMD_ROUNDS(4, 2, NVSHMEMI_AMD_ROUNDS_FULL);
             NVSHMEMI_AMD_ROUNDS(4, 1);
         }

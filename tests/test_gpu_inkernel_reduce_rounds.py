@@ -1,6 +1,6 @@
 """GPU parity of the in-kernel allreduce's fold of whole vectors, at the sizes where its rounds change: fewer vectors than
-lanes, remainders of every kind of round, the first size of wide rounds and of rounds that the block's wavefronts go
-through together, and team sizes on either side of the number of members fetched at a time."""
+lanes, remainders of every kind of round, 16 vectors per lane, the first size of rounds that the block's wavefronts go
+through together, and team sizes on either side of the numbers of members fetched at a time."""
 import numpy as np
 import pytest
 
@@ -10,7 +10,7 @@ from gpu_util import bits_equal, note, runtime
 
 pytestmark = pytest.mark.gpu
 
-PHASED_BYTES, WIDE_MIN = 512 << 10, 16
+PHASED_BYTES, MANY = 512 << 10, 16
 
 
 def _data(kind, shape, rng):
@@ -22,7 +22,7 @@ def _data(kind, shape, rng):
 def _slices(npes, threads):
     """Whole vectors that one PE folds."""
     phased = -(-PHASED_BYTES // (16 * npes))
-    return sorted({1, threads - 1, threads + 1, 3 * threads + 5, WIDE_MIN * threads - 1, WIDE_MIN * threads + threads // 2 + 3,
+    return sorted({1, threads - 1, threads + 1, 3 * threads + 5, MANY * threads - 1, MANY * threads + threads // 2 + 3,
                    phased - 1, phased, phased + 2 * threads + 7})
 
 

@@ -57,3 +57,13 @@ def _wavefronts(registers, kernel):
     ("moe_dispatch_kernelILb1E", 5), ("moe_dispatch_rowsignal_kernelILb1E", 4), ("moe_combine_kernelILb1E", 8)])
 def test_callers_of_the_copy_engine(registers, kernel, least):
     assert _wavefronts(registers, kernel) >= least
+
+
+@pytest.mark.parametrize("kernel,least", [("reduce_float_sum_kernel", 8), ("reduce_float_max_kernel", 8),
+                                          ("reduce_int32_sum_kernel", 8), ("reduce_int64_xor_kernel", 8),
+                                          ("reduce_uint64_and_kernel", 8), ("reduce_double_prod_kernel", 8),
+                                          ("reduce_int16_min_kernel", 8), ("reduce_bfloat16_sum_kernel", 8),
+                                          ("reduce_bfloat16_max_kernel", 7)])
+def test_in_kernel_allreduce(registers, kernel, least):
+    for scope in (THREAD, WARP, BLOCK):
+        assert _wavefronts(registers, kernel + "ILi%dE" % scope) >= least
