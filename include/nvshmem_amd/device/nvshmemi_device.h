@@ -425,7 +425,9 @@ NVSHMEMI_DEVICE_INLINE size_t nvshmemi_amd_copy_deep_rounds(char *__restrict__ d
     const unsigned shift = SHIFTED ? (unsigned)((uintptr_t)src & 3) : 0;
     const char *s0 = src - shift + wave_off;
     char *d0 = dst + wave_off;
-    const unsigned behind = (tid & (U - 1)) * (unsigned)step + 1024;  /* lane u fetches the word behind the u-th KiB */
+    /* lane u fetches the word behind the u-th KiB, the lanes from U on some of those again (U may be any depth up to 64) */
+    static_assert(!SHIFTED || U <= 64, "a lane for every KiB of a round");
+    const unsigned behind = (tid & 63) % U * (unsigned)step + 1024;
     /* In the first layout the rounds are walked from a start that differs from block to block, wrapping at
      * the end.  Blocks that each stream a slice of one large message otherwise march in step, at equal
      * offsets in slices that lie a power of two (or the PE distance) apart, and keep meeting on the same
@@ -478,9 +480,11 @@ NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_copy_vectors(char *__restrict__ dst,
                                                      size_t tid, size_t nthr, bool stream_loads) {
 #if NVSHMEMI_AMD_COPY_DEEP_UNROLL > NVSHMEMI_AMD_COPY_UNROLL
 #define NVSHMEMI_AMD_DEEP(SRC, NT) \
-    nvshmemi_amd_copy_deep_rounds<SRC, NT, STORE, NVSHMEMI_AMD_COPY_DEEP_UNROLL, BLOCK_WIDE>(dst, src, nvec, (unsigned)tid, nthr)
+    nvshmemi_amd_copy_deep_rounds<SRC, NT, STORE, (SRC == NVSHMEMI_AMD_SRC_SHIFTED && DEPTH > 64 ? 64 : DEPTH), BLOCK_WIDE>( \
+        dst, src, nvec, (unsigned)tid, nthr)
 #define NVSHMEMI_AMD_SHORT_DEEP(NT) \
     nvshmemi_amd_copy_deep_rounds<NVSHMEMI_AMD_SRC_SHIFTED, NT, STORE, 2, false>(dst, src, nvec, (unsigned)tid, nthr)
+    constexpr int DEPTH = NVSHMEMI_AMD_COPY_DEEP_UNROLL;
     constexpr int SRC = SRC_ALIGNED ? NVSHMEMI_AMD_SRC_ALIGNED : NVSHMEMI_AMD_SRC_UNALIGNED;
     const bool shifted = BLOCK_WIDE && !SRC_ALIGNED && ((uintptr_t)src & 3) != 0;
     /* (the second bound follows from the first for whole wavefronts; spelled out, it lets the compiler drop

@@ -44,6 +44,10 @@ enum { NVSHMEM_PERFTEST_LDS_PUT = 0, NVSHMEM_PERFTEST_LDS_GET = 1, NVSHMEM_PERFT
        NVSHMEM_PERFTEST_LDS_TILE = 8192 };
 int nvshmem_perftest_lds_rma(void *dest, const void *src, size_t bytes, size_t shift, int scope, int form, void *stream);
 
+/* nvshmemx_putmem_block of `bytes` from src to dest on PE (p+1)%npes by one block of `threads` threads per PE, in a translation
+ * unit built with a NVSHMEMI_AMD_COPY_DEEP_UNROLL that is no power of two (12). */
+int nvshmem_perftest_put_depth12(void *dest, const void *src, size_t bytes, int threads, void *stream);
+
 /* Counter calibration: PE 0's `src` -> PE 0's `dst`, `bytes` (multiple of 16) with a plain
  * one-vector-per-thread kernel that uses nothing of the NVSHMEM API.  Reads and writes exactly
  * `bytes` each. */

@@ -138,6 +138,7 @@ def load_perftest():
         "nvshmem_perftest_pe_identity": [vp, i32, vp],
         "nvshmem_perftest_api_matrix": [vp, vp, vp, vp, vp, i32, vp],
         "nvshmem_perftest_lds_rma": [vp, vp, sz, sz, i32, i32, vp],
+        "nvshmem_perftest_put_depth12": [vp, vp, sz, i32, vp],
         "nvshmem_perftest_signal_op": [vp, u64, i32, i32, i32, vp],
         "nvshmem_perftest_signal_wait": [vp, i32, u64, vp, vp],
         "nvshmem_perftest_put_signal_pingpong": [vp, vp, sz, i32, i32, vp],

@@ -184,6 +184,29 @@ def test_long_copies_from_another_offset(rt, scope, threads, lanes):
                 assert np.array_equal(got, want), (soff, doff, size, is_get)
 
 
+@pytest.mark.parametrize("threads", [64, 320, 512, 1024])
+def test_depth_of_the_long_rounds_that_is_no_power_of_two(rt, threads):
+    """Built with twelve vectors per lane and round: the last lane's bytes of every KiB come from the word behind it."""
+    perf = rt.perftest()
+    room = 16 * threads * 40 + 64
+    src, dst = rt.malloc(room), rt.malloc(room)
+    data = O.fill_all("bytes", NPES, room, 12)
+    rt.upload_all(src, data)
+    for soff in (0, 1, 2, 3, 7, 9, 14):
+        for doff, vectors, extra in ((0, 12, 0), (6, 13, 17), (4, 24, 1), (0, 39, 0)):
+            size = 16 * threads * vectors + extra
+            rt.fill(dst, 0x5A, room)
+            note("put at depth 12: %d threads, %d bytes from %d to %d" % (threads, size, soff, doff))
+            assert perf.nvshmem_perftest_put_depth12(dst + doff, src + soff, size, threads, None) == 0
+            rt.sync()
+            got = rt.download_all(dst, (room,), np.uint8)
+            for pe in range(NPES):
+                want = np.full(room, 0x5A, np.uint8)
+                want[doff:doff + size] = data[(pe - 1) % NPES][soff:soff + size]
+                assert np.array_equal(got[pe], want), (soff, doff, size, pe)
+    rt.free(src); rt.free(dst)
+
+
 @pytest.mark.parametrize("is_get", [0, 1])
 @pytest.mark.parametrize("shift", [0, 1, 9, 16 * 5, 16 * 63 + 15])
 def test_short_copies_by_a_wavefront(rt, is_get, shift):
