@@ -14,12 +14,23 @@ MODES = {"fcollect": 0, "alltoall": 1, "broadcast": 2}
 STREAMED = 2  # the store form of all three
 
 
+PERFTEST = os.path.join(ROOT, "nvshmem_amd", "lib", "libnvshmem_amd_perftest.so")
+
+
 @pytest.fixture(scope="module")
 def code_objects(tmp_path_factory):
     """The GPU code of the library, one ELF file per translation unit."""
-    d = tmp_path_factory.mktemp("code")
+    return _units(LIBRARY, tmp_path_factory.mktemp("code"))
+
+
+@pytest.fixture(scope="module")
+def perftest_objects(tmp_path_factory):
+    return _units(PERFTEST, tmp_path_factory.mktemp("perftest"))
+
+
+def _units(library, d):
     fat = str(d / "fatbin")
-    subprocess.run([LLVM + "llvm-objcopy", "--dump-section", ".hip_fatbin=" + fat, LIBRARY, str(d / "rest")], check=True)
+    subprocess.run([LLVM + "llvm-objcopy", "--dump-section", ".hip_fatbin=" + fat, library, str(d / "rest")], check=True)
     data = open(fat, "rb").read()
     out = []
     for m in re.finditer(b"__CLANG_OFFLOAD_BUNDLE__", data):
@@ -103,3 +114,14 @@ def test_kernels_of_small_calls_have_no_implicit_arguments(code_objects, kernel)
                 seen += 1
                 assert "hidden_" not in entry
     assert seen
+
+
+def test_rows_of_a_full_size_dispatch_are_spaced(perftest_objects):
+    """Long rows of much data: a wavefront asks for the row's place when the PE has arrived, behind a branch that others take."""
+    code = _code(perftest_objects, r"moe_dispatch_kernelILb1E")
+    places = _places(code, r"global_load_dwordx2")
+    spaced = [i for i in places if [j for j in _places(code, r"global_load_dword ") if i - 16 < j < i]]
+    assert spaced
+    between = code[[j for j in _places(code, r"global_load_dword ") if j < spaced[0]][-1] + 1:spaced[0]]
+    wait = [i for i, line in enumerate(between) if re.match(r"s_waitcnt.*vmcnt\(0\)", line)]
+    assert wait and any(re.match(r"s_cbranch", line) for line in between[:wait[0]])
