@@ -171,7 +171,8 @@ NVSHMEMI_DEVICE_INLINE void *nvshmemi_ptr(const void *ptr, int pe) {
  * head brings dst to a 16-byte boundary, the body issues four (long copies: eight) independent
  * dwordx4 loads per lane before the first store, and a byte tail finishes.  A src that is not
  * co-aligned is read with unaligned dwordx4 loads, which cost extra cache-line touches on a multiple of
- * 4 bytes and half the rate on any other; long copies read words there and shift them into place.
+ * 4 bytes and half the rate on any other; a block's copies of two vectors per lane and more read words
+ * there and shift them into place.
  * ---------------------------------------------------------------------------------------------- */
 typedef unsigned int nvshmemi_v4u __attribute__((ext_vector_type(4)));
 typedef nvshmemi_v4u __attribute__((aligned(1))) nvshmemi_v4u_unaligned;
@@ -189,12 +190,13 @@ typedef nvshmemi_v4u __attribute__((aligned(1))) nvshmemi_v4u_unaligned;
 #define NVSHMEMI_AMD_COPY_SKIP_MIN 256
 #endif
 /* Long copies - a lane owns at least NVSHMEMI_AMD_COPY_DEEP_MIN vectors - run rounds of
- * NVSHMEMI_AMD_COPY_DEEP_UNROLL vectors per lane first (0 switches them off).  Eight is what fits the
- * registers the rest of the engine needs anyway.  Sixteen takes 30 more vector registers (82 in all: five
- * wavefronts per SIMD instead of eight), which cost kernels of one-wavefront blocks that move 1-2 KiB each
- * 9-13 %, and buys nothing any more: large blocks, whose loads and stores run in separate runs (below),
- * measure the same at 8, 12 and 16.  (A block that streams a long slice alone on its compute unit moves
- * about 39 GB/s of payload whatever the depth: the unit keeps some 15 KiB of requests in flight.) */
+ * NVSHMEMI_AMD_COPY_DEEP_UNROLL vectors per lane first (0 switches them off; any depth moves the same bytes).
+ * They are what a caller's registers go to: a kernel of one put by a block has 46 vector registers at eight, 60
+ * at twelve and 76 at sixteen, a stream of puts with signals 71, 84 and 100, so eight, eight and six or seven,
+ * six and four wavefronts per SIMD.  That cost kernels of one-wavefront blocks that move 1-2 KiB each 9-13 % at
+ * sixteen, and buys nothing: large blocks, whose loads and stores run in separate runs (below), measure the same
+ * at 8, 12 and 16.  (A block that streams a long slice alone on its compute unit moves about 39 GB/s of payload
+ * whatever the depth: the unit keeps some 15 KiB of requests in flight.) */
 #ifndef NVSHMEMI_AMD_COPY_DEEP_UNROLL
 #define NVSHMEMI_AMD_COPY_DEEP_UNROLL 8
 #endif
@@ -320,8 +322,8 @@ NVSHMEMI_DEVICE_INLINE size_t nvshmemi_amd_copy_rounds(char *__restrict__ dst,
  * number of vectors.  The cascade above makes a round trip to memory for every power of two in that number, one behind
  * the other, and another for the vectors in front of the destination's next KiB.  Here lane and vector number are offsets
  * into buffer descriptors of just the bytes that are copied: what lies outside of them the hardware neither loads nor
- * stores, so no instruction needs a predicate, and instruction u covers the u-th KiB of memory that the copy touches
- * (from `skip` vectors in front of dst on), aligned.  A token dispatch with a signal per row, us, cascade / here: 8 x 1505
+ * stores, so no instruction needs a predicate, and instruction u covers the u-th KiB from `skip` vectors in front of
+ * dst on: on the destination's KiB boundaries from NVSHMEMI_AMD_COPY_SKIP_MIN vectors on, from dst itself (skip 0) below.  A token dispatch with a signal per row, us, cascade / here: 8 x 1505
  * tokens to 4 experts each in rows of 7424 bytes 100 / 71, 8 x 64 to 8 of 14 336 bytes 13.5 / 12.4; with the combine, of
  * whose pieces a row's last one is short, 8 x 1000 to 6 in rows of 4352 bytes 159 / 126, 8 x 218 to 8 of 11 776 104 / 98.
  * (Only for the wavefront scope.  A block's rounds are wide: few of its copies fit one, and the choice alone costs those
@@ -401,8 +403,10 @@ NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_copy_one_round(char *dst, const char *s
  * A source on another offset than the destination takes the same rounds in the block scope (in the wavefront scope they
  * cost the callers 14 to 36 registers and up to three of seven wavefronts per SIMD); where that is no multiple of 4, the
  * fifth word of a lane's vector is the first that the next lane loaded, and one more load per round fetches the
- * words behind each KiB for the last lane.  us for 8 PEs, byte loads in ordinary rounds / here / co-aligned: 16 MiB from one
- * block of 1024 threads 578 / 308 / 281, 256 MiB from 16 1166 / 761 / 711; on a multiple of 4 336 / 286 and 945 / 732.
+ * words behind each KiB for the last lane.  us for 8 PEs, unaligned loads in ordinary rounds / here / co-aligned: 16 MiB from one
+ * block of 1024 threads 577 / 302 / 271, 256 MiB from 16 1120 / 741 / 714; on a multiple of 4 334 / 281 and 917 / 737; 16 MiB
+ * from 16 of 64 threads 105 / 74 and, on a multiple of 4, 85 / 58; 64 MiB from 4 of 256 832 / 696 and 712 / 695.  (The one
+ * shape that loses: sources on a multiple of 4 and 16 blocks of 256 threads and more, which fill the GPU: 64 MiB 251 / 260.)
  * (Streamed loads of lines that two lanes share: 3 % faster here, where one wavefront reads on behind the other, and a
  * third slower in ordinary rounds, where it is another block.) */
 #ifndef NVSHMEMI_AMD_COPY_PHASED_THREADS
@@ -498,7 +502,7 @@ NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_copy_vectors(char *__restrict__ dst,
         src += 16 * done;
         nvec -= done;
     }
-    /* (what is left over too: 8 PEs, one block of 1024 threads, 128 KiB 7.0 -> 5.6 us, 200 000 bytes 9.1 -> 6.4) */
+    /* (what is left over too: 8 PEs, one block of 1024 threads, 128 KiB 7.2 -> 5.1 us, 200 000 bytes 9.1 -> 6.4) */
     if (shifted && (nthr & 63) == 0 && nvec >= 2 * nthr) {
         const size_t done = NVSHMEMI_AMD_SHORT_DEEP(false);
         dst += 16 * done;

@@ -366,7 +366,8 @@ namespace perftest {
 // be resident as a whole, and a cooperative launch runs in step with the stream on either side of it: 18 us a call more
 // (8 PEs, dispatch and combine of 64 tokens to 8 experts each in rows of 14 KiB 58.9 us, now 40.4; of 152 tokens to 4 in
 // rows of 2 KiB 38.4, now 19.7).  Blocks that only send end whatever else holds the GPU, and the wait behind them on the
-// stream has its signals when it starts.  A grid that could not have been resident is refused as before.
+// stream has its signals when it starts.  A grid that could not be resident is still refused: the limit belongs to the
+// call, whose other forms wait inside the kernel, and more blocks bring nothing, as they deal the rows out among themselves.
 int launch_senders(const void *fn, int blocks_per_pe, int threads, void **args, hipStream_t stream) {
     int cap = 0;
     const int rc = nvshmemx_collective_launch_query_gridsize(fn, dim3(threads), args, 0, &cap);

@@ -170,9 +170,10 @@ def test_copy_engine_all_mutual_alignments(rt):
             assert np.array_equal(got, want), (soff, doff, is_get)
 
 
-# A source on another offset than the destination is read in words, eight vectors per lane and round, then two: around
-# one round of each (the least that takes them) and 32 vectors per lane (the least for offsets that are a multiple of
-# 4), in blocks below and from 512 threads on, which lay a round out differently, and in wavefronts.
+# A block reads a source on another offset than the destination in words, eight vectors per lane and round, then two:
+# around one round of each (the least that takes them) and 32 vectors per lane (the least for offsets that are a multiple
+# of 4), in blocks below and from 512 threads on, which lay a round out differently; and a wavefront, which takes
+# ordinary rounds whatever the length.
 @pytest.mark.parametrize("scope,threads,lanes", [(N.SCOPE_BLOCK, 64, 64), (N.SCOPE_BLOCK, 192, 192), (N.SCOPE_BLOCK, 512, 512),
                                                  (N.SCOPE_BLOCK, 1024, 1024), (N.SCOPE_WARP, 64, 64)])
 def test_long_copies_from_another_offset(rt, scope, threads, lanes):
