@@ -113,6 +113,9 @@ NVSHMEMI_DEVICE_INLINE unsigned nvshmemi_amd_fresh(unsigned tid) {
 /* Wait until this wavefront's outstanding vector memory operations have completed
  * (s_waitcnt vmcnt(0), gfx9 encoding: lgkmcnt and expcnt left at their maxima). */
 NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_wait_vm() { __builtin_amdgcn_s_waitcnt(0x0F70); }
+/* ... until at most N (below 16) of them are outstanding. */
+template <int N>
+NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_wait_vm_but() { __builtin_amdgcn_s_waitcnt(0x0F70 | N); }
 
 /* ------------------------------------------------------------------------------------------------
  * PE identity and address translation
@@ -207,6 +210,14 @@ typedef nvshmemi_v4u __attribute__((aligned(1))) nvshmemi_v4u_unaligned;
  * twice as long: one round */
 #ifndef NVSHMEMI_AMD_COPY_SHIFTED_MIN
 #define NVSHMEMI_AMD_COPY_SHIFTED_MIN NVSHMEMI_AMD_COPY_DEEP_UNROLL
+#endif
+/* Stores that a wavefront's one-round copy of more than eight vectors per lane keeps outstanding where they are written
+ * through the L2, at most 16 (0: all go out together).  For a unit whose writes outrun the caches: a token dispatch with a
+ * signal per row, 8 x 8192 tokens to 8 experts in rows of 14 KiB 1702 us, with three 1660, with two 1645 in most processes and
+ * 1299, 1308, 1381 in those whose heap lies better in memory; where the caches take the writes they only cost: 8 x 64 tokens
+ * 13.2 us, 13.5 with three. */
+#ifndef NVSHMEMI_AMD_COPY_STORES
+#define NVSHMEMI_AMD_COPY_STORES 0
 #endif
 /* Cache policy of the vector body.  Stores stream (non-temporal): a copy never reads its destination
  * back.  Loads stay cacheable for short and medium copies, because callers often push the same source
@@ -366,9 +377,13 @@ NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_copy_one_round(char *dst, const char *s
 #pragma unroll
     for (int u = 0; u < U; ++u)
         v[u] = __builtin_amdgcn_raw_buffer_load_b128(from, (int)(u ? next + (unsigned)(u - 1) * 1024 : first), 0, LOAD_BITS);
+    constexpr int STORES = STORE == NVSHMEMI_AMD_STORE_WRITE_THROUGH && U > 8 ? NVSHMEMI_AMD_COPY_STORES : 0;
+    static_assert(STORES >= 0 && STORES <= 16, "what a wait can count");
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+    for (int u = 0; u < U; ++u) {
+        if (STORES > 0 && u >= STORES) nvshmemi_amd_wait_vm_but<(STORES > 0 ? STORES - 1 : 0)>();
         __builtin_amdgcn_raw_buffer_store_b128(v[u], to, (int)(u ? next + (unsigned)(u - 1) * 1024 : first), 0, STORE_BITS);
+    }
 }
 
 /* The translation unit's fixed choice for the loads of the ordinary rounds; the deep rounds of a long

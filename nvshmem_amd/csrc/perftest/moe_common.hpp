@@ -27,8 +27,10 @@ __device__ __forceinline__ unsigned wave_in_block_per_lane() { return threadIdx.
 }  // namespace
 
 namespace perftest {
-// moe_rowsignal.hip: the dispatch kernel that signals every row; `args` are its eleven arguments in order.
-int launch_moe_rowsignal(bool warp, int blocks_per_pe, int threads, void **args, hipStream_t stream);
+// moe_rowsignal.hip: the dispatch kernel that signals every row; `args` are its eleven arguments in order, `full` takes the
+// wavefronts' form that moe_rowsignal_full.hip builds.
+int launch_moe_rowsignal(bool warp, bool full, int blocks_per_pe, int threads, void **args, hipStream_t stream);
+const void *moe_rowsignal_full();
 // moe_shuffle.hip: launch of a kernel whose blocks send and never wait, one grid for all PEs.
 int launch_senders(const void *fn, int blocks_per_pe, int threads, void **args, hipStream_t stream);
 }  // namespace perftest

@@ -33,6 +33,11 @@ namespace {
 
 constexpr int kMaxPes = NVSHMEMI_AMD_MAX_PES;
 
+// A dispatch with a signal per row of more than this, all PEs together, takes the kernel of moe_rowsignal_full.hip.  us without
+// and with it: 8 x 64 tokens to 8 experts in rows of 14 KiB (59 MB) 13.2 / 13.5, 512 (0.5 GB) 92.6 / 93.5, 1024 (0.9 GB) 184 / 180,
+// 2048 in rows of 9216 bytes (1.2 GB) 235 / 224.
+constexpr size_t kFullDispatchBytes = (size_t)1 << 30;
+
 // Dispatch.  Rows are dealt round-robin to the thread groups of the PE's blocks.  Each group tallies
 // what it sent to every destination; once all its puts are complete it adds the tallies to the
 // destinations' signal words (one release + npes atomic adds per block instead of one per row).
@@ -414,7 +419,8 @@ int nvshmem_perftest_moe_dispatch_put_signal(void *recv, size_t recv_cap_rows, c
                         &sig_stride};
     void *args[] = {&r, &s, &dest_pe, &dest_row, &sig, &tokens, &topk, &row_bytes, &recv_cap_rows};
     const void *fn = warp ? (const void *)moe_dispatch_kernel<true> : (const void *)moe_dispatch_kernel<false>;
-    const int rc = per_row ? perftest::launch_moe_rowsignal(warp, blocks_per_pe, threads, row_args, (hipStream_t)stream)
+    const bool full = (size_t)tokens * (size_t)topk * row_bytes > kFullDispatchBytes / (size_t)nvshmem_n_pes();
+    const int rc = per_row ? perftest::launch_moe_rowsignal(warp, full, blocks_per_pe, threads, row_args, (hipStream_t)stream)
                            : perftest::launch_senders(fn, blocks_per_pe, threads, args, (hipStream_t)stream);
     if (rc != 0) return rc;
     hipLaunchKernelGGL(moe_receive_kernel, dim3(1, 1, (unsigned)nvshmem_n_pes()), dim3(NVSHMEMI_WARP_SIZE), 0,

@@ -125,3 +125,24 @@ def test_rows_of_a_full_size_dispatch_are_spaced(perftest_objects):
     between = code[[j for j in _places(code, r"global_load_dword ") if j < spaced[0]][-1] + 1:spaced[0]]
     wait = [i for i, line in enumerate(between) if re.match(r"s_waitcnt.*vmcnt\(0\)", line)]
     assert wait and any(re.match(r"s_cbranch", line) for line in between[:wait[0]])
+
+
+@pytest.mark.parametrize("full,outstanding", [(1, 2), (0, 13)])
+def test_stores_of_long_rows_with_a_signal(perftest_objects, full, outstanding):
+    """Fourteen write-through stores: in a full-size dispatch each from the fourth on waits until two are left, otherwise
+    each waits for its own load alone."""
+    code = _code(perftest_objects, r"moe_dispatch_rowsignal_kernelILb1ELb%dE" % full)
+    runs, waits = [], 15
+    for line in code:
+        count = re.match(r"s_waitcnt.*vmcnt\((\d+)\)", line)
+        if count:
+            waits = min(waits, int(count.group(1)))
+        elif line.startswith("buffer_load_dwordx4"):
+            runs.append([])
+        elif line.startswith("buffer_store_dwordx4") and " sc1" in line:
+            runs[-1].append(waits)
+            waits = 15
+    longest = max(runs, key=len)
+    assert len(longest) == 14 and set(longest[3:]) == {outstanding}
+    for run in runs:
+        assert 8 < len(run) or all(w >= len(run) - 1 for w in run[1:])

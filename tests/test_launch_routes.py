@@ -42,6 +42,22 @@ assert dispatch(1 << 20) != 0 and not launches()
 """ % scope)
 
 
+@pytest.mark.parametrize("scope,full", [(1 | 256, True), (2 | 256, False)])
+def test_full_size_dispatch_of_wavefronts_holds_its_stores_back(recorded, scope, full):  # noqa: F811
+    """More than 1 GiB of row copies, all PEs together."""
+    recorded("""
+perf = _lib.load_perftest()
+ok(lib.nvshmemx_amd_init(8, 32 << 20))
+a = lib.nvshmem_malloc(16 << 20)
+def sender(tokens):
+    launches()
+    assert perf.nvshmem_perftest_moe_dispatch_put_signal(a, 8, a, a, a, a, a, 1, tokens, 64, 16384, 64, 256, %d, None) == 0
+    return launches()[0][0]
+assert ("ILb1ELb1E" in sender(129)) == %s
+assert "ILb1ELb1E" not in sender(128)
+""" % (scope, full))
+
+
 def test_copies_that_are_in_flight_all_at_once_are_not_paced(recorded):  # noqa: F811
     """fcollect and broadcast of up to 32 pieces per compute unit (16 from 12 members on) store back to back, larger ones
     one destination at a time (third template argument of the kernel)."""
