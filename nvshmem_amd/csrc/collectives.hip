@@ -287,8 +287,7 @@ __device__ __forceinline__ T fold_next(int p, T acc, T x) {
 // elements in front of and behind them, fewer than 16 bytes on either side.  Stores are aligned that way whatever
 // the buffers are; a source on another offset is read with unaligned vector loads, which cost 3-4 % here (allreduce of
 // 8 x 25 MiB bf16: 73 us with both buffers on the same offset, aligned or not, 76 with different ones; an
-// element per lane and load takes 155 and 148 us.  reducescatter of 8 x 8 x 3 MB bf16 with blocks of an odd number of
-// elements: 42 us, an element per lane 91; with aligned blocks 39).
+// element per lane and load takes 155 and 148 us).
 struct reduce_shape_t {
     uint64_t dst, src;   // byte offsets of the destination and the source in a slice
     uint64_t nvec;       // whole vectors
@@ -511,31 +510,50 @@ __global__ __launch_bounds__(256) void reduce_element_kernel(char *base, uint64_
 // member order in registers and stores one vector into member q's destination.  The work is nearly all
 // loads, and for loads this shape beats the LDS-staged tile of the allreduce: 6.3 against 5.9 TB/s for
 // 8 members with 256 MiB of source each, 5.9 against 3.7 TB/s for 16 members.  NPES > 0 fixes the team
-// size at compile time; NPES == 0 reads it from the team.
+// size at compile time; NPES == 0 reads it from the team (16 members of bf16, sources of 6 | 12 | 24 MB in all, us
+// unknown / known: 5.0 / 3.5, 5.5 / 4.2, 9.5 / 8.1; sixteen loads in flight gain them nothing more).
+//
+// Pieces are cut on the SOURCE's boundaries: n loads and one store per vector, so where blocks of an odd number of
+// elements leave source and destination on different offsets, it is the store that straddles the lines and is
+// unaligned.  Cut on the destination's, every load was, and each piece touched one line more of every member, which
+// streamed loads fetch twice: us cached / streamed loads, 8 members of bf16 on odd elements, 100 MB of sources in all
+// 23.7 / 22.8 then and 23.0 / 19.8 now, 200 MB 43.7 / 42.1 and 42.9 / 36.3 (aligned blocks: 42.0 / 36.0).
+struct scatter_args_t {
+    char *base;
+    uint64_t slice_bytes;
+    team_arg_t team;
+    uint64_t dst, src;     // byte offsets of the destination and of the first source block in a slice
+    uint64_t nelems;       // reduced here, of every block
+    uint64_t block_bytes;  // from one source block to the next
+};
 template <typename T, int OP, int NPES, bool NTL>
-__global__ __launch_bounds__(64) void reducescatter_gather_kernel(char *base, uint64_t slice_bytes,
-                                                                  const nvshmemi_amd_team_view_t *groups,
-                                                                  reduce_shape_t s, uint64_t block_bytes) {
+__global__ __launch_bounds__(64) void reducescatter_gather_kernel(scatter_args_t a) {
     constexpr int VEC = 16 / sizeof(T);
     constexpr int kBatch = 8;  // loads in flight per lane
     union pack_t {
         nvshmemi_v4u v;
         T e[VEC];
     };
-    const nvshmemi_amd_team_view_t g = groups[blockIdx.z];
+    const nvshmemi_amd_team_view_t g = team_of(a.team, blockIdx.z);
     const int npes = NPES ? NPES : g.size;
     if ((int)blockIdx.y >= npes) return;
-    base += (uint64_t)g.start * slice_bytes;
-    const uint64_t pe_stride = (uint64_t)g.stride * slice_bytes;
-    const char *const block = base + s.src + (uint64_t)blockIdx.y * block_bytes;
-    char *const dst = base + (uint64_t)blockIdx.y * pe_stride + s.dst;
-    if (blockIdx.x == 0) reduce_edges<T, OP, true>(dst, block, s, pe_stride, npes, 1);
-    // pieces are cut on absolute 1 KiB boundaries of the source (up to the last 15 bytes, where it lies on another
-    // offset than the destination): `lead` slots of piece 0 lie in front
-    const char *const body = block + s.head * sizeof(T);
+    char *const base = a.base + (uint64_t)g.start * a.slice_bytes;
+    const uint64_t pe_stride = (uint64_t)g.stride * a.slice_bytes;
+    const char *const block = base + a.src + (uint64_t)blockIdx.y * a.block_bytes;
+    char *const dst = base + (uint64_t)blockIdx.y * pe_stride + a.dst;
+    // whole vectors from the source's first 16-byte boundary on, and the elements around them
+    uint64_t head = (-(uintptr_t)block & 15) / sizeof(T);
+    if (head > a.nelems) head = a.nelems;
+    const uint64_t nvec = (a.nelems - head) / VEC;
+    if (blockIdx.x == 0) {
+        const reduce_shape_t s = {0, 0, nvec, (uint32_t)head, (uint32_t)(a.nelems - head - nvec * VEC), 0};
+        reduce_edges<T, OP, true>(dst, block, s, pe_stride, npes, 1);
+    }
+    // pieces are cut on absolute 1 KiB boundaries: `lead` slots of piece 0 lie in front
+    const char *const body = block + head * sizeof(T);
     const uint64_t lead = ((uint64_t)(uintptr_t)body >> 4) & 63;
     const uint64_t v = (uint64_t)blockIdx.x * 64 + threadIdx.x - lead;
-    if (v >= s.nvec) return;  // also the slots in front of the block (wrapped)
+    if (v >= nvec) return;  // also the slots in front of the block (wrapped)
     const char *src = body + 16 * v;
     pack_t acc;
     for (int p0 = 0; p0 < npes; p0 += kBatch) {
@@ -554,7 +572,7 @@ __global__ __launch_bounds__(64) void reducescatter_gather_kernel(char *base, ui
                 }
             }
     }
-    stream_store<NVSHMEM_AMD_STORE_REDUCESCATTER>(dst + s.head * sizeof(T) + 16 * v, acc.v);
+    stream_store<NVSHMEM_AMD_STORE_REDUCESCATTER>(dst + head * sizeof(T) + 16 * v, acc.v);
 }
 
 // Tiles of a segment, wherever it starts.
@@ -774,20 +792,20 @@ void launch_reducescatter(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, u
                            tl.groups, dst_off, src_off, nelems);
         return;
     }
-    const reduce_shape_t shape = reduce_shape<T>(rt, dst_off, src_off, nelems);
-    const uint64_t blocks = (shape.nvec + 63 + 63) / 64;  // room for the lead-in; at least one block for the edges
+    const scatter_args_t args = {rt.base, rt.heap_size, team_arg(tl), dst_off, src_off, nelems, all * sizeof(T)};
+    const uint64_t blocks = (nelems / (16 / sizeof(T)) + 63 + 63) / 64;  // room for the lead-in; at least one block for the edges
     const dim3 grid((unsigned)blocks, (unsigned)tl.max_size, (unsigned)tl.ngroups);
     const bool stream_source = total_members(tl) * tl.max_size * all * sizeof(T) > rt.cacheable_source_bytes;
-#define NVSHMEM_AMD_LAUNCH_GATHER(N, NTL)                                                         \
-    hipLaunchKernelGGL((reducescatter_gather_kernel<T, OP, N, NTL>), grid, dim3(64), 0, stream,   \
-                       rt.base, rt.heap_size, tl.groups, shape, all * sizeof(T))
-    if (eight) {
-        if (stream_source) NVSHMEM_AMD_LAUNCH_GATHER(8, true);
-        else NVSHMEM_AMD_LAUNCH_GATHER(8, false);
-    } else {
-        if (stream_source) NVSHMEM_AMD_LAUNCH_GATHER(0, true);
-        else NVSHMEM_AMD_LAUNCH_GATHER(0, false);
-    }
+#define NVSHMEM_AMD_LAUNCH_GATHER(N)                                                                                   \
+    do {                                                                                                               \
+        if (stream_source)                                                                                             \
+            hipLaunchKernelGGL((reducescatter_gather_kernel<T, OP, N, true>), grid, dim3(64), 0, stream, args);        \
+        else                                                                                                           \
+            hipLaunchKernelGGL((reducescatter_gather_kernel<T, OP, N, false>), grid, dim3(64), 0, stream, args);       \
+    } while (0)
+    if (eight) NVSHMEM_AMD_LAUNCH_GATHER(8);
+    else if (tl.min_size == 16 && tl.max_size == 16) NVSHMEM_AMD_LAUNCH_GATHER(16);
+    else NVSHMEM_AMD_LAUNCH_GATHER(0);
 #undef NVSHMEM_AMD_LAUNCH_GATHER
 }
 

@@ -86,3 +86,28 @@ def test_ragged_reducescatter(npes, form, monkeypatch):
                     got, clean = _guarded(rt.download_all(dst, (n * es + 64,), np.uint8), storage, d, n)
                     assert clean and bits_equal(got, want), (name, n, d, s)
         rt.free(src); rt.free(dst)
+
+
+@pytest.mark.parametrize("npes", [3, 8, 16])
+def test_ragged_reducescatter_with_streamed_loads(npes, monkeypatch):
+    """The kernels of sources that the cache cannot hold, around the ends of a piece that is cut on the source's boundaries:
+    destinations on, before and behind theirs."""
+    monkeypatch.setenv("NVSHMEM_AMD_CACHEABLE_SOURCE_BYTES", "0")
+    monkeypatch.setenv("NVSHMEM_AMD_ELEMENT_REDUCE_BYTES", "0")
+    rng = np.random.default_rng(200 + npes)
+    with runtime(npes, 4 << 20) as rt:
+        src = rt.malloc(1 << 20); dst = rt.malloc(1 << 17)
+        for name, op, kind, storage, _ in KINDS:
+            es = np.dtype(storage).itemsize
+            vec = 16 // es
+            for n in (vec, 63 * vec + 1, 64 * vec, 65 * vec - 1, 128 * vec + 2):
+                data = _values(kind, rng, (npes, npes * n))
+                want = O.reducescatter(kind, op, data)
+                for d, s in ((0, 0), (0, vec - 1), (1, 0), (vec - 1, 1)):
+                    rt.upload_all(src, data, s * es)
+                    rt.fill(dst, 0xCD, n * es + 64)
+                    note("%s %s streamed reducescatter npes=%d n=%d dst+%d src+%d" % (name, op, npes, n, d, s))
+                    rt.reducescatter(name, op, dst + d * es, src + s * es, n)
+                    got, clean = _guarded(rt.download_all(dst, (n * es + 64,), np.uint8), storage, d, n)
+                    assert clean and bits_equal(got, want), (name, n, d, s)
+        rt.free(src); rt.free(dst)
