@@ -38,9 +38,10 @@ namespace {
  * elements (NARROW) and for wider ones (WIDE).  Narrow elements fold twice to four times as many elements
  * per byte, and a block has nothing in flight while it folds: with two members per wavefront the blocks
  * are half as large and twice as many share a compute unit, so more of them are in their load or store
- * phase at any time (bf16 sum and max, 8 x 128 MiB: 6.05-6.15 TB/s with one member per wavefront and two
- * vectors per thread, 6.21-6.25 with two members and one vector; four members 5.74-5.96).  4- and 8-byte
- * elements lose 5 % with two members per wavefront and 11 % with four. */
+ * phase at any time (16 members of bf16, cached sources of 70 MB in all: 22.2 us, 24.3 with one).  Streamed sources of 8
+ * members take one all the same: two loads of a wavefront, back to back, cost more than that gains (8 members of bf16,
+ * 100 | 200 | 400 | 1600 MB: 35.5 | 66.9 | 132.3 | 525 us with two members, 34.5 | 65.2 | 128.4 | 503 with one; four 36.8 | 69.8 |
+ * 137.6 | 548).  4- and 8-byte elements lose 5 % with two members per wavefront and 11 % with four. */
 #ifndef NVSHMEM_AMD_REDUCE_NARROW_MPW
 #define NVSHMEM_AMD_REDUCE_NARROW_MPW 2
 #endif
@@ -52,9 +53,18 @@ namespace {
 #endif
 /* Sources of up to Runtime::cacheable_source_bytes (all PEs together, 256 MiB unless the environment
  * says otherwise) are loaded with the default, cacheable policy: they fit the 256 MiB Infinity
- * Cache, so a source that is sent again (or was just produced) is served from it (measured +30 % on
+ * Cache, so a source that is sent again is served from it (measured +30 % on
  * the 1M-element reduce, +20..45 % on 256 MiB collectives).  Larger sources are streamed with
- * non-temporal loads (+5 % at 2 GiB).  Stores always stream. */
+ * non-temporal loads (+5 % at 2 GiB).  Stores always stream.
+ *
+ * Reductions stream from 3/8 of that on (96 MiB, streamed_reduction).  A streamed load is served from the Infinity
+ * Cache where the line is there - a source that was just produced - but brings none into it, so it does not push out
+ * what others have written there and not yet to memory.  us cached / streamed loads, fp32, sources in all of 100 | 128 | 200
+ * MB: a source just written, allreduce on 8 members 25.7 / 21.1 | 32.8 / 26.6 | 59.3 / 42.9, reducescatter 15.4 / 9.1 | 18.7 /
+ * 12.9 | 27.3 / 22.9; three buffers in turn 34.8 / 33.7 | 45.3 / 42.3 | 67.5 / 64.1 and 22.0 / 19.0 | 27.5 / 23.8 | 41.7 / 35.7;
+ * below, sources that are in use in turn are still there: of 64 MB 19.2 / 23.7 and 11.7 / 12.6.  What loses is a source that is
+ * reduced again as it is, with nothing in between: 29.1 / 33.2 | 36.6 / 41.6 | 56.0 / 63.6 and 17.4 / 16.3 | 21.5 / 21.9 | 33.2 /
+ * 33.3. */
 
 // (any byte alignment: one global_load_dwordx4 either way)
 template <bool NTL>
@@ -62,6 +72,35 @@ __device__ __forceinline__ nvshmemi_v4u stream_load(const char *p) {
     if (NTL && NVSHMEM_AMD_COLL_NT)
         return __builtin_nontemporal_load(reinterpret_cast<const nvshmemi_v4u_unaligned *>(p));
     return *reinterpret_cast<const nvshmemi_v4u_unaligned *>(p);
+}
+// A streamed load of a wavefront whose KiB does not start on a line of its own: the lines at its ends, which the wavefronts
+// on either side read too, possibly on another XCD, are brought into the caches (`shared`: the lanes on them), as
+// streamed ones come from memory twice.  (The empty statements keep the compiler from making one plain load of the two.)
+__device__ __forceinline__ nvshmemi_v4u stream_load_astride(const char *p, bool shared) {
+    nvshmemi_v4u v;
+    if (shared) {
+        asm volatile("");
+        v = stream_load<false>(p);
+        asm volatile("");
+    } else {
+        v = stream_load<true>(p);
+    }
+    return v;
+}
+// Blocks go to the eight XCDs in turn, and so would tiles that share lines of a source (it starts on another offset in
+// a line than the destination, on whose lines tiles are cut): each of these lines would come into two L2s.  The first
+// `dealt` blocks, a multiple of 8 * kDealtTiles, take tiles so that kDealtTiles consecutive ones share an XCD.  us in order /
+// dealt by 2 | 4 | 8 | 16, allreduce, sources on another offset: 8 members fp32 60 MB of sources in all 19.2 / 19.6 | 18.4 | 18.9 |
+// 18.2, 110 MB streamed 39.7 / 38.5 | 37.9 | 38.9 | 40.1, 420 MB 141.7 / 142.8 | 136.6 | 140.3 | 146.9; 2 members 110 MB 37.7 / 36.7 |
+// 36.1 | 36.4 | 36.2, 420 MB 134.7 / 131.7 | 129.0 | 131.6 | 131.8.  Where no line is shared it only widens what is read at a time
+// (8 members, 420 MB aligned: 132.4 in order, by 8 138.4).
+constexpr unsigned kDealtTiles = 4;
+__device__ __forceinline__ unsigned dealt_tile(unsigned block, unsigned dealt) {
+    constexpr unsigned kGroup = 8 * kDealtTiles;
+    return block < dealt ? block / kGroup * kGroup + block % 8 * kDealtTiles + block / 8 % kDealtTiles : block;
+}
+static uint32_t dealt_blocks(uint64_t dst_off, uint64_t src_off, uint64_t blocks) {
+    return (dst_off - src_off) % 128 ? (uint32_t)(blocks / (8 * kDealtTiles) * (8 * kDealtTiles)) : 0;
 }
 // How a kernel's result stores treat the caches.  Both forms write through (nothing here reads its output back): the
 // line leaves the L2 at once instead of queuing behind its eviction of streaming lines, and a write-only stream
@@ -293,6 +332,8 @@ struct reduce_shape_t {
     uint64_t nvec;       // whole vectors
     uint32_t head, tail; // elements in front of and behind them
     uint32_t lead;       // the first vector's place in its aligned 1 KiB of the destination
+    uint32_t dealt;      // blocks whose tiles are dealt to the XCDs (dealt_tile)
+    bool astride;        // streamed loads share the lines at a tile's ends (stream_load_astride)
 };
 template <typename T>
 reduce_shape_t reduce_shape(const Runtime &rt, uint64_t dst_off, uint64_t src_off, uint64_t nelems) {
@@ -301,7 +342,7 @@ reduce_shape_t reduce_shape(const Runtime &rt, uint64_t dst_off, uint64_t src_of
     if (head > nelems) head = nelems;
     const uint64_t nvec = (nelems - head) / (16 / sizeof(T));
     return {dst_off, src_off, nvec, (uint32_t)head, (uint32_t)(nelems - head - nvec * (16 / sizeof(T))),
-            (uint32_t)((at + head * sizeof(T)) >> 4 & 63)};
+            (uint32_t)((at + head * sizeof(T)) >> 4 & 63), 0, false};
 }
 // The elements around the vectors, one per thread of the calling block's first wavefront.
 template <typename T, int OP, bool SCATTER>
@@ -362,17 +403,25 @@ __global__ __launch_bounds__(NPES ? NPES / MPW * 64 : 1024) void reduce_vector_k
     constexpr unsigned tile_words = tile_vecs * VEC / EPW;
 
     // indices in front of the buffer wrap to huge values and are skipped like those behind it
-    const uint64_t v0 = (uint64_t)blockIdx.x * tile_vecs + i - s.lead;
+    const uint64_t v0 = (uint64_t)dealt_tile(blockIdx.x, s.dealt) * tile_vecs + i - s.lead;
+    auto fetch = [&](auto load) {
 #pragma unroll
-    for (int u = 0; u < VPT; ++u) {
-        const uint64_t v = v0 + ((uint64_t)u << lane_shift);
-        if (v < s.nvec) {
+        for (int u = 0; u < VPT; ++u) {
+            const uint64_t v = v0 + ((uint64_t)u << lane_shift);
+            if (v < s.nvec) {
 #pragma unroll
-            for (int m = 0; m < MPW; ++m)
-                if (member(m)) stage[(pe0 + m) * tile_vecs + ((unsigned)u << lane_shift) + i] =
-                    stream_load<NTL>(src + (uint64_t)(pe0 + m) * pe_stride + 16 * v);
+                for (int m = 0; m < MPW; ++m)
+                    if (member(m)) stage[(pe0 + m) * tile_vecs + ((unsigned)u << lane_shift) + i] =
+                        load(src + (uint64_t)(pe0 + m) * pe_stride + 16 * v);
+            }
         }
-    }
+    };
+    // (us streamed alone / here, tiles dealt, source on another offset, 110 MB | 200 MB of sources in all: 8 members fp32 in use in
+    // turn 37.8 / 37.5 | 65.5 / 65.7, just written 32.9 / 21.4 | 61.2 / 48.1, 4 members 36.9 / 35.8 | 64.8 / 62.2 and 29.7 / 25.3 |
+    // 57.5 / 49.5.  Sources beyond the Infinity Cache lose more by what this pushes out of it than they gain: 8 members, 300 MB just
+    // written 104 / 113, 420 MB 128 / 142, in turn 136.4 / 134.3.)
+    if (NTL && s.astride) fetch([i](const char *p) { return stream_load_astride(p, i - 8 >= 48); });
+    else fetch([](const char *p) { return stream_load<NTL>(p); });
     __syncthreads();
     // a thread folds one 4-byte word of the tile at a time - one element of 4 or 8 bytes, or the 2 or 4
     // narrower elements that share the word, each folded on its own in member order - so that a tile of
@@ -449,7 +498,7 @@ __global__ __launch_bounds__(64) void reduce_gather_kernel(char *base, uint64_t 
     const int npes = NPES ? NPES : g.size;
     base += (uint64_t)g.start * slice_bytes;
     const uint64_t pe_stride = (uint64_t)g.stride * slice_bytes;
-    const uint64_t v = (uint64_t)blockIdx.x * 64 + threadIdx.x - s.lead;
+    const uint64_t v = (uint64_t)dealt_tile(blockIdx.x, s.dealt) * 64 + threadIdx.x - s.lead;
     if (v < s.nvec) {
         const char *src = base + s.src + s.head * sizeof(T) + 16 * v;
         pack_t acc;
@@ -546,7 +595,7 @@ __global__ __launch_bounds__(64) void reducescatter_gather_kernel(scatter_args_t
     if (head > a.nelems) head = a.nelems;
     const uint64_t nvec = (a.nelems - head) / VEC;
     if (blockIdx.x == 0) {
-        const reduce_shape_t s = {0, 0, nvec, (uint32_t)head, (uint32_t)(a.nelems - head - nvec * VEC), 0};
+        const reduce_shape_t s = {0, 0, nvec, (uint32_t)head, (uint32_t)(a.nelems - head - nvec * VEC), 0, 0, false};
         reduce_edges<T, OP, true>(dst, block, s, pe_stride, npes, 1);
     }
     // pieces are cut on absolute 1 KiB boundaries: `lead` slots of piece 0 lie in front
@@ -676,7 +725,7 @@ template <typename T, int OP>
 void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t src_off,
                    uint64_t nelems, uint64_t all, hipStream_t stream) {
     const unsigned ngroups = (unsigned)tl.ngroups;
-    const reduce_shape_t shape = reduce_shape<T>(rt, dst_off, src_off, nelems);
+    reduce_shape_t shape = reduce_shape<T>(rt, dst_off, src_off, nelems);
     const uint64_t nvec = shape.nvec;
     // Which kernel.  From Runtime::lds_reduce_bytes of sources in all (64 MiB; a quarter
     // of that for teams of 17 to 32 members, four times for larger ones) the LDS-staged
@@ -696,7 +745,7 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
     // compile-time team size is worth 6 % at 32 members (6.17 against 5.82), nothing at 64.
     const uint64_t total_bytes = total_members(tl) * all * sizeof(T);
     const int fixed_size = tl.min_size == tl.max_size ? tl.max_size : 0;
-    const bool stream_source = total_bytes > rt.cacheable_source_bytes;
+    const bool stream_source = rt.streamed_reduction(total_bytes);
     // (in bytes whatever the element type: fp32, bf16 and int64 cross over at the same 64 MiB on 8 and 16 members)
     const uint64_t lds_from_bytes = tl.max_size > 32   ? rt.lds_reduce_bytes * 4
                                     : tl.max_size > 16 ? rt.lds_reduce_bytes / 4
@@ -704,7 +753,8 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
     // mpw: members per wavefront of the LDS-staged kernel; ct_size: a compile-time team size, if any
     int mpw = 0, ct_size = 0;
     constexpr int kNarrowMpw = sizeof(T) <= 2 ? NVSHMEM_AMD_REDUCE_NARROW_MPW : NVSHMEM_AMD_REDUCE_WIDE_MPW;
-    if (fixed_size == 8 || fixed_size == 16) ct_size = fixed_size, mpw = kNarrowMpw;
+    if (fixed_size == 8) ct_size = 8, mpw = stream_source ? NVSHMEM_AMD_REDUCE_WIDE_MPW : kNarrowMpw;
+    else if (fixed_size == 16) ct_size = 16, mpw = kNarrowMpw;
     else if (fixed_size == 32) ct_size = 32, mpw = 2;
     else if (tl.max_size >= 3 && tl.max_size <= 32) mpw = 2;
     else if (tl.max_size > 32 && tl.max_size <= 64) mpw = 4;
@@ -739,20 +789,22 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
         const int vpt = (ct_size == 8 || ct_size == 16) ? kVptNarrow : NVSHMEM_AMD_REDUCE_VPT;
         const uint64_t tile_vecs = (uint64_t)vpt << lane_shift;
         const uint64_t blocks = (nvec + (1u << lane_shift) + tile_vecs - 1) / tile_vecs;  // room for the lead-in
+        shape.dealt = dealt_blocks(dst_off, src_off, blocks);
+        shape.astride = (dst_off - src_off) % 128 && total_bytes <= rt.cacheable_source_bytes;
         const size_t lds = ((size_t)tl.max_size + 1) * 16 * tile_vecs;
         const dim3 grid((unsigned)blocks, 1, ngroups);
-#define NVSHMEM_AMD_LAUNCH_REDUCE(N, MPW) NVSHMEM_AMD_LAUNCH_REDUCE_V(N, MPW, NVSHMEM_AMD_REDUCE_VPT)
-#define NVSHMEM_AMD_LAUNCH_REDUCE_V(N, MPW, VPT)                                                  \
+#define NVSHMEM_AMD_LAUNCH_REDUCE(N, MPW) NVSHMEM_AMD_LAUNCH_REDUCE_V(N, MPW, MPW, NVSHMEM_AMD_REDUCE_VPT)
+#define NVSHMEM_AMD_LAUNCH_REDUCE_V(N, STREAM_MPW, MPW, VPT)                                      \
     do {                                                                                          \
         if (stream_source)                                                                        \
-            hipLaunchKernelGGL((reduce_vector_kernel<T, OP, N, true, VPT, MPW>), grid, dim3(threads), lds,  \
+            hipLaunchKernelGGL((reduce_vector_kernel<T, OP, N, true, VPT, STREAM_MPW>), grid, dim3(threads), lds,  \
                                stream, rt.base, rt.heap_size, tl.groups, shape);                                                  \
         else                                                                                      \
             hipLaunchKernelGGL((reduce_vector_kernel<T, OP, N, false, VPT, MPW>), grid, dim3(threads), lds, \
                                stream, rt.base, rt.heap_size, tl.groups, shape);                                                  \
     } while (0)
-        if (ct_size == 8) NVSHMEM_AMD_LAUNCH_REDUCE_V(8, kNarrowMpw, kVptNarrow);
-        else if (ct_size == 16) NVSHMEM_AMD_LAUNCH_REDUCE_V(16, kNarrowMpw, kVptNarrow);
+        if (ct_size == 8) NVSHMEM_AMD_LAUNCH_REDUCE_V(8, NVSHMEM_AMD_REDUCE_WIDE_MPW, kNarrowMpw, kVptNarrow);
+        else if (ct_size == 16) NVSHMEM_AMD_LAUNCH_REDUCE_V(16, kNarrowMpw, kNarrowMpw, kVptNarrow);
         else if (ct_size == 32) NVSHMEM_AMD_LAUNCH_REDUCE(32, 2);
         else if (mpw == 2) NVSHMEM_AMD_LAUNCH_REDUCE(0, 2);
         else NVSHMEM_AMD_LAUNCH_REDUCE(0, 4);
@@ -764,6 +816,7 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
     } else {
         // room for the lead-in; at least one block for the edges
         const dim3 grid((unsigned)((nvec + 63 + 63) / 64), 1, ngroups);
+        shape.dealt = dealt_blocks(dst_off, src_off, grid.x);
 #define NVSHMEM_AMD_LAUNCH_GATHER_REDUCE(N)                                                            \
     do {                                                                                               \
         if (stream_source)                                                                             \
@@ -795,7 +848,7 @@ void launch_reducescatter(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, u
     const scatter_args_t args = {rt.base, rt.heap_size, team_arg(tl), dst_off, src_off, nelems, all * sizeof(T)};
     const uint64_t blocks = (nelems / (16 / sizeof(T)) + 63 + 63) / 64;  // room for the lead-in; at least one block for the edges
     const dim3 grid((unsigned)blocks, (unsigned)tl.max_size, (unsigned)tl.ngroups);
-    const bool stream_source = total_members(tl) * tl.max_size * all * sizeof(T) > rt.cacheable_source_bytes;
+    const bool stream_source = rt.streamed_reduction(total_members(tl) * tl.max_size * all * sizeof(T));
 #define NVSHMEM_AMD_LAUNCH_GATHER(N)                                                                                   \
     do {                                                                                                               \
         if (stream_source)                                                                                             \

@@ -62,6 +62,8 @@ struct Runtime {
     // Host-launched collectives treat sources of more bytes than this (all PEs together) as too
     // large to stay in the Infinity Cache: NVSHMEM_AMD_CACHEABLE_SOURCE_BYTES, read at init
     uint64_t cacheable_source_bytes = (uint64_t)256 << 20;
+    // ... and reductions 3/8 of that (96 MiB): collectives.hip, where the loads are
+    bool streamed_reduction(uint64_t source_bytes) const { return source_bytes > cacheable_source_bytes / 8 * 3; }
     // fcollect and broadcast store to one destination after the other in grids of more blocks than this, to all of
     // them back to back in smaller ones: NVSHMEM_AMD_PACED_COPY_BLOCKS, read at init (default: 33 to a compute unit;
     // half of it from 12 destinations on)

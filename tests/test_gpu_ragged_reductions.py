@@ -111,3 +111,31 @@ def test_ragged_reducescatter_with_streamed_loads(npes, monkeypatch):
                     got, clean = _guarded(rt.download_all(dst, (n * es + 64,), np.uint8), storage, d, n)
                     assert clean and bits_equal(got, want), (name, n, d, s)
         rt.free(src); rt.free(dst)
+
+
+@pytest.mark.parametrize("npes,form", [(2, "gather"), (4, "lds"), (8, "lds"), (12, "lds"), (16, "lds"), (16, "two-step"), (33, "two-step")])
+def test_ragged_allreduce_with_streamed_loads(npes, form, monkeypatch):
+    """The kernels of sources that the cache cannot hold: source and destination on one offset in a line, on other ones a
+    whole number of vectors apart and not, around the ends of a tile."""
+    monkeypatch.setenv("NVSHMEM_AMD_CACHEABLE_SOURCE_BYTES", "0")
+    for k, v in FORMS[form].items():
+        monkeypatch.setenv(k, v)
+    rng = np.random.default_rng(300 + npes)
+    with runtime(npes, 2 << 20) as rt:
+        src = rt.malloc(1 << 16); dst = rt.malloc(1 << 16)
+        for name, op, kind, storage, _ in KINDS:
+            es = np.dtype(storage).itemsize
+            vec = 16 // es
+            for n in (vec, 57 * vec, 64 * vec, 64 * vec + 1, 3 * 64 * vec - 1):
+                data = _values(kind, rng, (npes, n))
+                want = O.reduce(kind, op, data)
+                for d, s in ((0, 0), (1, 1), (0, vec), (5 * vec, vec), (0, vec - 1), (vec - 1, 2)):
+                    rt.upload_all(src, data, s * es)
+                    rt.fill(dst, 0xCD, (n + 5 * vec) * es + 64)
+                    note("%s %s %s streamed reduce npes=%d n=%d dst+%d src+%d" % (form, name, op, npes, n, d, s))
+                    rt.reduce(name, op, dst + d * es, src + s * es, n)
+                    got, clean = _guarded(rt.download_all(dst, ((n + 5 * vec) * es + 64,), np.uint8), storage, d, n)
+                    assert clean and all(bits_equal(row, want) for row in got), (name, n, d, s)
+                rt.reduce(name, op, src + s * es, src + s * es, n)   # in place
+                assert bits_equal(rt.download(src, npes - 1, (n,), storage, s * es), want), (name, n, s)
+        rt.free(src); rt.free(dst)

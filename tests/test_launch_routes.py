@@ -152,3 +152,21 @@ for npes, mib, groups in ((15, 40, 0), (16, 16, 0), (16, 24, 8), (24, 16, 8), (6
     assert not groups or (grid[0] % 16384 == 0 and grid[0] // groups >= mib * 1024 > grid[0] // groups - 16384 // groups - 2)
     lib.nvshmem_finalize()
 """)
+
+
+def test_large_sources_of_reductions_are_streamed(recorded):  # noqa: F811
+    """More than 96 MiB of sources, all PEs together, take the kernels with streamed loads; an eighth of them being 1- or
+    2-byte elements then has a wavefront of its own."""
+    recorded("""
+ok(lib.nvshmemx_amd_init(8, 64 << 20))
+a, b = lib.nvshmem_malloc(16 << 20), lib.nvshmem_malloc(16 << 20)
+for name, es in (("float", 4), ("bfloat16", 2)):
+    for over in (0, 1):
+        n = (12 << 20) // es + over
+        launches()
+        ok(_lib.typed_coll(lib, "nvshmemx_%s_sum_reduce_on_stream" % name, True)(0, b, a, n, None))
+        ok(_lib.typed_coll(lib, "nvshmemx_%s_sum_reducescatter_on_stream" % name, True)(0, b, a, (12 << 20) // 8 // es + over, None))
+        (reduce, _, _, block, _), (scatter, _, _, _, _) = launches()
+        assert ("Li8ELb%dELi" % over) in reduce and ("Li8ELb%dEEE" % over) in scatter, (reduce, scatter)
+        assert block[0] == (512 if over or es == 4 else 256), block
+""")
