@@ -192,6 +192,7 @@ struct segment_args_t {
     uint32_t root;
     uint32_t members;                  // of the handle's largest team (gridDim would cost the host 0.6 us a launch: host_rma.hip)
     uint16_t part_shift, chunk_shift;  // chunked walk: 2^part_shift groups of destinations, chunks of 2^chunk_shift tiles
+    bool astride;                      // streamed alltoall: lanes at the ends of a piece load cacheable (segment_collective)
 };
 
 template <int MODE, bool NTL, bool PACED, int STORE, bool CHUNKED = false>
@@ -249,7 +250,11 @@ __global__ __launch_bounds__(64) void segment_copy_kernel(segment_args_t a) {
     const unsigned first = edges ? lead : 0, end = left < 64 ? (unsigned)left : 64;
     const bool body = lane - first < end - first;
     nvshmemi_v4u v = {};
-    if (body) v = stream_load<NTL>(src + head + 16 * v0 + 16 * lane);
+    if (body) {
+        const char *const from = src + head + 16 * v0 + 16 * lane;
+        if (MODE == kModeAlltoall && NTL && a.astride) v = stream_load_astride(from, lane - 8 >= 48);
+        else v = stream_load<NTL>(from);
+    }
     // at most 15 + 15 bytes, lane k the k-th of them, every second destination on either half of the lanes; they are
     // loaded beside the vectors
     const unsigned k = lane & 31;
@@ -683,7 +688,7 @@ static int launch_broadcast(Runtime &rt, const TeamLaunch &tl, uint64_t doff, ui
     }
     const dim3 grid((unsigned)tiles, 1, (unsigned)tl.ngroups);
     const segment_args_t args = {rt.base, rt.heap_size, team_arg(tl), doff, soff, bytes, (uint32_t)root,
-                                 (uint32_t)tl.max_size, 0, 0};
+                                 (uint32_t)tl.max_size, 0, 0, false};
     const bool paced = paced_copy(rt, tiles * (uint64_t)tl.ngroups, tl.max_size);
     const size_t lds = paced ? paced_lds_bytes(rt, sources, tl.max_size) : 0;
     // a source that cannot stay in the Infinity Cache is streamed
@@ -1049,8 +1054,18 @@ static int segment_collective(int mode, const char *what, nvshmem_team_t team, v
         set_error("%s: message too large", what);
         return NVSHMEMX_ERROR_INVALID_VALUE;
     }
-    const bool stream_source = sources > rt.cacheable_source_bytes;
-    const segment_args_t args = {rt.base, rt.heap_size, team_arg(tl), doff, soff, seg_bytes, 0, (uint32_t)n, 0, 0};
+    // Alltoalls that the Infinity Cache could just hold stream three quarters of a source and keep a quarter, the lines at
+    // the ends of its pieces, which on another offset than the destination's two wavefronts read.  Beside other buffers in turn
+    // a source kept whole is gone when it comes again, a quarter is not; and one that was just written loses less to what the
+    // loads bring in.  us kept / a quarter kept, fp32, sources of 110 | 160 | 240 MB in all: 8 members in turn 35.0 / 32.6 | 51.4 /
+    // 45.9 | 75.8 / 66.9, just written 28.3 / 21.9 | 41.5 / 33.0 | 59.8 / 56.5, on another offset 34.7 / 34.7 | 51.8 / 49.2 | 76.4 /
+    // 71.3; 16 members in turn 39.9 / 37.8 | 53.8 / 48.8 | 77.9 / 69.1, 4 34.7 / 32.3 | 51.2 / 45.7 | 76.4 / 67.4.  Not a buffer of just the
+    // cache's size: sent again and again as it is, it stays (16 members, 256 MiB: 72.4 / 78.5; in turn 85.4 / 78.1).  None
+    // kept: 200 MB 61.5, a quarter 56.6.  Below 112 MiB three buffers in turn are still there in part: 105 MB 31.9 / 31.2, on
+    // another offset 33.2 / 33.4, 16 members 37.2 / 38.8.  (Dealing the tiles to the XCDs, as in the reductions, loses 2 % here.)
+    const bool quarter = mode == kModeAlltoall && sources > rt.cacheable_source_bytes / 16 * 7 && sources < rt.cacheable_source_bytes;
+    const bool stream_source = quarter || sources > rt.cacheable_source_bytes;
+    const segment_args_t args = {rt.base, rt.heap_size, team_arg(tl), doff, soff, seg_bytes, 0, (uint32_t)n, 0, 0, quarter};
 #define NVSHMEM_AMD_LAUNCH_SEGCOPY(MODE, NTL, PACED, STORE) \
     hipLaunchKernelGGL((segment_copy_kernel<MODE, NTL, PACED, STORE>), grid, dim3(64), lds, stream, args)
     if (mode == kModeFcollect) {

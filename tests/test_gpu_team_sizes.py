@@ -334,3 +334,22 @@ def _allreduce_battery(npes, rng, tag):
             assert bits_equal(rt.download(dst, members[-1], (n,), np.float32), want), c
         rt.team_destroy(xt); rt.team_destroy(yt)
         rt.free(src); rt.free(dst)
+
+
+@pytest.mark.parametrize("npes,seg", [(2, 16384 + 7), (3, 5461), (4, 2 * 1024 + 1), (4, 4000), (5, 1300)])
+def test_alltoall_of_sources_that_nearly_fill_the_cache(npes, seg, monkeypatch):
+    """Streamed with a quarter of the loads cacheable: pieces whole, cut and off the lines of their source."""
+    monkeypatch.setenv("NVSHMEM_AMD_CACHEABLE_SOURCE_BYTES", str(npes * npes * seg * 3 // 2))
+    rng = np.random.default_rng(seg)
+    with runtime(npes, 4 << 20) as rt:
+        src = rt.malloc(1 << 17); dst = rt.malloc(1 << 17)
+        data = rng.integers(0, 256, (npes, npes * seg), dtype=np.uint8)
+        for doff, soff in ((0, 0), (0, 5), (64, 16), (3, 128), (1, 1)):
+            rt.upload_all(src, data, soff)
+            rt.fill(dst, 0xCD, npes * seg + 256)
+            note("streamed alltoallmem npes=%d seg=%d soff=%d doff=%d" % (npes, seg, soff, doff))
+            rt.alltoallmem(dst + doff, src + soff, seg)
+            got = rt.download_all(dst, (npes * seg + 256,), np.uint8)
+            assert np.array_equal(got[:, doff:doff + npes * seg], O.alltoall(data)), (seg, soff, doff)
+            assert (got[:, :doff] == 0xCD).all() and (got[:, doff + npes * seg:] == 0xCD).all()
+        rt.free(src); rt.free(dst)
