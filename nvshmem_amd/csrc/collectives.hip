@@ -487,8 +487,7 @@ __global__ __launch_bounds__(NPES ? NPES / MPW * 64 : 1024) void reduce_vector_k
 // wavefront, lane i loads vector i of a 1 KiB piece from every member, eight loads in flight at a time,
 // folds in member order and stores the result to every member.
 // NPES > 0 fixes the team size at compile time (loads, fold and stores fully unrolled).
-// ROOT_ONLY: the result goes to member 0's destination only (the first half of the two-step allreduce of large teams).
-template <typename T, int OP, int NPES, bool NTL, bool ROOT_ONLY = false>
+template <typename T, int OP, int NPES, bool NTL>
 __global__ __launch_bounds__(64) void reduce_gather_kernel(char *base, uint64_t slice_bytes,
                                                            const nvshmemi_amd_team_view_t *groups,
                                                            reduce_shape_t s) {
@@ -526,15 +525,11 @@ __global__ __launch_bounds__(64) void reduce_gather_kernel(char *base, uint64_t 
                 }
         }
         char *dst = base + s.dst + s.head * sizeof(T) + 16 * v;
-        if (ROOT_ONLY) {
-            stream_store<NVSHMEM_AMD_STORE_REDUCESCATTER>(dst, acc.v);
-        } else {
 #pragma unroll kStores
-            for (int p = 0; p < npes; ++p) stream_store<NVSHMEM_AMD_STORE_REDUCE>(dst + (uint64_t)p * pe_stride, acc.v);
-        }
+        for (int p = 0; p < npes; ++p) stream_store<NVSHMEM_AMD_STORE_REDUCE>(dst + (uint64_t)p * pe_stride, acc.v);
     }
     if (blockIdx.x == 0)
-        reduce_edges<T, OP, false>(base + s.dst, base + s.src, s, pe_stride, npes, ROOT_ONLY ? 1 : npes);
+        reduce_edges<T, OP, false>(base + s.dst, base + s.src, s, pe_stride, npes, npes);
 }
 
 // One element per lane and load, for small messages whose buffers are no whole vectors (element_at_a_time): what
@@ -580,7 +575,9 @@ struct scatter_args_t {
     uint64_t nelems;       // reduced here, of every block
     uint64_t block_bytes;  // from one source block to the next
 };
-template <typename T, int OP, int NPES, bool NTL>
+// SCATTER false: the first half of the two-step allreduce of large teams, one block into member 0's destination, in the
+// allreduce's operand order.
+template <typename T, int OP, int NPES, bool NTL, bool SCATTER>
 __global__ __launch_bounds__(64) void reducescatter_gather_kernel(scatter_args_t a) {
     constexpr int VEC = 16 / sizeof(T);
     constexpr int kBatch = 8;  // loads in flight per lane
@@ -601,7 +598,7 @@ __global__ __launch_bounds__(64) void reducescatter_gather_kernel(scatter_args_t
     const uint64_t nvec = (a.nelems - head) / VEC;
     if (blockIdx.x == 0) {
         const reduce_shape_t s = {0, 0, nvec, (uint32_t)head, (uint32_t)(a.nelems - head - nvec * VEC), 0, 0, false};
-        reduce_edges<T, OP, true>(dst, block, s, pe_stride, npes, 1);
+        reduce_edges<T, OP, SCATTER>(dst, block, s, pe_stride, npes, 1);
     }
     // pieces are cut on absolute 1 KiB boundaries: `lead` slots of piece 0 lie in front
     const char *const body = block + head * sizeof(T);
@@ -622,7 +619,7 @@ __global__ __launch_bounds__(64) void reducescatter_gather_kernel(scatter_args_t
                     acc = x[0];
                 } else {
 #pragma unroll
-                    for (int j = 0; j < VEC; ++j) acc.e[j] = nvshmemi_amd_reduce_op<T, OP>(acc.e[j], x[k].e[j]);
+                    for (int j = 0; j < VEC; ++j) acc.e[j] = fold_next<T, OP, SCATTER>(p0 + k, acc.e[j], x[k].e[j]);
                 }
             }
     }
@@ -747,7 +744,8 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
     // for the compile-time sizes 8 and 16, two members up to 32 and four beyond: one load and one store
     // per lane measured best where the block stays within 16 wavefronts, and wavefronts of fewer than
     // 64 lanes per member (512- or 256-byte accesses) lost 7-22 % against the gather kernel.  The
-    // compile-time team size is worth 6 % at 32 members (6.17 against 5.82), nothing at 64.
+    // compile-time team size is worth 6 % at 32 members (6.17 against 5.82), nothing at 64, and with a member per wavefront 3 to
+    // 8 % at 4 (70 | 200 | 800 MB of sources in all, fp32 22.4 / 20.9 | 63.6 / 61.8 | 248 / 240 us, bf16 alike).
     const uint64_t total_bytes = total_members(tl) * all * sizeof(T);
     const int fixed_size = tl.min_size == tl.max_size ? tl.max_size : 0;
     const bool stream_source = rt.streamed_reduction(total_bytes);
@@ -760,6 +758,7 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
     constexpr int kNarrowMpw = sizeof(T) <= 2 ? NVSHMEM_AMD_REDUCE_NARROW_MPW : NVSHMEM_AMD_REDUCE_WIDE_MPW;
     if (fixed_size == 8) ct_size = 8, mpw = stream_source ? NVSHMEM_AMD_REDUCE_WIDE_MPW : kNarrowMpw;
     else if (fixed_size == 16) ct_size = 16, mpw = kNarrowMpw;
+    else if (fixed_size == 4) ct_size = 4, mpw = 1;
     else if (fixed_size == 32) ct_size = 32, mpw = 2;
     else if (tl.max_size >= 3 && tl.max_size <= 32) mpw = 2;
     else if (tl.max_size > 32 && tl.max_size <= 64) mpw = 4;
@@ -774,13 +773,12 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
     if (rt.two_step_reduce_members && tl.min_size >= (int)rt.two_step_reduce_members &&
         (total_bytes >= rt.two_step_reduce_bytes || tl.min_size >= 3 * (int)rt.two_step_reduce_members) &&
         total_bytes >= lds_from_bytes) {
-        const dim3 grid((unsigned)((nvec + 63 + 63) / 64), 1, ngroups);
+        const scatter_args_t args = {rt.base, rt.heap_size, team_arg(tl), dst_off, src_off, nelems, 0};
+        const dim3 grid((unsigned)((nelems / (16 / sizeof(T)) + 63 + 63) / 64), 1, ngroups);
         if (stream_source)
-            hipLaunchKernelGGL((reduce_gather_kernel<T, OP, 0, true, true>), grid, dim3(64), 0, stream, rt.base,
-                               rt.heap_size, tl.groups, shape);
+            hipLaunchKernelGGL((reducescatter_gather_kernel<T, OP, 0, true, false>), grid, dim3(64), 0, stream, args);
         else
-            hipLaunchKernelGGL((reduce_gather_kernel<T, OP, 0, false, true>), grid, dim3(64), 0, stream, rt.base,
-                               rt.heap_size, tl.groups, shape);
+            hipLaunchKernelGGL((reducescatter_gather_kernel<T, OP, 0, false, false>), grid, dim3(64), 0, stream, args);
         (void)launch_broadcast(rt, tl, dst_off, dst_off, nelems * sizeof(T), 0, stream);
         return;
     }
@@ -810,6 +808,7 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
     } while (0)
         if (ct_size == 8) NVSHMEM_AMD_LAUNCH_REDUCE_V(8, NVSHMEM_AMD_REDUCE_WIDE_MPW, kNarrowMpw, kVptNarrow);
         else if (ct_size == 16) NVSHMEM_AMD_LAUNCH_REDUCE_V(16, kNarrowMpw, kNarrowMpw, kVptNarrow);
+        else if (ct_size == 4) NVSHMEM_AMD_LAUNCH_REDUCE(4, 1);
         else if (ct_size == 32) NVSHMEM_AMD_LAUNCH_REDUCE(32, 2);
         else if (mpw == 2) NVSHMEM_AMD_LAUNCH_REDUCE(0, 2);
         else NVSHMEM_AMD_LAUNCH_REDUCE(0, 4);
@@ -857,9 +856,9 @@ void launch_reducescatter(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, u
 #define NVSHMEM_AMD_LAUNCH_GATHER(N)                                                                                   \
     do {                                                                                                               \
         if (stream_source)                                                                                             \
-            hipLaunchKernelGGL((reducescatter_gather_kernel<T, OP, N, true>), grid, dim3(64), 0, stream, args);        \
+            hipLaunchKernelGGL((reducescatter_gather_kernel<T, OP, N, true, true>), grid, dim3(64), 0, stream, args);        \
         else                                                                                                           \
-            hipLaunchKernelGGL((reducescatter_gather_kernel<T, OP, N, false>), grid, dim3(64), 0, stream, args);       \
+            hipLaunchKernelGGL((reducescatter_gather_kernel<T, OP, N, false, true>), grid, dim3(64), 0, stream, args);       \
     } while (0)
     if (eight) NVSHMEM_AMD_LAUNCH_GATHER(8);
     else if (tl.min_size == 16 && tl.max_size == 16) NVSHMEM_AMD_LAUNCH_GATHER(16);
