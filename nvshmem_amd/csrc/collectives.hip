@@ -575,10 +575,9 @@ struct scatter_args_t {
     uint64_t nelems;       // reduced here, of every block
     uint64_t block_bytes;  // from one source block to the next
 };
-// SCATTER false: the first half of the two-step allreduce of large teams, one block into member 0's destination, in the
-// allreduce's operand order.
+// SCATTER false: the allreduce's operand order.
 template <typename T, int OP, int NPES, bool NTL, bool SCATTER>
-__global__ __launch_bounds__(64) void reducescatter_gather_kernel(scatter_args_t a) {
+__device__ __forceinline__ void fold_source_pieces(const scatter_args_t &a) {
     constexpr int VEC = 16 / sizeof(T);
     constexpr int kBatch = 8;  // loads in flight per lane
     union pack_t {
@@ -624,6 +623,16 @@ __global__ __launch_bounds__(64) void reducescatter_gather_kernel(scatter_args_t
             }
     }
     stream_store<NVSHMEM_AMD_STORE_REDUCESCATTER>(dst + head * sizeof(T) + 16 * v, acc.v);
+}
+
+template <typename T, int OP, int NPES, bool NTL>
+__global__ __launch_bounds__(64) void reducescatter_gather_kernel(scatter_args_t a) {
+    fold_source_pieces<T, OP, NPES, NTL, true>(a);
+}
+// The first half of the two-step allreduce of large teams: one block, into member 0's destination.
+template <typename T, int OP, bool NTL>
+__global__ __launch_bounds__(64) void reduce_root_kernel(scatter_args_t a) {
+    fold_source_pieces<T, OP, 0, NTL, false>(a);
 }
 
 // Tiles of a segment, wherever it starts.
@@ -768,17 +777,19 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
     // serialises n steps between two barriers.  fp32 sum of random data, TB/s, fused / two-step at about 512 MiB and 2 to
     // 4 GiB of sources in all: 12 members 6.02 / 6.03 and 6.23 / 6.20, 16: 6.12 / 6.25 and 6.12 / 6.32, 24: 5.72 / 6.24 and 5.79 /
     // 6.39, 32: 6.28 / 6.19 and 6.35 / 6.42, 48: 5.87 / 6.38 and 5.94 / 6.47, 64: 5.86 / 5.81 and 6.01 / 6.47; at 256 MiB 16
-    // members 6.98 / 6.10, 32 6.93 / 6.27, 64 6.37 / 6.31.  So: from Runtime::two_step_reduce_members (16) members on when the
-    // sources hold two_step_reduce_bytes (512 MiB) or more, and from three times that many members whatever the size.
-    if (rt.two_step_reduce_members && tl.min_size >= (int)rt.two_step_reduce_members &&
-        (total_bytes >= rt.two_step_reduce_bytes || tl.min_size >= 3 * (int)rt.two_step_reduce_members) &&
-        total_bytes >= lds_from_bytes) {
+    // members 6.98 / 6.10, 32 6.93 / 6.27, 64 6.37 / 6.31 for a source that is reduced again as it is.  Other buffers in turn,
+    // us fused / two-step, 104 | 160 | 240 MB of sources in all: 16 members fp32 51.6 / 37.1 | 75.8 / 55.4 | 95.3 / 78.7, bf16 50.0 / 38.3 |
+    // 68.3 / 56.7 | 96.5 / 79.8, 24 fp32 40.4 / 40.6 | 59.6 / 53.7 | 88.6 / 80.6, 32 48.9 / 40.0 | 69.6 / 61.4 | 99.7 / 79.9, against the gather
+    // kernel 40 39.5 / 38.4 | 63.0 / 58.8 | 93.1 / 81.4, 64 42.4 / 41.9 | 64.7 / 59.2 | 98.3 / 88.9; sources that are still in the cache lose
+    // (16 members, 80 MB: 26.8 / 31.5).  So: from Runtime::two_step_reduce_members (16) members on when the sources hold
+    // two_step_reduce_bytes (96 MiB, from where reductions stream) or more.
+    if (rt.two_step_reduce_members && tl.min_size >= (int)rt.two_step_reduce_members && total_bytes >= rt.two_step_reduce_bytes) {
         const scatter_args_t args = {rt.base, rt.heap_size, team_arg(tl), dst_off, src_off, nelems, 0};
         const dim3 grid((unsigned)((nelems / (16 / sizeof(T)) + 63 + 63) / 64), 1, ngroups);
         if (stream_source)
-            hipLaunchKernelGGL((reducescatter_gather_kernel<T, OP, 0, true, false>), grid, dim3(64), 0, stream, args);
+            hipLaunchKernelGGL((reduce_root_kernel<T, OP, true>), grid, dim3(64), 0, stream, args);
         else
-            hipLaunchKernelGGL((reducescatter_gather_kernel<T, OP, 0, false, false>), grid, dim3(64), 0, stream, args);
+            hipLaunchKernelGGL((reduce_root_kernel<T, OP, false>), grid, dim3(64), 0, stream, args);
         (void)launch_broadcast(rt, tl, dst_off, dst_off, nelems * sizeof(T), 0, stream);
         return;
     }
@@ -856,9 +867,9 @@ void launch_reducescatter(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, u
 #define NVSHMEM_AMD_LAUNCH_GATHER(N)                                                                                   \
     do {                                                                                                               \
         if (stream_source)                                                                                             \
-            hipLaunchKernelGGL((reducescatter_gather_kernel<T, OP, N, true, true>), grid, dim3(64), 0, stream, args);        \
+            hipLaunchKernelGGL((reducescatter_gather_kernel<T, OP, N, true>), grid, dim3(64), 0, stream, args);        \
         else                                                                                                           \
-            hipLaunchKernelGGL((reducescatter_gather_kernel<T, OP, N, false, true>), grid, dim3(64), 0, stream, args);       \
+            hipLaunchKernelGGL((reducescatter_gather_kernel<T, OP, N, false>), grid, dim3(64), 0, stream, args);       \
     } while (0)
     if (eight) NVSHMEM_AMD_LAUNCH_GATHER(8);
     else if (tl.min_size == 16 && tl.max_size == 16) NVSHMEM_AMD_LAUNCH_GATHER(16);

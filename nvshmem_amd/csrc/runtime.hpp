@@ -75,12 +75,11 @@ struct Runtime {
     // Reductions of ragged buffers with up to this many bytes of results fold one element per lane where that is the
     // faster way: NVSHMEM_AMD_ELEMENT_REDUCE_BYTES, read at init (0 = never)
     uint64_t element_reduce_bytes = (uint64_t)512 << 10;
-    // An allreduce beyond the cache takes two steps - fold into member 0, broadcast - instead of the fused
+    // An allreduce of streamed sources takes two steps - fold into member 0, broadcast - instead of the fused
     // kernel from this team size on (NVSHMEM_AMD_TWO_STEP_REDUCE_MEMBERS, read at init; 0 = never) when the
-    // sources of all members together hold at least two_step_reduce_bytes (NVSHMEM_AMD_TWO_STEP_REDUCE_BYTES), and
-    // from three times the team size at any size
+    // sources of all members together hold at least two_step_reduce_bytes (NVSHMEM_AMD_TWO_STEP_REDUCE_BYTES)
     unsigned two_step_reduce_members = 16;
-    uint64_t two_step_reduce_bytes = (uint64_t)512 << 20;
+    uint64_t two_step_reduce_bytes = (uint64_t)96 << 20;
     uint64_t timeouts_seen = 0;  // bounded waits that gave up, as far as the host has reported them
     // pinned host word the GPU writes a timeout's number to (null if it could not be allocated), and the value
     // the host found there at its last report: equal values mean nothing gave up since

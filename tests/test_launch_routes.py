@@ -183,3 +183,18 @@ for mib, streamed in ((28, 0), (29, 1), (63, 1), (64, 0), (65, 1)):
     (kernel, _, _, _, _), = launches()
     assert "ILi1ELb%dELb0E" % streamed in kernel, (mib, kernel)
 """)
+
+
+def test_large_teams_fold_into_one_member_and_broadcast(recorded):  # noqa: F811
+    """From 16 members and 96 MiB of sources in all on: two launches, the second from the first member's destination."""
+    recorded("""
+for npes, mib, two in ((15, 8, 0), (16, 5, 0), (16, 6, 1), (16, 32, 1), (32, 3, 1), (33, 2, 0), (64, 2, 1)):
+    ok(lib.nvshmemx_amd_init(npes, 80 << 20))
+    a, b = lib.nvshmem_malloc(32 << 20), lib.nvshmem_malloc(32 << 20)
+    launches()
+    ok(_lib.typed_coll(lib, "nvshmemx_float_sum_reduce_on_stream", True)(0, b, a, mib << 18, None))
+    names = [l[0] for l in launches()]
+    assert len(names) == 1 + two, (npes, mib, names)
+    assert not two or ("reduce_root_kernel" in names[0] and "segment_copy_kernelILi2" in names[1]), names
+    lib.nvshmem_finalize()
+""")
