@@ -2009,6 +2009,85 @@ NVSHMEMI_DEVICE_INLINE size_t nvshmemi_amd_reduce_rounds(T *dst, const T *src, s
     return base;
 }
 
+/* A pointer that is the same for all lanes, as a scalar. */
+NVSHMEMI_DEVICE_INLINE const char *nvshmemi_amd_uniform(const void *p) {
+    const uint64_t a = (uint64_t)(uintptr_t)p;
+    return (const char *)(uintptr_t)((uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)a) |
+                                     (uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(a >> 32)) << 32);
+}
+/* The same FULL rounds for a team of a whole number of M members, with the loads of the next round in front of the stores of
+ * the last: behind them, a wait for the loads is one for the stores' acknowledgements as well, which is what a block of few
+ * wavefronts spends its time on.  No more registers than the rounds above (fp32 55, bf16 sum 59, max 71); with the loads in
+ * front of the fold too they would be 105.  us, kernel and barriers, three sets of buffers in turn, rounds above / here: 256
+ * threads, 8 members fp32 max 341 766 elements 49.9 / 38.0, bf16 sum 700 000 52 / 44.6, 16 members bf16 59 / 46, 4 members bf16 sum 786 111
+ * 57 / 47, max 60 / 54, fp32 500 000 56.7 / 50.8; 1024 threads, 16 members bf16 700 000 39.5 / 37.1, 8 114 688 9.4 / 9.2.  What is bound
+ * by the place of its data stays: 16 members fp32 903 614 170 / 168.  Wavefronts that go through their rounds together
+ * (PHASED) do as well as this from 512 threads on (8 members fp32 827 072: 69.7, 79.6 so). */
+template <typename T, int OP, int M, int V>
+NVSHMEMI_DEVICE_INLINE size_t nvshmemi_amd_reduce_rounds_ahead(T *dst, const T *src, size_t pe_stride, int npes, size_t nvec,
+                                                               size_t tid, size_t nthr, size_t base) {
+    constexpr size_t VEC = 16 / sizeof(T);
+    union pack_t { nvshmemi_v4u bits; T e[VEC]; __device__ pack_t() {} };
+    if (base + V * nthr > nvec) return base;
+    /* (addresses as a scalar base and a lane's offset: one pair of vector registers per member would be 32 of them) */
+    const char *const s0 = nvshmemi_amd_uniform(src);
+    char *const d0 = const_cast<char *>(nvshmemi_amd_uniform(dst));
+    const size_t stride = pe_stride * sizeof(T);
+    const unsigned lane = (unsigned)tid * 16;
+    pack_t x[V][M];
+    /* the place of member p0's vector; the compiler does not see how it goes on from round to round, which it would keep a
+     * pointer per member for */
+    typedef __attribute__((address_space(1))) char *global_t; /* (symmetric memory: no flat instructions) */
+    typedef __attribute__((address_space(1))) nvshmemi_v4u *global_vec_t;
+    auto place = [&](const char *p, size_t at, int p0) {
+        p = nvshmemi_amd_uniform(p + (size_t)p0 * stride + at * 16);
+        asm volatile("" : "+s"(p));
+        return (global_t)(uintptr_t)p;
+    };
+    auto fetch = [&](size_t at, int p0) {
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+            global_t from = place(s0, at + j * nthr, p0);
+#pragma unroll
+            for (int k = 0; k < M; ++k, from += stride) x[j][k].bits = *(global_vec_t)(from + lane);
+        }
+    };
+    fetch(base, 0);
+    for (;;) {
+        pack_t acc[V];
+        for (int p0 = 0;;) {
+#pragma unroll
+            for (int k = 0; k < M; ++k)
+#pragma unroll
+                for (int j = 0; j < V; ++j)
+                    if (p0 + k == 0) {
+                        acc[j].bits = x[j][0].bits;
+                    } else {
+#pragma unroll
+                        for (size_t e = 0; e < VEC; ++e) acc[j].e[e] = nvshmemi_amd_fold_step<T, OP>(p0 + k, acc[j].e[e], x[j][k].e[e]);
+                    }
+            /* (the fold is over before the registers are loaded again: sooner, they would be twice as many) */
+#pragma unroll
+            for (int j = 0; j < V; ++j) asm volatile("" : "+v"(acc[j].bits) : : "memory");
+            p0 += M;
+            if (p0 >= npes) break;
+            fetch(base, p0);
+        }
+        const size_t next = base + V * nthr;
+        const bool more = next + V * nthr <= nvec;
+        if (more) fetch(next, 0);
+        for (int p0 = 0; p0 < npes; p0 += M)
+#pragma unroll
+            for (int j = 0; j < V; ++j) {
+                global_t to = place(d0, base + j * nthr, p0);
+#pragma unroll
+                for (int k = 0; k < M; ++k, to += stride) *(global_vec_t)(to + lane) = acc[j].bits;
+            }
+        base = next;
+        if (!more) return base;
+    }
+}
+
 /* The fold of `nvec` whole vectors by a thread group.  Bound by what one compute unit keeps in flight, so by the loads of a
  * lane that wait together: eight, of as many members as there are, and with four or fewer of two vectors each.
  *  - Eight are what leaves every caller its wavefronts.  Sixteen take 79 to 101 vector registers where these take 51 (bf16
@@ -2035,9 +2114,11 @@ NVSHMEMI_DEVICE_INLINE void nvshmemi_amd_reduce_vectors(T *dst, const T *src, si
         const bool phased = sizeof(T) >= 4 && nthr >= NVSHMEMI_AMD_COPY_PHASED_THREADS && nvec * 16 * npes >= PHASED_BYTES;
         if (npes > 4) {
             if (phased) NVSHMEMI_AMD_ROUNDS(8, 1, NVSHMEMI_AMD_ROUNDS_PHASED);
+            else if (npes % 8 == 0) base = nvshmemi_amd_reduce_rounds_ahead<T, OP, 8, 1>(dst, src, pe_stride, npes, nvec, tid, nthr, base);
             NVSHMEMI_AMD_ROUNDS(8, 1);
         } else {
             if (phased) NVSHMEMI_AMD_ROUNDS(4, 2, NVSHMEMI_AMD_ROUNDS_PHASED);
+            else if (npes == 4) base = nvshmemi_amd_reduce_rounds_ahead<T, OP, 4, 2>(dst, src, pe_stride, npes, nvec, tid, nthr, base);
             NVSHMEMI_AMD_ROUNDS(4, 2, NVSHMEMI_AMD_ROUNDS_FULL);
             NVSHMEMI_AMD_ROUNDS(4, 1);
         }
