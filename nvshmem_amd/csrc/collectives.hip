@@ -487,7 +487,8 @@ __global__ __launch_bounds__(NPES ? NPES / MPW * 64 : 1024) void reduce_vector_k
 // wavefront, lane i loads vector i of a 1 KiB piece from every member, eight loads in flight at a time,
 // folds in member order and stores the result to every member.
 // NPES > 0 fixes the team size at compile time (loads, fold and stores fully unrolled).
-template <typename T, int OP, int NPES, bool NTL>
+// ASTRIDE: streamed loads that share the lines at a tile's ends (as in the LDS-staged kernel's fetch).
+template <typename T, int OP, int NPES, bool NTL, bool ASTRIDE = false>
 __global__ __launch_bounds__(64) void reduce_gather_kernel(char *base, uint64_t slice_bytes,
                                                            const nvshmemi_amd_team_view_t *groups,
                                                            reduce_shape_t s) {
@@ -511,7 +512,10 @@ __global__ __launch_bounds__(64) void reduce_gather_kernel(char *base, uint64_t 
             pack_t x[kBatch];
 #pragma unroll
             for (int k = 0; k < kBatch; ++k)
-                if (p0 + k < npes) x[k].v = stream_load<NTL>(src + (uint64_t)(p0 + k) * pe_stride);
+                if (p0 + k < npes) {
+                    const char *const from = src + (uint64_t)(p0 + k) * pe_stride;
+                    x[k].v = ASTRIDE ? stream_load_astride(from, threadIdx.x - 8 >= 48) : stream_load<NTL>(from);
+                }
 #pragma unroll
             for (int k = 0; k < kBatch; ++k)
                 if (p0 + k < npes) {
@@ -832,9 +836,13 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
         // room for the lead-in; at least one block for the edges
         const dim3 grid((unsigned)((nvec + 63 + 63) / 64), 1, ngroups);
         shape.dealt = dealt_blocks(dst_off, src_off, grid.x);
+        const bool astride = stream_source && (dst_off - src_off) % 128 && total_bytes <= rt.cacheable_source_bytes;
 #define NVSHMEM_AMD_LAUNCH_GATHER_REDUCE(N)                                                            \
     do {                                                                                               \
-        if (stream_source)                                                                             \
+        if (astride)                                                                                   \
+            hipLaunchKernelGGL((reduce_gather_kernel<T, OP, 0, true, true>), grid, dim3(64), 0, stream, rt.base, \
+                               rt.heap_size, tl.groups, shape);                                        \
+        else if (stream_source)                                                                        \
             hipLaunchKernelGGL((reduce_gather_kernel<T, OP, N, true>), grid, dim3(64), 0, stream, rt.base, \
                                rt.heap_size, tl.groups, shape);                    \
         else                                                                                           \
