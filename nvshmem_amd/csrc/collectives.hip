@@ -22,6 +22,7 @@
 #include <cstdio>
 
 #include "nvshmem.h"
+#include "launch.hpp"
 #include "runtime.hpp"
 
 namespace nvshmem_amd {
@@ -703,7 +704,7 @@ static int launch_broadcast(Runtime &rt, const TeamLaunch &tl, uint64_t doff, ui
     const size_t lds = paced ? paced_lds_bytes(rt, sources, tl.max_size) : 0;
     // a source that cannot stay in the Infinity Cache is streamed
 #define NVSHMEM_AMD_LAUNCH_BROADCAST(NTL, PACED)                                                                \
-    hipLaunchKernelGGL((segment_copy_kernel<kModeBroadcast, NTL, PACED, NVSHMEM_AMD_STORE_REPLICATE>), grid,      \
+    launch_kernel((segment_copy_kernel<kModeBroadcast, NTL, PACED, NVSHMEM_AMD_STORE_REPLICATE>), grid,      \
                        dim3(64), lds, stream, args)
     if (!paced) NVSHMEM_AMD_LAUNCH_BROADCAST(false, false);
     else if (sources > rt.cacheable_source_bytes) NVSHMEM_AMD_LAUNCH_BROADCAST(true, true);
@@ -791,9 +792,9 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
         const scatter_args_t args = {rt.base, rt.heap_size, team_arg(tl), dst_off, src_off, nelems, 0};
         const dim3 grid((unsigned)((nelems / (16 / sizeof(T)) + 63 + 63) / 64), 1, ngroups);
         if (stream_source)
-            hipLaunchKernelGGL((reduce_root_kernel<T, OP, true>), grid, dim3(64), 0, stream, args);
+            launch_kernel((reduce_root_kernel<T, OP, true>), grid, dim3(64), 0, stream, args);
         else
-            hipLaunchKernelGGL((reduce_root_kernel<T, OP, false>), grid, dim3(64), 0, stream, args);
+            launch_kernel((reduce_root_kernel<T, OP, false>), grid, dim3(64), 0, stream, args);
         (void)launch_broadcast(rt, tl, dst_off, dst_off, nelems * sizeof(T), 0, stream);
         return;
     }
@@ -815,10 +816,10 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
 #define NVSHMEM_AMD_LAUNCH_REDUCE_V(N, STREAM_MPW, MPW, VPT)                                      \
     do {                                                                                          \
         if (stream_source)                                                                        \
-            hipLaunchKernelGGL((reduce_vector_kernel<T, OP, N, true, VPT, STREAM_MPW>), grid, dim3(threads), lds,  \
+            launch_kernel((reduce_vector_kernel<T, OP, N, true, VPT, STREAM_MPW>), grid, dim3(threads), lds,  \
                                stream, rt.base, rt.heap_size, tl.groups, shape);                                                  \
         else                                                                                      \
-            hipLaunchKernelGGL((reduce_vector_kernel<T, OP, N, false, VPT, MPW>), grid, dim3(threads), lds, \
+            launch_kernel((reduce_vector_kernel<T, OP, N, false, VPT, MPW>), grid, dim3(threads), lds, \
                                stream, rt.base, rt.heap_size, tl.groups, shape);                                                  \
     } while (0)
         if (ct_size == 8) NVSHMEM_AMD_LAUNCH_REDUCE_V(8, NVSHMEM_AMD_REDUCE_WIDE_MPW, kNarrowMpw, kVptNarrow);
@@ -830,7 +831,7 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
 #undef NVSHMEM_AMD_LAUNCH_REDUCE
 #undef NVSHMEM_AMD_LAUNCH_REDUCE_V
     } else if (element_at_a_time<T, false>(rt, tl, fixed_size == 4 || fixed_size == 8, dst_off, src_off, nelems)) {
-        hipLaunchKernelGGL((reduce_element_kernel<T, OP>), dim3((unsigned)((nelems + 255) / 256), 1, ngroups), dim3(256), 0,
+        launch_kernel((reduce_element_kernel<T, OP>), dim3((unsigned)((nelems + 255) / 256), 1, ngroups), dim3(256), 0,
                            stream, rt.base, rt.heap_size, tl.groups, dst_off, src_off, nelems);
     } else {
         // room for the lead-in; at least one block for the edges
@@ -840,13 +841,13 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
 #define NVSHMEM_AMD_LAUNCH_GATHER_REDUCE(N)                                                            \
     do {                                                                                               \
         if (astride)                                                                                   \
-            hipLaunchKernelGGL((reduce_gather_kernel<T, OP, 0, true, true>), grid, dim3(64), 0, stream, rt.base, \
+            launch_kernel((reduce_gather_kernel<T, OP, 0, true, true>), grid, dim3(64), 0, stream, rt.base, \
                                rt.heap_size, tl.groups, shape);                                        \
         else if (stream_source)                                                                        \
-            hipLaunchKernelGGL((reduce_gather_kernel<T, OP, N, true>), grid, dim3(64), 0, stream, rt.base, \
+            launch_kernel((reduce_gather_kernel<T, OP, N, true>), grid, dim3(64), 0, stream, rt.base, \
                                rt.heap_size, tl.groups, shape);                    \
         else                                                                                           \
-            hipLaunchKernelGGL((reduce_gather_kernel<T, OP, N, false>), grid, dim3(64), 0, stream, rt.base, \
+            launch_kernel((reduce_gather_kernel<T, OP, N, false>), grid, dim3(64), 0, stream, rt.base, \
                                rt.heap_size, tl.groups, shape);                    \
     } while (0)
         // (sixteen members unrolled measured slower than the loop: 5.2 against 5.4 TB/s)
@@ -864,7 +865,7 @@ void launch_reducescatter(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, u
     const bool eight = tl.min_size == 8 && tl.max_size == 8;
     if (nelems == all && element_at_a_time<T, true>(rt, tl, eight, dst_off, src_off, nelems)) {
         const dim3 grid((unsigned)((nelems + 255) / 256), (unsigned)tl.max_size, (unsigned)tl.ngroups);
-        hipLaunchKernelGGL((reduce_element_kernel<T, OP, true>), grid, dim3(256), 0, stream, rt.base, rt.heap_size,
+        launch_kernel((reduce_element_kernel<T, OP, true>), grid, dim3(256), 0, stream, rt.base, rt.heap_size,
                            tl.groups, dst_off, src_off, nelems);
         return;
     }
@@ -875,9 +876,9 @@ void launch_reducescatter(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, u
 #define NVSHMEM_AMD_LAUNCH_GATHER(N)                                                                                   \
     do {                                                                                                               \
         if (stream_source)                                                                                             \
-            hipLaunchKernelGGL((reducescatter_gather_kernel<T, OP, N, true>), grid, dim3(64), 0, stream, args);        \
+            launch_kernel((reducescatter_gather_kernel<T, OP, N, true>), grid, dim3(64), 0, stream, args);        \
         else                                                                                                           \
-            hipLaunchKernelGGL((reducescatter_gather_kernel<T, OP, N, false>), grid, dim3(64), 0, stream, args);       \
+            launch_kernel((reducescatter_gather_kernel<T, OP, N, false>), grid, dim3(64), 0, stream, args);       \
     } while (0)
     if (eight) NVSHMEM_AMD_LAUNCH_GATHER(8);
     else if (tl.min_size == 16 && tl.max_size == 16) NVSHMEM_AMD_LAUNCH_GATHER(16);
@@ -1085,7 +1086,7 @@ static int segment_collective(int mode, const char *what, nvshmem_team_t team, v
     const bool stream_source = quarter || sources > rt.cacheable_source_bytes;
     const segment_args_t args = {rt.base, rt.heap_size, team_arg(tl), doff, soff, seg_bytes, 0, (uint32_t)n, 0, 0, quarter};
 #define NVSHMEM_AMD_LAUNCH_SEGCOPY(MODE, NTL, PACED, STORE) \
-    hipLaunchKernelGGL((segment_copy_kernel<MODE, NTL, PACED, STORE>), grid, dim3(64), lds, stream, args)
+    launch_kernel((segment_copy_kernel<MODE, NTL, PACED, STORE>), grid, dim3(64), lds, stream, args)
     if (mode == kModeFcollect) {
         const dim3 grid((unsigned)tiles, (unsigned)n, (unsigned)tl.ngroups);
         const bool paced = paced_copy(rt, tiles * n * (uint64_t)tl.ngroups, tl.max_size);
@@ -1093,7 +1094,7 @@ static int segment_collective(int mode, const char *what, nvshmem_team_t team, v
         segment_args_t chunked = args;
         const uint64_t chunked_blocks = paced && stream_source ? chunked_copy(&chunked, tl.max_size, tiles) : 0;
         if (chunked_blocks) {
-            hipLaunchKernelGGL((segment_copy_kernel<kModeFcollect, false, true, NVSHMEM_AMD_STORE_REPLICATE, true>),
+            launch_kernel((segment_copy_kernel<kModeFcollect, false, true, NVSHMEM_AMD_STORE_REPLICATE, true>),
                                dim3((unsigned)chunked_blocks, grid.y, grid.z), dim3(64), 0, stream, chunked);
         } else if (!paced) NVSHMEM_AMD_LAUNCH_SEGCOPY(kModeFcollect, false, false, NVSHMEM_AMD_STORE_REPLICATE);
         else if (stream_source) NVSHMEM_AMD_LAUNCH_SEGCOPY(kModeFcollect, true, true, NVSHMEM_AMD_STORE_REPLICATE);

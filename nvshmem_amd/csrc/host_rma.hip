@@ -9,6 +9,7 @@
 #include <type_traits>
 
 #include "nvshmem.h"
+#include "launch.hpp"
 #include "runtime.hpp"
 
 namespace nvshmem_amd {
@@ -66,10 +67,10 @@ constexpr size_t kKernelElements = (size_t)1 << 31;
 template <typename T>
 void launch_strided(void *dst, size_t dst_stride, const void *src, size_t src_stride, size_t nelems, hipStream_t stream) {
     if (nelems > kNarrowBlockElements)
-        hipLaunchKernelGGL((strided_copy_kernel<T, 256>), dim3((unsigned)((nelems + 255) / 256)), dim3(256), 0, stream, (T *)dst,
+        launch_kernel((strided_copy_kernel<T, 256>), dim3((unsigned)((nelems + 255) / 256)), dim3(256), 0, stream, (T *)dst,
                            dst_stride, (const T *)src, src_stride, nelems);
     else
-        hipLaunchKernelGGL((strided_copy_kernel<T, 64>), dim3((unsigned)((nelems + 63) / 64)), dim3(64), 0, stream, (T *)dst,
+        launch_kernel((strided_copy_kernel<T, 64>), dim3((unsigned)((nelems + 63) / 64)), dim3(64), 0, stream, (T *)dst,
                            dst_stride, (const T *)src, src_stride, nelems);
     NVSHMEM_AMD_HIP_CHECK(hipGetLastError());
 }
@@ -145,7 +146,7 @@ void p_on_stream(void *dest, const void *value, size_t es, int pe, hipStream_t s
     if (!check_symmetric_range(rt, "p", dest, es, &off)) return;
     uint64_t bits = 0;
     memcpy(&bits, value, es);
-    hipLaunchKernelGGL(scalar_p_kernel, dim3(1), dim3(1), 0, stream, dest, bits, (int)es, pe);
+    launch_kernel(scalar_p_kernel, dim3(1), dim3(1), 0, stream, dest, bits, (int)es, pe);
     NVSHMEM_AMD_HIP_CHECK(hipGetLastError());
 }
 
@@ -179,7 +180,7 @@ void wait_until_on_stream(T *ivar, int cmp, T value, hipStream_t stream) {
         set_error("wait_until_on_stream: unknown comparison %d", cmp);
         return;
     }
-    hipLaunchKernelGGL(wait_until_kernel<T>, dim3(1), dim3(1), 0, stream, ivar, cmp, value);
+    launch_kernel(wait_until_kernel<T>, dim3(1), dim3(1), 0, stream, ivar, cmp, value);
     NVSHMEM_AMD_HIP_CHECK(hipGetLastError());
 }
 
@@ -196,7 +197,7 @@ void wait_until_all_on_stream(T *ivars, size_t nelems, const int *status, int cm
         return;
     }
     // `status` is read by the kernel: it must be device-accessible memory (or NULL), as in the reference
-    hipLaunchKernelGGL(wait_until_all_kernel<T>, dim3(1), dim3(kWaitThreads), 0, stream, ivars, nelems, status, cmp, value);
+    launch_kernel(wait_until_all_kernel<T>, dim3(1), dim3(kWaitThreads), 0, stream, ivars, nelems, status, cmp, value);
     NVSHMEM_AMD_HIP_CHECK(hipGetLastError());
 }
 
@@ -225,7 +226,7 @@ void wait_until_all_vector_on_stream(T *ivars, size_t nelems, const int *status,
         set_error("wait_until_all_vector_on_stream: cmp_values is NULL");
         return;
     }
-    hipLaunchKernelGGL(wait_until_all_vector_kernel<T>, dim3(1), dim3(kWaitThreads), 0, stream, ivars, nelems, status, cmp,
+    launch_kernel(wait_until_all_vector_kernel<T>, dim3(1), dim3(kWaitThreads), 0, stream, ivars, nelems, status, cmp,
                        values);
     NVSHMEM_AMD_HIP_CHECK(hipGetLastError());
 }
@@ -278,7 +279,7 @@ T host_amo(const char *what, int op, const T *target, T value, T cond, int pe) {
     static uint64_t *slot = nullptr;  // pinned, lives until the process ends
     if (!slot) NVSHMEM_AMD_HIP_CHECK(hipHostMalloc((void **)&slot, sizeof(uint64_t), hipHostMallocDefault));
     *slot = 0;
-    hipLaunchKernelGGL(host_amo_kernel<T>, dim3(1), dim3(1), 0, nullptr, op, const_cast<T *>(target), value, cond,
+    launch_kernel(host_amo_kernel<T>, dim3(1), dim3(1), 0, nullptr, op, const_cast<T *>(target), value, cond,
                        pe, reinterpret_cast<T *>(slot));
     NVSHMEM_AMD_HIP_CHECK(hipGetLastError());
     sync0();

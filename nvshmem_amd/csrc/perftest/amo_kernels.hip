@@ -114,7 +114,7 @@ int nvshmem_perftest_amo_matrix(uint64_t *slots, const uint64_t *val, const uint
         !perftest::check_range(val, bytes) || !perftest::check_range(cond, bytes) ||
         !perftest::check_range(out, bytes) || !perftest::check_range(ncases, sizeof(int)))
         return NVSHMEMX_ERROR_INVALID_VALUE;
-    hipLaunchKernelGGL(amo_matrix_kernel, dim3(1, 1, (unsigned)nvshmem_n_pes()), dim3(64), 0,
+    nvshmem_amd::launch_kernel(amo_matrix_kernel, dim3(1, 1, (unsigned)nvshmem_n_pes()), dim3(64), 0,
                        (hipStream_t)stream, slots, val, cond, out, ncases);
     return perftest::launch_status("amo_matrix");
 }
@@ -129,7 +129,7 @@ int nvshmem_perftest_amo_contend(uint64_t *words, unsigned int *seen, unsigned l
         !perftest::check_range(seen, total * sizeof(unsigned int)) ||
         !perftest::check_range(chain, total * sizeof(unsigned long long)))
         return NVSHMEMX_ERROR_INVALID_VALUE;
-    hipLaunchKernelGGL(amo_contend_kernel, dim3((unsigned)blocks, 1, (unsigned)nvshmem_n_pes()),
+    nvshmem_amd::launch_kernel(amo_contend_kernel, dim3((unsigned)blocks, 1, (unsigned)nvshmem_n_pes()),
                        dim3((unsigned)threads), 0, (hipStream_t)stream, words, seen, chain, home);
     return perftest::launch_status("amo_contend");
 }

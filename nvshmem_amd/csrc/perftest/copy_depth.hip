@@ -21,7 +21,7 @@ extern "C" int nvshmem_perftest_put_depth12(void *dest, const void *src, size_t 
     if (!perftest::ready() || !perftest::check_launch(1, threads) || !perftest::check_range(dest, bytes) ||
         !perftest::check_range(src, bytes))
         return NVSHMEMX_ERROR_INVALID_VALUE;
-    hipLaunchKernelGGL(put_depth12_kernel, dim3(1, 1, (unsigned)nvshmem_n_pes()), dim3(threads), 0, (hipStream_t)stream,
+    nvshmem_amd::launch_kernel(put_depth12_kernel, dim3(1, 1, (unsigned)nvshmem_n_pes()), dim3(threads), 0, (hipStream_t)stream,
                        (char *)dest, (const char *)src, bytes);
     return perftest::launch_status("put_depth12");
 }

@@ -423,7 +423,7 @@ int nvshmem_perftest_moe_dispatch_put_signal(void *recv, size_t recv_cap_rows, c
     const int rc = per_row ? perftest::launch_moe_rowsignal(warp, full, blocks_per_pe, threads, row_args, (hipStream_t)stream)
                            : perftest::launch_senders(fn, blocks_per_pe, threads, args, (hipStream_t)stream);
     if (rc != 0) return rc;
-    hipLaunchKernelGGL(moe_receive_kernel, dim3(1, 1, (unsigned)nvshmem_n_pes()), dim3(NVSHMEMI_WARP_SIZE), 0,
+    nvshmem_amd::launch_kernel(moe_receive_kernel, dim3(1, 1, (unsigned)nvshmem_n_pes()), dim3(NVSHMEMI_WARP_SIZE), 0,
                        (hipStream_t)stream, expected, sig, sig_stride);
     return perftest::launch_status("moe_receive");
 }
@@ -478,16 +478,16 @@ static int dispatch_pieces(void *recv, size_t recv_cap_rows, const void *send, c
     const dim3 dgrid(grid.x << kshift, grid.y, grid.z);
     if (static_sig) {
         const unsigned n = (unsigned)(nvshmem_n_pes() * nvshmem_n_pes());
-        hipLaunchKernelGGL(clear_words_kernel, dim3((n + 255) / 256), dim3(256), 0, (hipStream_t)stream, static_sig, n);
+        nvshmem_amd::launch_kernel(clear_words_kernel, dim3((n + 255) / 256), dim3(256), 0, (hipStream_t)stream, static_sig, n);
         const int rc0 = perftest::launch_status("clear_words");
         if (rc0 != 0) return rc0;
     }
 #define LAUNCH_DIRECT(V)                                                                           \
-    hipLaunchKernelGGL((moe_dispatch_direct_kernel<V>), dgrid, dim3(threads), 0, (hipStream_t)stream, \
+    nvshmem_amd::launch_kernel((moe_dispatch_direct_kernel<V>), dgrid, dim3(threads), 0, (hipStream_t)stream, \
                        (char *)recv, (const char *)send, dest_pe, dest_row, tokens, topk, row_bytes, \
                        recv_cap_rows, kshift)
 #define LAUNCH_DISPATCH(P)                                                                         \
-    hipLaunchKernelGGL((moe_dispatch_pieces_kernel<P>), grid, dim3(threads), 0, (hipStream_t)stream, \
+    nvshmem_amd::launch_kernel((moe_dispatch_pieces_kernel<P>), grid, dim3(threads), 0, (hipStream_t)stream, \
                        (char *)recv, (const char *)send, dest_pe, dest_row, tokens, topk, row_bytes, \
                        recv_cap_rows)
     if (direct) {
@@ -507,10 +507,10 @@ static int dispatch_pieces(void *recv, size_t recv_cap_rows, const void *send, c
     // most 64) can never keep a block that still has to announce off the GPU
     const unsigned sig_blocks = (unsigned)(((size_t)tokens * (size_t)topk + 8191) / 8192 < 8 ? ((size_t)tokens * (size_t)topk + 8191) / 8192 : 8);
     if (static_sig)
-        hipLaunchKernelGGL(moe_dispatch_signal_kernel<false>, dim3(sig_blocks, 1, (unsigned)nvshmem_n_pes()), dim3(1024),
+        nvshmem_amd::launch_kernel(moe_dispatch_signal_kernel<false>, dim3(sig_blocks, 1, (unsigned)nvshmem_n_pes()), dim3(1024),
                            0, (hipStream_t)stream, dest_pe, dest_row, expected, static_sig, tokens, topk, recv_cap_rows);
     else
-        hipLaunchKernelGGL(moe_dispatch_signal_kernel<true>, dim3(sig_blocks, 1, (unsigned)nvshmem_n_pes()), dim3(1024),
+        nvshmem_amd::launch_kernel(moe_dispatch_signal_kernel<true>, dim3(sig_blocks, 1, (unsigned)nvshmem_n_pes()), dim3(1024),
                            0, (hipStream_t)stream, dest_pe, dest_row, expected, sig, tokens, topk, recv_cap_rows);
     return perftest::launch_status("moe_dispatch_signal");
 }
@@ -587,7 +587,7 @@ int nvshmem_perftest_moe_combine_pieces(void *out, const void *recv, size_t recv
         return NVSHMEMX_ERROR_INVALID_VALUE;   // the kernel counts work items in 32 bits
     const dim3 grid((unsigned)blocks_per_pe, 1, (unsigned)nvshmem_n_pes());
 #define LAUNCH_COMBINE(...)                                                                        \
-    hipLaunchKernelGGL((moe_combine_kernel<__VA_ARGS__>), grid, dim3(threads), 0, (hipStream_t)stream, \
+    nvshmem_amd::launch_kernel((moe_combine_kernel<__VA_ARGS__>), grid, dim3(threads), 0, (hipStream_t)stream, \
                        (char *)out, (const char *)recv, dest_pe, dest_row, tokens, topk, row_bytes,    \
                        recv_cap_rows)
     if (piece_bytes == 1024) LAUNCH_COMBINE(true, 1024);
@@ -624,7 +624,7 @@ int nvshmem_perftest_moe_exchange_offsets(const int64_t *counts, int64_t *seg_ba
         !perftest::check_range(seg_base, sizeof(int64_t) * (size_t)num_experts * np) ||
         !perftest::check_range(recv_rows, sizeof(int64_t)))
         return NVSHMEMX_ERROR_INVALID_VALUE;
-    hipLaunchKernelGGL(moe_exchange_offsets_kernel, dim3(1, 1, (unsigned)np), dim3(256),
+    nvshmem_amd::launch_kernel(moe_exchange_offsets_kernel, dim3(1, 1, (unsigned)np), dim3(256),
                        (size_t)num_experts * np * sizeof(int64_t), (hipStream_t)stream, counts,
                        seg_base, recv_rows, num_experts);
     return perftest::launch_status("moe_exchange_offsets");

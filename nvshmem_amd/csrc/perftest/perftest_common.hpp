@@ -6,6 +6,7 @@
 
 #include <cstdio>
 
+#include "launch.hpp"
 #include "nvshmem.h"
 
 namespace perftest {

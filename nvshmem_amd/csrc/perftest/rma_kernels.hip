@@ -366,16 +366,16 @@ int launch_element(int what, void *dest, const void *src, size_t n, int blocks, 
     const dim3 grid((unsigned)blocks, 1, (unsigned)nvshmem_n_pes());
     switch (what) {
         case NVSHMEM_PERFTEST_ELEMENT_P:
-            hipLaunchKernelGGL((element_bw_kernel<T, NVSHMEM_PERFTEST_ELEMENT_P>), grid, dim3(threads), 0, stream, (T *)dest, (const T *)src, n);
+            nvshmem_amd::launch_kernel((element_bw_kernel<T, NVSHMEM_PERFTEST_ELEMENT_P>), grid, dim3(threads), 0, stream, (T *)dest, (const T *)src, n);
             break;
         case NVSHMEM_PERFTEST_ELEMENT_G:
-            hipLaunchKernelGGL((element_bw_kernel<T, NVSHMEM_PERFTEST_ELEMENT_G>), grid, dim3(threads), 0, stream, (T *)dest, (const T *)src, n);
+            nvshmem_amd::launch_kernel((element_bw_kernel<T, NVSHMEM_PERFTEST_ELEMENT_G>), grid, dim3(threads), 0, stream, (T *)dest, (const T *)src, n);
             break;
         case NVSHMEM_PERFTEST_ELEMENT_ST:
-            hipLaunchKernelGGL((element_bw_kernel<T, NVSHMEM_PERFTEST_ELEMENT_ST>), grid, dim3(threads), 0, stream, (T *)dest, (const T *)src, n);
+            nvshmem_amd::launch_kernel((element_bw_kernel<T, NVSHMEM_PERFTEST_ELEMENT_ST>), grid, dim3(threads), 0, stream, (T *)dest, (const T *)src, n);
             break;
         default:
-            hipLaunchKernelGGL((element_bw_kernel<T, NVSHMEM_PERFTEST_ELEMENT_ADD>), grid, dim3(threads), 0, stream, (T *)dest, (const T *)src, n);
+            nvshmem_amd::launch_kernel((element_bw_kernel<T, NVSHMEM_PERFTEST_ELEMENT_ADD>), grid, dim3(threads), 0, stream, (T *)dest, (const T *)src, n);
             break;
     }
     return perftest::launch_status("element_bw");
@@ -387,10 +387,10 @@ int launch_ring(bool is_get, char *dest, const char *src, size_t bytes, int bloc
     const dim3 grid((unsigned)blocks, 1, (unsigned)nvshmem_n_pes());
     const size_t per_block = bytes / (size_t)blocks;
     if (is_get)
-        hipLaunchKernelGGL((ring_rma_kernel<SCOPE, true>), grid, dim3(threads), 0, stream, dest, src, bytes,
+        nvshmem_amd::launch_kernel((ring_rma_kernel<SCOPE, true>), grid, dim3(threads), 0, stream, dest, src, bytes,
                            per_block);
     else
-        hipLaunchKernelGGL((ring_rma_kernel<SCOPE, false>), grid, dim3(threads), 0, stream, dest, src, bytes,
+        nvshmem_amd::launch_kernel((ring_rma_kernel<SCOPE, false>), grid, dim3(threads), 0, stream, dest, src, bytes,
                            per_block);
     return perftest::launch_status("ring_rma");
 }
@@ -437,7 +437,7 @@ int nvshmem_perftest_lds_rma(void *dest, const void *src, size_t bytes, size_t s
         return NVSHMEMX_ERROR_INVALID_VALUE;
     const auto kernel = scope == NVSHMEM_PERFTEST_SCOPE_WARP ? lds_rma_kernel<NVSHMEM_PERFTEST_SCOPE_WARP>
                                                              : lds_rma_kernel<NVSHMEM_PERFTEST_SCOPE_BLOCK>;
-    hipLaunchKernelGGL(kernel, dim3(1, 1, (unsigned)nvshmem_n_pes()), dim3(NVSHMEMI_WARP_SIZE), 0, (hipStream_t)stream,
+    nvshmem_amd::launch_kernel(kernel, dim3(1, 1, (unsigned)nvshmem_n_pes()), dim3(NVSHMEMI_WARP_SIZE), 0, (hipStream_t)stream,
                        (char *)dest, (const char *)src, (unsigned)bytes, (unsigned)shift, form);
     return perftest::launch_status("lds_rma");
 }
@@ -466,7 +466,7 @@ int nvshmem_perftest_plain_copy(void *dst, const void *src, size_t bytes, void *
         return NVSHMEMX_ERROR_INVALID_VALUE;
     const size_t nvec = bytes / 16;
     if (nvec == 0) return 0;
-    hipLaunchKernelGGL(plain_copy_kernel, dim3((unsigned)((nvec + 255) / 256)), dim3(256), 0,
+    nvshmem_amd::launch_kernel(plain_copy_kernel, dim3((unsigned)((nvec + 255) / 256)), dim3(256), 0,
                        (hipStream_t)stream, (nvshmemi_v4u *)dst, (const nvshmemi_v4u *)src, nvec);
     return perftest::launch_status("plain_copy");
 }
@@ -479,14 +479,14 @@ int nvshmem_perftest_stream_probe(void *buf, size_t bytes, int blocks_per_pe, in
     const size_t per_block = bytes / (size_t)blocks_per_pe / round * round;  // whole rounds only
     if (per_block == 0) return NVSHMEMX_ERROR_INVALID_VALUE;
     const dim3 grid((unsigned)blocks_per_pe, 1, (unsigned)nvshmem_n_pes());
-    if (write == 2) hipLaunchKernelGGL(stream_probe_kernel<2>, grid, dim3(threads), 0, (hipStream_t)stream, (char *)buf, bytes, per_block);
-    else if (write) hipLaunchKernelGGL(stream_probe_kernel<1>, grid, dim3(threads), 0, (hipStream_t)stream, (char *)buf, bytes, per_block);
-    else hipLaunchKernelGGL(stream_probe_kernel<0>, grid, dim3(threads), 0, (hipStream_t)stream, (char *)buf, bytes, per_block);
+    if (write == 2) nvshmem_amd::launch_kernel(stream_probe_kernel<2>, grid, dim3(threads), 0, (hipStream_t)stream, (char *)buf, bytes, per_block);
+    else if (write) nvshmem_amd::launch_kernel(stream_probe_kernel<1>, grid, dim3(threads), 0, (hipStream_t)stream, (char *)buf, bytes, per_block);
+    else nvshmem_amd::launch_kernel(stream_probe_kernel<0>, grid, dim3(threads), 0, (hipStream_t)stream, (char *)buf, bytes, per_block);
     return perftest::launch_status("stream_probe");
 }
 
 int nvshmem_perftest_profile_marker(void *stream) {
-    hipLaunchKernelGGL(profile_marker_kernel, dim3(1), dim3(1), 0, (hipStream_t)stream);
+    nvshmem_amd::launch_kernel(profile_marker_kernel, dim3(1), dim3(1), 0, (hipStream_t)stream);
     return perftest::launch_status("profile_marker");
 }
 
@@ -501,7 +501,7 @@ int nvshmem_perftest_p_g(uint64_t *words, uint64_t *out, uint64_t value_base, vo
 
 int nvshmem_perftest_pe_identity(int *out, int grid_z, void *stream) {
     if (!perftest::ready() || !out || grid_z < 1 || grid_z > 64) return NVSHMEMX_ERROR_INVALID_VALUE;
-    hipLaunchKernelGGL(pe_identity_kernel, dim3(1, 1, (unsigned)grid_z), dim3(1), 0, (hipStream_t)stream, out);
+    nvshmem_amd::launch_kernel(pe_identity_kernel, dim3(1, 1, (unsigned)grid_z), dim3(1), 0, (hipStream_t)stream, out);
     return perftest::launch_status("pe_identity");
 }
 
@@ -512,7 +512,7 @@ int nvshmem_perftest_signal_op(uint64_t *sig, uint64_t value, int sig_op, int th
         return NVSHMEMX_ERROR_INVALID_VALUE;
     if (sig_op != NVSHMEM_SIGNAL_SET && sig_op != NVSHMEM_SIGNAL_ADD)
         return NVSHMEMX_ERROR_INVALID_VALUE;
-    hipLaunchKernelGGL(signal_op_kernel, dim3(1, 1, (unsigned)nvshmem_n_pes()), dim3(threads), 0,
+    nvshmem_amd::launch_kernel(signal_op_kernel, dim3(1, 1, (unsigned)nvshmem_n_pes()), dim3(threads), 0,
                        (hipStream_t)stream, sig, value, sig_op, reps);
     return perftest::launch_status("signal_op");
 }
@@ -522,7 +522,7 @@ int nvshmem_perftest_signal_wait(uint64_t *sig, int cmp, uint64_t cmp_value, uin
     if (!perftest::ready() || !perftest::check_range(sig, sizeof(uint64_t)) ||
         !perftest::check_range(out, sizeof(uint64_t)))
         return NVSHMEMX_ERROR_INVALID_VALUE;
-    hipLaunchKernelGGL(signal_wait_kernel, dim3(1, 1, (unsigned)nvshmem_n_pes()), dim3(1), 0,
+    nvshmem_amd::launch_kernel(signal_wait_kernel, dim3(1, 1, (unsigned)nvshmem_n_pes()), dim3(1), 0,
                        (hipStream_t)stream, sig, cmp, cmp_value, out);
     return perftest::launch_status("signal_wait");
 }
@@ -565,7 +565,7 @@ int nvshmem_perftest_fill_words(uint64_t *words, uint64_t value, size_t nwords, 
         return NVSHMEMX_ERROR_INVALID_VALUE;
     if (nwords == 0) return 0;
     const unsigned blocks = (unsigned)((nwords + 255) / 256 < 1024 ? (nwords + 255) / 256 : 1024);
-    hipLaunchKernelGGL(fill_words_kernel, dim3(blocks, 1, (unsigned)nvshmem_n_pes()), dim3(256), 0,
+    nvshmem_amd::launch_kernel(fill_words_kernel, dim3(blocks, 1, (unsigned)nvshmem_n_pes()), dim3(256), 0,
                        (hipStream_t)stream, words, value, nwords);
     return perftest::launch_status("fill_words");
 }

@@ -5,6 +5,7 @@
 // (:2288-2387 public heap calls), src/host/comm/putget.cpp (:48-185 on-stream RMA),
 // src/host/comm/sync.cpp (:60-115 on-stream signal ops),
 // src/device/launch/collective_launch.cpp (:72-260).
+#include "launch.hpp"
 #include "runtime.hpp"
 
 #include <cstdio>
@@ -582,7 +583,7 @@ static void stream_copy(char *dst, const char *src, size_t bytes, bool other_is_
     constexpr size_t kBulk = (size_t)128 << 20;  // source + destination no longer fit the 256 MiB cache
     const size_t blocks = (bytes + 1023) / 1024;
     if (bytes > kBulk && blocks <= 0x7fffffffull && other_is_device) {
-        hipLaunchKernelGGL(bulk_copy_kernel, dim3((unsigned)blocks), dim3(64), 0, stream, dst, src, bytes);
+        launch_kernel(bulk_copy_kernel, dim3((unsigned)blocks), dim3(64), 0, stream, dst, src, bytes);
         NVSHMEM_AMD_HIP_CHECK(hipGetLastError());
         return;
     }
@@ -663,7 +664,7 @@ void nvshmemx_signal_op_on_stream(uint64_t *sig_addr, uint64_t signal, int sig_o
         std::lock_guard<std::recursive_mutex> lock(rt.mu);
         refresh_symbols(rt, false);
     }
-    hipLaunchKernelGGL(signal_op_kernel, dim3(1), dim3(1), 0, (hipStream_t)stream, sig_addr, signal,
+    launch_kernel(signal_op_kernel, dim3(1), dim3(1), 0, (hipStream_t)stream, sig_addr, signal,
                        sig_op, pe);
     NVSHMEM_AMD_HIP_CHECK(hipGetLastError());
 }
@@ -684,7 +685,7 @@ void nvshmemx_signal_wait_until_on_stream(uint64_t *sig_addr, int cmp, uint64_t 
         std::lock_guard<std::recursive_mutex> lock(rt.mu);
         refresh_symbols(rt, false);
     }
-    hipLaunchKernelGGL(signal_wait_kernel, dim3(1), dim3(1), 0, (hipStream_t)stream, sig_addr, 0, cmp, cmp_value);
+    launch_kernel(signal_wait_kernel, dim3(1), dim3(1), 0, (hipStream_t)stream, sig_addr, 0, cmp, cmp_value);
     NVSHMEM_AMD_HIP_CHECK(hipGetLastError());
 }
 
@@ -708,7 +709,7 @@ void nvshmemx_putmem_signal_on_stream(void *dest, const void *source, size_t byt
             }
             const size_t vecs = (bytes + 15) / 16;
             const unsigned threads = vecs >= 1024 ? 1024 : (unsigned)(vecs + 63) & ~63u;
-            hipLaunchKernelGGL(put_signal_kernel, dim3(1), dim3(threads), 0, (hipStream_t)stream, dst, src,
+            launch_kernel(put_signal_kernel, dim3(1), dim3(threads), 0, (hipStream_t)stream, dst, src,
                                (uint32_t)bytes, threads, sig_addr, signal, op, pe);
             NVSHMEM_AMD_HIP_CHECK(hipGetLastError());
             return;
