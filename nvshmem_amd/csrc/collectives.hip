@@ -1073,16 +1073,17 @@ static int segment_collective(int mode, const char *what, nvshmem_team_t team, v
         set_error("%s: message too large", what);
         return NVSHMEMX_ERROR_INVALID_VALUE;
     }
-    // Alltoalls that the Infinity Cache could just hold stream three quarters of a source and keep a quarter, the lines at
-    // the ends of its pieces, which on another offset than the destination's two wavefronts read.  Beside other buffers in turn
-    // a source kept whole is gone when it comes again, a quarter is not; and one that was just written loses less to what the
-    // loads bring in.  us kept / a quarter kept, fp32, sources of 110 | 160 | 240 MB in all: 8 members in turn 35.0 / 32.6 | 51.4 /
-    // 45.9 | 75.8 / 66.9, just written 28.3 / 21.9 | 41.5 / 33.0 | 59.8 / 56.5, on another offset 34.7 / 34.7 | 51.8 / 49.2 | 76.4 /
-    // 71.3; 16 members in turn 39.9 / 37.8 | 53.8 / 48.8 | 77.9 / 69.1, 4 34.7 / 32.3 | 51.2 / 45.7 | 76.4 / 67.4.  Not a buffer of just the
-    // cache's size: sent again and again as it is, it stays (16 members, 256 MiB: 72.4 / 78.5; in turn 85.4 / 78.1).  None
-    // kept: 200 MB 61.5, a quarter 56.6.  Below 112 MiB three buffers in turn are still there in part: 105 MB 31.9 / 31.2, on
-    // another offset 33.2 / 33.4, 16 members 37.2 / 38.8.  (Dealing the tiles to the XCDs, as in the reductions, loses 2 % here.)
-    const bool quarter = mode == kModeAlltoall && sources > rt.cacheable_source_bytes / 16 * 7 && sources < rt.cacheable_source_bytes;
+    // Alltoalls of 7/16 (112 MiB) to all of what the Infinity Cache could hold stream three quarters of a source and keep a
+    // quarter, the lines at the ends of its pieces, which on another offset than the destination's two wavefronts read.  Beside
+    // other buffers in turn a source kept whole is gone when it comes again, a quarter is not.  us kept / a quarter kept, fp32
+    // normal data, 120 | 200 | 240 | 256 MiB of sources in all, 8 members, three sets of buffers in turn 39.2 / 36.5 | 66.3 / 59.3 | 79.5 /
+    // 70.5 | 84.5 / 75.2, each filled in front of its call (both kernels) 74.5 / 70.6 | 110.0 / 107.0 | 124.8 / 125.8 | 129.0 / 133.4; what
+    // loses is a source sent again as it is, with nothing in between: 34.9 / 36.2 | 58.2 / 59.6 | 68.6 / 70.2 | 72.8 / 75.3.  256 MiB on 4
+    // and 16 members: in turn 84.4 / 74.8 and 84.5 / 77.5, filled 117.9 / 118.8 and 143.1 / 146.8, again as it is 72.8 / 74.7 and 72.4 /
+    // 77.8; on another offset, 8 members, 85.2 / 80.7, 132.5 / 136.2 and 76.0 / 80.6.  None kept: 200 MiB in turn 63.3.  Below 112
+    // MiB three buffers in turn are still there in part: 105 MB 31.9 / 31.2, on another offset 33.2 / 33.4, 16 members 37.2 / 38.8.
+    // (Dealing the tiles to the XCDs, as in the reductions, loses 2 % here.)
+    const bool quarter = mode == kModeAlltoall && sources > rt.cacheable_source_bytes / 16 * 7 && sources <= rt.cacheable_source_bytes;
     const bool stream_source = quarter || sources > rt.cacheable_source_bytes;
     const segment_args_t args = {rt.base, rt.heap_size, team_arg(tl), doff, soff, seg_bytes, 0, (uint32_t)n, 0, 0, quarter};
 #define NVSHMEM_AMD_LAUNCH_SEGCOPY(MODE, NTL, PACED, STORE) \

@@ -173,11 +173,11 @@ for name, es in (("float", 4), ("bfloat16", 2)):
 
 
 def test_alltoalls_that_nearly_fill_the_cache_are_streamed(recorded):  # noqa: F811
-    """From 112 MiB of sources on, but not a source of the cache's size (second template argument)."""
+    """From 112 MiB of sources on, without a gap where the cache ends (second template argument)."""
     recorded("""
 ok(lib.nvshmemx_amd_init(4, 256 << 20))
 a, b = lib.nvshmem_malloc(96 << 20), lib.nvshmem_malloc(96 << 20)
-for mib, streamed in ((28, 0), (29, 1), (63, 1), (64, 0), (65, 1)):
+for mib, streamed in ((28, 0), (29, 1), (63, 1), (64, 1), (65, 1)):
     launches()
     ok(lib.nvshmemx_alltoallmem_on_stream(0, b, a, mib << 18, None))
     (kernel, _, _, _, _), = launches()
