@@ -8,6 +8,7 @@
 #include "launch.hpp"
 #include "runtime.hpp"
 
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -284,7 +285,8 @@ int nvshmemx_amd_init(int npes, size_t symmetric_size) {
     rt.lds_reduce_bytes = env_size("NVSHMEM_AMD_LDS_REDUCE_BYTES", (size_t)64 << 20);
     rt.element_reduce_bytes = env_size("NVSHMEM_AMD_ELEMENT_REDUCE_BYTES", (size_t)512 << 10);
     rt.two_step_reduce_members = (unsigned)env_size("NVSHMEM_AMD_TWO_STEP_REDUCE_MEMBERS", 16);
-    rt.two_step_reduce_bytes = env_size("NVSHMEM_AMD_TWO_STEP_REDUCE_BYTES", (size_t)96 << 20);
+    rt.two_step_reduce_bytes = env_size("NVSHMEM_AMD_TWO_STEP_REDUCE_BYTES",
+                                        std::max((uint64_t)96 << 20, rt.cacheable_source_bytes / 8 * 3));
     if (!teams_init(rt)) {
         teams_finalize(rt);
         (void)hipFree(rt.base);

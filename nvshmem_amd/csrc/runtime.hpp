@@ -77,7 +77,8 @@ struct Runtime {
     uint64_t element_reduce_bytes = (uint64_t)512 << 10;
     // An allreduce of streamed sources takes two steps - fold into member 0, broadcast - instead of the fused
     // kernel from this team size on (NVSHMEM_AMD_TWO_STEP_REDUCE_MEMBERS, read at init; 0 = never) when the
-    // sources of all members together hold at least two_step_reduce_bytes (NVSHMEM_AMD_TWO_STEP_REDUCE_BYTES)
+    // sources of all members together hold at least two_step_reduce_bytes (NVSHMEM_AMD_TWO_STEP_REDUCE_BYTES, by
+    // default where reductions start to stream, but never below the 96 MiB that the form was measured from)
     unsigned two_step_reduce_members = 16;
     uint64_t two_step_reduce_bytes = (uint64_t)96 << 20;
     uint64_t timeouts_seen = 0;  // bounded waits that gave up, as far as the host has reported them

@@ -198,3 +198,21 @@ for npes, mib, two in ((15, 8, 0), (16, 5, 0), (16, 6, 1), (16, 32, 1), (32, 3, 
     assert not two or ("reduce_root_kernel" in names[0] and "segment_copy_kernelILi2" in names[1]), names
     lib.nvshmem_finalize()
 """)
+
+
+def test_sources_that_a_program_keeps_in_the_cache_stay_with_the_fused_reduction(recorded):  # noqa: F811
+    """With a larger NVSHMEM_AMD_CACHEABLE_SOURCE_BYTES large teams take two steps from 3/8 of that on, as their sources are
+    streamed from there; with a smaller one still from 96 MiB.  A threshold of its own wins."""
+    code = """
+ok(lib.nvshmemx_amd_init(16, 80 << 20))
+a, b = lib.nvshmem_malloc(32 << 20), lib.nvshmem_malloc(32 << 20)
+for mib, two in %s:
+    launches()
+    ok(_lib.typed_coll(lib, "nvshmemx_float_sum_reduce_on_stream", True)(0, b, a, mib << 18, None))
+    names = [l[0] for l in launches()]
+    assert len(names) == 1 + two and ("reduce_root_kernel" in names[0]) == bool(two), (mib, names)
+"""
+    cacheable = {"NVSHMEM_AMD_CACHEABLE_SOURCE_BYTES": str(1 << 30)}
+    recorded(code % "((6, 0), (16, 0), (23, 0), (24, 1))", **cacheable)
+    recorded(code % "((1, 0), (5, 0), (6, 1))", NVSHMEM_AMD_CACHEABLE_SOURCE_BYTES="0")
+    recorded(code % "((7, 0), (8, 1), (16, 1))", NVSHMEM_AMD_TWO_STEP_REDUCE_BYTES=str(128 << 20), **cacheable)
