@@ -139,3 +139,31 @@ def test_ragged_allreduce_with_streamed_loads(npes, form, monkeypatch):
                 rt.reduce(name, op, src + s * es, src + s * es, n)   # in place
                 assert bits_equal(rt.download(src, npes - 1, (n,), storage, s * es), want), (name, n, s)
         rt.free(src); rt.free(dst)
+
+
+@pytest.mark.parametrize("cacheable", ["none", "all"])
+@pytest.mark.parametrize("npes,form", [(2, "gather"), (3, "gather"), (4, "lds"), (8, "lds"), (12, "lds"), (16, "lds")])
+def test_ragged_allreduce_whose_tiles_share_lines(npes, form, cacheable, monkeypatch):
+    """Streamed sources on another offset in a line than the destination, in the sizes where the lanes at a tile's ends load
+    cacheable (the cache could hold them: 2/3 of it) and beyond: fewer tiles than are dealt to the XCDs, and a round of 32 of
+    them with some left over."""
+    for k, v in FORMS[form].items():
+        monkeypatch.setenv(k, v)
+    for nbytes in (1024 + 8, 41 * 1024 + 8):   # of every PE, whatever the element type
+        monkeypatch.setenv("NVSHMEM_AMD_CACHEABLE_SOURCE_BYTES", "0" if cacheable == "none" else str(npes * nbytes * 3 // 2))
+        rng = np.random.default_rng(npes * nbytes)
+        with runtime(npes, 2 << 20) as rt:
+            src = rt.malloc(1 << 16); dst = rt.malloc(1 << 16)
+            for name, op, kind, storage, _ in KINDS:
+                es = np.dtype(storage).itemsize
+                vec, n = 16 // es, nbytes // es
+                data = _values(kind, rng, (npes, n))
+                want = O.reduce(kind, op, data)
+                for d, s in ((0, 0), (0, vec), (5 * vec, vec), (0, vec - 1), (vec - 1, 2)):
+                    rt.upload_all(src, data, s * es)
+                    rt.fill(dst, 0xCD, (n + 5 * vec) * es + 64)
+                    note("%s %s %s shared lines npes=%d n=%d dst+%d src+%d %s" % (form, name, op, npes, n, d, s, cacheable))
+                    rt.reduce(name, op, dst + d * es, src + s * es, n)
+                    got, clean = _guarded(rt.download_all(dst, ((n + 5 * vec) * es + 64,), np.uint8), storage, d, n)
+                    assert clean and all(bits_equal(row, want) for row in got), (name, n, d, s)
+            rt.free(src); rt.free(dst)

@@ -216,3 +216,18 @@ for mib, two in %s:
     recorded(code % "((6, 0), (16, 0), (23, 0), (24, 1))", **cacheable)
     recorded(code % "((1, 0), (5, 0), (6, 1))", NVSHMEM_AMD_CACHEABLE_SOURCE_BYTES="0")
     recorded(code % "((7, 0), (8, 1), (16, 1))", NVSHMEM_AMD_TWO_STEP_REDUCE_BYTES=str(128 << 20), **cacheable)
+
+
+def test_streamed_sources_on_another_offset_share_their_lines(recorded):  # noqa: F811
+    """Two members: the gather kernel whose lanes at a tile's ends load cacheable (fifth template argument), as long as the
+    cache could hold the sources.  A whole number of lines apart there are none to share."""
+    recorded("""
+ok(lib.nvshmemx_amd_init(2, 512 << 20))
+a, b = lib.nvshmem_malloc(160 << 20), lib.nvshmem_malloc(160 << 20)
+for mib, offset, kernel in ((48, 4, "Li0ELb0ELb0E"), (49, 0, "Li0ELb1ELb0E"), (49, 128, "Li0ELb1ELb0E"), (49, 4, "Li0ELb1ELb1E"),
+                            (49, 16, "Li0ELb1ELb1E"), (128, 4, "Li0ELb1ELb1E"), (129, 4, "Li0ELb1ELb0E")):
+    launches()
+    ok(_lib.typed_coll(lib, "nvshmemx_float_sum_reduce_on_stream", True)(0, b, a + offset, mib << 18, None))
+    (name, _, _, _, _), = launches()
+    assert "reduce_gather_kernel" in name and kernel in name, (mib, offset, name)
+""")
