@@ -634,10 +634,11 @@ template <typename T, int OP, int NPES, bool NTL>
 __global__ __launch_bounds__(64) void reducescatter_gather_kernel(scatter_args_t a) {
     fold_source_pieces<T, OP, NPES, NTL, true>(a);
 }
-// The first half of the two-step allreduce of large teams: one block, into member 0's destination.
-template <typename T, int OP, bool NTL>
+// The first half of the two-step allreduce of large teams: one block, into member 0's destination.  Always streamed: by
+// default the form starts where streaming does (at exactly that size a byte earlier).
+template <typename T, int OP>
 __global__ __launch_bounds__(64) void reduce_root_kernel(scatter_args_t a) {
-    fold_source_pieces<T, OP, 0, NTL, false>(a);
+    fold_source_pieces<T, OP, 0, true, false>(a);
 }
 
 // Tiles of a segment, wherever it starts.
@@ -771,9 +772,9 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
     int mpw = 0, ct_size = 0;
     constexpr int kNarrowMpw = sizeof(T) <= 2 ? NVSHMEM_AMD_REDUCE_NARROW_MPW : NVSHMEM_AMD_REDUCE_WIDE_MPW;
     if (fixed_size == 8) ct_size = 8, mpw = stream_source ? NVSHMEM_AMD_REDUCE_WIDE_MPW : kNarrowMpw;
-    else if (fixed_size == 16) ct_size = 16, mpw = kNarrowMpw;
     else if (fixed_size == 4) ct_size = 4, mpw = 1;
-    else if (fixed_size == 32) ct_size = 32, mpw = 2;
+    else if (fixed_size == 16 && !stream_source) ct_size = 16, mpw = kNarrowMpw;
+    else if (fixed_size == 32 && !stream_source) ct_size = 32, mpw = 2;
     else if (tl.max_size >= 3 && tl.max_size <= 32) mpw = 2;
     else if (tl.max_size > 32 && tl.max_size <= 64) mpw = 4;
     // Two-step allreduce of large teams: fold into member 0's destination (n loads and ONE store per vector, the
@@ -791,10 +792,7 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
     if (rt.two_step_reduce_members && tl.min_size >= (int)rt.two_step_reduce_members && total_bytes >= rt.two_step_reduce_bytes) {
         const scatter_args_t args = {rt.base, rt.heap_size, team_arg(tl), dst_off, src_off, nelems, 0};
         const dim3 grid((unsigned)((nelems / (16 / sizeof(T)) + 63 + 63) / 64), 1, ngroups);
-        if (stream_source)
-            launch_kernel((reduce_root_kernel<T, OP, true>), grid, dim3(64), 0, stream, args);
-        else
-            launch_kernel((reduce_root_kernel<T, OP, false>), grid, dim3(64), 0, stream, args);
+        launch_kernel((reduce_root_kernel<T, OP>), grid, dim3(64), 0, stream, args);
         (void)launch_broadcast(rt, tl, dst_off, dst_off, nelems * sizeof(T), 0, stream);
         return;
     }
@@ -812,24 +810,23 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
         shape.astride = (dst_off - src_off) % 128 && total_bytes <= rt.cacheable_source_bytes;
         const size_t lds = ((size_t)tl.max_size + 1) * 16 * tile_vecs;
         const dim3 grid((unsigned)blocks, 1, ngroups);
-#define NVSHMEM_AMD_LAUNCH_REDUCE(N, MPW) NVSHMEM_AMD_LAUNCH_REDUCE_V(N, MPW, MPW, NVSHMEM_AMD_REDUCE_VPT)
-#define NVSHMEM_AMD_LAUNCH_REDUCE_V(N, STREAM_MPW, MPW, VPT)                                      \
-    do {                                                                                          \
-        if (stream_source)                                                                        \
-            launch_kernel((reduce_vector_kernel<T, OP, N, true, VPT, STREAM_MPW>), grid, dim3(threads), lds,  \
-                               stream, rt.base, rt.heap_size, tl.groups, shape);                                                  \
-        else                                                                                      \
-            launch_kernel((reduce_vector_kernel<T, OP, N, false, VPT, MPW>), grid, dim3(threads), lds, \
-                               stream, rt.base, rt.heap_size, tl.groups, shape);                                                  \
+#define NVSHMEM_AMD_LAUNCH_REDUCE(N, NTL, MPW, VPT)                                                      \
+    launch_kernel((reduce_vector_kernel<T, OP, N, NTL, VPT, MPW>), grid, dim3(threads), lds, stream, rt.base, \
+                  rt.heap_size, tl.groups, shape)
+#define NVSHMEM_AMD_LAUNCH_REDUCE_EITHER(N, MPW)                                          \
+    do {                                                                                  \
+        if (stream_source) NVSHMEM_AMD_LAUNCH_REDUCE(N, true, MPW, NVSHMEM_AMD_REDUCE_VPT); \
+        else NVSHMEM_AMD_LAUNCH_REDUCE(N, false, MPW, NVSHMEM_AMD_REDUCE_VPT);              \
     } while (0)
-        if (ct_size == 8) NVSHMEM_AMD_LAUNCH_REDUCE_V(8, NVSHMEM_AMD_REDUCE_WIDE_MPW, kNarrowMpw, kVptNarrow);
-        else if (ct_size == 16) NVSHMEM_AMD_LAUNCH_REDUCE_V(16, kNarrowMpw, kNarrowMpw, kVptNarrow);
-        else if (ct_size == 4) NVSHMEM_AMD_LAUNCH_REDUCE(4, 1);
-        else if (ct_size == 32) NVSHMEM_AMD_LAUNCH_REDUCE(32, 2);
-        else if (mpw == 2) NVSHMEM_AMD_LAUNCH_REDUCE(0, 2);
-        else NVSHMEM_AMD_LAUNCH_REDUCE(0, 4);
+        if (ct_size == 8 && stream_source) NVSHMEM_AMD_LAUNCH_REDUCE(8, true, NVSHMEM_AMD_REDUCE_WIDE_MPW, kVptNarrow);
+        else if (ct_size == 8) NVSHMEM_AMD_LAUNCH_REDUCE(8, false, kNarrowMpw, kVptNarrow);
+        else if (ct_size == 16) NVSHMEM_AMD_LAUNCH_REDUCE(16, false, kNarrowMpw, kVptNarrow);
+        else if (ct_size == 32) NVSHMEM_AMD_LAUNCH_REDUCE(32, false, 2, NVSHMEM_AMD_REDUCE_VPT);
+        else if (ct_size == 4) NVSHMEM_AMD_LAUNCH_REDUCE_EITHER(4, 1);
+        else if (mpw == 2) NVSHMEM_AMD_LAUNCH_REDUCE_EITHER(0, 2);
+        else NVSHMEM_AMD_LAUNCH_REDUCE_EITHER(0, 4);
+#undef NVSHMEM_AMD_LAUNCH_REDUCE_EITHER
 #undef NVSHMEM_AMD_LAUNCH_REDUCE
-#undef NVSHMEM_AMD_LAUNCH_REDUCE_V
     } else if (element_at_a_time<T, false>(rt, tl, fixed_size == 4 || fixed_size == 8, dst_off, src_off, nelems)) {
         launch_kernel((reduce_element_kernel<T, OP>), dim3((unsigned)((nelems + 255) / 256), 1, ngroups), dim3(256), 0,
                            stream, rt.base, rt.heap_size, tl.groups, dst_off, src_off, nelems);
@@ -838,22 +835,15 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
         const dim3 grid((unsigned)((nvec + 63 + 63) / 64), 1, ngroups);
         shape.dealt = dealt_blocks(dst_off, src_off, grid.x);
         const bool astride = stream_source && (dst_off - src_off) % 128 && total_bytes <= rt.cacheable_source_bytes;
-#define NVSHMEM_AMD_LAUNCH_GATHER_REDUCE(N)                                                            \
-    do {                                                                                               \
-        if (astride)                                                                                   \
-            launch_kernel((reduce_gather_kernel<T, OP, 0, true, true>), grid, dim3(64), 0, stream, rt.base, \
-                               rt.heap_size, tl.groups, shape);                                        \
-        else if (stream_source)                                                                        \
-            launch_kernel((reduce_gather_kernel<T, OP, N, true>), grid, dim3(64), 0, stream, rt.base, \
-                               rt.heap_size, tl.groups, shape);                    \
-        else                                                                                           \
-            launch_kernel((reduce_gather_kernel<T, OP, N, false>), grid, dim3(64), 0, stream, rt.base, \
-                               rt.heap_size, tl.groups, shape);                    \
-    } while (0)
-        // (sixteen members unrolled measured slower than the loop: 5.2 against 5.4 TB/s)
-        if (fixed_size == 4) NVSHMEM_AMD_LAUNCH_GATHER_REDUCE(4);
-        else if (fixed_size == 8) NVSHMEM_AMD_LAUNCH_GATHER_REDUCE(8);
-        else NVSHMEM_AMD_LAUNCH_GATHER_REDUCE(0);
+#define NVSHMEM_AMD_LAUNCH_GATHER_REDUCE(...)                                                                          \
+    launch_kernel((reduce_gather_kernel<T, OP, __VA_ARGS__>), grid, dim3(64), 0, stream, rt.base, rt.heap_size, tl.groups, shape)
+        // (streamed sources of 4 and 8 members come here only with a larger NVSHMEM_AMD_LDS_REDUCE_BYTES; sixteen members
+        // unrolled measured slower than the loop: 5.2 against 5.4 TB/s)
+        if (astride) NVSHMEM_AMD_LAUNCH_GATHER_REDUCE(0, true, true);
+        else if (stream_source) NVSHMEM_AMD_LAUNCH_GATHER_REDUCE(0, true);
+        else if (fixed_size == 4) NVSHMEM_AMD_LAUNCH_GATHER_REDUCE(4, false);
+        else if (fixed_size == 8) NVSHMEM_AMD_LAUNCH_GATHER_REDUCE(8, false);
+        else NVSHMEM_AMD_LAUNCH_GATHER_REDUCE(0, false);
 #undef NVSHMEM_AMD_LAUNCH_GATHER_REDUCE
     }
 }

@@ -231,3 +231,19 @@ for mib, offset, kernel in ((48, 4, "Li0ELb0ELb0E"), (49, 0, "Li0ELb1ELb0E"), (4
     (name, _, _, _, _), = launches()
     assert "reduce_gather_kernel" in name and kernel in name, (mib, offset, name)
 """)
+
+
+def test_streamed_sources_of_large_teams_share_the_kernels_of_any_team_size(recorded):  # noqa: F811
+    """A program that switches the two-step form off: the staged kernel that reads the team size, two members to a wavefront."""
+    recorded("""
+for npes, mib in ((16, 7), (32, 4)):
+    ok(lib.nvshmemx_amd_init(npes, 80 << 20))
+    a, b = lib.nvshmem_malloc(32 << 20), lib.nvshmem_malloc(32 << 20)
+    launches()
+    for per_pe in (mib, 5 if npes == 16 else 2):
+        ok(_lib.typed_coll(lib, "nvshmemx_float_sum_reduce_on_stream", True)(0, b, a, per_pe << 18, None))
+    (streamed, _, _, block, _), (cached, _, _, _, _) = launches()
+    assert "reduce_vector_kernelIfLi5ELi0ELb1ELi1ELi2E" in streamed and block[0] == 32 * npes, (streamed, block)
+    assert "reduce_vector_kernelIfLi5ELi%dELb0E" % npes in cached, cached
+    lib.nvshmem_finalize()
+""", NVSHMEM_AMD_TWO_STEP_REDUCE_MEMBERS="0")
