@@ -2017,12 +2017,14 @@ NVSHMEMI_DEVICE_INLINE const char *nvshmemi_amd_uniform(const void *p) {
 }
 /* The same FULL rounds for a team of a whole number of M members, with the loads of the next round in front of the stores of
  * the last: behind them, a wait for the loads is one for the stores' acknowledgements as well, which is what a block of few
- * wavefronts spends its time on.  No more registers than the rounds above (fp32 55, bf16 sum 59, max 71); with the loads in
- * front of the fold too they would be 105.  us, kernel and barriers, three sets of buffers in turn, rounds above / here: 256
+ * wavefronts spends its time on.  Registers 53 to 55 for 4- and 8-byte elements, 51 in the rounds above, and as many as there
+ * for narrower ones (bf16 sum 59, max 71), so the wavefronts per SIMD are the same; with the loads in front of the fold too they
+ * would be 105.  us, kernel and barriers, three sets of buffers in turn, rounds above / here: 256
  * threads, 8 members fp32 max 341 766 elements 49.9 / 38.0, bf16 sum 700 000 52 / 44.6, 16 members bf16 59 / 46, 4 members bf16 sum 786 111
  * 57 / 47, max 60 / 54, fp32 500 000 56.7 / 50.8; 1024 threads, 16 members bf16 700 000 39.5 / 37.1, 8 114 688 9.4 / 9.2.  What is bound
  * by the place of its data stays: 16 members fp32 903 614 170 / 168.  Wavefronts that go through their rounds together
- * (PHASED) do as well as this from 512 threads on (8 members fp32 827 072: 69.7, 79.6 so). */
+ * (PHASED) do as well as this from 512 threads on (8 members fp32 827 072: 69.7, 79.6 so).  Other team sizes stay with the rounds
+ * above, which fetch the last member again to fill a round: such rounds ahead of the stores were not built. */
 template <typename T, int OP, int M, int V>
 NVSHMEMI_DEVICE_INLINE size_t nvshmemi_amd_reduce_rounds_ahead(T *dst, const T *src, size_t pe_stride, int npes, size_t nvec,
                                                                size_t tid, size_t nthr, size_t base) {

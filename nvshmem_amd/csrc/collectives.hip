@@ -35,7 +35,7 @@ namespace {
 #ifndef NVSHMEM_AMD_REDUCE_VPT_NARROW /* the same for 1- and 2-byte elements on the compile-time team sizes 8 and 16 */
 #define NVSHMEM_AMD_REDUCE_VPT_NARROW 1
 #endif
-/* Members per wavefront of the fused reduce on the compile-time team sizes 8 and 16, for 1- and 2-byte
+/* Members per wavefront of the fused reduce on teams of 8 and on cached sources of 16, for 1- and 2-byte
  * elements (NARROW) and for wider ones (WIDE).  Narrow elements fold twice to four times as many elements
  * per byte, and a block has nothing in flight while it folds: with two members per wavefront the blocks
  * are half as large and twice as many share a compute unit, so more of them are in their load or store
@@ -60,12 +60,25 @@ namespace {
  *
  * Reductions stream from 3/8 of that on (96 MiB, streamed_reduction).  A streamed load is served from the Infinity
  * Cache where the line is there - a source that was just produced - but brings none into it, so it does not push out
- * what others have written there and not yet to memory.  us cached / streamed loads, fp32, sources in all of 100 | 128 | 200
- * MB: a source just written, allreduce on 8 members 25.7 / 21.1 | 32.8 / 26.6 | 59.3 / 42.9, reducescatter 15.4 / 9.1 | 18.7 /
- * 12.9 | 27.3 / 22.9; three buffers in turn 34.8 / 33.7 | 45.3 / 42.3 | 67.5 / 64.1 and 22.0 / 19.0 | 27.5 / 23.8 | 41.7 / 35.7;
- * below, sources that are in use in turn are still there: of 64 MB 19.2 / 23.7 and 11.7 / 12.6.  What loses is a source that is
- * reduced again as it is, with nothing in between: 29.1 / 33.2 | 36.6 / 41.6 | 56.0 / 63.6 and 17.4 / 16.3 | 21.5 / 21.9 | 33.2 /
- * 33.3. */
+ * what others have written there and not yet to memory.  us cached / streamed loads, fp32 normal data, sources in all of 110 | 160 |
+ * 200 MB | 256 MiB (16 members cached on the fused kernel, streamed in two steps):
+ *  - three sets of buffers in turn, each source filled in front of its call, both kernels: allreduce on 4 members 57.9 / 55.2 | 86.4 /
+ *    75.1 | 105.6 / 90.6 | 118.8 / 117.7, 8 members 73.2 / 70.1 | 104.8 / 87.0 | 122.9 / 102.4 | 133.2 / 132.2, 16 members 88.5 / 80.8 |
+ *    119.3 / 103.2 | 143.4 / 123.6 | 146.4 / 152.2; reducescatter on 8 members 54.1 / 52.1 | 68.6 / 67.9 | 80.4 / 79.5 | 104.6 / 100.7.
+ *  - in turn without the fills: allreduce on 4 members 39.1 / 37.8 | 54.0 / 52.9 | 67.7 / 65.7 | 89.1 / 85.9, 8 members 43.7 / 42.7 |
+ *    58.4 / 54.5 | 72.2 / 67.4 | 97.4 / 88.0; reducescatter on 8 members, 128 MiB | 200 MB | 256 MiB, 30.2 / 27.3 | 43.7 / 37.6 | 56.3 / 49.5.
+ *  - below 96 MiB sources that are in use in turn are still there: of 64 MB allreduce 19.2 / 23.7, reducescatter 11.7 / 12.6.
+ * What loses:
+ *  - A source that is reduced again as it is, with nothing in between (a sum and then a maximum of one buffer): 128 MiB | 200 MB | 256
+ *    MiB on 4 members 37.9 / 43.6 | 55.2 / 65.6 | 73.5 / 85.5, 8 members 43.0 / 47.3 | 60.6 / 68.7 | 79.0 / 89.0, 16 members 39.9 / 45.3 |
+ *    57.9 / 63.4 | 76.5 / 83.3, 32 members 39.6 / 48.7 | 57.7 / 68.5 | 76.6 / 88.8; reducescatter on 8 members 25.8 / 25.7 | 35.8 / 37.4 |
+ *    48.9 / 50.1.  Buffers of zeros, which the cache serves faster, lose up to 40 % (8 members 36.4 / 43.4 and 67.2 / 84.6, 32 34.5 / 48.2).
+ *  - ONE source that is filled again in front of each call on 8 and 16 members (both kernels less the fill alone): 8 members 51.1 /
+ *    55.8 | 60.2 / 66.4 | 68.8 / 73.9 | 87.8 / 86.2, 16 members 39.5 / 41.5 | 50.1 / 57.8 | 64.5 / 69.5 | 81.6 / 87.2; 4 members gain, 41.7 /
+ *    39.7 | 58.1 / 51.5 | 66.9 / 61.7 | 86.7 / 81.0.
+ *  - Sources on another offset in a line near the cache's size: stream_load_astride.
+ * A larger cacheable_source_bytes is for programs of these kinds.  (A quarter kept, as an alltoall's: in turn without fills 86.1
+ * instead of 88.0, 8 members of 256 MiB; with them 162 instead of 132.) */
 
 // (any byte alignment: one global_load_dwordx4 either way)
 template <bool NTL>
@@ -76,7 +89,13 @@ __device__ __forceinline__ nvshmemi_v4u stream_load(const char *p) {
 }
 // A streamed load of a wavefront whose KiB does not start on a line of its own: the lines at its ends, which the wavefronts
 // on either side read too, possibly on another XCD, are brought into the caches (`shared`: the lanes on them), as
-// streamed ones come from memory twice.  (The empty statements keep the compiler from making one plain load of the two.)
+// streamed ones come from memory twice.  us cached / streamed / so, allreduce, source on another offset, 110 | 160 | 200 MB | 256 MiB of
+// sources in all, fp32 normal data: three sets in turn, each filled in front of its call (both kernels), 2 members 51.9 / 58.5 / 52.6 |
+// 78.0 / 82.3 / 73.8 | 93.6 / 101.3 / 92.4 | 115.6 / 134.4 / 127.8, 4 members 60.7 / 68.5 / 60.2 | 91.1 / 93.5 / 80.5 | 108.5 / 110.3 /
+// 101.2 | 125.4 / 145.2 / 149.9, 8 members 71.4 / 77.4 / 67.8 | 106.1 / 101.1 / 92.7 | 124.4 / 122.5 / 122.7 | 139.2 / 161.0 / 167.6: at
+// the cache's own size it is the whole of streaming that loses.  In turn without fills 8 members 42.9 / 42.5 / 41.5 | 61.7 / 58.4 /
+// 58.6 | 80.5 / 76.5 / 75.2 | 110.0 / 99.7 / 98.3; reduced again as it is 36.1 / 45.6 / 43.8 | 51.0 / 60.5 / 58.5 | 65.2 / 78.4 / 74.9 |
+// 88.0 / 106.1 / 106.1.  (The empty statements keep the compiler from making one plain load of the two.)
 __device__ __forceinline__ nvshmemi_v4u stream_load_astride(const char *p, bool shared) {
     nvshmemi_v4u v;
     if (shared) {
@@ -94,7 +113,9 @@ __device__ __forceinline__ nvshmemi_v4u stream_load_astride(const char *p, bool 
 // dealt by 2 | 4 | 8 | 16, allreduce, sources on another offset: 8 members fp32 60 MB of sources in all 19.2 / 19.6 | 18.4 | 18.9 |
 // 18.2, 110 MB streamed 39.7 / 38.5 | 37.9 | 38.9 | 40.1, 420 MB 141.7 / 142.8 | 136.6 | 140.3 | 146.9; 2 members 110 MB 37.7 / 36.7 |
 // 36.1 | 36.4 | 36.2, 420 MB 134.7 / 131.7 | 129.0 | 131.6 | 131.8.  Where no line is shared it only widens what is read at a time
-// (8 members, 420 MB aligned: 132.4 in order, by 8 138.4).
+// (8 members, 420 MB aligned: 132.4 in order, by 8 138.4).  Small ones, in order / dealt by 4, three sets in turn in a graph: 2 to
+// 16 members the same below 1 MiB per PE; 1 MiB 4 members fp32 2.80 / 2.33, 8 bf16 4.73 / 4.05, 16 bf16 8.88 / 8.34, 2 bf16 2.55 /
+// 2.57; 4 MiB 8 members fp32 13.3 / 11.9, 16 members 22.3 / 22.6, bf16 21.8 / 23.0, the most that loses (sent again as it is 21.8 / 21.5).
 constexpr unsigned kDealtTiles = 4;
 __device__ __forceinline__ unsigned dealt_tile(unsigned block, unsigned dealt) {
     constexpr unsigned kGroup = 8 * kDealtTiles;
@@ -422,10 +443,8 @@ __global__ __launch_bounds__(NPES ? NPES / MPW * 64 : 1024) void reduce_vector_k
             }
         }
     };
-    // (us streamed alone / here, tiles dealt, source on another offset, 110 MB | 200 MB of sources in all: 8 members fp32 in use in
-    // turn 37.8 / 37.5 | 65.5 / 65.7, just written 32.9 / 21.4 | 61.2 / 48.1, 4 members 36.9 / 35.8 | 64.8 / 62.2 and 29.7 / 25.3 |
-    // 57.5 / 49.5.  Sources beyond the Infinity Cache lose more by what this pushes out of it than they gain: 8 members, 300 MB just
-    // written 104 / 113, 420 MB 128 / 142, in turn 136.4 / 134.3.)
+    // (stream_load_astride has the figures.  Sources beyond the Infinity Cache lose more by what this pushes out of it than they
+    // gain: 8 members, 300 MB just written 104 / 113 us, 420 MB 128 / 142, in turn 136.4 / 134.3.)
     if (NTL && s.astride) fetch([i](const char *p) { return stream_load_astride(p, i - 8 >= 48); });
     else fetch([](const char *p) { return stream_load<NTL>(p); });
     __syncthreads();
@@ -755,12 +774,20 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
     // 512 MiB / 2 GiB of sources: 4 members 6.54 / 6.55 against 6.19 / 6.24, 6 members 6.37 / 6.44
     // against 5.89 / 5.58, 8 members 6.46 / 6.53 against 6.03 / 6.09, 12 members 6.28 / 6.28 against
     // 5.73 / 5.83, 16 members 6.21 / 6.12 against 5.44 / 5.57, 32 members 6.17 / 6.10 against 5.22 / 5.49,
-    // 64 members 5.64 / 5.64 against 5.15 / 5.26.  A wavefront of the LDS kernel serves one member
-    // for the compile-time sizes 8 and 16, two members up to 32 and four beyond: one load and one store
-    // per lane measured best where the block stays within 16 wavefronts, and wavefronts of fewer than
-    // 64 lanes per member (512- or 256-byte accesses) lost 7-22 % against the gather kernel.  The
-    // compile-time team size is worth 6 % at 32 members (6.17 against 5.82), nothing at 64, and with a member per wavefront 3 to
-    // 8 % at 4 (70 | 200 | 800 MB of sources in all, fp32 22.4 / 20.9 | 63.6 / 61.8 | 248 / 240 us, bf16 alike).
+    // 64 members 5.64 / 5.64 against 5.15 / 5.26.  A wavefront of the LDS kernel serves
+    //   4 members   one                                        (team size known at compile time)
+    //   8 members   one; cached sources of 1- and 2-byte elements two   (known)
+    //   16 members  cached: one, 1- and 2-byte elements two    (known); streamed: two
+    //   32 members  two                                        (cached: known)
+    //   others      two up to 32 members, four beyond (there: handles whose smallest team has fewer than
+    //               two_step_reduce_members, and programs without the two-step form)
+    // One load and one store per lane measured best where the block stays within 16 wavefronts (narrow elements:
+    // NVSHMEM_AMD_REDUCE_NARROW_MPW), and wavefronts of fewer than 64 lanes per member (512- or 256-byte accesses) lost
+    // 7-22 % against the gather kernel.  The compile-time size is worth 6 % at 32 members (6.17 against 5.82), nothing at 64,
+    // and with a member per wavefront 3 to 8 % at 4 (70 | 200 | 800 MB of sources in all, fp32 22.4 / 20.9 | 63.6 / 61.8 | 248 / 240
+    // us, bf16 alike).  Streamed sources of 16 and 32 members take two steps (below); for programs that switch those off the size read
+    // from the team does, us known / read, 110 | 200 | 600 MB in turn: 16 members fp32 38.5 / 39.0 | 67.4 / 68.0 | 193.6 / 198.0, bf16 39.7 /
+    // 39.1 | 69.0 / 68.3 | 201.2 / 198.4, 32 members fp32 40.3 / 41.4 | 69.5 / 71.8 | 207.1 / 212.7.
     const uint64_t total_bytes = total_members(tl) * all * sizeof(T);
     const int fixed_size = tl.min_size == tl.max_size ? tl.max_size : 0;
     const bool stream_source = rt.streamed_reduction(total_bytes);
@@ -788,7 +815,7 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
     // 68.3 / 56.7 | 96.5 / 79.8, 24 fp32 40.4 / 40.6 | 59.6 / 53.7 | 88.6 / 80.6, 32 48.9 / 40.0 | 69.6 / 61.4 | 99.7 / 79.9, against the gather
     // kernel 40 39.5 / 38.4 | 63.0 / 58.8 | 93.1 / 81.4, 64 42.4 / 41.9 | 64.7 / 59.2 | 98.3 / 88.9; sources that are still in the cache lose
     // (16 members, 80 MB: 26.8 / 31.5).  So: from Runtime::two_step_reduce_members (16) members on when the sources hold
-    // two_step_reduce_bytes (96 MiB, from where reductions stream) or more.
+    // two_step_reduce_bytes or more (96 MiB, from where reductions stream; with a larger cacheable_source_bytes 3/8 of that).
     if (rt.two_step_reduce_members && tl.min_size >= (int)rt.two_step_reduce_members && total_bytes >= rt.two_step_reduce_bytes) {
         const scatter_args_t args = {rt.base, rt.heap_size, team_arg(tl), dst_off, src_off, nelems, 0};
         const dim3 grid((unsigned)((nelems / (16 / sizeof(T)) + 63 + 63) / 64), 1, ngroups);
@@ -799,9 +826,9 @@ void launch_reduce(Runtime &rt, const TeamLaunch &tl, uint64_t dst_off, uint64_t
     if (mpw && total_bytes >= lds_from_bytes) {
         const uint32_t lane_shift = 6;
         const unsigned threads = (unsigned)((tl.max_size + mpw - 1) / mpw) << lane_shift;
-        // A tile of two vectors per thread halves the barriers per byte: worth 5 % for 16-bit elements with one
-        // member per wavefront (bf16 sum at 8 x 128 MiB 5.83 -> 6.14 TB/s), less than the two members per
-        // wavefront they now use with one vector; it costs 4-byte and 8-byte elements 3-4 %.
+        // A tile of two vectors per thread halves the barriers per byte and loses all the same: 4-byte and 8-byte elements 3-4 %;
+        // bf16 on 8 members, streamed with a member per wavefront, one / two vectors, us at 110 | 200 | 400 | 1600 MB of sources in all
+        // in turn 42.5 / 44.6 | 68.5 / 72.6 | 131.8 / 143.8 | 517 / 581.
         constexpr int kVptNarrow = sizeof(T) <= 2 ? NVSHMEM_AMD_REDUCE_VPT_NARROW : NVSHMEM_AMD_REDUCE_VPT;
         const int vpt = (ct_size == 8 || ct_size == 16) ? kVptNarrow : NVSHMEM_AMD_REDUCE_VPT;
         const uint64_t tile_vecs = (uint64_t)vpt << lane_shift;

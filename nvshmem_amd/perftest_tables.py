@@ -143,8 +143,10 @@ def collectives(iters):
             lines.append("%-34s" % label + "".join("%8.0f" % rows.get(s, float("nan")) for s in sizes))
     head = ["Host-launched collectives by size on one MI355X: what the library's kernel choice gives, and what each of",
             "the two forms it chooses between gives when forced through the environment.  Algorithmic bytes as in",
-            "bench.py; host wall time over back-to-back calls (a call costs at least a launch, ~3 us; sources up to",
-            "256 MiB in all stay in the Infinity Cache between calls).", "",
+            "bench.py; host wall time over back-to-back calls on the same buffers (a call costs at least a launch, ~3 us).",
+            "They hold what the heap is allocated with, which the caches serve faster than data, and what is not streamed",
+            "stays in the Infinity Cache between calls: sources of up to 96 MiB in all in a reduction, 112 in an alltoall",
+            "(a quarter of it up to 256), 256 in the others.", "",
             "Commands (repository root, after python3 -m nvshmem_amd.build):",
             "  python3 nvshmem_amd/perftest_tables.py --what collectives --out profiles/collective_size_sweep.txt", "which runs"]
     return head + ["  " + c for c in commands] + lines
